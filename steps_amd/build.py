@@ -31,7 +31,7 @@ SHIM_VARIANTS = {"r3": [], "t3": ["-DPERIODIC"], "s1r2": ["-DPERIODIC_Z", "-DEWA
                  "s1r2_bh_rand": ["-DPERIODIC_Z", "-DEWALD_INTERPOLATION_ORDER=2", "-DUSE_BH=0.5", "-DRANDOMIZE_BH=7"]}
 
 HIP_SOURCES = ["pair_kernels.hip", "engine.hip", "kdk_kernels.hip", "table_kernels.hip", "order_kernels.hip",
-               "server.hip", "noalloc.hip", "bh_kernels.hip"]
+               "server.hip", "noalloc.hip", "bh_kernels.hip", "sym_kernels.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -42,6 +42,13 @@ int cu_count(int device) {
     return n;
 }
 
+int reserve_scratch(DevBuf &b, EvalPlan &p) {
+    if (b.reserve(scratch_bytes(p), "alloc partials") == STEPS_OK) return STEPS_OK;
+    // the slots of fewer cells at a time take less (and give the same sums)
+    if (p.sym) p.sym_launch_cells = 1;
+    return b.reserve(scratch_bytes(p), "alloc partials");
+}
+
 int DevBuf::reserve(size_t bytes, const char *what) {
     if (bytes <= cap && ptr) return STEPS_OK;
     if (ptr) (void)hipFree(ptr);
@@ -297,6 +304,7 @@ int make_plan(const steps_force_desc &d, int64_t N, int64_t id_min, int64_t id_m
         p.jchunk = ((N + 7) / 8 + kTile - 1) / kTile * kTile;
         p.splits = 8;
     }
+    sym_plan(p);
     return STEPS_OK;
 }
 
@@ -324,13 +332,15 @@ int check_finite(const double *x, int64_t n) {
 // resident simulation
 // ---------------------------------------------------------------------------
 
-int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, steps_sim **out) {
+int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool lean, steps_sim **out) {
     *out = nullptr;
     if (N <= 0) return fail(STEPS_ERR_ARG, "N must be positive");
     EvalPlan p;
     int rc = make_plan(d, N, 0, N - 1, p);
     if (rc) return rc;
     size_t scratch = scratch_bytes(p);
+    p.sym_launch_cells = std::min(p.sym_launch_cells, 1);
+    size_t least = scratch_bytes(p);
     if (both_precisions && desc_mixed_capable(d)) {
         // the scratch serves either precision (neither plan's need bounds the other's)
         steps_force_desc dd = d;
@@ -338,6 +348,8 @@ int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, steps
         EvalPlan q;
         if ((rc = make_plan(dd, N, 0, N - 1, q))) return rc;
         scratch = std::max(scratch, scratch_bytes(q));
+        q.sym_launch_cells = std::min(q.sym_launch_cells, 1);
+        least = std::max(least, scratch_bytes(q));
     }
     if ((rc = set_device(d.device))) return rc;
     steps_sim *s = new (std::nothrow) steps_sim();
@@ -353,7 +365,8 @@ int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, steps
     };
     if ((rc = s->jrec.reserve((size_t)N * sizeof(double4), "alloc jrec")) ||
         (rc = s->jsoft.reserve(nb, "alloc soft")) || (rc = s->v.reserve(3 * nb, "alloc v")) ||
-        (rc = s->F.reserve(3 * nb, "alloc F")) || (rc = s->part.reserve(scratch, "alloc partials")) ||
+        (rc = s->F.reserve(3 * nb, "alloc F")) ||
+        (rc = s->part.reserve(lean ? least : scratch, "alloc partials") && (rc = s->part.reserve(least, "alloc partials"))) ||
         (rc = s->stage.reserve(std::max(3 * nb, (size_t)1024), "alloc stage")) ||
         (rc = s->blockmax.reserve((size_t)(kdk_reduce_blocks(N) + 1) * sizeof(double), "alloc blockmax")) ||
         (rc = s->dparams.reserve(sizeof(KdkParams), "alloc step params")))
@@ -422,7 +435,7 @@ int sim_plan(steps_sim *s, int64_t id_min, int64_t id_max, int precision, EvalPl
     d.precision = precision;
     int rc = make_plan(d, s->N, id_min, id_max, p);
     if (rc) return rc;
-    if (scratch_bytes(p) > s->part.cap) return fail(STEPS_ERR_STATE, "scratch too small for this precision");
+    if (!sym_fit(p, s->part.cap) || scratch_bytes(p) > s->part.cap) return fail(STEPS_ERR_STATE, "scratch too small for this precision");
     p.t3 = s->t3.ptr();
     p.t3_lo = s->t3.lo;
     p.s1r2 = s->s1r2.ptr();
@@ -579,7 +592,7 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
     const size_t nb = (size_t)N * sizeof(double);
     if ((rc = o.x.reserve(3 * nb, "alloc x")) || (rc = o.M.reserve(nb, "alloc M")) ||
         (rc = o.soft.reserve(nb, "alloc soft")) || (rc = o.jrec.reserve((size_t)N * sizeof(double4), "alloc jrec")) ||
-        (rc = o.jsoft.reserve(nb, "alloc jsoft")) || (rc = o.part.reserve(scratch_bytes(p), "alloc partials")) ||
+        (rc = o.jsoft.reserve(nb, "alloc jsoft")) || (rc = reserve_scratch(o.part, p)) ||
         (rc = o.F.reserve(3 * (size_t)p.nrows * sizeof(double), "alloc F")))
         return rc;
     hipStream_t st = o.stream;
@@ -614,7 +627,7 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
 
 int steps_sim_create(const steps_force_desc *d, int64_t N, steps_sim **out) {
     if (!d || !out) return fail(STEPS_ERR_ARG, "null argument");
-    return sim_create(*d, N, true, out);
+    return sim_create(*d, N, true, false, out);
 }
 
 int steps_sim_destroy(steps_sim *s) {

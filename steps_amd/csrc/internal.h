@@ -92,16 +92,44 @@ struct EvalPlan {
     // the radial octree correction table (device), applied with the
     // comoving external term of R3 and S1R2
     const double *bh_radial = nullptr; int bh_radial_size = 0;
+    // every unordered pair once (sym_kernels.hip): blocks of block_rows rows,
+    // tasks of task_tiles source tiles, cells of whole tasks and offsets,
+    // launch_cells cells a launch
+    bool sym = false;
+    int sym_blocks = 0, sym_block_rows = 0, sym_task_tiles = 0;
+    int sym_cells = 0, sym_launch_cells = 0;
 };
 
 // The T3 Ewald evaluation deals its sources out to the eight XCDs by table
 // slab (pair_kernels.hip, body_t3_slab): make_plan then sets eight splits.
 bool t3_slab_plan(const EvalPlan &p);
 
+// The pair-symmetric evaluation (sym_kernels.hip).  sym_plan fills the plan's
+// sym fields where it applies; sym_fit lowers the cells per launch until the
+// evaluation's scratch is at most `bytes` (false when even one cell does not
+// fit); neither changes results beyond the choice sym / not sym.
+struct SymBuffers {
+    const double4 *rec;    // sources: sorted or scaled copies, or the input records
+    const double *soft;
+    const double4 *tiles, *ext;
+    const double *table;
+    const uint32_t *keys;
+    const uint32_t *perm;  // sorted -> input row, or null
+    const double4 *jrec;   // input records (external term)
+    double *part;
+};
+void sym_plan(EvalPlan &p);
+bool sym_fit(EvalPlan &p, size_t bytes);
+size_t sym_bytes(const EvalPlan &p);  // of the partial sums; 0 without sym
+bool sym_selected(const EvalPlan &p);
+hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t stream);
+hipError_t launch_sym_finish(const EvalPlan &p, const SymBuffers &b, double *F, hipStream_t stream);
+
 // Scratch of one evaluation: partial sums [splits][3][nrows] (FP64), followed
 // (256-byte aligned) by the source-tile table and, for STEPS_PREC_MIXED, the
 // FP32 tile-recentred source records and an FP32 copy of the S1R2 table.
 size_t partial_bytes(const EvalPlan &p);
+size_t scratch_bytes(const EvalPlan &p);
 size_t tile_extra_bytes(const EvalPlan &p);
 constexpr int kTile = 64;  // sources per tile (one wave64 prepares one tile)
 constexpr int kSub = 8;    // sources per sub-tile of the mixed S1R2 table kernels

@@ -120,10 +120,21 @@ extern "C" int steps_force_eval_noalloc(const steps_force_desc *d, int64_t N, co
     }
     if (radial) rad = (size_t)d->radial_table_size * sizeof(double);
     const size_t rbh = (size_t)p.bh_radial_size * sizeof(double);
-    const size_t pieces[] = {3 * nb, nb, nb, (size_t)N * sizeof(double4), nb, 3 * (size_t)p.nrows * sizeof(double),
+    size_t pieces[] = {3 * nb, nb, nb, (size_t)N * sizeof(double4), nb, 3 * (size_t)p.nrows * sizeof(double),
                              scratch_bytes(p), t3_raw, t3_dev, s1_raw, s1_dev, rad, rbh};
-    size_t need = 0;
-    for (size_t b : pieces) need += (b + 255) & ~(size_t)255;
+    auto total = [&] {
+        size_t n = 0;
+        for (size_t b : pieces) n += (b + 255) & ~(size_t)255;
+        return n;
+    };
+    size_t need = total();
+    if (need > kNoAllocScratchBytes && p.sym) {
+        // fewer cells of a pair-symmetric evaluation at a time: the same sums
+        const size_t rest = need - ((pieces[6] + 255) & ~(size_t)255);
+        if (rest < kNoAllocScratchBytes) (void)sym_fit(p, (kNoAllocScratchBytes - rest) & ~(size_t)255);
+        pieces[6] = scratch_bytes(p);
+        need = total();
+    }
     if (need > kNoAllocScratchBytes)
         return fail(STEPS_ERR_ARG, "evaluation needs " + std::to_string(need) + " bytes of device scratch; " +
                                        "steps_force_eval_noalloc has " + std::to_string(kNoAllocScratchBytes));

@@ -911,6 +911,37 @@ __device__ __forceinline__ float t3_mixed_disp(const KScalars &k, const double4 
     return fmaf(dx, dx, fmaf(dy, dy, dz * dz));
 }
 
+__device__ __forceinline__ double radial_correction(double r, double R, const double *T,
+                                                    int size) {
+    // forces_cuda.cu:41-70 (linear interpolation; nodes assumed at R/size*i)
+    const double step = R / (double)size;
+    const int i = (int)floor(r / R * (size - 1));
+    double c = T[size - 1];
+    if (i < size - 1) {
+        const double X1 = step * i, Y1 = T[i], X2 = step * (i + 1), Y2 = T[i + 1];
+        const double A = (Y2 - Y1) / (X2 - X1);
+        const double B = Y1 - A * X1;
+        c = A * r + B;
+    }
+    return c;
+}
+
+// The external term of a row at x (modes of EvalPlan::ext_mode).
+__device__ __forceinline__ void add_external(double f[3], const double4 &x, const double *radial, int ext_mode,
+                                             double ext_coeff, double Rsim, int radial_size) {
+    if (ext_mode == 3) {
+        // forces_cuda.cu:698-701: mass_in_unit_sphere * x * correction(r_xy), x and y only
+        const double corr = radial_correction(sqrt(x.x * x.x + x.y * x.y), Rsim, radial, radial_size);
+        f[0] += ext_coeff * x.x * corr;
+        f[1] += ext_coeff * x.y * corr;
+    } else if (ext_mode != 0) {
+        // forces_cuda.cu:545-556 (mode 1, xyz) and :848-857 (mode 2, xy)
+        f[0] += ext_coeff * x.x;
+        f[1] += ext_coeff * x.y;
+        if (ext_mode == 1) f[2] += ext_coeff * x.z;
+    }
+}
+
 // The launch scalars of an evaluation.
 inline KScalars make_scalars(const EvalPlan &p) {
     KScalars k{};

@@ -1088,21 +1088,6 @@ __global__ void t3_f32_kernel(const double *__restrict__ T, float4 *__restrict__
 // ---------------------------------------------------------------------------
 // fixed-order reduction of the splits + external term, AoS output
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double radial_correction(double r, double R, const double *T,
-                                                    int size) {
-    // forces_cuda.cu:41-70 (linear interpolation; nodes assumed at R/size*i)
-    const double step = R / (double)size;
-    const int i = (int)floor(r / R * (size - 1));
-    double c = T[size - 1];
-    if (i < size - 1) {
-        const double X1 = step * i, Y1 = T[i], X2 = step * (i + 1), Y2 = T[i + 1];
-        const double A = (Y2 - Y1) / (X2 - X1);
-        const double B = Y1 - A * X1;
-        c = A * r + B;
-    }
-    return c;
-}
-
 // perm (or null): partial-sum row r belongs to input row perm[r] (rows taken
 // in spatial order; id_min is 0 then).
 __global__ __launch_bounds__(256) void reduce_kernel(const double *__restrict__ part,
@@ -1123,19 +1108,7 @@ __global__ __launch_bounds__(256) void reduce_kernel(const double *__restrict__ 
         f[1] += p[nrows + k];
         f[2] += p[2 * nrows + k];
     }
-    if (ext_mode == 3) {
-        // forces_cuda.cu:698-701: mass_in_unit_sphere * x * correction(r_xy), x and y only
-        const double4 x = jrec[id_min + r];
-        const double corr = radial_correction(sqrt(x.x * x.x + x.y * x.y), Rsim, radial, radial_size);
-        f[0] += ext_coeff * x.x * corr;
-        f[1] += ext_coeff * x.y * corr;
-    } else if (ext_mode != 0) {
-        // forces_cuda.cu:545-556 (mode 1, xyz) and :848-857 (mode 2, xy)
-        const double4 x = jrec[id_min + r];
-        f[0] += ext_coeff * x.x;
-        f[1] += ext_coeff * x.y;
-        if (ext_mode == 1) f[2] += ext_coeff * x.z;
-    }
+    add_external(f, jrec[id_min + r], radial, ext_mode, ext_coeff, Rsim, radial_size);
     F[3 * r + 0] = f[0];
     F[3 * r + 1] = f[1];
     F[3 * r + 2] = f[2];
@@ -1411,6 +1384,15 @@ PairArgs make_args(const EvalPlan &p, const DeviceParticles &dp, const ScratchVi
     return a;
 }
 
+// What the pair-symmetric kernels read and write (launch_sym_pairs / _finish).
+SymBuffers sym_buffers(const EvalPlan &p, const DeviceParticles &dp, double *partials) {
+    const ScratchView v = scratch_view(p, partials);
+    const PairArgs a = make_args(p, dp, v);
+    const bool sorted = sorted_sources(p);
+    return SymBuffers{a.jrec, a.soft, a.tiles, a.tile_ext, a.table, a.keys,
+                      sorted ? spatial_order_perm(v.order, p.N) : nullptr, dp.jrec, v.part};
+}
+
 unsigned row_blocks(const EvalPlan &p) {
     const int64_t rpb = (int64_t)kBlock * rows_per_lane(p.variant, p.precision);
     return (unsigned)((p.nrows + rpb - 1) / rpb);
@@ -1485,7 +1467,7 @@ void s1r2_device_layout(const double *T, int nrho, int nz, std::vector<double> &
 }
 
 size_t partial_bytes(const EvalPlan &p) {
-    return (size_t)p.splits * 3u * (size_t)std::max<int64_t>(p.nrows, 1) * sizeof(double);
+    return std::max((size_t)p.splits * 3u * (size_t)std::max<int64_t>(p.nrows, 1) * sizeof(double), sym_bytes(p));
 }
 
 // Scratch after the partial sums (same buffer, 256-byte aligned pieces, in
@@ -1562,6 +1544,7 @@ hipError_t launch_forces_prepare(const EvalPlan &p, const DeviceParticles &dp, d
 
 hipError_t launch_forces_pairs(const EvalPlan &p, const DeviceParticles &dp, double *partials, hipStream_t st) {
     if (!has_pairs(p)) return hipSuccess;
+    if (sym_selected(p)) return launch_sym_pairs(p, sym_buffers(p, dp, partials), st);
     const PairArgs a = make_args(p, dp, scratch_view(p, partials));
     if (t3_window(p)) return launch_pair_t<BK_T3_WIN, PV_T3_EWALD>(&a, nullptr, 0, row_blocks(p), (unsigned)p.splits, st);
     if (t3_slab(p)) return launch_pair_t<BK_T3_SLAB, PV_T3_EWALD>(&a, nullptr, 0, row_blocks(p) * kXcds, 1, st);
@@ -1574,6 +1557,7 @@ hipError_t launch_forces_pairs(const EvalPlan &p, const DeviceParticles &dp, dou
 hipError_t launch_forces_finish(const EvalPlan &p, const DeviceParticles &dp, double *partials, double *F,
                                 hipStream_t st) {
     if (p.nrows <= 0) return hipSuccess;
+    if (sym_selected(p)) return launch_sym_finish(p, sym_buffers(p, dp, partials), F, st);
     const int splits = (p.N > 0) ? p.splits : 0;
     const uint32_t *perm =
         (sorted_rows(p) && has_pairs(p)) ? spatial_order_perm(scratch_view(p, partials).order, p.N) : nullptr;
@@ -1611,7 +1595,8 @@ int64_t pack_describe(const EvalPlan &p, const DeviceParticles &dp, double *part
     g.nbx = std::max(1u, row_blocks(p));
     g.blk_begin = (int)blk_begin;
     ((PackSeg *)host_descs)[idx] = g;
-    return has_pairs(p) ? (int64_t)g.nbx * p.splits : 0;  // an empty segment owns no workgroup
+    // a pair-symmetric evaluation is launched by itself (its segment owns no workgroup)
+    return (has_pairs(p) && !sym_selected(p)) ? (int64_t)g.nbx * p.splits : 0;
 }
 
 hipError_t launch_pair_packed(int variant, int precision, const void *dev_descs, int nseg, int64_t total_blocks,

@@ -60,6 +60,7 @@ struct SimEntry {
     std::vector<double> t3, s1r2, radial;   // host tables, needed to (re)admit
     steps_sim *res = nullptr;
     size_t bytes = 0;
+    bool lean = false;            // resident with the least scratch (it would not fit the budget otherwise)
     // busy: its device state is in use (a request in flight, an admission
     // or eviction in progress, a get_state copy); has_F: the host F copy is
     // the forces of the host positions; lost: an eviction failed to copy the
@@ -79,7 +80,7 @@ struct Slot {
 };
 
 // Device bytes a resident simulation takes (what sim_create allocates).
-size_t footprint(const steps_force_desc &d, int64_t N) {
+size_t footprint(const steps_force_desc &d, int64_t N, bool lean) {
     EvalPlan p;
     steps_force_desc dd = d;
     // tables only have to look present for the size computation
@@ -93,7 +94,9 @@ size_t footprint(const steps_force_desc &d, int64_t N) {
     for (int prec : {STEPS_PREC_FP64, STEPS_PREC_MIXED}) {
         if (prec == STEPS_PREC_MIXED && !desc_mixed_capable(d)) continue;
         dd.precision = prec;
-        if (make_plan(dd, N, 0, N - 1, p) == STEPS_OK) scratch = std::max(scratch, scratch_bytes(p));
+        if (make_plan(dd, N, 0, N - 1, p) != STEPS_OK) continue;
+        if (lean) p.sym_launch_cells = std::min(p.sym_launch_cells, 1);
+        scratch = std::max(scratch, scratch_bytes(p));
     }
     b += scratch;
     b += (size_t)(kdk_reduce_blocks(N) + 1) * 8;
@@ -413,6 +416,11 @@ struct steps_server {
         if (he == hipSuccess)
             he = hipMemcpyAsync(sl.dseg.ptr, sl.hseg, n * pack_desc_bytes(), hipMemcpyHostToDevice, qs);
         if (he == hipSuccess) he = launch_pair_packed(plans[0].variant, plans[0].precision, sl.dseg.ptr, (int)n, blocks, qs);
+        for (size_t i = 0; i < n && he == hipSuccess; ++i)
+            if (sym_selected(plans[i])) {  // owns no workgroup of the packed launch
+                steps_sim *s = a.es[i]->res;
+                he = launch_forces_pairs(plans[i], s->dp, s->part.as<double>(), qs);
+            }
         for (size_t i = 0; i < n && he == hipSuccess; ++i) {
             steps_sim *s = a.es[i]->res;
             he = launch_forces_finish(plans[i], s->dp, s->part.as<double>(), s->F.as<double>(), qs);
@@ -446,7 +454,7 @@ struct steps_server {
             d.s1r2_table = e.s1r2.empty() ? nullptr : e.s1r2.data();
             d.radial_table = e.radial.empty() ? nullptr : e.radial.data();
             steps_sim *s = nullptr;
-            a.rc = sim_create(d, e.N, true, &s);
+            a.rc = sim_create(d, e.N, true, e.lean, &s);
             if (!a.rc) {
                 a.rc = sim_upload(s, e.x.data(), e.v.data(), e.M.data(), e.soft.data(), e.has_F ? e.F.data() : nullptr);
                 if (a.rc) sim_destroy(s);
@@ -661,7 +669,9 @@ int steps_server_add_sim(steps_server *S, const steps_force_desc *d, int64_t N, 
     if (p.ext_mode == 3) e.radial.assign(d->radial_table, d->radial_table + d->radial_table_size);
     e.desc.t3_table = e.desc.s1r2_table = e.desc.radial_table = nullptr;
     e.variant = p.variant;
-    e.bytes = footprint(*d, N);
+    e.bytes = footprint(*d, N, false);
+    e.lean = (int64_t)e.bytes > S->cfg.hbm_budget_bytes;
+    if (e.lean) e.bytes = footprint(*d, N, true);
     if ((int64_t)e.bytes > S->cfg.hbm_budget_bytes)
         return fail(STEPS_ERR_ADMISSION, "simulation larger than the whole memory budget");
     std::lock_guard<std::mutex> lk(S->mu);

@@ -52,7 +52,6 @@ inline bool desc_mixed_capable(const steps_force_desc &d) {
            (d.topology == STEPS_TOPO_S1R2 &&
             (d.is_periodic == 1 || (d.is_periodic >= 2 && d.s1r2_lookup && d.interp_order != 0)));
 }
-size_t scratch_bytes(const EvalPlan &p);
 
 }  // namespace steps
 
@@ -81,7 +80,9 @@ struct steps_sim {
 namespace steps {
 
 // Create/destroy without touching the global error state of other sims.
-int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, steps_sim **out);
+// lean: the least scratch its evaluations can do with (one cell of a
+// pair-symmetric evaluation at a time; the same results).
+int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool lean, steps_sim **out);
 void sim_destroy(steps_sim *s);
 // Plan of one evaluation of this sim at the given precision.
 int sim_plan(steps_sim *s, int64_t id_min, int64_t id_max, int precision, EvalPlan &p);

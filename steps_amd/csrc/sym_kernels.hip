@@ -1,0 +1,563 @@
+// sym_kernels.hip -- direct pair forces with every unordered pair evaluated
+// once (Newton's third law), for evaluations of (nearly) all rows.
+//
+// The one-sided kernels (pair_kernels.hip) evaluate each pair twice, once per
+// row, and run at the VALU issue limit: the only way to less time is less
+// arithmetic per interaction.  Displacement, r^2, the reciprocal square root
+// and the softening are the same for both sides of a pair, and only the two
+// mass products and six accumulations belong to one side, so one evaluation
+// for both costs 18 FP64 VALU + one v_rsq_f64 per two interactions instead of
+// 14 + 1 per one.  What makes it pay on a wave64 machine is how the second
+// side is summed:
+//   * a lane holds NI target rows in VGPRs with their FP64 sums; a tile of 64
+//     sources is staged in LDS and at step s lane l takes source
+//     (l + s) mod 64, so the 64 lanes always hold 64 different sources and
+//     each source's partial sum rides along in VGPRs: after every step it
+//     moves one lane down (v_mov_b32 with DPP wave_rol:1, six dwords for NI
+//     pairs), and after 64 steps it is back in its own lane, complete for
+//     the wave's 64*NI rows.  No atomics and no cross-lane reduction;
+//   * the four waves of a workgroup take the same tile with their own rows;
+//     their four source sums are added through LDS in wave order.
+// Blocks of kSymBlock rows are paired cyclically: block b takes the source
+// blocks b, b+1 .. b+H (mod S), H = S/2, with the last offset taken by half
+// of the blocks when S is even, so every unordered block pair is evaluated
+// exactly once and all workgroups do the same work.  A (block, offset) pair's
+// source sums go to a slot of their own, [offset][3][N], the row sums of a
+// task (a run of tiles) to another, and the reduction adds the slots in a
+// fixed order, so two evaluations are bitwise equal.  When the slots of all
+// offsets do not fit the scratch, the offsets are done in groups of launches,
+// each followed by a reduction onto running sums; the additions and their
+// order do not depend on the grouping.
+//
+// Measured against the one-sided kernels (resident or one-shot calls, copies
+// included): R3 N = 16384 KDK runs 1.33 -> 1.04 ms, N = 100003 6.8 -> 4.5 ms,
+// N = 10^6 511 -> 387 ms (1.34 T pair evaluations/s, 2.67 T interactions/s;
+// the loop alone reaches 1.41); T3 nearest image at 64^3 50.0 -> 32.5 ms.
+// Errors against 64-bit sums are smaller (shorter addition chains).  Bound by
+// FP64 VALU issue: ~100 of the ~107 cycles a pair evaluation takes per SIMD
+// are its 18 FP64 instructions and the quarter-rate v_rsq_f64.
+#include "pair_device.h"
+
+#include <algorithm>
+
+namespace steps {
+
+namespace {
+
+constexpr int kSymWaves = kBlock / 64;
+
+struct SymArgs {
+    const double4 *rec;   // sources and rows: (x, y, z, -1.5 m)
+    const double *soft;
+    const double4 *tiles;  // per 64 records: bounding-box centre, largest softening length
+    const double4 *ext;    // half extents
+    double *part;
+    KScalars k;
+    int blocks, half;      // S and H
+    int tb, tpt;           // tiles per block, tiles per task
+    int cell_tasks, cell_offs;
+    int cell0;             // first cell of this launch
+};
+
+// Slot layout of one cell: cell_tasks row-sum slots, then cell_offs
+// source-sum slots, each [3][N].
+__host__ __device__ inline size_t sym_slot(int64_t n, int cell, int cell_tasks, int cell_offs, int slot) {
+    return ((size_t)cell * (size_t)(cell_tasks + cell_offs) + (size_t)slot) * 3u * (size_t)n;
+}
+
+__device__ __forceinline__ double from_next_lane(double v) {
+    // lane l receives lane (l + 1) mod 64's value
+    union { double d; int i[2]; } u;
+    u.d = v;
+    u.i[0] = __builtin_amdgcn_update_dpp(u.i[0], u.i[0], 0x134, 0xf, 0xf, false);
+    u.i[1] = __builtin_amdgcn_update_dpp(u.i[1], u.i[1], 0x134, 0xf, 0xf, false);
+    return u.d;
+}
+
+// Walks the tiles of a task: relative tile r counts from the block's own
+// first tile (offset r / tb, tile r mod tb of that source block).
+struct SymWalk {
+    int r, end;
+    int tile, off;
+    __device__ __forceinline__ bool settle(const SymArgs &a, int b, int ntiles) {
+        for (; r < end; ++r) {
+            off = r / a.tb;
+            if (off > a.half) return false;
+            // the last offset of an even number of blocks: half of the blocks
+            if (off > 0 && 2 * off == a.blocks && b >= off) {
+                r = (off + 1) * a.tb - 1;
+                continue;
+            }
+            int jb = b + off;
+            if (jb >= a.blocks) jb -= a.blocks;
+            tile = jb * a.tb + (r - off * a.tb);
+            if (tile < ntiles) return true;
+            r = (off + 1) * a.tb - 1;  // the rest of the (last) source block is empty
+        }
+        return false;
+    }
+};
+
+// One pair for both sides: u = -(2/3) r^-3 (mr3_scaled's correction without
+// the mass), the row's sum gets m_j r^-3 d, the source's m_i r^-3 d (its sign
+// is applied in the reduction).  NEAR: a pair within the bound B is left to
+// sym_close_pair (r2 may be 0 here) and reported.  NEAR = 2, a block with
+// itself: a pair at r2 <= rskip is not worth reporting (rskip is 0 where the
+// row is softened: the self pair's force is 0 then; else negative).
+template <int NEAR>
+__device__ __forceinline__ void sym_pair(const double dx, const double dy, const double dz, const double mi,
+                                         const double mj, const double cm53, const double B, const double rskip,
+                                         bool &close, double &fx,
+                                         double &fy, double &fz, double &gx, double &gy, double &gz) {
+    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double t = y * y;
+    double u = (t * y) * fma(r2, t, cm53);
+    if (NEAR) {
+        const bool c = r2 < B;
+        close = close || (NEAR == 2 ? (c && r2 > rskip) : c);
+        u = c ? 0.0 : u;
+    }
+    const double sj = u * mj, si = u * mi;
+    fx = fma(sj, dx, fx);
+    fy = fma(sj, dy, fy);
+    fz = fma(sj, dz, fz);
+    gx = fma(si, dx, gx);
+    gy = fma(si, dy, gy);
+    gz = fma(si, dz, gz);
+}
+
+// A pair within the tile's softening bound, exact test and spline.
+__device__ __forceinline__ void sym_close_pair(const double r2, const double dx, const double dy, const double dz,
+                                               const double mi, const double mj, const double *__restrict__ soft,
+                                               const int64_t i, const int64_t j, const double cm53, double &fx,
+                                               double &fy, double &fz, double &gx, double &gy, double &gz) {
+    const double beta = soft[i] + soft[j];
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double t = y * y;
+    double u = (t * y) * fma(r2, t, cm53);
+    if (r2 < beta * beta) u = softening_exact(sqrt(r2), beta) * (-2.0 / 3.0);
+    const double sj = u * mj, si = u * mi;
+    fx = fma(sj, dx, fx);
+    fy = fma(sj, dy, fy);
+    fz = fma(sj, dz, fz);
+    gx = fma(si, dx, gx);
+    gy = fma(si, dy, gy);
+    gz = fma(si, dz, gz);
+}
+
+template <int K> struct IntC { static constexpr int value = K; };
+
+template <int V, int NI>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_kernel(const SymArgs a) {
+    __shared__ __align__(2048) double2 jbuf[2][2][kTile];  // (x, y) and (z, -1.5 m) of the tile's sources
+    __shared__ double gsum[2][kSymWaves][3][kTile];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t N = a.k.N;
+    const int ntiles = (int)((N + kTile - 1) / kTile);
+    const int b = blockIdx.x;
+    const int cell_l = blockIdx.y / a.cell_tasks, task = blockIdx.y % a.cell_tasks;
+    const int cell = a.cell0 + cell_l;
+    SymWalk w;
+    w.r = cell * a.cell_offs * a.tb + task * a.tpt;
+    w.end = w.r + a.tpt;
+
+    const int64_t row0 = ((int64_t)b * kSymWaves + wave) * (64 * NI) + lane;
+    double x[NI], y[NI], z[NI], m[NI], fx[NI], fy[NI], fz[NI];
+#pragma unroll
+    for (int q = 0; q < NI; ++q) {
+        const int64_t r = row0 + q * 64;
+        const double4 p = a.rec[min(r, N - 1)];
+        x[q] = p.x;
+        y[q] = p.y;
+        z[q] = p.z;
+        m[q] = r < N ? p.w : 0.0;  // rows past the end: the last particle again, without mass
+        fx[q] = fy[q] = fz[q] = 0.0;
+    }
+    const double cm53 = a.k.cm53;
+
+    auto stage = [&](int buf, int tile) {  // wave 0: one source per lane
+        const int64_t j = (int64_t)tile * kTile + lane;
+        const double4 p = a.rec[min(j, N - 1)];
+        jbuf[buf][0][lane] = make_double2(p.x, p.y);
+        jbuf[buf][1][lane] = make_double2(p.z, j < N ? p.w : 0.0);
+    };
+    // source (lane + s) mod 64 of a tile at byte offset o = 16 ((lane + s) mod 64)
+    auto source = [&](int buf, unsigned o, double2 &pa, double2 &pb) {
+        const char *p = (const char *)&jbuf[buf][0][0] + o;
+        pa = *(const double2 *)p;
+        pb = *(const double2 *)(p + sizeof(double2) * kTile);
+    };
+    constexpr unsigned kWrap = sizeof(double2) * kTile - 1;
+    bool have = w.settle(a, b, ntiles);
+    if (have && wave == 0) stage(0, w.tile);
+    __syncthreads();
+
+    for (int it = 0; have; ++it) {
+        const int buf = it & 1;
+        const int tile = w.tile, off = w.off;
+        // the next tile's records, stored to the other buffer after this tile
+        SymWalk nw = w;
+        ++nw.r;
+        const bool more = nw.settle(a, b, ntiles);
+        if (more && wave == 0) stage(buf ^ 1, nw.tile);
+
+        const double4 tc = a.tiles[tile], te = a.ext[tile];
+        // far: no source of the tile within any row's softening bound (widened
+        // by 1e-9 for rounding); wrap: an axis on which some lane sees the
+        // tile on both sides of a period wrap.  Other axes take the row's
+        // image on the tile's side (tile_shift).
+        bool far = true, wx = false, wy = false, wz = false;
+        double B = 0.0;  // the largest of the lane's softening bounds
+        double rskip = 0.0;
+        if (V != PV_R3) {
+#pragma unroll
+            for (int q = 0; q < NI; ++q) {
+                const double4 p = a.rec[min(row0 + q * 64, N - 1)];
+                double sh;
+                if (V == PV_T3_NEAREST) {
+                    wx = !tile_shift(p.x, tc.x, te.x, a.k, sh) || wx;
+                    wy = !tile_shift(p.y, tc.y, te.y, a.k, sh) || wy;
+                }
+                wz = !tile_shift(p.z, tc.z, te.z, a.k, sh) || wz;
+            }
+            wx = __any(wx);
+            wy = __any(wy);
+            wz = __any(wz);
+        }
+#pragma unroll
+        for (int q = 0; q < NI; ++q) {
+            const int64_t r = min(row0 + q * 64, N - 1);
+            if (V != PV_R3) {
+                const double4 p = a.rec[r];
+                double sx = 0.0, sy = 0.0, sz = 0.0;
+                if (!wz) tile_shift(p.z, tc.z, te.z, a.k, sz);
+                if (V == PV_T3_NEAREST) {
+                    if (!wx) tile_shift(p.x, tc.x, te.x, a.k, sx);
+                    if (!wy) tile_shift(p.y, tc.y, te.y, a.k, sy);
+                }
+                x[q] = p.x - sx;
+                y[q] = p.y - sy;
+                z[q] = p.z - sz;
+            }
+            const double h = a.soft[r], bb = h + tc.w;
+            if (!(h > 0.0)) rskip = -1.0;
+            const double Bq = bb * bb;
+            B = fmax(B, Bq);
+            // distance to the box over the axes that are on one side
+            const double ax = wx ? 0.0 : fmax(fabs(x[q] - tc.x) - te.x, 0.0);
+            const double ay = wy ? 0.0 : fmax(fabs(y[q] - tc.y) - te.y, 0.0);
+            const double az = wz ? 0.0 : fmax(fabs(z[q] - tc.z) - te.z, 0.0);
+            far = far && fma(ax, ax, fma(ay, ay, az * az)) > Bq * (1.0 + 1e-9);
+        }
+        far = __all(far);
+
+        double gx = 0.0, gy = 0.0, gz = 0.0;
+        bool close = false;
+        // the 64 steps; WM: axes wrapped per pair (bit 0 x, 1 y, 2 z)
+        auto steps = [&](auto near, auto wm) {
+            constexpr int NEAR = decltype(near)::value;
+            constexpr int WM = decltype(wm)::value;
+            unsigned o = (unsigned)lane * 16u;
+            double2 na, nb;
+            source(buf, o, na, nb);
+#pragma unroll 2
+            for (int s = 0; s < kTile; ++s) {
+                const double2 pa = na, pb = nb;
+                o = (o + 16u) & kWrap;
+                source(buf, o, na, nb);  // the next step's (the last one re-reads the first)
+#pragma unroll
+                for (int q = 0; q < NI; ++q) {
+                    double dx = pa.x - x[q], dy = pa.y - y[q], dz = pb.x - z[q];
+                    if (WM & 1) dx = wrap_half(dx, a.k);
+                    if (WM & 2) dy = wrap_half(dy, a.k);
+                    if (WM & 4) dz = wrap_half(dz, a.k);
+                    sym_pair<NEAR>(dx, dy, dz, m[q], pb.y, cm53, B, rskip, close, fx[q], fy[q], fz[q], gx, gy, gz);
+                }
+                gx = from_next_lane(gx);
+                gy = from_next_lane(gy);
+                gz = from_next_lane(gz);
+            }
+        };
+        auto variants = [&](auto near) {
+            const int wm = (wx ? 1 : 0) | (wy ? 2 : 0) | (wz ? 4 : 0);
+            if (wm == 0) steps(near, IntC<0>{});
+            else if (V == PV_S1R2_NEAREST) steps(near, IntC<4>{});
+            else if (V == PV_T3_NEAREST) {
+                if (wm == 1) steps(near, IntC<1>{});
+                else if (wm == 2) steps(near, IntC<2>{});
+                else if (wm == 4) steps(near, IntC<4>{});
+                else steps(near, IntC<7>{});
+            }
+        };
+        if (far) variants(IntC<0>{});
+        else if (V == PV_R3 && off == 0) variants(IntC<2>{});
+        else variants(IntC<1>{});
+        if (__any(close)) {
+            // rare: the pairs within the bound, with the exact softening
+            // (every lane goes round, so that the source sums do)
+#pragma unroll 1
+            for (int s = 0; s < kTile; ++s) {
+                const int id = (lane + s) & 63;
+                double2 pa, pb;
+                source(buf, (unsigned)id * 16u, pa, pb);
+                const int64_t j = min((int64_t)tile * kTile + id, N - 1);
+#pragma unroll
+                for (int q = 0; q < NI; ++q) {
+                    double dx = pa.x - x[q], dy = pa.y - y[q], dz = pb.x - z[q];
+                    if (V == PV_T3_NEAREST && wx) dx = wrap_half(dx, a.k);
+                    if (V == PV_T3_NEAREST && wy) dy = wrap_half(dy, a.k);
+                    if (V != PV_R3 && wz) dz = wrap_half(dz, a.k);
+                    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+                    if (r2 < B) sym_close_pair(r2, dx, dy, dz, m[q], pb.y, a.soft, min(row0 + q * 64, N - 1), j, cm53,
+                                               fx[q], fy[q], fz[q], gx, gy, gz);
+                }
+                gx = from_next_lane(gx);
+                gy = from_next_lane(gy);
+                gz = from_next_lane(gz);
+            }
+        }
+        if (off > 0) {
+            gsum[buf][wave][0][lane] = gx;
+            gsum[buf][wave][1][lane] = gy;
+            gsum[buf][wave][2][lane] = gz;
+        }
+        // one barrier a tile: closes the source sums and the next tile's
+        // records; both buffers are reused two tiles on, past the next barrier
+        __syncthreads();
+        if (off > 0 && tid < 3 * kTile) {
+            const int c = tid >> 6;
+            const int64_t j = (int64_t)tile * kTile + lane;
+            double g = gsum[buf][0][c][lane];
+#pragma unroll
+            for (int v = 1; v < kSymWaves; ++v) g += gsum[buf][v][c][lane];
+            if (j < N)
+                a.part[sym_slot(N, cell_l, a.cell_tasks, a.cell_offs, a.cell_tasks + off - cell * a.cell_offs) +
+                       (size_t)c * N + j] = g;
+        }
+        w = nw;
+        have = more;
+    }
+
+    double *out = a.part + sym_slot(N, cell_l, a.cell_tasks, a.cell_offs, task);
+#pragma unroll
+    for (int q = 0; q < NI; ++q) {
+        const int64_t r = row0 + q * 64;
+        if (r < N) {
+            out[r] = fx[q];
+            out[N + r] = fy[q];
+            out[2 * N + r] = fz[q];
+        }
+    }
+}
+
+// The slots of one launch onto the running sums: cell by cell, the row sums
+// of its tasks, then its source sums (with the sign of the other side).  The
+// last launch's reduction adds the external term (reduce_kernel's) and writes
+// F for the rows asked for, in input order.
+struct SymReduceArgs {
+    const double *part;
+    double *acc;           // running sums [3][N]
+    const uint32_t *perm;  // sorted row -> input row, or null
+    const double4 *jrec;   // input order
+    const double *radial;
+    double *F;
+    int64_t N, id_min, nrows;
+    int blocks, half, block_rows, cell_tasks, cell_offs, cell0, cells;
+    int first, last;
+    int ext_mode, radial_size;
+    double ext_coeff, Rsim;
+};
+
+// One thread per row and component (blockIdx.y): at N = 16384 the slots are
+// 144 deep and the row count alone would leave most CUs idle.
+__global__ __launch_bounds__(256) void sym_reduce_kernel(const SymReduceArgs a) {
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= a.N) return;
+    const int c = blockIdx.y;
+    const int b = (int)(k / a.block_rows);
+    const size_t slot = 3u * (size_t)a.N;
+    const double *p = a.part + (size_t)c * a.N + k;
+    double f = a.first ? 0.0 : a.acc[(size_t)c * a.N + k];
+    for (int cl = 0; cl < a.cells; ++cl) {
+#pragma unroll 8
+        for (int t = 0; t < a.cell_tasks; ++t, p += slot) f += *p;
+        const int off0 = (a.cell0 + cl) * a.cell_offs;
+#pragma unroll 4
+        for (int o = 0; o < a.cell_offs; ++o, p += slot) {
+            const int off = off0 + o;
+            // slots nobody wrote: the block's own offset, offsets past H, and
+            // the half of the blocks that took the last offset as rows
+            if (off == 0 || off > a.half || (2 * off == a.blocks && b < off)) continue;
+            f -= *p;
+        }
+    }
+    if (!a.last) {
+        a.acc[(size_t)c * a.N + k] = f;
+        return;
+    }
+    const int64_t r = a.perm ? (int64_t)a.perm[k] : k;
+    if (r < a.id_min || r >= a.id_min + a.nrows) return;
+    double g[3] = {f, f, f};
+    add_external(g, a.jrec[r], a.radial, a.ext_mode, a.ext_coeff, a.Rsim, a.radial_size);
+    a.F[3 * (r - a.id_min) + c] = c == 0 ? g[0] : (c == 1 ? g[1] : g[2]);
+}
+
+}  // namespace
+
+namespace {
+
+// Rows per lane: the moving sums, the LDS reads and the address arithmetic of
+// a step are paid once per NI pairs.  2 rows measured 1.25 T evaluations/s in
+// the bare loop, 4 1.41 T (128 VGPRs, 4 waves per SIMD); 8 rows (168 VGPRs, 3
+// waves) 1.48 T there, but the tested loops spill and fewer tiles are far of
+// a 512-row wave: 402 against 387 ms at N = 10^6.
+constexpr int kSymNI = 4;
+// Below this many particles the triangle of block pairs leaves too few equal
+// tasks to fill the chip (N = 9000: 0.129 against 0.167 ms).
+constexpr int64_t kSymMinN = 8192;
+// Scratch the slots may take; the offsets go in as many launches as that
+// needs (128 MiB: 4.5 against 4.3 ms at N = 100003, 33.2 against 31.0 ms for
+// the 64^3 nearest image).
+constexpr size_t kSymBytes = (size_t)256 << 20;
+
+bool sym_variant(const EvalPlan &p) {
+    return p.precision == STEPS_PREC_FP64 &&
+           (p.variant == PV_R3 || p.variant == PV_T3_NEAREST || p.variant == PV_S1R2_NEAREST);
+}
+
+struct SymShape {
+    int tb, cell_tasks, cell_offs, half, cells;
+};
+
+SymShape sym_shape(const EvalPlan &p) {
+    SymShape s;
+    s.tb = p.sym_block_rows / kTile;
+    s.cell_tasks = std::max(1, s.tb / p.sym_task_tiles);
+    s.cell_offs = std::max(1, p.sym_task_tiles / s.tb);
+    s.half = p.sym_blocks / 2;
+    s.cells = (s.half + s.cell_offs) / s.cell_offs;  // offsets 0 .. half
+    return s;
+}
+
+size_t sym_cell_bytes(const EvalPlan &p) {
+    const SymShape s = sym_shape(p);
+    return (size_t)(s.cell_tasks + s.cell_offs) * 3u * (size_t)p.N * sizeof(double);
+}
+
+size_t sym_acc_bytes(const EvalPlan &p) {
+    return p.sym_launch_cells < p.sym_cells ? 3u * (size_t)p.N * sizeof(double) : 0;
+}
+
+void launch_sym_kernel(const EvalPlan &p, const SymArgs &a, int cells, hipStream_t st) {
+    const dim3 grid((unsigned)a.blocks, (unsigned)(cells * a.cell_tasks));
+    switch (p.variant) {
+    case PV_R3: hipLaunchKernelGGL((sym_kernel<PV_R3, kSymNI>), grid, dim3(kBlock), 0, st, a); break;
+    case PV_T3_NEAREST: hipLaunchKernelGGL((sym_kernel<PV_T3_NEAREST, kSymNI>), grid, dim3(kBlock), 0, st, a); break;
+    default: hipLaunchKernelGGL((sym_kernel<PV_S1R2_NEAREST, kSymNI>), grid, dim3(kBlock), 0, st, a); break;
+    }
+}
+
+hipError_t launch_sym_reduce(const EvalPlan &p, const SymBuffers &b, int cell0, int cells, double *F, hipStream_t st) {
+    const SymShape s = sym_shape(p);
+    SymReduceArgs r{};
+    r.part = b.part;
+    r.acc = b.part + sym_cell_bytes(p) / sizeof(double) * (size_t)p.sym_launch_cells;
+    r.perm = b.perm;
+    r.jrec = b.jrec;
+    r.radial = p.radial;
+    r.F = F;
+    r.N = p.N;
+    r.id_min = p.id_min;
+    r.nrows = p.nrows;
+    r.blocks = p.sym_blocks;
+    r.half = s.half;
+    r.block_rows = p.sym_block_rows;
+    r.cell_tasks = s.cell_tasks;
+    r.cell_offs = s.cell_offs;
+    r.cell0 = cell0;
+    r.cells = cells;
+    r.first = cell0 == 0;
+    r.last = F != nullptr;
+    r.ext_mode = p.ext_mode;
+    r.radial_size = p.radial_size;
+    r.ext_coeff = p.ext_coeff;
+    r.Rsim = p.Rsim;
+    hipLaunchKernelGGL(sym_reduce_kernel, dim3((unsigned)((p.N + 255) / 256), 3), dim3(256), 0, st, r);
+    return hipGetLastError();
+}
+
+// First cell of the last launch.
+int sym_last_cell0(const EvalPlan &p) { return (p.sym_cells - 1) / p.sym_launch_cells * p.sym_launch_cells; }
+
+}  // namespace
+
+// The triangle pays when (nearly) every row is asked for: it evaluates
+// N^2 / 2 pairs at ~1.45 times the cost of a one-sided pair, the one-sided
+// kernel nrows N of them.
+void sym_plan(EvalPlan &p) {
+    p.sym = false;
+    if (p.bh || p.N < kSymMinN || p.N > INT32_MAX || 3 * p.nrows < 2 * p.N || !sym_variant(p)) return;
+    p.sym = true;
+    p.sym_block_rows = kBlock * kSymNI;
+    p.sym_blocks = (int)((p.N + p.sym_block_rows - 1) / p.sym_block_rows);
+    const int tb = p.sym_block_rows / kTile, offsets = p.sym_blocks / 2 + 1;
+    // Tasks of several offsets where there are plenty (fewer row-sum slots),
+    // of parts of an offset where there are few (workgroups to fill the chip).
+    int tiles = tb;
+    if ((int64_t)p.sym_blocks * offsets >= 16384) tiles = 2 * tb;
+    if ((int64_t)p.sym_blocks * offsets >= 4 * 16384) tiles = 4 * tb;
+    while (tiles > 1 && tiles <= tb && (int64_t)p.sym_blocks * offsets * (tb / tiles) < 1100) tiles /= 2;
+    p.sym_task_tiles = tiles;
+    const SymShape s = sym_shape(p);
+    p.sym_cells = s.cells;
+    const size_t most = std::max(kSymBytes, (size_t)p.splits * 3u * (size_t)p.nrows * sizeof(double));
+    p.sym_launch_cells = (int)std::min<size_t>((size_t)s.cells, std::max<size_t>(1, most / sym_cell_bytes(p)));
+}
+
+size_t sym_bytes(const EvalPlan &p) {
+    return p.sym ? sym_cell_bytes(p) * (size_t)p.sym_launch_cells + sym_acc_bytes(p) : 0;
+}
+
+bool sym_fit(EvalPlan &p, size_t bytes) {
+    while (p.sym && scratch_bytes(p) > bytes) {
+        if (p.sym_launch_cells == 1) return false;
+        p.sym_launch_cells = p.sym_launch_cells > 8 ? p.sym_launch_cells * 7 / 8 : p.sym_launch_cells - 1;
+    }
+    return true;
+}
+
+bool sym_selected(const EvalPlan &p) { return p.sym; }
+
+hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t st) {
+    const SymShape s = sym_shape(p);
+    SymArgs a{};
+    a.rec = b.rec;
+    a.soft = b.soft;
+    a.tiles = b.tiles;
+    a.ext = b.ext;
+    a.part = b.part;
+    a.k = make_scalars(p);
+    a.blocks = p.sym_blocks;
+    a.half = s.half;
+    a.tb = s.tb;
+    a.tpt = p.sym_task_tiles;
+    a.cell_tasks = s.cell_tasks;
+    a.cell_offs = s.cell_offs;
+    for (int c0 = 0; c0 < p.sym_cells; c0 += p.sym_launch_cells) {
+        const int cells = std::min(p.sym_launch_cells, p.sym_cells - c0);
+        a.cell0 = c0;
+        launch_sym_kernel(p, a, cells, st);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess && c0 + cells < p.sym_cells) e = launch_sym_reduce(p, b, c0, cells, nullptr, st);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+hipError_t launch_sym_finish(const EvalPlan &p, const SymBuffers &b, double *F, hipStream_t st) {
+    const int c0 = sym_last_cell0(p);
+    return launch_sym_reduce(p, b, c0, p.sym_cells - c0, F, st);
+}
+
+}  // namespace steps
