@@ -76,6 +76,7 @@ struct EvalPlan {
     // tables (device)
     const double *t3 = nullptr; int t3_ng = 0;
     int t3_lo = 0;         // first x/y node of the T3 device layout (t3_device_layout)
+    bool t3_odd = false;   // the table in use is odd (t3_table_odd)
     const double *s1r2 = nullptr; int s1r2_nrho = 0, s1r2_nz = 0;
     const double *radial = nullptr; int radial_size = 0;
     int images = 0;        // S1R2 image-sum: ewald_max
@@ -233,6 +234,9 @@ int kdk_reduce_blocks(int64_t n);
 int t3_device_layout(const double *T, int ng, std::vector<double> &out);
 // The lo t3_device_layout picks for this table (Ng/2 when it folds, else 0).
 int t3_layout_lo(const double *T, int ng);
+// The table is odd through its centre, T(-d) = -T(d) (components below 2^-52
+// max|T| count as zero): the correction of a pair then serves both sides.
+bool t3_table_odd(const double *T, int ng);
 inline size_t t3_device_entries(int ng, int lo) {
     return (size_t)(ng - lo) * (size_t)(ng - lo) * (size_t)(ng + 3) * 3u;
 }

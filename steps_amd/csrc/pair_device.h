@@ -802,14 +802,16 @@ __device__ __forceinline__ void mixed_far_tile_z(const float4 *__restrict__ tr, 
 // odd multiples of 128 bytes: 32.4).
 __host__ __device__ constexpr unsigned t3_win_stride(unsigned nz3) { return (nz3 + 1u) & ~1u; }
 
-// Layout nodes one axis of the window needs: sources in cell column s, rows
-// in columns [bmin, bmax].  d / h lies in (s - b - 1, s - b + 1) (mod Ng), so
-// the stencils' unfolded nodes lie in [s - bmax + (Ng-1)/2 - 2,
-// s - bmin + Ng/2 + 2] (mod Ng); their images in the folded layout are a
-// contiguous range [f0, f0 + nf).  False when the range is too wide to be one.
-__device__ __forceinline__ bool t3_win_axis(int s, int bmin, int bmax, int Ng, int lo, int &f0, int &nf) {
-    const int nlo = (s - bmax) + (Ng - 1) / 2 - 2;
-    const int nhi = (s - bmin) + Ng / 2 + 2;
+// Layout nodes one axis of the window needs: sources in cell columns
+// [smin, smax], rows in columns [bmin, bmax].  d / h lies in (s - b - 1,
+// s - b + 1) (mod Ng), so the stencils' unfolded nodes lie in
+// [smin - bmax + (Ng-1)/2 - 2, smax - bmin + Ng/2 + 2] (mod Ng); their images
+// in the folded layout are a contiguous range [f0, f0 + nf).  False when the
+// range is too wide to be one.
+__device__ __forceinline__ bool t3_win_axis(int smin, int smax, int bmin, int bmax, int Ng, int lo, int &f0,
+                                            int &nf) {
+    const int nlo = (smin - bmax) + (Ng - 1) / 2 - 2;
+    const int nhi = (smax - bmin) + Ng / 2 + 2;
     if (nhi - nlo >= Ng / 2) return false;
     int mn = Ng, mxv = -1;
     for (int n = nlo; n <= nhi; ++n) {

@@ -703,8 +703,8 @@ __device__ __forceinline__ void body_t3_win(const PairArgs &a, const int bx, con
             const int pk = (int)(kj >> 10);
             if (pk != cur) {
                 cur = pk;
-                wok = t3_win_axis(pk >> 10, bxmin, bxmax, Ng, lo, fx0, nxw) &&
-                      t3_win_axis(pencil_y(kj, Ng), bymin, bymax, Ng, lo, fy0, nyw) &&
+                wok = t3_win_axis(pk >> 10, pk >> 10, bxmin, bxmax, Ng, lo, fx0, nxw) &&
+                      t3_win_axis(pencil_y(kj, Ng), pencil_y(kj, Ng), bymin, bymax, Ng, lo, fy0, nyw) &&
                       (int64_t)nxw * nyw * WS <= kT3WinDoubles;
                 __syncthreads();  // every wave is done with the previous window
                 if (wok) {
@@ -955,8 +955,8 @@ __device__ __forceinline__ void body_t3_mixed(const PairArgs &a, const int bx, c
                 const int pk = (int)(kj >> 10);
                 if (pk != cur) {  // the same for every wave: both barriers are reached by all
                     cur = pk;
-                    wok = win_share && t3_win_axis(pk >> 10, bxmin, bxmax, Ng, lo, fx0, nxw) &&
-                          t3_win_axis(pencil_y(kj, Ng), bymin, bymax, Ng, lo, fy0, nyw) &&
+                    wok = win_share && t3_win_axis(pk >> 10, pk >> 10, bxmin, bxmax, Ng, lo, fx0, nxw) &&
+                          t3_win_axis(pencil_y(kj, Ng), pencil_y(kj, Ng), bymin, bymax, Ng, lo, fy0, nyw) &&
                           (int64_t)nxw * nyw * NZ <= kT3WinNodes32;
                     __syncthreads();  // every wave is done with the previous window
                     if (wok) {
@@ -1431,6 +1431,20 @@ static bool t3_antisymmetric_xy(const double *T, int ng) {
                 if (!(same(by[0], a[0]) && (2 * iy + 1 == n || same(by[1], -a[1])) && same(by[2], a[2])))
                     return false;
             }
+    return true;
+}
+
+bool t3_table_odd(const double *T, int ng) {
+    const size_t n3 = (size_t)ng * ng * ng;
+    double tmax = 0.0;
+    for (size_t i = 0; i < n3 * 3u; ++i) tmax = std::max(tmax, std::fabs(T[i]));
+    if (!(tmax < INFINITY)) return false;
+    const double eps0 = std::ldexp(tmax, -52);
+    for (size_t i = 0; i < n3; ++i) {  // node n3 - 1 - i is node i seen through the centre
+        const double *a = T + 3u * i, *b = T + 3u * (n3 - 1 - i);
+        for (int c = 0; c < 3; ++c)
+            if (!(b[c] == -a[c] || (std::fabs(a[c]) <= eps0 && std::fabs(b[c]) <= eps0))) return false;
+    }
     return true;
 }
 

@@ -34,7 +34,8 @@ struct TableCopy {
     size_t n = 0;
     uint64_t fp = 0;
     DevBuf dev;
-    int lo = 0;  // T3 tables: first x/y node of the device layout
+    int lo = 0;        // T3 tables: first x/y node of the device layout
+    bool odd = false;  // T3 tables: t3_table_odd
     int sync(const double *h, size_t count, hipStream_t st, const char *what);
     // T3 / S1R2: upload the table in the pair kernels' layout
     // (t3_device_layout, s1r2_device_layout)

@@ -51,6 +51,8 @@ struct SymArgs {
     const double *soft;
     const double4 *tiles;  // per 64 records: bounding-box centre, largest softening length
     const double4 *ext;    // half extents
+    const double *table;   // T3 Ewald table, device layout
+    const uint32_t *keys;  // pencil keys of the records (T3 Ewald)
     double *part;
     KScalars k;
     int blocks, half;      // S and H
@@ -351,6 +353,303 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     }
 }
 
+// ---------------------------------------------------------------------------
+// T3 Ewald: the same scheme, one row per lane.  The tricubic correction reads
+// 192 table values per pair, and those reads are what the pair costs; here
+// they serve both sides.  Records are in z pencils.  Before each source tile
+// the workgroup copies the table window that its rows' and the tile's cell
+// columns can reach into LDS, unfolded, so that a stencil is 16 rows at fixed
+// strides from one address: no mirror or wrap per row (638 -> 468 VALU per
+// pair against the folded window of body_t3_win).  A window that does not fit
+// leaves the tile on the global table, and so does a lane whose stencil
+// leaves the window.  The eight waves of a workgroup are W / G sets of 64
+// rows times G groups of 64 / G steps: fewer rows make a smaller window, so
+// sparse boxes (few particles per column) take G = 4 or 8.  After the tile
+// the window's memory takes the waves' source sums.
+//
+// Bound by LDS: ~107 reads of 16 bytes per pair, 4.3 cycles each, and as much
+// again in bank conflicts (876 LDS cycles of 978 per wave step at 60^3).  In
+// the lanes of one read the source and row indices both advance, so their
+// stencils sit a few z nodes apart on 2 x 2 neighbouring rows; the (x, y)
+// nodes are therefore stored by z mod 4 (lanes a few nodes apart then share
+// words) and rows 4, planes 8 words apart mod 16.  Measured at 60^3: folded
+// body_t3_win rows 737 ms, this layout 615; planes at 4 or 2 mod 16 695 / 652,
+// rows of 104 or 108 words 630 / 633, z components as single 8-byte reads 710.
+// Measured against the one-sided kernels (ms): 24^3 22.8 -> 9.7, 40^3 310 ->
+// 86, 48^3 739 -> 206, 56^3 1440 -> 443, 64^3 2000 -> 850.
+// ---------------------------------------------------------------------------
+constexpr int kSymT3Win = 9800;   // 16-byte words: 153 KB, one workgroup per CU
+constexpr int kT3Waves = 8;
+constexpr int kT3MaxWinNg = 63;   // the window row is laid out for tables up to this grid
+constexpr int kT3Row = 100;       // words a window row: 66 (x, y) nodes and 34 z pairs
+constexpr int kT3RunOff[4] = {0, 17, 34, 50};  // (x, y) nodes by z mod 4: start of each run
+constexpr int kT3ZPairs = 66;     // start of the z components, two nodes a word
+
+// Words from one x plane of window rows to the next: 8 (mod 16), which with
+// rows 4 (mod 16) apart spreads the 2 x 2 neighbouring rows that the lanes
+// of a read mostly sit on over different banks.
+__device__ __forceinline__ int t3_plane(int ny) { return ny * kT3Row + ((8 - ny * kT3Row) & 15); }
+
+// Unfolded nodes one axis of the window holds: n0 .. n0 + n - 1 (mod Ng), n0
+// in [0, Ng), for sources in cell columns [smin, smax] and rows in [bmin,
+// bmax] (see t3_win_axis).  n <= Ng + 3 keeps every node at most twice.
+__device__ __forceinline__ void t3_win_nodes(int smin, int smax, int bmin, int bmax, int Ng, int &n0, int &n) {
+    const int nlo = (smin - bmax) + (Ng - 1) / 2 - 2, nhi = (smax - bmin) + Ng / 2 + 2;
+    n = nhi - nlo + 1;
+    n0 = imodp(nlo, Ng);
+}
+
+// Stencil start of one axis relative to the window's first node: node
+// floor(u) - 1 is window node rel; false when the four nodes leave the window
+// (or the displacement the box).
+__device__ __forceinline__ bool t3_win_rel(int i, int n0, int n, int Ng, unsigned &rel) {
+    const int d = i - 1 - n0;
+    rel = min((unsigned)d, (unsigned)(d + Ng));
+    return (int)rel <= n - 4 && (int)rel >= 0;
+}
+
+// Catmull-Rom weights of one axis (t3_axis without the index wrap).
+__device__ __forceinline__ int t3_weights(double d, const KScalars &k, double w[4]) {
+    const double u = (d + k.L * 0.5) * k.inv_gs - 0.5;
+    const double uf = floor(u);
+    const double t = u - uf;
+    const double t2 = t * t, t3 = t * t2;
+    w[0] = -0.5 * t3 + t2 - 0.5 * t;
+    w[1] = 1.5 * t3 - 2.5 * t2 + 1.0;
+    w[2] = -1.5 * t3 + 2.0 * t2 + 0.5 * t;
+    w[3] = 0.5 * t3 - 0.5 * t2;
+    return (int)uf;
+}
+
+template <int G>
+__global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) {
+    constexpr int W = kT3Waves, RW = W / G;  // waves; waves of different rows
+    constexpr int kSteps = kTile / G;
+    __shared__ __align__(16) double win[2 * kSymT3Win];
+    __shared__ __align__(16) double2 jbuf[2][kTile];
+    __shared__ int brange[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t N = a.k.N;
+    const int ntiles = (int)((N + kTile - 1) / kTile);
+    const int b = blockIdx.x;
+    const int cell_l = blockIdx.y / a.cell_tasks, task = blockIdx.y % a.cell_tasks;
+    const int cell = a.cell0 + cell_l;
+    SymWalk w;
+    w.r = cell * a.cell_offs * a.tb + task * a.tpt;
+    w.end = w.r + a.tpt;
+
+    KScalars k = a.k;
+    k.c15 = in_vgpr(a.k.c15);
+    const int64_t row = (int64_t)b * (64 * RW) + (wave % RW) * 64 + lane;
+    const int s0 = wave / RW * kSteps;  // the wave's first step
+    const int64_t rowc = min(row, N - 1);
+    const double4 p = a.rec[rowc];
+    const double xi = p.x, yi = p.y, zi = p.z, mi = row < N ? p.w : 0.0, hi = a.soft[rowc];
+    double fx = 0.0, fy = 0.0, fz = 0.0;
+    const int Ng = k.ng, lo = k.t3_lo;
+    const unsigned NY = (unsigned)(Ng - lo), NZ = (unsigned)(Ng + 3), NZ3 = 3u * NZ;
+
+    int bxmin = 0, bxmax = 0, bymin = 0, bymax = 0;  // the rows' cell columns
+    {
+        if (tid == 0) {
+            brange[0] = brange[2] = INT32_MAX;
+            brange[1] = brange[3] = -1;
+        }
+        __syncthreads();
+        const uint32_t kr = a.keys[rowc];
+        const int rbx = (int)(kr >> 20), rby = pencil_y(kr, Ng);
+        atomicMin(&brange[0], rbx);
+        atomicMax(&brange[1], rbx);
+        atomicMin(&brange[2], rby);
+        atomicMax(&brange[3], rby);
+        __syncthreads();
+        bxmin = brange[0];
+        bxmax = brange[1];
+        bymin = brange[2];
+        bymax = brange[3];
+    }
+    auto stage = [&](int tile) {  // wave 0: one source per lane
+        const int64_t j = (int64_t)tile * kTile + lane;
+        const double4 q = a.rec[min(j, N - 1)];
+        jbuf[0][lane] = make_double2(q.x, q.y);
+        jbuf[1][lane] = make_double2(q.z, j < N ? q.w : 0.0);
+    };
+    bool have = w.settle(a, b, ntiles);
+    if (have && wave == 0) stage(w.tile);
+
+    while (have) {
+        const int tile = w.tile, off = w.off;
+        __syncthreads();  // records in place; the window's memory is free
+        bool wok = false;
+        int wx0 = 0, nx = 0, wy0 = 0, ny = 0, plane = 0;
+        {
+            const uint32_t kj = a.keys[min((int64_t)tile * kTile + lane, N - 1)];
+            int sx0 = (int)(kj >> 20), sx1 = sx0, sy0 = pencil_y(kj, Ng), sy1 = sy0;
+#pragma unroll
+            for (int m = 32; m > 0; m >>= 1) {
+                sx0 = min(sx0, __shfl_xor(sx0, m, 64));
+                sx1 = max(sx1, __shfl_xor(sx1, m, 64));
+                sy0 = min(sy0, __shfl_xor(sy0, m, 64));
+                sy1 = max(sy1, __shfl_xor(sy1, m, 64));
+            }
+            t3_win_nodes(sx0, sx1, bxmin, bxmax, Ng, wx0, nx);
+            t3_win_nodes(sy0, sy1, bymin, bymax, Ng, wy0, ny);
+            wx0 = __builtin_amdgcn_readfirstlane(wx0);
+            wy0 = __builtin_amdgcn_readfirstlane(wy0);
+            nx = __builtin_amdgcn_readfirstlane(nx);
+            ny = __builtin_amdgcn_readfirstlane(ny);
+            plane = t3_plane(ny);
+            wok = nx <= Ng && ny <= Ng && nx * plane <= kSymT3Win;
+            if (wok) {
+                // a wave copies whole rows (lanes along the z run), unfolding
+                // them: a node below lo is its mirror with that component negated
+                for (int rw = wave; rw < nx * ny; rw += W) {
+                    const int ax = rw / ny, ay = rw - ax * ny;
+                    int jx = wx0 + ax, jy = wy0 + ay;
+                    if (jx >= Ng) jx -= Ng;
+                    if (jy >= Ng) jy -= Ng;
+                    const bool fx_ = jx < lo, fy_ = jy < lo;
+                    const unsigned mx = (unsigned)(fx_ ? Ng - 1 - lo - jx : jx - lo);
+                    const unsigned my = (unsigned)(fy_ ? Ng - 1 - lo - jy : jy - lo);
+                    const double *src = a.table + (mx * NY + my) * NZ3;
+                    double *dst = win + 2 * (ax * plane + ay * kT3Row);
+                    for (unsigned o = lane; o < 2u * kT3Row; o += 64) {
+                        if (o < NZ3) {
+                            const unsigned z = o / 3u, c = o - 3u * z;
+                            double v = src[o];
+                            if (c == 0u && fx_) v = -v;
+                            if (c == 1u && fy_) v = -v;
+                            const unsigned run = z & 3u;
+                            const unsigned start = run == 0u ? 0u : (run == 1u ? 17u : (run == 2u ? 34u : 50u));
+                            dst[c < 2u ? 2u * (start + (z >> 2)) + c : 2u * kT3ZPairs + z] = v;
+                        }
+                    }
+                    // z values past the run meet zero weights
+                    const unsigned pad = 2u * kT3ZPairs + NZ + lane;
+                    if (pad < 2u * kT3Row) dst[pad] = 0.0;
+                }
+            }
+            __syncthreads();  // the window is complete
+        }
+        const double bb = hi + a.tiles[tile].w;
+        const double B = bb * bb;
+        double gx = 0.0, gy = 0.0, gz = 0.0;
+#pragma unroll 1
+        for (int s = 0; s < kSteps; ++s) {
+            const int id = (lane + s0 + s) & 63;
+            const double2 pa = jbuf[0][id], pb = jbuf[1][id];
+            const double dx = wrap_half(pa.x - xi, k), dy = wrap_half(pa.y - yi, k), dz = wrap_half(pb.x - zi, k);
+            const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+            const double wp = pair_w_tile(r2, B, hi, a.soft, min((int64_t)tile * kTile + id, N - 1), k);
+            double Dx, Dy, Dz;
+            bool in = false;
+            double wxs[4], wys[4], wzs[4];
+            unsigned rx = 0, ry = 0, iz = 0;
+            if (wok) {
+                const int ix = t3_weights(dx, k, wxs), iy = t3_weights(dy, k, wys), izi = t3_weights(dz, k, wzs);
+                iz = min((unsigned)izi, (unsigned)(izi + Ng));  // layout z index of the stencil's first node
+                const bool inx = t3_win_rel(ix, wx0, nx, Ng, rx), iny = t3_win_rel(iy, wy0, ny, Ng, ry);
+                in = inx && iny && iz < (unsigned)Ng;
+            }
+            if (in) {
+                // (x, y) nodes by z mod 4: read k takes the stencil's node with
+                // z = k (mod 4), so lanes a few nodes apart read the same word
+                // or neighbouring ones
+                const unsigned r = iz & 3u, blk = iz >> 2;
+                double v0 = wzs[0], v1 = wzs[1], v2 = wzs[2], v3 = wzs[3];
+                const bool r1 = (r & 1u) != 0u, r2b = (r & 2u) != 0u;
+                const double p0 = r1 ? v3 : v0, p1 = r1 ? v0 : v1, p2 = r1 ? v1 : v2, p3 = r1 ? v2 : v3;
+                const double wk[4] = {r2b ? p2 : p0, r2b ? p3 : p1, r2b ? p0 : p2, r2b ? p1 : p3};
+                const double wz5[5] = {r1 ? 0.0 : v0, r1 ? v0 : v1, r1 ? v1 : v2, r1 ? v2 : v3, r1 ? v3 : 0.0};
+                const unsigned base = rx * (unsigned)plane + ry * (unsigned)kT3Row;
+                const double2 *w2 = (const double2 *)win;
+                const double2 *pk[4], *pz = w2 + base + kT3ZPairs + (iz >> 1);
+#pragma unroll
+                for (unsigned q = 0; q < 4; ++q) pk[q] = w2 + base + kT3RunOff[q] + blk + (q < r ? 1u : 0u);
+                double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    double u0 = 0.0, u1 = 0.0, u2 = 0.0;
+#pragma unroll
+                    for (int jj = 0; jj < 4; ++jj) {
+                        const double2 a0 = pk[0][jj * kT3Row], a1 = pk[1][jj * kT3Row], a2 = pk[2][jj * kT3Row],
+                                      a3 = pk[3][jj * kT3Row];
+                        const double2 z0 = pz[jj * kT3Row], z1 = pz[jj * kT3Row + 1], z2 = pz[jj * kT3Row + 2];
+                        const double t0 = fma(wk[3], a3.x, fma(wk[2], a2.x, fma(wk[1], a1.x, wk[0] * a0.x)));
+                        const double t1 = fma(wk[3], a3.y, fma(wk[2], a2.y, fma(wk[1], a1.y, wk[0] * a0.y)));
+                        const double t2 = fma(wz5[4], z2.x,
+                                              fma(wz5[3], z1.y, fma(wz5[2], z1.x, fma(wz5[1], z0.y, wz5[0] * z0.x))));
+                        u0 = fma(wys[jj], t0, u0);
+                        u1 = fma(wys[jj], t1, u1);
+                        u2 = fma(wys[jj], t2, u2);
+                    }
+                    s0 = fma(wxs[i], u0, s0);
+                    s1 = fma(wxs[i], u1, s1);
+                    s2 = fma(wxs[i], u2, s2);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) pk[q] += plane;
+                    pz += plane;
+                }
+                Dx = s0;
+                Dy = s1;
+                Dz = s2;
+            } else {
+                t3_interp(a.table, k, dx, dy, dz, Dx, Dy, Dz);
+            }
+            const double px = fma(wp, dx, -Dx), py = fma(wp, dy, -Dy), pz = fma(wp, dz, -Dz);
+            fx = fma(pb.y, px, fx);
+            fy = fma(pb.y, py, fy);
+            fz = fma(pb.y, pz, fz);
+            gx = from_next_lane(fma(mi, px, gx));
+            gy = from_next_lane(fma(mi, py, gy));
+            gz = from_next_lane(fma(mi, pz, gz));
+        }
+        SymWalk nw = w;
+        ++nw.r;
+        have = nw.settle(a, b, ntiles);
+        __syncthreads();  // every wave is done with the window and the records
+        if (off > 0) {
+            const int id = (lane + s0 + kSteps) & 63;  // the source whose sums this lane holds now
+            win[(3 * wave + 0) * kTile + id] = gx;
+            win[(3 * wave + 1) * kTile + id] = gy;
+            win[(3 * wave + 2) * kTile + id] = gz;
+        }
+        if (have && wave == 0) stage(nw.tile);
+        __syncthreads();
+        for (int c = wave; off > 0 && c < 3; c += W) {
+            const int64_t j = (int64_t)tile * kTile + lane;
+            double g = win[c * kTile + lane];
+#pragma unroll
+            for (int v = 1; v < W; ++v) g += win[(3 * v + c) * kTile + lane];
+            if (j < N)
+                a.part[sym_slot(N, cell_l, a.cell_tasks, a.cell_offs, a.cell_tasks + off - cell * a.cell_offs) +
+                       (size_t)c * N + j] = g;
+        }
+        w = nw;
+    }
+    if (G > 1) {
+        // the row sums of the step groups, added in their order
+        __syncthreads();
+        win[(3 * wave + 0) * kTile + lane] = fx;
+        win[(3 * wave + 1) * kTile + lane] = fy;
+        win[(3 * wave + 2) * kTile + lane] = fz;
+        __syncthreads();
+        if (wave >= RW) return;
+#pragma unroll
+        for (int g = 1; g < G; ++g) {
+            fx += win[(3 * (wave + g * RW) + 0) * kTile + lane];
+            fy += win[(3 * (wave + g * RW) + 1) * kTile + lane];
+            fz += win[(3 * (wave + g * RW) + 2) * kTile + lane];
+        }
+    }
+    if (row < N) {
+        double *out = a.part + sym_slot(N, cell_l, a.cell_tasks, a.cell_offs, task);
+        out[row] = fx;
+        out[N + row] = fy;
+        out[2 * N + row] = fz;
+    }
+}
+
 // The slots of one launch onto the running sums: cell by cell, the row sums
 // of its tasks, then its source sums (with the sign of the other side).  The
 // last launch's reduction adds the external term (reduce_kernel's) and writes
@@ -416,6 +715,7 @@ constexpr int kSymNI = 4;
 // Below this many particles the triangle of block pairs leaves too few equal
 // tasks to fill the chip (N = 9000: 0.129 against 0.167 ms).
 constexpr int64_t kSymMinN = 8192;
+constexpr int64_t kSymT3MinN = 1024;  // T3 Ewald (13^3: 0.57 against 2.8 ms)
 // Scratch the slots may take; the offsets go in as many launches as that
 // needs (128 MiB: 4.5 against 4.3 ms at N = 100003, 33.2 against 31.0 ms for
 // the 64^3 nearest image).
@@ -423,7 +723,19 @@ constexpr size_t kSymBytes = (size_t)256 << 20;
 
 bool sym_variant(const EvalPlan &p) {
     return p.precision == STEPS_PREC_FP64 &&
-           (p.variant == PV_R3 || p.variant == PV_T3_NEAREST || p.variant == PV_S1R2_NEAREST);
+           (p.variant == PV_R3 || p.variant == PV_T3_NEAREST || p.variant == PV_S1R2_NEAREST ||
+            (p.variant == PV_T3_EWALD && p.t3_ng <= kT3MaxWinNg));
+}
+
+// Rows of a T3 Ewald workgroup: with c particles per cell column, R rows and
+// a tile span about (R + 64) / c columns in y, and a window of 5 planes holds
+// 98 / 5 = 19 rows of it, 5 + 2 of them the stencil's and the partial columns.
+// Measured (ms, 256 / 128 / 64 rows): 56^3 (c = 44) 443 / 471 / -, 48^3 (28)
+// 216 / 207 / 239, 44^3 (21) 251 / 131 / 150, 40^3 (16) 172 / 86 / 90, 36^3
+// (12) 95 / 92 / 52; 512 rows: 618 against 621 at 60^3, 538 against 443 at 56^3.
+int sym_t3_rows(const EvalPlan &p) {
+    const double c = (double)p.N / ((double)p.t3_ng * p.t3_ng);
+    return 320 <= 12 * c ? 256 : (192 <= 12 * c ? 128 : 64);
 }
 
 struct SymShape {
@@ -451,6 +763,15 @@ size_t sym_acc_bytes(const EvalPlan &p) {
 
 void launch_sym_kernel(const EvalPlan &p, const SymArgs &a, int cells, hipStream_t st) {
     const dim3 grid((unsigned)a.blocks, (unsigned)(cells * a.cell_tasks));
+    if (p.variant == PV_T3_EWALD) {
+        const dim3 block(64 * kT3Waves);
+        switch (p.sym_block_rows) {
+        case 256: hipLaunchKernelGGL(sym_t3_kernel<2>, grid, block, 0, st, a); break;
+        case 128: hipLaunchKernelGGL(sym_t3_kernel<4>, grid, block, 0, st, a); break;
+        default: hipLaunchKernelGGL(sym_t3_kernel<8>, grid, block, 0, st, a); break;
+        }
+        return;
+    }
     switch (p.variant) {
     case PV_R3: hipLaunchKernelGGL((sym_kernel<PV_R3, kSymNI>), grid, dim3(kBlock), 0, st, a); break;
     case PV_T3_NEAREST: hipLaunchKernelGGL((sym_kernel<PV_T3_NEAREST, kSymNI>), grid, dim3(kBlock), 0, st, a); break;
@@ -497,9 +818,9 @@ int sym_last_cell0(const EvalPlan &p) { return (p.sym_cells - 1) / p.sym_launch_
 // kernel nrows N of them.
 void sym_plan(EvalPlan &p) {
     p.sym = false;
-    if (p.bh || p.N < kSymMinN || p.N > INT32_MAX || 3 * p.nrows < 2 * p.N || !sym_variant(p)) return;
+    if (p.bh || p.N < (p.variant == PV_T3_EWALD ? kSymT3MinN : kSymMinN) || p.N > INT32_MAX || 3 * p.nrows < 2 * p.N || !sym_variant(p)) return;
     p.sym = true;
-    p.sym_block_rows = kBlock * kSymNI;
+    p.sym_block_rows = p.variant == PV_T3_EWALD ? sym_t3_rows(p) : kBlock * kSymNI;
     p.sym_blocks = (int)((p.N + p.sym_block_rows - 1) / p.sym_block_rows);
     const int tb = p.sym_block_rows / kTile, offsets = p.sym_blocks / 2 + 1;
     // Tasks of several offsets where there are plenty (fewer row-sum slots),
@@ -527,7 +848,7 @@ bool sym_fit(EvalPlan &p, size_t bytes) {
     return true;
 }
 
-bool sym_selected(const EvalPlan &p) { return p.sym; }
+bool sym_selected(const EvalPlan &p) { return p.sym && (p.variant != PV_T3_EWALD || p.t3_odd); }
 
 hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t st) {
     const SymShape s = sym_shape(p);
@@ -536,6 +857,8 @@ hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t 
     a.soft = b.soft;
     a.tiles = b.tiles;
     a.ext = b.ext;
+    a.table = b.table;
+    a.keys = b.keys;
     a.part = b.part;
     a.k = make_scalars(p);
     a.blocks = p.sym_blocks;

@@ -64,6 +64,31 @@ def test_against_oracle(steps, oracle, mode, N):
     assert np.median(rel_err(few, F[:N // 2 + 1])) <= 1e-12
 
 
+@pytest.mark.parametrize("N", [1024, 1087, 3000, 40001, 66000, 107001])
+def test_t3_ewald_against_oracle(steps, oracle, N):
+    """Every rows-per-workgroup choice of the T3 Ewald kernel (64, 128, 256
+    by particles per table column), windows that fit and that do not, ragged
+    ends, close pairs; and a table that is not odd through its centre, which
+    has to take the one-sided kernel."""
+    print(f"case pair-symmetric t3 ewald N={N}", flush=True)
+    x, M, h, L = particles("t3", N, N)
+    T = steps.t3_table(2, L)
+    rows = np.unique(np.concatenate([np.arange(0, 12), np.arange(N - 12, N),
+                                     np.linspace(0, N - 1, 24).astype(int)])).astype(np.int32)
+    bent = T.reshape(63, 63, 63, 3).copy()
+    bent[:, :, 40:, 2] *= 1.25                            # even in x and y still, not odd in z
+    for label, tab in (("odd", T), ("bent", bent.reshape(-1))):
+        if label == "bent" and N > 3000:
+            continue
+        d, keep = steps.make_desc(steps.TOPO_T3, is_periodic=2, L=L, t3_table=tab)
+        F = steps.force_eval(d, x, M, h)
+        p = oracle.params(1, is_periodic=2, L=L, t3_table=tab, interp_order=4)
+        e = rel_err(F[rows], oracle.forces_rows(p, x, M, h, rows))
+        report(f"pair-symmetric t3 ewald {label} N={N}", e)
+        assert np.all(np.isfinite(F)) and np.median(e) <= 1e-12 and e.max() <= 1e-9
+        assert np.array_equal(steps.force_eval(d, x, M, h), F)
+
+
 @pytest.mark.parametrize("N", [150001, 300000])
 def test_scratch_does_not_change_the_sums(steps, N):
     """The entry point with 256 MiB of static scratch runs fewer offsets a
