@@ -114,6 +114,7 @@ struct SymBuffers {
     const double *soft;
     const double4 *tiles, *ext;
     const double *table;
+    const float4 *tab32;   // FP32 T3 table (mixed precision)
     const uint32_t *keys;
     const uint32_t *perm;  // sorted -> input row, or null
     const double4 *jrec;   // input records (external term)

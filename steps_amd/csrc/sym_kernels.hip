@@ -39,6 +39,7 @@
 #include "pair_device.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace steps {
 
@@ -52,6 +53,7 @@ struct SymArgs {
     const double4 *tiles;  // per 64 records: bounding-box centre, largest softening length
     const double4 *ext;    // half extents
     const double *table;   // T3 Ewald table, device layout
+    const float4 *tab32;   // ... its FP32 copy, 16-byte nodes (mixed precision)
     const uint32_t *keys;  // pencil keys of the records (T3 Ewald)
     double *part;
     KScalars k;
@@ -74,6 +76,13 @@ __device__ __forceinline__ double from_next_lane(double v) {
     u.i[0] = __builtin_amdgcn_update_dpp(u.i[0], u.i[0], 0x134, 0xf, 0xf, false);
     u.i[1] = __builtin_amdgcn_update_dpp(u.i[1], u.i[1], 0x134, 0xf, 0xf, false);
     return u.d;
+}
+
+__device__ __forceinline__ float from_next_lane(float v) {
+    union { float f; int i; } u;
+    u.f = v;
+    u.i = __builtin_amdgcn_update_dpp(u.i, u.i, 0x134, 0xf, 0xf, false);
+    return u.f;
 }
 
 // Walks the tiles of a task: relative tile r counts from the block's own
@@ -382,13 +391,18 @@ constexpr int kSymT3Win = 9800;   // 16-byte words: 153 KB, one workgroup per CU
 constexpr int kT3Waves = 8;
 constexpr int kT3MaxWinNg = 63;   // the window row is laid out for tables up to this grid
 constexpr int kT3Row = 100;       // words a window row: 66 (x, y) nodes and 34 z pairs
+constexpr int kT3Row32 = 68;      // ... of FP32 nodes, one word each
 constexpr int kT3RunOff[4] = {0, 17, 34, 50};  // (x, y) nodes by z mod 4: start of each run
 constexpr int kT3ZPairs = 66;     // start of the z components, two nodes a word
+
+__device__ __forceinline__ unsigned t3_run_start(unsigned r) {
+    return r == 0u ? kT3RunOff[0] : (r == 1u ? kT3RunOff[1] : (r == 2u ? kT3RunOff[2] : kT3RunOff[3]));
+}
 
 // Words from one x plane of window rows to the next: 8 (mod 16), which with
 // rows 4 (mod 16) apart spreads the 2 x 2 neighbouring rows that the lanes
 // of a read mostly sit on over different banks.
-__device__ __forceinline__ int t3_plane(int ny) { return ny * kT3Row + ((8 - ny * kT3Row) & 15); }
+__device__ __forceinline__ int t3_plane(int ny, int row) { return ny * row + ((8 - ny * row) & 15); }
 
 // Unfolded nodes one axis of the window holds: n0 .. n0 + n - 1 (mod Ng), n0
 // in [0, Ng), for sources in cell columns [smin, smax] and rows in [bmin,
@@ -408,7 +422,7 @@ __device__ __forceinline__ bool t3_win_rel(int i, int n0, int n, int Ng, unsigne
     return (int)rel <= n - 4 && (int)rel >= 0;
 }
 
-// Catmull-Rom weights of one axis (t3_axis without the index wrap).
+// Catmull-Rom weights of one axis (t3_axis, t3_axis_f32 without the index wrap).
 __device__ __forceinline__ int t3_weights(double d, const KScalars &k, double w[4]) {
     const double u = (d + k.L * 0.5) * k.inv_gs - 0.5;
     const double uf = floor(u);
@@ -420,11 +434,24 @@ __device__ __forceinline__ int t3_weights(double d, const KScalars &k, double w[
     w[3] = 0.5 * t3 - 0.5 * t2;
     return (int)uf;
 }
+__device__ __forceinline__ int t3_weights(float d, const KScalars &k, float w[4]) {
+    const float u = (d + k.halfLf) * k.inv_gsf - 0.5f;
+    const float uf = floorf(u);
+    const float t = u - uf;
+    const float t2 = t * t, t3 = t * t2;
+    w[0] = -0.5f * t3 + t2 - 0.5f * t;
+    w[1] = 1.5f * t3 - 2.5f * t2 + 1.0f;
+    w[2] = -1.5f * t3 + 2.0f * t2 + 0.5f * t;
+    w[3] = 0.5f * t3 - 0.5f * t2;
+    return (int)uf;
+}
 
-template <int G>
+template <int G, bool MX>
 __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) {
     constexpr int W = kT3Waves, RW = W / G;  // waves; waves of different rows
     constexpr int kSteps = kTile / G;
+    constexpr int kRow = MX ? kT3Row32 : kT3Row;
+    using real = std::conditional_t<MX, float, double>;
     __shared__ __align__(16) double win[2 * kSymT3Win];
     __shared__ __align__(16) double2 jbuf[2][kTile];
     __shared__ int brange[4];
@@ -498,7 +525,7 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
             wy0 = __builtin_amdgcn_readfirstlane(wy0);
             nx = __builtin_amdgcn_readfirstlane(nx);
             ny = __builtin_amdgcn_readfirstlane(ny);
-            plane = t3_plane(ny);
+            plane = t3_plane(ny, kRow);
             wok = nx <= Ng && ny <= Ng && nx * plane <= kSymT3Win;
             if (wok) {
                 // a wave copies whole rows (lanes along the z run), unfolding
@@ -511,39 +538,64 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                     const bool fx_ = jx < lo, fy_ = jy < lo;
                     const unsigned mx = (unsigned)(fx_ ? Ng - 1 - lo - jx : jx - lo);
                     const unsigned my = (unsigned)(fy_ ? Ng - 1 - lo - jy : jy - lo);
-                    const double *src = a.table + (mx * NY + my) * NZ3;
-                    double *dst = win + 2 * (ax * plane + ay * kT3Row);
-                    for (unsigned o = lane; o < 2u * kT3Row; o += 64) {
-                        if (o < NZ3) {
+                    if constexpr (MX) {
+                        const float4 *src = a.tab32 + (mx * NY + my) * NZ;
+                        float4 *dst = (float4 *)win + ax * plane + ay * kRow;
+                        for (unsigned z = lane; z < NZ; z += 64) {
+                            float4 v = src[z];
+                            if (fx_) v.x = -v.x;
+                            if (fy_) v.y = -v.y;
+                            dst[t3_run_start(z & 3u) + (z >> 2)] = v;
+                        }
+                    } else {
+                        const double *src = a.table + (mx * NY + my) * NZ3;
+                        double *dst = win + 2 * (ax * plane + ay * kRow);
+                        for (unsigned o = lane; o < NZ3; o += 64) {
                             const unsigned z = o / 3u, c = o - 3u * z;
                             double v = src[o];
                             if (c == 0u && fx_) v = -v;
                             if (c == 1u && fy_) v = -v;
-                            const unsigned run = z & 3u;
-                            const unsigned start = run == 0u ? 0u : (run == 1u ? 17u : (run == 2u ? 34u : 50u));
-                            dst[c < 2u ? 2u * (start + (z >> 2)) + c : 2u * kT3ZPairs + z] = v;
+                            dst[c < 2u ? 2u * (t3_run_start(z & 3u) + (z >> 2)) + c : 2u * kT3ZPairs + z] = v;
                         }
+                        // z values past the run meet zero weights
+                        const unsigned pad = 2u * kT3ZPairs + NZ + lane;
+                        if (pad < 2u * kRow) dst[pad] = 0.0;
                     }
-                    // z values past the run meet zero weights
-                    const unsigned pad = 2u * kT3ZPairs + NZ + lane;
-                    if (pad < 2u * kT3Row) dst[pad] = 0.0;
                 }
             }
             __syncthreads();  // the window is complete
         }
         const double bb = hi + a.tiles[tile].w;
         const double B = bb * bb;
-        double gx = 0.0, gy = 0.0, gz = 0.0;
+        // mixed: the FP32 bound, widened so that rounding cannot hide a pair
+        const float Bf = (float)(bb * (1.0 + 1e-5)) * (float)(bb * (1.0 + 1e-5));
+        real gx = 0, gy = 0, gz = 0, ax = 0, ay = 0, az = 0;
+        bool near = false;
 #pragma unroll 1
         for (int s = 0; s < kSteps; ++s) {
             const int id = (lane + s0 + s) & 63;
             const double2 pa = jbuf[0][id], pb = jbuf[1][id];
-            const double dx = wrap_half(pa.x - xi, k), dy = wrap_half(pa.y - yi, k), dz = wrap_half(pb.x - zi, k);
-            const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-            const double wp = pair_w_tile(r2, B, hi, a.soft, min((int64_t)tile * kTile + id, N - 1), k);
-            double Dx, Dy, Dz;
+            // the displacement is formed and wrapped in FP64 (mixed: then rounded once)
+            const real dx = (real)wrap_half(pa.x - xi, k), dy = (real)wrap_half(pa.y - yi, k),
+                       dz = (real)wrap_half(pb.x - zi, k);
+            real wp, mj, mr;
+            if constexpr (MX) {
+                const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                const bool nr = r2 < Bf;  // left to the FP64 redo (r2 may be 0 here)
+                near = near || nr;
+                const float y = __builtin_amdgcn_rsqf(r2);
+                wp = nr ? 0.0f : (y * y) * y;
+                mj = nr ? 0.0f : (float)pb.y;
+                mr = nr ? 0.0f : (float)mi;
+            } else {
+                const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+                wp = pair_w_tile(r2, B, hi, a.soft, min((int64_t)tile * kTile + id, N - 1), k);
+                mj = pb.y;
+                mr = mi;
+            }
+            real Dx, Dy, Dz;
             bool in = false;
-            double wxs[4], wys[4], wzs[4];
+            real wxs[4], wys[4], wzs[4];
             unsigned rx = 0, ry = 0, iz = 0;
             if (wok) {
                 const int ix = t3_weights(dx, k, wxs), iy = t3_weights(dy, k, wys), izi = t3_weights(dz, k, wzs);
@@ -556,53 +608,133 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                 // z = k (mod 4), so lanes a few nodes apart read the same word
                 // or neighbouring ones
                 const unsigned r = iz & 3u, blk = iz >> 2;
-                double v0 = wzs[0], v1 = wzs[1], v2 = wzs[2], v3 = wzs[3];
                 const bool r1 = (r & 1u) != 0u, r2b = (r & 2u) != 0u;
-                const double p0 = r1 ? v3 : v0, p1 = r1 ? v0 : v1, p2 = r1 ? v1 : v2, p3 = r1 ? v2 : v3;
-                const double wk[4] = {r2b ? p2 : p0, r2b ? p3 : p1, r2b ? p0 : p2, r2b ? p1 : p3};
-                const double wz5[5] = {r1 ? 0.0 : v0, r1 ? v0 : v1, r1 ? v1 : v2, r1 ? v2 : v3, r1 ? v3 : 0.0};
-                const unsigned base = rx * (unsigned)plane + ry * (unsigned)kT3Row;
-                const double2 *w2 = (const double2 *)win;
-                const double2 *pk[4], *pz = w2 + base + kT3ZPairs + (iz >> 1);
+                const real p0 = r1 ? wzs[3] : wzs[0], p1 = r1 ? wzs[0] : wzs[1], p2 = r1 ? wzs[1] : wzs[2],
+                           p3 = r1 ? wzs[2] : wzs[3];
+                const real wk[4] = {r2b ? p2 : p0, r2b ? p3 : p1, r2b ? p0 : p2, r2b ? p1 : p3};
+                const unsigned base = rx * (unsigned)plane + ry * (unsigned)kRow;
+                unsigned at[4];
 #pragma unroll
-                for (unsigned q = 0; q < 4; ++q) pk[q] = w2 + base + kT3RunOff[q] + blk + (q < r ? 1u : 0u);
-                double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+                for (unsigned q = 0; q < 4; ++q) at[q] = base + kT3RunOff[q] + blk + (q < r ? 1u : 0u);
+                real s0 = 0, s1 = 0, s2 = 0;
+                if constexpr (MX) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    double u0 = 0.0, u1 = 0.0, u2 = 0.0;
+                    for (int i = 0; i < 4; ++i) {
+                        const float4 *pk[4];
 #pragma unroll
-                    for (int jj = 0; jj < 4; ++jj) {
-                        const double2 a0 = pk[0][jj * kT3Row], a1 = pk[1][jj * kT3Row], a2 = pk[2][jj * kT3Row],
-                                      a3 = pk[3][jj * kT3Row];
-                        const double2 z0 = pz[jj * kT3Row], z1 = pz[jj * kT3Row + 1], z2 = pz[jj * kT3Row + 2];
-                        const double t0 = fma(wk[3], a3.x, fma(wk[2], a2.x, fma(wk[1], a1.x, wk[0] * a0.x)));
-                        const double t1 = fma(wk[3], a3.y, fma(wk[2], a2.y, fma(wk[1], a1.y, wk[0] * a0.y)));
-                        const double t2 = fma(wz5[4], z2.x,
-                                              fma(wz5[3], z1.y, fma(wz5[2], z1.x, fma(wz5[1], z0.y, wz5[0] * z0.x))));
-                        u0 = fma(wys[jj], t0, u0);
-                        u1 = fma(wys[jj], t1, u1);
-                        u2 = fma(wys[jj], t2, u2);
+                        for (int q = 0; q < 4; ++q) pk[q] = (const float4 *)win + at[q] + i * plane;
+                        float u0 = 0.0f, u1 = 0.0f, u2 = 0.0f;
+#pragma unroll
+                        for (int jj = 0; jj < 4; ++jj) {
+                            const float4 a0 = pk[0][jj * kRow], a1 = pk[1][jj * kRow], a2 = pk[2][jj * kRow],
+                                         a3 = pk[3][jj * kRow];
+                            // the unused fourth component keeps the reads 16 bytes wide:
+                            // a 12-byte LDS read takes twice the cycles (8 against 4.3)
+                            asm volatile("" ::"v"(a0.w), "v"(a1.w), "v"(a2.w), "v"(a3.w));
+                            const float t0 = fmaf(wk[3], a3.x, fmaf(wk[2], a2.x, fmaf(wk[1], a1.x, wk[0] * a0.x)));
+                            const float t1 = fmaf(wk[3], a3.y, fmaf(wk[2], a2.y, fmaf(wk[1], a1.y, wk[0] * a0.y)));
+                            const float t2 = fmaf(wk[3], a3.z, fmaf(wk[2], a2.z, fmaf(wk[1], a1.z, wk[0] * a0.z)));
+                            u0 = fmaf(wys[jj], t0, u0);
+                            u1 = fmaf(wys[jj], t1, u1);
+                            u2 = fmaf(wys[jj], t2, u2);
+                        }
+                        s0 = fmaf(wxs[i], u0, s0);
+                        s1 = fmaf(wxs[i], u1, s1);
+                        s2 = fmaf(wxs[i], u2, s2);
                     }
-                    s0 = fma(wxs[i], u0, s0);
-                    s1 = fma(wxs[i], u1, s1);
-                    s2 = fma(wxs[i], u2, s2);
+                } else {
+                    // z components: six nodes from the even start as three words, the extra two with weight 0
+                    const double wz5[5] = {r1 ? 0.0 : wzs[0], r1 ? wzs[0] : wzs[1], r1 ? wzs[1] : wzs[2],
+                                           r1 ? wzs[2] : wzs[3], r1 ? wzs[3] : 0.0};
+                    const double2 *w2 = (const double2 *)win;
+                    const unsigned zat = base + kT3ZPairs + (iz >> 1);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) pk[q] += plane;
-                    pz += plane;
+                    for (int i = 0; i < 4; ++i) {
+                        const double2 *pk[4], *pz = w2 + zat + i * plane;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) pk[q] = w2 + at[q] + i * plane;
+                        double u0 = 0.0, u1 = 0.0, u2 = 0.0;
+#pragma unroll
+                        for (int jj = 0; jj < 4; ++jj) {
+                            const double2 a0 = pk[0][jj * kRow], a1 = pk[1][jj * kRow], a2 = pk[2][jj * kRow],
+                                          a3 = pk[3][jj * kRow];
+                            const double2 z0 = pz[jj * kRow], z1 = pz[jj * kRow + 1], z2 = pz[jj * kRow + 2];
+                            const double t0 = fma(wk[3], a3.x, fma(wk[2], a2.x, fma(wk[1], a1.x, wk[0] * a0.x)));
+                            const double t1 = fma(wk[3], a3.y, fma(wk[2], a2.y, fma(wk[1], a1.y, wk[0] * a0.y)));
+                            const double t2 = fma(wz5[4], z2.x,
+                                                  fma(wz5[3], z1.y, fma(wz5[2], z1.x, fma(wz5[1], z0.y, wz5[0] * z0.x))));
+                            u0 = fma(wys[jj], t0, u0);
+                            u1 = fma(wys[jj], t1, u1);
+                            u2 = fma(wys[jj], t2, u2);
+                        }
+                        s0 = fma(wxs[i], u0, s0);
+                        s1 = fma(wxs[i], u1, s1);
+                        s2 = fma(wxs[i], u2, s2);
+                    }
                 }
                 Dx = s0;
                 Dy = s1;
                 Dz = s2;
+            } else if constexpr (MX) {
+                T3Stencil32 st;
+                t3_stencil_f32(k, dx, dy, dz, st);
+                t3_contract_f32(
+                    st,
+                    [&](int i, int jj, float4 *n) {
+                        const float4 *g = a.tab32 + (st.mx[i] * NY + st.my[jj]) * NZ + (unsigned)st.iz0;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) n[q] = g[q];
+                    },
+                    Dx, Dy, Dz);
             } else {
                 t3_interp(a.table, k, dx, dy, dz, Dx, Dy, Dz);
             }
-            const double px = fma(wp, dx, -Dx), py = fma(wp, dy, -Dy), pz = fma(wp, dz, -Dz);
-            fx = fma(pb.y, px, fx);
-            fy = fma(pb.y, py, fy);
-            fz = fma(pb.y, pz, fz);
-            gx = from_next_lane(fma(mi, px, gx));
-            gy = from_next_lane(fma(mi, py, gy));
-            gz = from_next_lane(fma(mi, pz, gz));
+            auto mad = [](real m, real v, real acc) {
+                if constexpr (MX) return fmaf(m, v, acc);
+                else return fma(m, v, acc);
+            };
+            const real px = mad(wp, dx, -Dx), py = mad(wp, dy, -Dy), pz = mad(wp, dz, -Dz);
+            ax = mad(mj, px, ax);
+            ay = mad(mj, py, ay);
+            az = mad(mj, pz, az);
+            gx = from_next_lane(mad(mr, px, gx));
+            gy = from_next_lane(mad(mr, py, gy));
+            gz = from_next_lane(mad(mr, pz, gz));
+        }
+        // the tile's sums (mixed: FP32 over at most 64 pairs) onto the FP64 ones
+        fx += (double)ax;
+        fy += (double)ay;
+        fz += (double)az;
+        double hx = (double)gx, hy = (double)gy, hz = (double)gz;
+        if (MX && __any(near)) {
+            // rare: the pairs within the bound, in FP64 with the FP64 table
+            double cx = 0.0, cy = 0.0, cz = 0.0;
+#pragma unroll 1
+            for (int s = 0; s < kSteps; ++s) {
+                const int id = (lane + s0 + s) & 63;
+                const double2 pa = jbuf[0][id], pb = jbuf[1][id];
+                const double ex = wrap_half(pa.x - xi, k), ey = wrap_half(pa.y - yi, k), ez = wrap_half(pb.x - zi, k);
+                const float dx = (float)ex, dy = (float)ey, dz = (float)ez;
+                if (fmaf(dx, dx, fmaf(dy, dy, dz * dz)) < Bf) {
+                    const double r2 = fma(ex, ex, fma(ey, ey, ez * ez));
+                    const double wp = pair_w_tile(r2, B, hi, a.soft, min((int64_t)tile * kTile + id, N - 1), k);
+                    double Dx, Dy, Dz;
+                    t3_interp(a.table, k, ex, ey, ez, Dx, Dy, Dz);
+                    const double px = fma(wp, ex, -Dx), py = fma(wp, ey, -Dy), pz = fma(wp, ez, -Dz);
+                    fx = fma(pb.y, px, fx);
+                    fy = fma(pb.y, py, fy);
+                    fz = fma(pb.y, pz, fz);
+                    cx = fma(mi, px, cx);
+                    cy = fma(mi, py, cy);
+                    cz = fma(mi, pz, cz);
+                }
+                cx = from_next_lane(cx);
+                cy = from_next_lane(cy);
+                cz = from_next_lane(cz);
+            }
+            hx += cx;
+            hy += cy;
+            hz += cz;
         }
         SymWalk nw = w;
         ++nw.r;
@@ -610,9 +742,9 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
         __syncthreads();  // every wave is done with the window and the records
         if (off > 0) {
             const int id = (lane + s0 + kSteps) & 63;  // the source whose sums this lane holds now
-            win[(3 * wave + 0) * kTile + id] = gx;
-            win[(3 * wave + 1) * kTile + id] = gy;
-            win[(3 * wave + 2) * kTile + id] = gz;
+            win[(3 * wave + 0) * kTile + id] = hx;
+            win[(3 * wave + 1) * kTile + id] = hy;
+            win[(3 * wave + 2) * kTile + id] = hz;
         }
         if (have && wave == 0) stage(nw.tile);
         __syncthreads();
@@ -722,9 +854,9 @@ constexpr int64_t kSymT3MinN = 1024;  // T3 Ewald (13^3: 0.57 against 2.8 ms)
 constexpr size_t kSymBytes = (size_t)256 << 20;
 
 bool sym_variant(const EvalPlan &p) {
+    if (p.variant == PV_T3_EWALD) return p.t3_ng <= kT3MaxWinNg;  // either precision
     return p.precision == STEPS_PREC_FP64 &&
-           (p.variant == PV_R3 || p.variant == PV_T3_NEAREST || p.variant == PV_S1R2_NEAREST ||
-            (p.variant == PV_T3_EWALD && p.t3_ng <= kT3MaxWinNg));
+           (p.variant == PV_R3 || p.variant == PV_T3_NEAREST || p.variant == PV_S1R2_NEAREST);
 }
 
 // Rows of a T3 Ewald workgroup: with c particles per cell column, R rows and
@@ -735,7 +867,10 @@ bool sym_variant(const EvalPlan &p) {
 // (12) 95 / 92 / 52; 512 rows: 618 against 621 at 60^3, 538 against 443 at 56^3.
 int sym_t3_rows(const EvalPlan &p) {
     const double c = (double)p.N / ((double)p.t3_ng * p.t3_ng);
-    return 320 <= 12 * c ? 256 : (192 <= 12 * c ? 128 : 64);
+    // FP32 nodes: 144 rows of one word a node, 28 in y
+    const double span = p.precision == STEPS_PREC_MIXED ? 20 : 12;
+    const double t = getenv("T3S") ? atof(getenv("T3S")) : span;
+    return 320 <= t * c ? 256 : (192 <= t * c ? 128 : 64);
 }
 
 struct SymShape {
@@ -765,10 +900,17 @@ void launch_sym_kernel(const EvalPlan &p, const SymArgs &a, int cells, hipStream
     const dim3 grid((unsigned)a.blocks, (unsigned)(cells * a.cell_tasks));
     if (p.variant == PV_T3_EWALD) {
         const dim3 block(64 * kT3Waves);
-        switch (p.sym_block_rows) {
-        case 256: hipLaunchKernelGGL(sym_t3_kernel<2>, grid, block, 0, st, a); break;
-        case 128: hipLaunchKernelGGL(sym_t3_kernel<4>, grid, block, 0, st, a); break;
-        default: hipLaunchKernelGGL(sym_t3_kernel<8>, grid, block, 0, st, a); break;
+        const bool mx = p.precision == STEPS_PREC_MIXED;
+        const int rows = p.sym_block_rows;
+        if (rows == 256) {
+            if (mx) hipLaunchKernelGGL((sym_t3_kernel<2, true>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((sym_t3_kernel<2, false>), grid, block, 0, st, a);
+        } else if (rows == 128) {
+            if (mx) hipLaunchKernelGGL((sym_t3_kernel<4, true>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((sym_t3_kernel<4, false>), grid, block, 0, st, a);
+        } else {
+            if (mx) hipLaunchKernelGGL((sym_t3_kernel<8, true>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((sym_t3_kernel<8, false>), grid, block, 0, st, a);
         }
         return;
     }
@@ -859,6 +1001,7 @@ hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t 
     a.ext = b.ext;
     a.table = b.table;
     a.keys = b.keys;
+    a.tab32 = b.tab32;
     a.part = b.part;
     a.k = make_scalars(p);
     a.blocks = p.sym_blocks;
