@@ -370,8 +370,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // columns can reach into LDS, unfolded, so that a stencil is 16 rows at fixed
 // strides from one address: no mirror or wrap per row (638 -> 468 VALU per
 // pair against the folded window of body_t3_win).  A window that does not fit
-// leaves the tile on the global table, and so does a lane whose stencil
-// leaves the window.  The eight waves of a workgroup are W / G sets of 64
+// is taken in up to three bands of y rows, each its own pass over the steps in
+// which the lanes whose stencils lie in the band take part (32^3 46 -> 34 ms;
+// more bands gain nothing); a wider one leaves the tile on the global table,
+// and so does a lane whose stencil leaves the window.  The eight waves of a workgroup are W / G sets of 64
 // rows times G groups of 64 / G steps: fewer rows make a smaller window, so
 // sparse boxes (few particles per column) take G = 4 or 8.  After the tile
 // the window's memory takes the waves' source sums.
@@ -384,11 +386,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // words) and rows 4, planes 8 words apart mod 16.  Measured at 60^3: folded
 // body_t3_win rows 737 ms, this layout 615; planes at 4 or 2 mod 16 695 / 652,
 // rows of 104 or 108 words 630 / 633, z components as single 8-byte reads 710.
-// Measured against the one-sided kernels (ms): 24^3 22.8 -> 9.7, 40^3 310 ->
-// 86, 48^3 739 -> 206, 56^3 1440 -> 443, 64^3 2000 -> 850.
+// Measured against the one-sided kernels (ms): 24^3 22.8 -> 9.7, 32^3 91 -> 34,
+// 40^3 310 -> 80, 48^3 739 -> 194, 56^3 1440 -> 443, 64^3 2000 -> 850.
+//
+// MX, mixed precision: the displacement is formed and wrapped in FP64 and
+// rounded once, the rest of a pair is FP32, with 16-byte nodes (64 reads a
+// pair); FP32 sums run over one wave's steps of a tile and are added in FP64,
+// pairs within the softening bound are done again in FP64 (body_t3_mixed's
+// scheme).  VALU (420 per pair) and LDS (490 cycles) are about even there:
+// 24^3 14.6 -> 5.0 ms, 40^3 190 -> 42, 48^3 490 -> 103, 56^3 1092 -> 235.
 // ---------------------------------------------------------------------------
 constexpr int kSymT3Win = 9800;   // 16-byte words: 153 KB, one workgroup per CU
 constexpr int kT3Waves = 8;
+constexpr int kT3Bands = 3;       // most bands of a window (see sym_t3_kernel)
 constexpr int kT3MaxWinNg = 63;   // the window row is laid out for tables up to this grid
 constexpr int kT3Row = 100;       // words a window row: 66 (x, y) nodes and 34 z pairs
 constexpr int kT3Row32 = 68;      // ... of FP32 nodes, one word each
@@ -507,8 +517,9 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
     while (have) {
         const int tile = w.tile, off = w.off;
         __syncthreads();  // records in place; the window's memory is free
-        bool wok = false;
-        int wx0 = 0, nx = 0, wy0 = 0, ny = 0, plane = 0;
+        // The window's nodes, in bands of bys + 3 y rows that fit LDS: band b
+        // serves the stencils that start at y rows [b bys, (b + 1) bys).
+        int wx0 = 0, nx = 0, wy0 = 0, ny = 0, bys = 0, bands = 0;
         {
             const uint32_t kj = a.keys[min((int64_t)tile * kTile + lane, N - 1)];
             int sx0 = (int)(kj >> 20), sx1 = sx0, sy0 = pencil_y(kj, Ng), sy1 = sy0;
@@ -525,16 +536,28 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
             wy0 = __builtin_amdgcn_readfirstlane(wy0);
             nx = __builtin_amdgcn_readfirstlane(nx);
             ny = __builtin_amdgcn_readfirstlane(ny);
-            plane = t3_plane(ny, kRow);
-            wok = nx <= Ng && ny <= Ng && nx * plane <= kSymT3Win;
-            if (wok) {
+            bys = min(ny, (kSymT3Win / nx - 12) / kRow) - 3;  // 12: the most t3_plane adds
+            bands = bys > 0 ? (ny - 3 + bys - 1) / bys : INT32_MAX;
+            if (bands > kT3Bands) bands = 0;  // the global table
+        }
+        const double bb = hi + a.tiles[tile].w;
+        const double B = bb * bb;
+        // mixed: the FP32 bound, widened so that rounding cannot hide a pair
+        const float Bf = (float)(bb * (1.0 + 1e-5)) * (float)(bb * (1.0 + 1e-5));
+        double hx = 0.0, hy = 0.0, hz = 0.0;
+        bool near = false;
+        for (int band = 0; band == 0 || band < bands; ++band) {
+            if (band > 0) __syncthreads();  // every wave is done with the previous band
+            const int y0 = band * bys, nyb = min(bys + 3, ny - y0);
+            const int plane = t3_plane(nyb, kRow);
+            if (bands > 0) {
                 // a wave copies whole rows (lanes along the z run), unfolding
                 // them: a node below lo is its mirror with that component negated
-                for (int rw = wave; rw < nx * ny; rw += W) {
-                    const int ax = rw / ny, ay = rw - ax * ny;
-                    int jx = wx0 + ax, jy = wy0 + ay;
-                    if (jx >= Ng) jx -= Ng;
-                    if (jy >= Ng) jy -= Ng;
+                for (int rw = wave; rw < nx * nyb; rw += W) {
+                    const int ax = rw / nyb, ay = rw - ax * nyb;
+                    int jx = wx0 + ax, jy = wy0 + y0 + ay;
+                    while (jx >= Ng) jx -= Ng;
+                    while (jy >= Ng) jy -= Ng;
                     const bool fx_ = jx < lo, fy_ = jy < lo;
                     const unsigned mx = (unsigned)(fx_ ? Ng - 1 - lo - jx : jx - lo);
                     const unsigned my = (unsigned)(fy_ ? Ng - 1 - lo - jy : jy - lo);
@@ -564,148 +587,153 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                 }
             }
             __syncthreads();  // the window is complete
-        }
-        const double bb = hi + a.tiles[tile].w;
-        const double B = bb * bb;
-        // mixed: the FP32 bound, widened so that rounding cannot hide a pair
-        const float Bf = (float)(bb * (1.0 + 1e-5)) * (float)(bb * (1.0 + 1e-5));
-        real gx = 0, gy = 0, gz = 0, ax = 0, ay = 0, az = 0;
-        bool near = false;
+            real gx = 0, gy = 0, gz = 0, ax = 0, ay = 0, az = 0;
 #pragma unroll 1
-        for (int s = 0; s < kSteps; ++s) {
-            const int id = (lane + s0 + s) & 63;
-            const double2 pa = jbuf[0][id], pb = jbuf[1][id];
-            // the displacement is formed and wrapped in FP64 (mixed: then rounded once)
-            const real dx = (real)wrap_half(pa.x - xi, k), dy = (real)wrap_half(pa.y - yi, k),
-                       dz = (real)wrap_half(pb.x - zi, k);
-            real wp, mj, mr;
-            if constexpr (MX) {
-                const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                const bool nr = r2 < Bf;  // left to the FP64 redo (r2 may be 0 here)
-                near = near || nr;
-                const float y = __builtin_amdgcn_rsqf(r2);
-                wp = nr ? 0.0f : (y * y) * y;
-                mj = nr ? 0.0f : (float)pb.y;
-                mr = nr ? 0.0f : (float)mi;
-            } else {
-                const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-                wp = pair_w_tile(r2, B, hi, a.soft, min((int64_t)tile * kTile + id, N - 1), k);
-                mj = pb.y;
-                mr = mi;
-            }
-            real Dx, Dy, Dz;
-            bool in = false;
-            real wxs[4], wys[4], wzs[4];
-            unsigned rx = 0, ry = 0, iz = 0;
-            if (wok) {
-                const int ix = t3_weights(dx, k, wxs), iy = t3_weights(dy, k, wys), izi = t3_weights(dz, k, wzs);
-                iz = min((unsigned)izi, (unsigned)(izi + Ng));  // layout z index of the stencil's first node
-                const bool inx = t3_win_rel(ix, wx0, nx, Ng, rx), iny = t3_win_rel(iy, wy0, ny, Ng, ry);
-                in = inx && iny && iz < (unsigned)Ng;
-            }
-            if (in) {
-                // (x, y) nodes by z mod 4: read k takes the stencil's node with
-                // z = k (mod 4), so lanes a few nodes apart read the same word
-                // or neighbouring ones
-                const unsigned r = iz & 3u, blk = iz >> 2;
-                const bool r1 = (r & 1u) != 0u, r2b = (r & 2u) != 0u;
-                const real p0 = r1 ? wzs[3] : wzs[0], p1 = r1 ? wzs[0] : wzs[1], p2 = r1 ? wzs[1] : wzs[2],
-                           p3 = r1 ? wzs[2] : wzs[3];
-                const real wk[4] = {r2b ? p2 : p0, r2b ? p3 : p1, r2b ? p0 : p2, r2b ? p1 : p3};
-                const unsigned base = rx * (unsigned)plane + ry * (unsigned)kRow;
-                unsigned at[4];
-#pragma unroll
-                for (unsigned q = 0; q < 4; ++q) at[q] = base + kT3RunOff[q] + blk + (q < r ? 1u : 0u);
-                real s0 = 0, s1 = 0, s2 = 0;
+            for (int s = 0; s < kSteps; ++s) {
+                const int id = (lane + s0 + s) & 63;
+                const double2 pa = jbuf[0][id], pb = jbuf[1][id];
+                // the displacement is formed and wrapped in FP64 (mixed: then rounded once)
+                const real dx = (real)wrap_half(pa.x - xi, k), dy = (real)wrap_half(pa.y - yi, k),
+                           dz = (real)wrap_half(pb.x - zi, k);
+                // the band that holds this pair's stencil: its share of the pair is
+                // the correction, and band 0 also has the direct force (and, from
+                // the global table, the corrections of stencils no band holds)
+                real wxs[4], wys[4], wzs[4];
+                unsigned rx = 0, ry = 0, iz = 0;
+                bool in = false, out = band == 0;
+                if (bands > 0) {
+                    const int ix = t3_weights(dx, k, wxs), iy = t3_weights(dy, k, wys), izi = t3_weights(dz, k, wzs);
+                    iz = min((unsigned)izi, (unsigned)(izi + Ng));  // layout z index of the stencil's first node
+                    const bool inx = t3_win_rel(ix, wx0, nx, Ng, rx), iny = t3_win_rel(iy, wy0, ny, Ng, ry);
+                    const bool held = inx && iny && iz < (unsigned)Ng;
+                    ry -= (unsigned)y0;
+                    in = held && ry < (unsigned)bys;
+                    out = band == 0 && !held;
+                }
+                real wp = 0, mj, mr;
                 if constexpr (MX) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float4 *pk[4];
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) pk[q] = (const float4 *)win + at[q] + i * plane;
-                        float u0 = 0.0f, u1 = 0.0f, u2 = 0.0f;
-#pragma unroll
-                        for (int jj = 0; jj < 4; ++jj) {
-                            const float4 a0 = pk[0][jj * kRow], a1 = pk[1][jj * kRow], a2 = pk[2][jj * kRow],
-                                         a3 = pk[3][jj * kRow];
-                            // the unused fourth component keeps the reads 16 bytes wide:
-                            // a 12-byte LDS read takes twice the cycles (8 against 4.3)
-                            asm volatile("" ::"v"(a0.w), "v"(a1.w), "v"(a2.w), "v"(a3.w));
-                            const float t0 = fmaf(wk[3], a3.x, fmaf(wk[2], a2.x, fmaf(wk[1], a1.x, wk[0] * a0.x)));
-                            const float t1 = fmaf(wk[3], a3.y, fmaf(wk[2], a2.y, fmaf(wk[1], a1.y, wk[0] * a0.y)));
-                            const float t2 = fmaf(wk[3], a3.z, fmaf(wk[2], a2.z, fmaf(wk[1], a1.z, wk[0] * a0.z)));
-                            u0 = fmaf(wys[jj], t0, u0);
-                            u1 = fmaf(wys[jj], t1, u1);
-                            u2 = fmaf(wys[jj], t2, u2);
-                        }
-                        s0 = fmaf(wxs[i], u0, s0);
-                        s1 = fmaf(wxs[i], u1, s1);
-                        s2 = fmaf(wxs[i], u2, s2);
-                    }
+                    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                    const bool nr = r2 < Bf;  // left to the FP64 redo (r2 may be 0 here)
+                    near = near || nr;
+                    const float y = __builtin_amdgcn_rsqf(r2);
+                    wp = (nr || band > 0) ? 0.0f : (y * y) * y;
+                    mj = nr ? 0.0f : (float)pb.y;
+                    mr = nr ? 0.0f : (float)mi;
                 } else {
-                    // z components: six nodes from the even start as three words, the extra two with weight 0
-                    const double wz5[5] = {r1 ? 0.0 : wzs[0], r1 ? wzs[0] : wzs[1], r1 ? wzs[1] : wzs[2],
-                                           r1 ? wzs[2] : wzs[3], r1 ? wzs[3] : 0.0};
-                    const double2 *w2 = (const double2 *)win;
-                    const unsigned zat = base + kT3ZPairs + (iz >> 1);
+                    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+                    if (band == 0) wp = pair_w_tile(r2, B, hi, a.soft, min((int64_t)tile * kTile + id, N - 1), k);
+                    mj = pb.y;
+                    mr = mi;
+                }
+                real Dx = 0, Dy = 0, Dz = 0;
+                if (in) {
+                    // (x, y) nodes by z mod 4: read k takes the stencil's node with
+                    // z = k (mod 4), so lanes a few nodes apart read the same word
+                    // or neighbouring ones
+                    const unsigned r = iz & 3u, blk = iz >> 2;
+                    const bool r1 = (r & 1u) != 0u, r2b = (r & 2u) != 0u;
+                    const real p0 = r1 ? wzs[3] : wzs[0], p1 = r1 ? wzs[0] : wzs[1], p2 = r1 ? wzs[1] : wzs[2],
+                               p3 = r1 ? wzs[2] : wzs[3];
+                    const real wk[4] = {r2b ? p2 : p0, r2b ? p3 : p1, r2b ? p0 : p2, r2b ? p1 : p3};
+                    const unsigned base = rx * (unsigned)plane + ry * (unsigned)kRow;
+                    unsigned at[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const double2 *pk[4], *pz = w2 + zat + i * plane;
+                    for (unsigned q = 0; q < 4; ++q) at[q] = base + kT3RunOff[q] + blk + (q < r ? 1u : 0u);
+                    real s0 = 0, s1 = 0, s2 = 0;
+                    if constexpr (MX) {
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) pk[q] = w2 + at[q] + i * plane;
-                        double u0 = 0.0, u1 = 0.0, u2 = 0.0;
+                        for (int i = 0; i < 4; ++i) {
+                            const float4 *pk[4];
 #pragma unroll
-                        for (int jj = 0; jj < 4; ++jj) {
-                            const double2 a0 = pk[0][jj * kRow], a1 = pk[1][jj * kRow], a2 = pk[2][jj * kRow],
-                                          a3 = pk[3][jj * kRow];
-                            const double2 z0 = pz[jj * kRow], z1 = pz[jj * kRow + 1], z2 = pz[jj * kRow + 2];
-                            const double t0 = fma(wk[3], a3.x, fma(wk[2], a2.x, fma(wk[1], a1.x, wk[0] * a0.x)));
-                            const double t1 = fma(wk[3], a3.y, fma(wk[2], a2.y, fma(wk[1], a1.y, wk[0] * a0.y)));
-                            const double t2 = fma(wz5[4], z2.x,
-                                                  fma(wz5[3], z1.y, fma(wz5[2], z1.x, fma(wz5[1], z0.y, wz5[0] * z0.x))));
-                            u0 = fma(wys[jj], t0, u0);
-                            u1 = fma(wys[jj], t1, u1);
-                            u2 = fma(wys[jj], t2, u2);
+                            for (int q = 0; q < 4; ++q) pk[q] = (const float4 *)win + at[q] + i * plane;
+                            float u0 = 0.0f, u1 = 0.0f, u2 = 0.0f;
+#pragma unroll
+                            for (int jj = 0; jj < 4; ++jj) {
+                                const float4 a0 = pk[0][jj * kRow], a1 = pk[1][jj * kRow], a2 = pk[2][jj * kRow],
+                                             a3 = pk[3][jj * kRow];
+                                // the unused fourth component keeps the reads 16 bytes wide:
+                                // a 12-byte LDS read takes twice the cycles (8 against 4.3)
+                                asm volatile("" ::"v"(a0.w), "v"(a1.w), "v"(a2.w), "v"(a3.w));
+                                const float t0 = fmaf(wk[3], a3.x, fmaf(wk[2], a2.x, fmaf(wk[1], a1.x, wk[0] * a0.x)));
+                                const float t1 = fmaf(wk[3], a3.y, fmaf(wk[2], a2.y, fmaf(wk[1], a1.y, wk[0] * a0.y)));
+                                const float t2 = fmaf(wk[3], a3.z, fmaf(wk[2], a2.z, fmaf(wk[1], a1.z, wk[0] * a0.z)));
+                                u0 = fmaf(wys[jj], t0, u0);
+                                u1 = fmaf(wys[jj], t1, u1);
+                                u2 = fmaf(wys[jj], t2, u2);
+                            }
+                            s0 = fmaf(wxs[i], u0, s0);
+                            s1 = fmaf(wxs[i], u1, s1);
+                            s2 = fmaf(wxs[i], u2, s2);
                         }
-                        s0 = fma(wxs[i], u0, s0);
-                        s1 = fma(wxs[i], u1, s1);
-                        s2 = fma(wxs[i], u2, s2);
+                    } else {
+                        // z components: six nodes from the even start as three words, the extra two with weight 0
+                        const double wz5[5] = {r1 ? 0.0 : wzs[0], r1 ? wzs[0] : wzs[1], r1 ? wzs[1] : wzs[2],
+                                               r1 ? wzs[2] : wzs[3], r1 ? wzs[3] : 0.0};
+                        const double2 *w2 = (const double2 *)win;
+                        const unsigned zat = base + kT3ZPairs + (iz >> 1);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const double2 *pk[4], *pz = w2 + zat + i * plane;
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) pk[q] = w2 + at[q] + i * plane;
+                            double u0 = 0.0, u1 = 0.0, u2 = 0.0;
+#pragma unroll
+                            for (int jj = 0; jj < 4; ++jj) {
+                                const double2 a0 = pk[0][jj * kRow], a1 = pk[1][jj * kRow], a2 = pk[2][jj * kRow],
+                                              a3 = pk[3][jj * kRow];
+                                const double2 z0 = pz[jj * kRow], z1 = pz[jj * kRow + 1], z2 = pz[jj * kRow + 2];
+                                const double t0 = fma(wk[3], a3.x, fma(wk[2], a2.x, fma(wk[1], a1.x, wk[0] * a0.x)));
+                                const double t1 = fma(wk[3], a3.y, fma(wk[2], a2.y, fma(wk[1], a1.y, wk[0] * a0.y)));
+                                const double t2 = fma(wz5[4], z2.x,
+                                                      fma(wz5[3], z1.y, fma(wz5[2], z1.x, fma(wz5[1], z0.y, wz5[0] * z0.x))));
+                                u0 = fma(wys[jj], t0, u0);
+                                u1 = fma(wys[jj], t1, u1);
+                                u2 = fma(wys[jj], t2, u2);
+                            }
+                            s0 = fma(wxs[i], u0, s0);
+                            s1 = fma(wxs[i], u1, s1);
+                            s2 = fma(wxs[i], u2, s2);
+                        }
+                    }
+                    Dx = s0;
+                    Dy = s1;
+                    Dz = s2;
+                } else if (out) {
+                    if constexpr (MX) {
+                        T3Stencil32 st;
+                        t3_stencil_f32(k, dx, dy, dz, st);
+                        t3_contract_f32(
+                            st,
+                            [&](int i, int jj, float4 *n) {
+                                const float4 *g = a.tab32 + (st.mx[i] * NY + st.my[jj]) * NZ + (unsigned)st.iz0;
+#pragma unroll
+                                for (int q = 0; q < 4; ++q) n[q] = g[q];
+                            },
+                            Dx, Dy, Dz);
+                    } else {
+                        t3_interp(a.table, k, dx, dy, dz, Dx, Dy, Dz);
                     }
                 }
-                Dx = s0;
-                Dy = s1;
-                Dz = s2;
-            } else if constexpr (MX) {
-                T3Stencil32 st;
-                t3_stencil_f32(k, dx, dy, dz, st);
-                t3_contract_f32(
-                    st,
-                    [&](int i, int jj, float4 *n) {
-                        const float4 *g = a.tab32 + (st.mx[i] * NY + st.my[jj]) * NZ + (unsigned)st.iz0;
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) n[q] = g[q];
-                    },
-                    Dx, Dy, Dz);
-            } else {
-                t3_interp(a.table, k, dx, dy, dz, Dx, Dy, Dz);
+                auto mad = [](real m, real v, real acc) {
+                    if constexpr (MX) return fmaf(m, v, acc);
+                    else return fma(m, v, acc);
+                };
+                const real px = mad(wp, dx, -Dx), py = mad(wp, dy, -Dy), pz = mad(wp, dz, -Dz);
+                ax = mad(mj, px, ax);
+                ay = mad(mj, py, ay);
+                az = mad(mj, pz, az);
+                gx = from_next_lane(mad(mr, px, gx));
+                gy = from_next_lane(mad(mr, py, gy));
+                gz = from_next_lane(mad(mr, pz, gz));
             }
-            auto mad = [](real m, real v, real acc) {
-                if constexpr (MX) return fmaf(m, v, acc);
-                else return fma(m, v, acc);
-            };
-            const real px = mad(wp, dx, -Dx), py = mad(wp, dy, -Dy), pz = mad(wp, dz, -Dz);
-            ax = mad(mj, px, ax);
-            ay = mad(mj, py, ay);
-            az = mad(mj, pz, az);
-            gx = from_next_lane(mad(mr, px, gx));
-            gy = from_next_lane(mad(mr, py, gy));
-            gz = from_next_lane(mad(mr, pz, gz));
+            // the tile's sums (mixed: FP32 over at most 64 pairs) onto the FP64 ones
+            fx += (double)ax;
+            fy += (double)ay;
+            fz += (double)az;
+            hx += (double)gx;
+            hy += (double)gy;
+            hz += (double)gz;
         }
-        // the tile's sums (mixed: FP32 over at most 64 pairs) onto the FP64 ones
-        fx += (double)ax;
-        fy += (double)ay;
-        fz += (double)az;
-        double hx = (double)gx, hy = (double)gy, hz = (double)gz;
         if (MX && __any(near)) {
             // rare: the pairs within the bound, in FP64 with the FP64 table
             double cx = 0.0, cy = 0.0, cz = 0.0;
@@ -861,16 +889,15 @@ bool sym_variant(const EvalPlan &p) {
 
 // Rows of a T3 Ewald workgroup: with c particles per cell column, R rows and
 // a tile span about (R + 64) / c columns in y, and a window of 5 planes holds
-// 98 / 5 = 19 rows of it, 5 + 2 of them the stencil's and the partial columns.
+// 98 / 5 = 19 rows of it, 5 + 2 of them the stencil's and the partial columns
+// (FP32 nodes: 28).
 // Measured (ms, 256 / 128 / 64 rows): 56^3 (c = 44) 443 / 471 / -, 48^3 (28)
 // 216 / 207 / 239, 44^3 (21) 251 / 131 / 150, 40^3 (16) 172 / 86 / 90, 36^3
 // (12) 95 / 92 / 52; 512 rows: 618 against 621 at 60^3, 538 against 443 at 56^3.
 int sym_t3_rows(const EvalPlan &p) {
     const double c = (double)p.N / ((double)p.t3_ng * p.t3_ng);
-    // FP32 nodes: 144 rows of one word a node, 28 in y
-    const double span = p.precision == STEPS_PREC_MIXED ? 20 : 12;
-    const double t = getenv("T3S") ? atof(getenv("T3S")) : span;
-    return 320 <= t * c ? 256 : (192 <= t * c ? 128 : 64);
+    const bool mx = p.precision == STEPS_PREC_MIXED;
+    return 320 <= (mx ? 14 : 12) * c ? 256 : (192 <= (mx ? 18 : 12) * c ? 128 : 64);
 }
 
 struct SymShape {

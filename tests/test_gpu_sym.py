@@ -87,6 +87,13 @@ def test_t3_ewald_against_oracle(steps, oracle, N):
         report(f"pair-symmetric t3 ewald {label} N={N}", e)
         assert np.all(np.isfinite(F)) and np.median(e) <= 1e-12 and e.max() <= 1e-9
         assert np.array_equal(steps.force_eval(d, x, M, h), F)
+        dm, keepm = steps.make_desc(steps.TOPO_T3, is_periodic=2, L=L, t3_table=tab, precision=steps.PREC_MIXED)
+        Fm = steps.force_eval(dm, x, M, h)
+        em = rel_err(Fm, F)
+        report(f"pair-symmetric t3 ewald {label} N={N} mixed vs fp64", em)
+        # the mixed path's bar, p99 1e-5 (uniform particles, no cancelling lattice)
+        assert np.all(np.isfinite(Fm)) and np.median(em) <= 2e-6 and np.percentile(em, 99) <= 1e-5
+        assert not np.array_equal(Fm, F) and np.array_equal(steps.force_eval(dm, x, M, h), Fm)
 
 
 @pytest.mark.parametrize("N", [150001, 300000])
