@@ -136,11 +136,11 @@ int TableCopy::sync_t3(const double *h, int ng, hipStream_t st) {
     return STEPS_OK;
 }
 
-int TableCopy::sync_s1r2(const double *h, int nrho, int nz, hipStream_t st) {
+int TableCopy::sync_s1r2(const double *h, int nrho, int nz, double L_, double Rsim_, hipStream_t st) {
     const size_t count = (size_t)nrho * nz * 2;
     if (!h || nrho < 1 || nz < 1) return STEPS_OK;
     const uint64_t f = fingerprint(h, count);
-    if (h == host && count == n && f == fp && dev.ptr) return STEPS_OK;
+    if (h == host && count == n && f == fp && dev.ptr && L_ == L && Rsim_ == Rsim) return STEPS_OK;
     std::vector<double> layout;
     s1r2_device_layout(h, nrho, nz, layout);
     int rc = dev.reserve(layout.size() * sizeof(double), "S1R2 table");
@@ -151,6 +151,9 @@ int TableCopy::sync_s1r2(const double *h, int nrho, int nz, hipStream_t st) {
     host = h;
     n = count;
     fp = f;
+    L = L_;
+    Rsim = Rsim_;
+    odd = s1r2_table_odd(h, nrho, nz, L_, Rsim_);
     return STEPS_OK;
 }
 
@@ -387,7 +390,7 @@ int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool 
     if (p.variant == PV_T3_EWALD && (rc = s->t3.sync_t3(d.t3_table, d.t3_ngrid, s->stream)))
         return cleanup(rc);
     if (p.variant >= PV_S1R2_NGP && p.variant <= PV_S1R2_TSC &&
-        (rc = s->s1r2.sync_s1r2(d.s1r2_table, d.s1r2_nrho, d.s1r2_nz, s->stream)))
+        (rc = s->s1r2.sync_s1r2(d.s1r2_table, d.s1r2_nrho, d.s1r2_nz, d.L, d.Rsim, s->stream)))
         return cleanup(rc);
     if (p.ext_mode == 3 &&
         (rc = s->radial.sync(d.radial_table, (size_t)d.radial_table_size, s->stream, "radial table")))
@@ -441,6 +444,7 @@ int sim_plan(steps_sim *s, int64_t id_min, int64_t id_max, int precision, EvalPl
     p.t3_lo = s->t3.lo;
     p.t3_odd = s->t3.odd;
     p.s1r2 = s->s1r2.ptr();
+    p.s1r2_odd = s->s1r2.odd;
     p.radial = s->radial.ptr();
     p.bh_radial = s->radial_bh.ptr();
     return STEPS_OK;
@@ -600,7 +604,7 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
     hipStream_t st = o.stream;
     if (p.variant == PV_T3_EWALD && (rc = o.t3.sync_t3(d->t3_table, d->t3_ngrid, st))) return rc;
     if (p.variant >= PV_S1R2_NGP && p.variant <= PV_S1R2_TSC &&
-        (rc = o.s1r2.sync_s1r2(d->s1r2_table, d->s1r2_nrho, d->s1r2_nz, st)))
+        (rc = o.s1r2.sync_s1r2(d->s1r2_table, d->s1r2_nrho, d->s1r2_nz, d->L, d->Rsim, st)))
         return rc;
     if (p.ext_mode == 3 && (rc = o.radial.sync(d->radial_table, (size_t)d->radial_table_size, st, "radial table")))
         return rc;
@@ -611,6 +615,7 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
     p.t3_lo = o.t3.lo;
     p.t3_odd = o.t3.odd;
     p.s1r2 = o.s1r2.ptr();
+    p.s1r2_odd = o.s1r2.odd;
     p.radial = o.radial.ptr();
     p.bh_radial = o.radial_bh.ptr();
     STEPS_HIP(hipMemcpyAsync(o.x.ptr, x, 3 * nb, hipMemcpyHostToDevice, st), "copy x");

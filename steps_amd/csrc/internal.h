@@ -78,6 +78,7 @@ struct EvalPlan {
     int t3_lo = 0;         // first x/y node of the T3 device layout (t3_device_layout)
     bool t3_odd = false;   // the table in use is odd (t3_table_odd)
     const double *s1r2 = nullptr; int s1r2_nrho = 0, s1r2_nz = 0;
+    bool s1r2_odd = false; // the table in use is odd in z (s1r2_table_odd)
     const double *radial = nullptr; int radial_size = 0;
     int images = 0;        // S1R2 image-sum: ewald_max
     // Barnes-Hut octree instead of the direct sum (USE_BH; forces.cc:373-506,
@@ -249,6 +250,11 @@ constexpr int kT3MaxGrid = 1023;  // element offsets of the layout stay below 2^
 // (ir, iz) at ((ir + 1)*(Nz + 3) + iz + 1)*2 + c, so no stencil needs a wrap
 // or a clamp.
 void s1r2_device_layout(const double *T, int nrho, int nz, std::vector<double> &out);
+// D_rho is even and D_z odd in z, to 16 ulp of the larger of max|D| and the
+// Newtonian force at the node (what the builders' own rounding leaves: 6 ulp
+// on the reference's tables).  A pair near a node has at least that force, so
+// taking one side's correction for the other moves it by its own rounding.
+bool s1r2_table_odd(const double *T, int nrho, int nz, double L, double Rsim);
 inline size_t s1r2_device_nodes(int nrho, int nz) { return ((size_t)nrho + 2) * ((size_t)nz + 3); }
 
 // Table builders (table_kernels.hip); all buffers host memory.

@@ -163,6 +163,7 @@ extern "C" int steps_force_eval_noalloc(const steps_force_desc *d, int64_t N, co
                            d->s1r2_nz, s1d);
         STEPS_HIP(hipGetLastError(), "S1R2 table layout");
         p.s1r2 = s1d;
+        p.s1r2_odd = s1r2_table_odd(d->s1r2_table, d->s1r2_nrho, d->s1r2_nz, d->L, d->Rsim);
     }
     if (radial) {
         STEPS_HIP(hipMemcpyAsync(radd, d->radial_table, rad, hipMemcpyHostToDevice, st), "copy radial table");

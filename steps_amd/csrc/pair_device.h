@@ -387,6 +387,38 @@ __device__ __forceinline__ void s1r2_interp(const double *__restrict__ T, const 
     Dz = Dzv;
 }
 
+// An LDS copy of the S1R2 table rows for rho nodes w0 .. w0 + nw - 1 (each
+// the full z run of the device layout), valid when ok.
+struct S1R2Win {
+    const double2 *win;
+    int w0, nw;
+    bool ok;
+};
+
+// s1r2_interp reading the rho rows from the window when they all lie in it,
+// else from the global table (the same values either way).
+template <int ORDER>
+__device__ __forceinline__ void s1r2_interp_win(const double *__restrict__ T, const KScalars &k, double dx, double dy,
+                                                double dz, double &q, double &Dz, const S1R2Win sw) {
+    double rho, inv_rho, uz, Dr, Dzv;
+    s1r2_coords(k, dx, dy, dz, rho, inv_rho, uz);
+    bool in = false;
+    if (sw.ok) {
+        int lo, hi;
+        s1r2_rows<ORDER>(k, rho, lo, hi);
+        in = lo >= sw.w0 && hi < sw.w0 + sw.nw;
+    }
+    if (in) {
+        const unsigned nz3 = (unsigned)(k.nz + 3);
+        s1r2_gather<ORDER>([&](int ir) { return sw.win + __umul24((unsigned)(ir - sw.w0), nz3); }, k, rho, uz, Dr,
+                           Dzv);
+    } else {
+        s1r2_gather<ORDER>([&](int ir) { return s1r2_row(T, k, ir); }, k, rho, uz, Dr, Dzv);
+    }
+    q = Dr * inv_rho;
+    Dz = Dzv;
+}
+
 // Softened coefficient for a pair, with the tile bound B = (h_i + h_max,tile)^2:
 // only pairs with r2 < B can be inside h_i + h_j, so the exact test (and the
 // softening_exact evaluation) runs in a branch that almost no wave takes.
@@ -411,14 +443,6 @@ __device__ __forceinline__ double pair_s_tile(double r2, double B, double hi, do
     }
     return s;
 }
-
-// An LDS copy of the S1R2 table rows for rho nodes w0 .. w0 + nw - 1 (each
-// the full z run of the device layout), valid when ok.
-struct S1R2Win {
-    const double2 *win;
-    int w0, nw;
-    bool ok;
-};
 
 // One pair (i = lane row, j = uniform source) for variant V, FP64.  WIN: an
 // S1R2 lookup pair reads its rho rows from the window when they all lie in
@@ -494,22 +518,8 @@ __device__ __forceinline__ void pair_f64(const KScalars &k, const double *__rest
             const double w = pair_w_tile(r2, B, hi, soft, j, k);
             // m (w d - D) with D_x = q dx, D_y = q dy: x and y share m (w - q)
             constexpr int ORD = (V == PV_S1R2_NGP) ? 0 : ((V == PV_S1R2_CIC) ? 2 : 4);
-            double rho, inv_rho, uz, Dr, Dzv;
-            s1r2_coords(k, dx, dy, dz, rho, inv_rho, uz);
-            bool in = false;
-            if (WIN && sw.ok) {
-                int lo, hi;
-                s1r2_rows<ORD>(k, rho, lo, hi);
-                in = lo >= sw.w0 && hi < sw.w0 + sw.nw;
-            }
-            if (in) {
-                const unsigned nz3 = (unsigned)(k.nz + 3);
-                s1r2_gather<ORD>([&](int ir) { return sw.win + __umul24((unsigned)(ir - sw.w0), nz3); }, k, rho, uz, Dr,
-                                 Dzv);
-            } else {
-                s1r2_gather<ORD>([&](int ir) { return s1r2_row(table, k, ir); }, k, rho, uz, Dr, Dzv);
-            }
-            const double q = Dr * inv_rho, Dz = Dzv;
+            double q, Dz;
+            s1r2_interp_win<ORD>(table, k, dx, dy, dz, q, Dz, WIN ? sw : S1R2Win{});
             const double sxy = pj.w * (w - q);
             fx = fma(sxy, dx, fx);
             fy = fma(sxy, dy, fy);

@@ -1266,6 +1266,8 @@ bool is_mixed(const EvalPlan &p) { return p.precision == STEPS_PREC_MIXED && mix
 constexpr int64_t kR3SortMinN = 65536;
 bool sorted_sources(const EvalPlan &p) {
     const bool far_tiles = p.variant == PV_R3 || p.variant == PV_T3_NEAREST || p.variant == PV_S1R2_NEAREST;
+    // pair-symmetric S1R2 table kernels take rows and sources in input order
+    if (is_s1r2_lookup(p.variant) && sym_selected(p)) return false;
     const bool mixed_sorted = is_mixed(p) && p.variant != PV_S1R2_TSC && !(p.variant == PV_R3 && p.N < kR3SortMinN);
     return mixed_sorted || (far_tiles && p.N >= kR3SortMinN) || p.variant == PV_T3_EWALD;
 }
@@ -1464,6 +1466,21 @@ int t3_device_layout(const double *T, int ng, std::vector<double> &out) {
             }
         }
     return lo;
+}
+
+bool s1r2_table_odd(const double *T, int nrho, int nz, double L, double Rsim) {
+    double tmax = 0.0;
+    for (size_t i = 0; i < (size_t)nrho * nz * 2u; ++i) tmax = std::max(tmax, std::fabs(T[i]));
+    if (!(tmax < INFINITY)) return false;
+    const double ulp16 = std::ldexp(1.0, -49), drho = kRadialExtent * Rsim / (double)std::max(1, nrho - 1);
+    for (int ir = 0; ir < nrho; ++ir)
+        for (int iz = 0; 2 * iz < nz; ++iz) {
+            const double *a = T + ((size_t)ir * nz + iz) * 2u, *b = T + ((size_t)ir * nz + (nz - 1 - iz)) * 2u;
+            const double rho = ir * drho, z = ((double)iz + 0.5) * (L / nz) - 0.5 * L, r2 = rho * rho + z * z;
+            const double tol = ulp16 * std::max(tmax, r2 > 0.0 ? 1.0 / r2 : 0.0);
+            if (!(std::fabs(a[0] - b[0]) <= tol && std::fabs(a[1] + b[1]) <= tol)) return false;
+        }
+    return true;
 }
 
 void s1r2_device_layout(const double *T, int nrho, int nz, std::vector<double> &out) {

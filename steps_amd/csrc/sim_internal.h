@@ -33,14 +33,15 @@ struct TableCopy {
     const double *host = nullptr;
     size_t n = 0;
     uint64_t fp = 0;
+    double L = 0, Rsim = 0;  // S1R2 tables: the box the oddness was checked for
     DevBuf dev;
     int lo = 0;        // T3 tables: first x/y node of the device layout
-    bool odd = false;  // T3 tables: t3_table_odd
+    bool odd = false;  // T3 / S1R2 tables: t3_table_odd, s1r2_table_odd
     int sync(const double *h, size_t count, hipStream_t st, const char *what);
     // T3 / S1R2: upload the table in the pair kernels' layout
     // (t3_device_layout, s1r2_device_layout)
     int sync_t3(const double *h, int ng, hipStream_t st);
-    int sync_s1r2(const double *h, int nrho, int nz, hipStream_t st);
+    int sync_s1r2(const double *h, int nrho, int nz, double L, double Rsim, hipStream_t st);
     const double *ptr() const { return dev.as<const double>(); }
 };
 

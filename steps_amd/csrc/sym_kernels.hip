@@ -52,8 +52,9 @@ struct SymArgs {
     const double *soft;
     const double4 *tiles;  // per 64 records: bounding-box centre, largest softening length
     const double4 *ext;    // half extents
-    const double *table;   // T3 Ewald table, device layout
+    const double *table;   // T3 Ewald or S1R2 table, device layout
     const float4 *tab32;   // ... its FP32 copy, 16-byte nodes (mixed precision)
+    const float2 *tab32s;  // S1R2: the FP32 copy of the table (mixed precision)
     const uint32_t *keys;  // pencil keys of the records (T3 Ewald)
     double *part;
     KScalars k;
@@ -810,6 +811,205 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
     }
 }
 
+// ---------------------------------------------------------------------------
+// S1R2 with the tabulated correction (CIC, TSC): the same scheme, one row per
+// lane, records in input order, and the rho rows of each source tile staged in
+// LDS as in body_f64 (all waves on the same tile).  D_rho is even and D_z odd
+// in dz (s1r2_table_odd), so one interpolation serves both sides.  MX: the
+// displacement is formed and wrapped in FP64 and rounded once -- the lanes of
+// a step hold different sources, so there is no common centre to take FP32
+// offsets from, and no image can be chosen differently than in FP64 -- the
+// rest of a pair is FP32 (FP32 copy of the table), FP32 sums run over the 64
+// pairs of a tile and are added in FP64, and pairs within the softening bound
+// are done again in FP64.  Measured against the one-sided kernels (resident
+// calls on the cylinder, ms): N = 262144 FP64 CIC 182 -> 92, TSC 296 -> 146,
+// mixed CIC 111 -> 66, TSC 183 -> 94; N = 32799 FP64 CIC 6.6 -> 2.1, TSC 10.3
+// -> 4.3, mixed TSC 7.0 -> 2.6.  Bound by VALU issue.
+// ---------------------------------------------------------------------------
+constexpr int kSymS1Win = 2368;  // 16-byte words (37 KB: four workgroups per CU), two FP32 nodes a word
+
+template <int V, bool MX>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_s1r2_kernel(const SymArgs a) {
+    constexpr int W = kSymWaves;
+    constexpr int ORD = V == PV_S1R2_CIC ? 2 : 4;
+    constexpr int kNodes = MX ? 2 * kSymS1Win : kSymS1Win;
+    using real = std::conditional_t<MX, float, double>;
+    using node = std::conditional_t<MX, float2, double2>;
+    __shared__ __align__(16) double2 win[kSymS1Win];
+    __shared__ __align__(16) double2 jbuf[2][kTile];
+    __shared__ int rng[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t N = a.k.N;
+    const int ntiles = (int)((N + kTile - 1) / kTile);
+    const int b = blockIdx.x;
+    const int cell_l = blockIdx.y / a.cell_tasks, task = blockIdx.y % a.cell_tasks;
+    const int cell = a.cell0 + cell_l;
+    SymWalk w;
+    w.r = cell * a.cell_offs * a.tb + task * a.tpt;
+    w.end = w.r + a.tpt;
+
+    KScalars k = a.k;
+    k.c15 = in_vgpr(a.k.c15);
+    const int64_t row = (int64_t)b * kBlock + tid;
+    const int64_t rowc = min(row, N - 1);
+    const double4 p = a.rec[rowc];
+    const double xi = p.x, yi = p.y, zi = p.z, mi = row < N ? p.w : 0.0, hi = a.soft[rowc];
+    double fx = 0.0, fy = 0.0, fz = 0.0;
+    const unsigned nz3 = (unsigned)(k.nz + 3);
+
+    auto stage = [&](int tile) {  // wave 0: one source per lane
+        const int64_t j = (int64_t)tile * kTile + lane;
+        const double4 q = a.rec[min(j, N - 1)];
+        jbuf[0][lane] = make_double2(q.x, q.y);
+        jbuf[1][lane] = make_double2(q.z, j < N ? q.w : 0.0);
+    };
+    bool have = w.settle(a, b, ntiles);
+    if (have && wave == 0) stage(w.tile);
+    if (tid < 4) rng[tid] = (tid & 1) ? INT32_MIN : INT32_MAX;
+
+    for (int it = 0; have; ++it) {
+        const int tile = w.tile, off = w.off;
+        const double4 tc = a.tiles[tile], te = a.ext[tile];
+        __syncthreads();  // records and range slot in place; the window's memory is free
+        // rho of every pair lies between the distances from the row to the
+        // near and far sides of the tile's xy box; the stencils read rho nodes
+        // floor(rho / drho) - 1 .. floor + 2
+        {
+            const double ax = fabs(xi - tc.x), ay = fabs(yi - tc.y);
+            const double gx = fmax(ax - te.x, 0.0), gy = fmax(ay - te.y, 0.0);
+            const double ex = ax + te.x, ey = ay + te.y;
+            int lo = (int)floor(fmin(sqrt(fma(gx, gx, gy * gy)) * k.inv_drho, k.last_r)) - 1;
+            int up = (int)floor(fmin(sqrt(fma(ex, ex, ey * ey)) * k.inv_drho, k.last_r)) + 2;
+#pragma unroll
+            for (int m = 32; m > 0; m >>= 1) {
+                lo = min(lo, __shfl_xor(lo, m, 64));
+                up = max(up, __shfl_xor(up, m, 64));
+            }
+            if (lane == 0) {
+                atomicMin(&rng[2 * (it & 1)], lo);
+                atomicMax(&rng[2 * (it & 1) + 1], up);
+            }
+        }
+        __syncthreads();
+        const int w0 = max(rng[2 * (it & 1)], -1), w1 = min(rng[2 * (it & 1) + 1], k.nrho);  // ghost rows -1, Nrho
+        const int nw = w1 - w0 + 1;
+        const bool wok = (int64_t)nw * nz3 <= kNodes;
+        if (tid < 2) rng[2 * ((it + 1) & 1) + tid] = tid ? INT32_MIN : INT32_MAX;  // the next tile's slot
+        if (wok) {
+            const unsigned nn = (unsigned)nw * nz3;  // rows w0 .. w1 are contiguous
+            node *dst = (node *)win;
+            const node *src;
+            if constexpr (MX) src = s1r2_row32(a.tab32s, k, w0);
+            else src = s1r2_row(a.table, k, w0);
+            for (unsigned o = tid; o < nn; o += kBlock) dst[o] = src[o];
+        }
+        __syncthreads();  // the window is complete
+        const double bb = hi + tc.w;
+        const double B = bb * bb;
+        const float Bf = (float)(bb * (1.0 + 1e-5)) * (float)(bb * (1.0 + 1e-5));  // mixed: widened
+        real gx = 0, gy = 0, gz = 0, ax = 0, ay = 0, az = 0;
+        bool near = false;
+#pragma unroll 1
+        for (int s = 0; s < kTile; ++s) {
+            const int id = (lane + s) & 63;
+            const double2 pa = jbuf[0][id], pb = jbuf[1][id];
+            const real dx = (real)(pa.x - xi), dy = (real)(pa.y - yi), dz = (real)wrap_half(pb.x - zi, k);
+            real wp, mj, mr, qd, Dz;
+            if constexpr (MX) {
+                const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                const bool nr = r2 < Bf;  // left to the FP64 redo (r2 may be 0 here)
+                near = near || nr;
+                const float y = __builtin_amdgcn_rsqf(r2);
+                wp = nr ? 0.0f : (y * y) * y;
+                mj = nr ? 0.0f : (float)pb.y;
+                mr = nr ? 0.0f : (float)mi;
+                s1r2_interp_f32<ORD, true>(a.tab32s, k, dx, dy, dz, qd, Dz,
+                                           S1R2Win32{(const float2 *)win, w0, nw, wok});
+            } else {
+                const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+                wp = pair_w_tile(r2, B, hi, a.soft, min((int64_t)tile * kTile + id, N - 1), k);
+                mj = pb.y;
+                mr = mi;
+                s1r2_interp_win<ORD>(a.table, k, dx, dy, dz, qd, Dz, S1R2Win{win, w0, nw, wok});
+            }
+            // m (w d - D) with D_x = q dx, D_y = q dy: x and y share m (w - q)
+            auto mad = [](real m, real v, real acc) {
+                if constexpr (MX) return fmaf(m, v, acc);
+                else return fma(m, v, acc);
+            };
+            const real sxy = wp - qd, pz = mad(wp, dz, -Dz), sj = mj * sxy, si = mr * sxy;
+            ax = mad(sj, dx, ax);
+            ay = mad(sj, dy, ay);
+            az = mad(mj, pz, az);
+            gx = from_next_lane(mad(si, dx, gx));
+            gy = from_next_lane(mad(si, dy, gy));
+            gz = from_next_lane(mad(mr, pz, gz));
+        }
+        fx += (double)ax;
+        fy += (double)ay;
+        fz += (double)az;
+        double hx = (double)gx, hy = (double)gy, hz = (double)gz;
+        if (MX && __any(near)) {
+            // rare: the pairs within the bound, in FP64 with the FP64 table
+            double cx = 0.0, cy = 0.0, cz = 0.0;
+#pragma unroll 1
+            for (int s = 0; s < kTile; ++s) {
+                const int id = (lane + s) & 63;
+                const double2 pa = jbuf[0][id], pb = jbuf[1][id];
+                const double ex = pa.x - xi, ey = pa.y - yi, ez = wrap_half(pb.x - zi, k);
+                const float dx = (float)ex, dy = (float)ey, dz = (float)ez;
+                if (fmaf(dx, dx, fmaf(dy, dy, dz * dz)) < Bf) {
+                    const double r2 = fma(ex, ex, fma(ey, ey, ez * ez));
+                    const double wp = pair_w_tile(r2, B, hi, a.soft, min((int64_t)tile * kTile + id, N - 1), k);
+                    double qd, Dz;
+                    s1r2_interp<ORD>(a.table, k, ex, ey, ez, qd, Dz);
+                    const double sxy = wp - qd, pz = fma(wp, ez, -Dz);
+                    fx = fma(pb.y * sxy, ex, fx);
+                    fy = fma(pb.y * sxy, ey, fy);
+                    fz = fma(pb.y, pz, fz);
+                    cx = fma(mi * sxy, ex, cx);
+                    cy = fma(mi * sxy, ey, cy);
+                    cz = fma(mi, pz, cz);
+                }
+                cx = from_next_lane(cx);
+                cy = from_next_lane(cy);
+                cz = from_next_lane(cz);
+            }
+            hx += cx;
+            hy += cy;
+            hz += cz;
+        }
+        SymWalk nw_ = w;
+        ++nw_.r;
+        have = nw_.settle(a, b, ntiles);
+        __syncthreads();  // every wave is done with the window and the records
+        double *gsum = (double *)win;
+        if (off > 0) {
+            gsum[(3 * wave + 0) * kTile + lane] = hx;
+            gsum[(3 * wave + 1) * kTile + lane] = hy;
+            gsum[(3 * wave + 2) * kTile + lane] = hz;
+        }
+        if (have && wave == 0) stage(nw_.tile);
+        __syncthreads();
+        if (off > 0 && wave < 3) {
+            const int64_t j = (int64_t)tile * kTile + lane;
+            double g = gsum[wave * kTile + lane];
+#pragma unroll
+            for (int v = 1; v < W; ++v) g += gsum[(3 * v + wave) * kTile + lane];
+            if (j < N)
+                a.part[sym_slot(N, cell_l, a.cell_tasks, a.cell_offs, a.cell_tasks + off - cell * a.cell_offs) +
+                       (size_t)wave * N + j] = g;
+        }
+        w = nw_;
+    }
+    if (row < N) {
+        double *out = a.part + sym_slot(N, cell_l, a.cell_tasks, a.cell_offs, task);
+        out[row] = fx;
+        out[N + row] = fy;
+        out[2 * N + row] = fz;
+    }
+}
+
 // The slots of one launch onto the running sums: cell by cell, the row sums
 // of its tasks, then its source sums (with the sign of the other side).  The
 // last launch's reduction adds the external term (reduce_kernel's) and writes
@@ -875,6 +1075,7 @@ constexpr int kSymNI = 4;
 // Below this many particles the triangle of block pairs leaves too few equal
 // tasks to fill the chip (N = 9000: 0.129 against 0.167 ms).
 constexpr int64_t kSymMinN = 8192;
+constexpr int64_t kSymS1MinN = 4096;  // S1R2 with a table
 constexpr int64_t kSymT3MinN = 1024;  // T3 Ewald (13^3: 0.57 against 2.8 ms)
 // Scratch the slots may take; the offsets go in as many launches as that
 // needs (128 MiB: 4.5 against 4.3 ms at N = 100003, 33.2 against 31.0 ms for
@@ -883,6 +1084,7 @@ constexpr size_t kSymBytes = (size_t)256 << 20;
 
 bool sym_variant(const EvalPlan &p) {
     if (p.variant == PV_T3_EWALD) return p.t3_ng <= kT3MaxWinNg;  // either precision
+    if (p.variant == PV_S1R2_CIC || p.variant == PV_S1R2_TSC) return true;
     return p.precision == STEPS_PREC_FP64 &&
            (p.variant == PV_R3 || p.variant == PV_T3_NEAREST || p.variant == PV_S1R2_NEAREST);
 }
@@ -898,6 +1100,10 @@ int sym_t3_rows(const EvalPlan &p) {
     const double c = (double)p.N / ((double)p.t3_ng * p.t3_ng);
     const bool mx = p.precision == STEPS_PREC_MIXED;
     return 320 <= (mx ? 14 : 12) * c ? 256 : (192 <= (mx ? 18 : 12) * c ? 128 : 64);
+}
+
+int64_t sym_min_n(const EvalPlan &p) {
+    return p.variant == PV_T3_EWALD ? kSymT3MinN : is_s1r2_lookup(p.variant) ? kSymS1MinN : kSymMinN;
 }
 
 struct SymShape {
@@ -938,6 +1144,17 @@ void launch_sym_kernel(const EvalPlan &p, const SymArgs &a, int cells, hipStream
         } else {
             if (mx) hipLaunchKernelGGL((sym_t3_kernel<8, true>), grid, block, 0, st, a);
             else hipLaunchKernelGGL((sym_t3_kernel<8, false>), grid, block, 0, st, a);
+        }
+        return;
+    }
+    if (is_s1r2_lookup(p.variant)) {
+        const bool mx = p.precision == STEPS_PREC_MIXED;
+        if (p.variant == PV_S1R2_CIC) {
+            if (mx) hipLaunchKernelGGL((sym_s1r2_kernel<PV_S1R2_CIC, true>), grid, dim3(kBlock), 0, st, a);
+            else hipLaunchKernelGGL((sym_s1r2_kernel<PV_S1R2_CIC, false>), grid, dim3(kBlock), 0, st, a);
+        } else {
+            if (mx) hipLaunchKernelGGL((sym_s1r2_kernel<PV_S1R2_TSC, true>), grid, dim3(kBlock), 0, st, a);
+            else hipLaunchKernelGGL((sym_s1r2_kernel<PV_S1R2_TSC, false>), grid, dim3(kBlock), 0, st, a);
         }
         return;
     }
@@ -987,9 +1204,11 @@ int sym_last_cell0(const EvalPlan &p) { return (p.sym_cells - 1) / p.sym_launch_
 // kernel nrows N of them.
 void sym_plan(EvalPlan &p) {
     p.sym = false;
-    if (p.bh || p.N < (p.variant == PV_T3_EWALD ? kSymT3MinN : kSymMinN) || p.N > INT32_MAX || 3 * p.nrows < 2 * p.N || !sym_variant(p)) return;
+    if (p.bh || p.N < sym_min_n(p) || p.N > INT32_MAX || 3 * p.nrows < 2 * p.N || !sym_variant(p)) return;
     p.sym = true;
-    p.sym_block_rows = p.variant == PV_T3_EWALD ? sym_t3_rows(p) : kBlock * kSymNI;
+    p.sym_block_rows = p.variant == PV_T3_EWALD ? sym_t3_rows(p)
+                       : is_s1r2_lookup(p.variant) ? kBlock
+                                                   : kBlock * kSymNI;
     p.sym_blocks = (int)((p.N + p.sym_block_rows - 1) / p.sym_block_rows);
     const int tb = p.sym_block_rows / kTile, offsets = p.sym_blocks / 2 + 1;
     // Tasks of several offsets where there are plenty (fewer row-sum slots),
@@ -1017,7 +1236,9 @@ bool sym_fit(EvalPlan &p, size_t bytes) {
     return true;
 }
 
-bool sym_selected(const EvalPlan &p) { return p.sym && (p.variant != PV_T3_EWALD || p.t3_odd); }
+bool sym_selected(const EvalPlan &p) {
+    return p.sym && (p.variant != PV_T3_EWALD || p.t3_odd) && (!is_s1r2_lookup(p.variant) || p.s1r2_odd);
+}
 
 hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t st) {
     const SymShape s = sym_shape(p);
@@ -1029,6 +1250,7 @@ hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t 
     a.table = b.table;
     a.keys = b.keys;
     a.tab32 = b.tab32;
+    a.tab32s = (const float2 *)b.tab32;
     a.part = b.part;
     a.k = make_scalars(p);
     a.blocks = p.sym_blocks;

@@ -96,6 +96,38 @@ def test_t3_ewald_against_oracle(steps, oracle, N):
         assert not np.array_equal(Fm, F) and np.array_equal(steps.force_eval(dm, x, M, h), Fm)
 
 
+@pytest.mark.parametrize("N", [4096, 4097, 5 * 256 + 4096 - 63, 20011])
+@pytest.mark.parametrize("order", [2, 4])
+def test_s1r2_table_against_oracle(steps, oracle, order, N):
+    """CIC and TSC, windows of rho rows that fit (particles sorted by radius)
+    and that do not (shuffled), ragged ends and close pairs, both precisions;
+    and a table that is not odd in z, which takes the one-sided kernel."""
+    print(f"case pair-symmetric s1r2 order={order} N={N}", flush=True)
+    x, M, h, L = particles("s1r2", N, N)
+    Rsim = 300.0
+    T, shape = steps.s1r2_table(2, L, Rsim)
+    bent = T.reshape(*shape, 2).copy()
+    bent[:, 3 * shape[1] // 4:, 1] *= 1.25
+    by_radius = np.argsort(np.hypot(x[:, 0], x[:, 1]), kind="stable")
+    rows = np.unique(np.concatenate([np.arange(0, 20), np.arange(N - 20, N),
+                                     np.linspace(0, N - 1, 40).astype(int)])).astype(np.int32)
+    for label, tab, o in (("by radius", T, by_radius), ("shuffled", T, np.arange(N)), ("bent", bent.reshape(-1), by_radius)):
+        kw = dict(is_periodic=2, L=L, Rsim=Rsim, s1r2_lookup=1, interp_order=order, s1r2_table=tab, s1r2_shape=shape)
+        d, keep = steps.make_desc(steps.TOPO_S1R2, **kw)
+        dm, keepm = steps.make_desc(steps.TOPO_S1R2, precision=steps.PREC_MIXED, **kw)
+        xo, Mo, ho = x[o], M[o], h[o]
+        F = steps.force_eval(d, xo, Mo, ho)
+        e = rel_err(F[rows], oracle.forces_rows(oracle.params(2, **kw), xo, Mo, ho, rows))
+        report(f"pair-symmetric s1r2 order={order} N={N} {label}", e)
+        assert np.all(np.isfinite(F)) and np.median(e) <= 1e-12 and e.max() <= 1e-9
+        Fm = steps.force_eval(dm, xo, Mo, ho)
+        em = rel_err(Fm, F)
+        report(f"pair-symmetric s1r2 order={order} N={N} {label} mixed vs fp64", em)
+        # the mixed path's bar on the pair sum
+        assert np.all(np.isfinite(Fm)) and np.median(em) <= 2e-6 and np.percentile(em, 99) <= 1e-5
+        assert not np.array_equal(Fm, F)
+
+
 @pytest.mark.parametrize("N", [150001, 300000])
 def test_scratch_does_not_change_the_sums(steps, N):
     """The entry point with 256 MiB of static scratch runs fewer offsets a
