@@ -115,7 +115,8 @@ struct SymBuffers {
     const double *soft;
     const double4 *tiles, *ext;
     const double *table;
-    const float4 *tab32;   // FP32 T3 table (mixed precision)
+    const float4 *tab32;   // FP32 T3 or S1R2 table (mixed precision)
+    const float4 *jrel;    // FP32 records relative to the tiles (mixed precision)
     const uint32_t *keys;
     const uint32_t *perm;  // sorted -> input row, or null
     const double4 *jrec;   // input records (external term)

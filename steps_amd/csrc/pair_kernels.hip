@@ -1391,7 +1391,7 @@ SymBuffers sym_buffers(const EvalPlan &p, const DeviceParticles &dp, double *par
     const ScratchView v = scratch_view(p, partials);
     const PairArgs a = make_args(p, dp, v);
     const bool sorted = sorted_sources(p);
-    return SymBuffers{a.jrec, a.soft, a.tiles, a.tile_ext, a.table, a.t3tab32, a.keys,
+    return SymBuffers{a.jrec, a.soft, a.tiles, a.tile_ext, a.table, a.t3tab32, a.jrel, a.keys,
                       sorted ? spatial_order_perm(v.order, p.N) : nullptr, dp.jrec, v.part};
 }
 

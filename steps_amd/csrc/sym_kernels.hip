@@ -52,6 +52,7 @@ struct SymArgs {
     const double *soft;
     const double4 *tiles;  // per 64 records: bounding-box centre, largest softening length
     const double4 *ext;    // half extents
+    const float4 *jrel;    // mixed: FP32 offsets from the tile's centre, and the mass
     const double *table;   // T3 Ewald or S1R2 table, device layout
     const float4 *tab32;   // ... its FP32 copy, 16-byte nodes (mixed precision)
     const float2 *tab32s;  // S1R2: the FP32 copy of the table (mixed precision)
@@ -346,6 +347,273 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             if (j < N)
                 a.part[sym_slot(N, cell_l, a.cell_tasks, a.cell_offs, a.cell_tasks + off - cell * a.cell_offs) +
                        (size_t)c * N + j] = g;
+        }
+        w = nw;
+        have = more;
+    }
+
+    double *out = a.part + sym_slot(N, cell_l, a.cell_tasks, a.cell_offs, task);
+#pragma unroll
+    for (int q = 0; q < NI; ++q) {
+        const int64_t r = row0 + q * 64;
+        if (r < N) {
+            out[r] = fx[q];
+            out[N + r] = fy[q];
+            out[2 * N + r] = fz[q];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Mixed precision, R3 and nearest image: the scheme of sym_kernel with FP32
+// pairs.  A tile's sources are FP32 offsets from the tile's centre (jrel), a
+// row's offset is formed in FP64 (its image nearest the tile on periodic
+// axes) and rounded once per tile.  FP32 sums: a row's run over the 64 sources
+// of a tile, a source's over kFlush steps of NI rows (at most 64 pairs); both
+// are then added in FP64, the source's in LDS.  Pairs within the bound, or
+// within 1e-6 L of half a period on an axis that is wrapped per pair (where
+// FP32 could take the other image), are done again in FP64.
+//
+// Measured against the one-sided kernels (ms): R3 N = 16384 0.235 -> 0.192,
+// 100003 4.0 -> 2.8, 1.5 10^6 575 -> 468; T3 nearest 24^3 0.471 -> 0.423,
+// 45^3 6.3 -> 3.8, 64^3 38.3 -> 27.5; below N = 12288 the one-sided kernel is
+// as fast (R3 N = 9000: 0.189 against 0.217).  Bound by VALU issue at ~65
+// cycles a pair evaluation and SIMD for 17.5 instructions: fewer or more waves
+// (2, 3, 5, 6 per SIMD) and 8 rows per lane all measured 0-15% slower.  Six of
+// them are FMAs on three VGPR operands, where the one-sided kernel has three
+// and takes its sources from SGPRs, so the gain stays below FP64's.
+// ---------------------------------------------------------------------------
+template <int V, int NI>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_mixed_kernel(const SymArgs a) {
+    constexpr int kFlush = 64 / NI;
+    __shared__ __align__(1024) float4 jbuf[2][kTile];
+    __shared__ double gsum[2][kSymWaves][3][kTile];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t N = a.k.N;
+    const int ntiles = (int)((N + kTile - 1) / kTile);
+    const int b = blockIdx.x;
+    const int cell_l = blockIdx.y / a.cell_tasks, task = blockIdx.y % a.cell_tasks;
+    const int cell = a.cell0 + cell_l;
+    SymWalk w;
+    w.r = cell * a.cell_offs * a.tb + task * a.tpt;
+    w.end = w.r + a.tpt;
+
+    KScalars k = a.k;
+    const int64_t row0 = ((int64_t)b * kSymWaves + wave) * (64 * NI) + lane;
+    double fx[NI], fy[NI], fz[NI];
+    float m[NI];
+#pragma unroll
+    for (int q = 0; q < NI; ++q) {
+        const int64_t r = row0 + q * 64;
+        m[q] = r < N ? (float)a.rec[min(r, N - 1)].w : 0.0f;
+        fx[q] = fy[q] = fz[q] = 0.0;
+    }
+    auto stage = [&](int buf, int tile) {  // wave 0: one source per lane
+        const int64_t j = (int64_t)tile * kTile + lane;
+        float4 p = a.jrel[min(j, N - 1)];
+        if (j >= N) p.w = 0.0f;
+        jbuf[buf][lane] = p;
+    };
+    bool have = w.settle(a, b, ntiles);
+    if (have && wave == 0) stage(0, w.tile);
+    __syncthreads();
+
+    for (int it = 0; have; ++it) {
+        const int buf = it & 1;
+        const int tile = w.tile, off = w.off;
+        SymWalk nw = w;
+        ++nw.r;
+        const bool more = nw.settle(a, b, ntiles);
+        if (more && wave == 0) stage(buf ^ 1, nw.tile);
+
+        const double4 tc = a.tiles[tile], te = a.ext[tile];
+        bool far = true, wx = false, wy = false, wz = false;  // as in sym_kernel
+        float B = 0.0f;
+        if (V != PV_R3) {
+#pragma unroll
+            for (int q = 0; q < NI; ++q) {
+                const double4 p = a.rec[min(row0 + q * 64, N - 1)];
+                double sh;
+                if (V == PV_T3_NEAREST) {
+                    wx = !tile_shift(p.x, tc.x, te.x, k, sh, 1e-5) || wx;
+                    wy = !tile_shift(p.y, tc.y, te.y, k, sh, 1e-5) || wy;
+                }
+                wz = !tile_shift(p.z, tc.z, te.z, k, sh, 1e-5) || wz;
+            }
+            wx = __any(wx);
+            wy = __any(wy);
+            wz = __any(wz);
+        }
+        // the row's coordinate on one axis: its image on the tile's side, or
+        // (wrapped per pair) the one nearest the tile's centre
+        auto place = [&](double x, double c, double e, bool wrapped) {
+            if (wrapped) return near_image(x, c, k);
+            double sh = 0.0;
+            tile_shift(x, c, e, k, sh, 1e-5);
+            return x - sh;
+        };
+        float x[NI], y[NI], z[NI], ax[NI], ay[NI], az[NI];
+#pragma unroll
+        for (int q = 0; q < NI; ++q) {
+            const int64_t r = min(row0 + q * 64, N - 1);
+            double4 p = a.rec[r];
+            if (V == PV_T3_NEAREST) {
+                p.x = place(p.x, tc.x, te.x, wx);
+                p.y = place(p.y, tc.y, te.y, wy);
+            }
+            if (V != PV_R3) p.z = place(p.z, tc.z, te.z, wz);
+            x[q] = (float)(p.x - tc.x);
+            y[q] = (float)(p.y - tc.y);
+            z[q] = (float)(p.z - tc.z);
+            ax[q] = ay[q] = az[q] = 0.0f;
+            // widened by 1e-5: FP32 rounding of r2 cannot hide a pair within the bound
+            const float bq = (float)((a.soft[r] + tc.w) * (1.0 + 1e-5));
+            B = fmaxf(B, bq * bq);
+            const double gx = wx ? 0.0 : fmax(fabs(p.x - tc.x) - te.x, 0.0);
+            const double gy = wy ? 0.0 : fmax(fabs(p.y - tc.y) - te.y, 0.0);
+            const double gz = wz ? 0.0 : fmax(fabs(p.z - tc.z) - te.z, 0.0);
+            far = far && fma(gx, gx, fma(gy, gy, gz * gz)) > (double)(bq * bq) * (1.0 + 1e-3);
+        }
+        far = __all(far);
+        if (off > 0) gsum[buf][wave][0][lane] = gsum[buf][wave][1][lane] = gsum[buf][wave][2][lane] = 0.0;
+
+        bool close = false;
+        float gx = 0.0f, gy = 0.0f, gz = 0.0f;
+        // one axis' nearest image in FP32; bnd: within 1e-6 L of half a period
+        auto wrap = [&](float d, bool &bnd) {
+            const float h = fabsf(d) - k.halfLf;
+            bnd = bnd || fabsf(h) < k.wrap_epsf;
+            return h > 0.0f ? d - copysignf(k.Lf, d) : d;
+        };
+        auto steps = [&](auto near, auto wm) {
+            constexpr int NEAR = decltype(near)::value;
+            constexpr int WM = decltype(wm)::value;
+            unsigned o = (unsigned)lane * 16u;
+            const char *base = (const char *)&jbuf[buf][0];
+            float4 nj = *(const float4 *)(base + o);
+            for (int s0 = 0; s0 < kTile; s0 += kFlush) {
+#pragma unroll 2
+                for (int s = 0; s < kFlush; ++s) {
+                    const float4 pj = nj;
+                    o = (o + 16u) & 1023u;
+                    nj = *(const float4 *)(base + o);  // the next step's (the last one re-reads the first)
+#pragma unroll
+                    for (int q = 0; q < NI; ++q) {
+                        float dx = pj.x - x[q], dy = pj.y - y[q], dz = pj.z - z[q];
+                        bool c = false;
+                        if (WM & 1) dx = wrap(dx, c);
+                        if (WM & 2) dy = wrap(dy, c);
+                        if (WM & 4) dz = wrap(dz, c);
+                        const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                        const float yr = __builtin_amdgcn_rsqf(r2);
+                        float y3 = (yr * yr) * yr;
+                        if (NEAR || WM) {
+                            if (NEAR) c = c || r2 < B;
+                            close = close || c;
+                            y3 = c ? 0.0f : y3;
+                        }
+                        const float sj = y3 * pj.w, si = y3 * m[q];
+                        ax[q] = fmaf(sj, dx, ax[q]);
+                        ay[q] = fmaf(sj, dy, ay[q]);
+                        az[q] = fmaf(sj, dz, az[q]);
+                        gx = fmaf(si, dx, gx);
+                        gy = fmaf(si, dy, gy);
+                        gz = fmaf(si, dz, gz);
+                    }
+                    gx = from_next_lane(gx);
+                    gy = from_next_lane(gy);
+                    gz = from_next_lane(gz);
+                }
+                if (off > 0) {
+                    // lane l holds source (l + s0 + kFlush) mod 64's sums; the
+                    // wave's LDS operations are in order
+                    const int id = (lane + s0 + kFlush) & 63;
+                    __builtin_amdgcn_wave_barrier();
+                    gsum[buf][wave][0][id] += (double)gx;
+                    gsum[buf][wave][1][id] += (double)gy;
+                    gsum[buf][wave][2][id] += (double)gz;
+                    __builtin_amdgcn_wave_barrier();
+                }
+                gx = gy = gz = 0.0f;
+            }
+        };
+        auto variants = [&](auto near) {
+            const int wm = (wx ? 1 : 0) | (wy ? 2 : 0) | (wz ? 4 : 0);
+            if (wm == 0) steps(near, IntC<0>{});
+            else if (V == PV_S1R2_NEAREST) steps(near, IntC<4>{});
+            else if (V == PV_T3_NEAREST) {
+                if (wm == 1) steps(near, IntC<1>{});
+                else if (wm == 2) steps(near, IntC<2>{});
+                else if (wm == 4) steps(near, IntC<4>{});
+                else steps(near, IntC<7>{});
+            }
+        };
+        if (far) variants(IntC<0>{});
+        else variants(IntC<1>{});
+#pragma unroll
+        for (int q = 0; q < NI; ++q) {
+            fx[q] += (double)ax[q];
+            fy[q] += (double)ay[q];
+            fz[q] += (double)az[q];
+        }
+        if (__any(close)) {
+            // rare: those pairs in FP64 from the FP64 records
+            double cx = 0.0, cy = 0.0, cz = 0.0;
+#pragma unroll 1
+            for (int s = 0; s < kTile; ++s) {
+                const int id = (lane + s) & 63;
+                const float4 pj = jbuf[buf][id];
+                const int64_t j = min((int64_t)tile * kTile + id, N - 1);
+#pragma unroll
+                for (int q = 0; q < NI; ++q) {
+                    float dx = pj.x - x[q], dy = pj.y - y[q], dz = pj.z - z[q];
+                    bool c = false;
+                    if (V == PV_T3_NEAREST && wx) dx = wrap(dx, c);
+                    if (V == PV_T3_NEAREST && wy) dy = wrap(dy, c);
+                    if (V != PV_R3 && wz) dz = wrap(dz, c);
+                    c = c || (!far && fmaf(dx, dx, fmaf(dy, dy, dz * dz)) < B);
+                    if (c) {
+                        const int64_t i = min(row0 + q * 64, N - 1);
+                        const double4 pi = a.rec[i], pd = a.rec[j];
+                        double ex = pd.x - pi.x, ey = pd.y - pi.y, ez = pd.z - pi.z;
+                        if (V == PV_T3_NEAREST) {
+                            ex = wrap_half(ex, k);
+                            ey = wrap_half(ey, k);
+                        }
+                        if (V != PV_R3) ez = wrap_half(ez, k);
+                        const double r2 = fma(ex, ex, fma(ey, ey, ez * ez));
+                        const double beta = a.soft[i] + a.soft[j];
+                        double u = inv_r3(r2, 1.5);
+                        if (r2 < beta * beta) u = softening_exact(sqrt(r2), beta);
+                        const double sj = (pj.w == 0.0f ? 0.0 : pd.w) * u, si = (m[q] == 0.0f ? 0.0 : pi.w) * u;
+                        fx[q] = fma(sj, ex, fx[q]);
+                        fy[q] = fma(sj, ey, fy[q]);
+                        fz[q] = fma(sj, ez, fz[q]);
+                        cx = fma(si, ex, cx);
+                        cy = fma(si, ey, cy);
+                        cz = fma(si, ez, cz);
+                    }
+                }
+                cx = from_next_lane(cx);
+                cy = from_next_lane(cy);
+                cz = from_next_lane(cz);
+            }
+            if (off > 0) {
+                __builtin_amdgcn_wave_barrier();
+                gsum[buf][wave][0][lane] += cx;
+                gsum[buf][wave][1][lane] += cy;
+                gsum[buf][wave][2][lane] += cz;
+            }
+        }
+        __syncthreads();  // as in sym_kernel
+        if (off > 0 && tid < 3 * kTile) {
+            const int64_t j = (int64_t)tile * kTile + lane;
+            double g = gsum[buf][0][wave][lane];
+#pragma unroll
+            for (int v = 1; v < kSymWaves; ++v) g += gsum[buf][v][wave][lane];
+            if (j < N)
+                a.part[sym_slot(N, cell_l, a.cell_tasks, a.cell_offs, a.cell_tasks + off - cell * a.cell_offs) +
+                       (size_t)wave * N + j] = g;
         }
         w = nw;
         have = more;
@@ -1075,6 +1343,7 @@ constexpr int kSymNI = 4;
 // Below this many particles the triangle of block pairs leaves too few equal
 // tasks to fill the chip (N = 9000: 0.129 against 0.167 ms).
 constexpr int64_t kSymMinN = 8192;
+constexpr int64_t kSymMixedMinN = 12288;  // the same in mixed precision (sym_mixed_kernel)
 constexpr int64_t kSymS1MinN = 4096;  // S1R2 with a table
 constexpr int64_t kSymT3MinN = 1024;  // T3 Ewald (13^3: 0.57 against 2.8 ms)
 // Scratch the slots may take; the offsets go in as many launches as that
@@ -1085,8 +1354,7 @@ constexpr size_t kSymBytes = (size_t)256 << 20;
 bool sym_variant(const EvalPlan &p) {
     if (p.variant == PV_T3_EWALD) return p.t3_ng <= kT3MaxWinNg;  // either precision
     if (p.variant == PV_S1R2_CIC || p.variant == PV_S1R2_TSC) return true;
-    return p.precision == STEPS_PREC_FP64 &&
-           (p.variant == PV_R3 || p.variant == PV_T3_NEAREST || p.variant == PV_S1R2_NEAREST);
+    return p.variant == PV_R3 || p.variant == PV_T3_NEAREST || p.variant == PV_S1R2_NEAREST;
 }
 
 // Rows of a T3 Ewald workgroup: with c particles per cell column, R rows and
@@ -1103,7 +1371,9 @@ int sym_t3_rows(const EvalPlan &p) {
 }
 
 int64_t sym_min_n(const EvalPlan &p) {
-    return p.variant == PV_T3_EWALD ? kSymT3MinN : is_s1r2_lookup(p.variant) ? kSymS1MinN : kSymMinN;
+    if (p.variant == PV_T3_EWALD) return kSymT3MinN;
+    if (is_s1r2_lookup(p.variant)) return kSymS1MinN;
+    return p.precision == STEPS_PREC_MIXED ? kSymMixedMinN : kSymMinN;
 }
 
 struct SymShape {
@@ -1155,6 +1425,16 @@ void launch_sym_kernel(const EvalPlan &p, const SymArgs &a, int cells, hipStream
         } else {
             if (mx) hipLaunchKernelGGL((sym_s1r2_kernel<PV_S1R2_TSC, true>), grid, dim3(kBlock), 0, st, a);
             else hipLaunchKernelGGL((sym_s1r2_kernel<PV_S1R2_TSC, false>), grid, dim3(kBlock), 0, st, a);
+        }
+        return;
+    }
+    if (p.precision == STEPS_PREC_MIXED) {
+        switch (p.variant) {
+        case PV_R3: hipLaunchKernelGGL((sym_mixed_kernel<PV_R3, kSymNI>), grid, dim3(kBlock), 0, st, a); break;
+        case PV_T3_NEAREST:
+            hipLaunchKernelGGL((sym_mixed_kernel<PV_T3_NEAREST, kSymNI>), grid, dim3(kBlock), 0, st, a);
+            break;
+        default: hipLaunchKernelGGL((sym_mixed_kernel<PV_S1R2_NEAREST, kSymNI>), grid, dim3(kBlock), 0, st, a); break;
         }
         return;
     }
@@ -1250,6 +1530,7 @@ hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t 
     a.table = b.table;
     a.keys = b.keys;
     a.tab32 = b.tab32;
+    a.jrel = b.jrel;
     a.tab32s = (const float2 *)b.tab32;
     a.part = b.part;
     a.k = make_scalars(p);

@@ -64,6 +64,27 @@ def test_against_oracle(steps, oracle, mode, N):
     assert np.median(rel_err(few, F[:N // 2 + 1])) <= 1e-12
 
 
+@pytest.mark.parametrize("N", [12288, 12289, 15 * 1024 - 63, 66001])
+@pytest.mark.parametrize("mode", ["r3", "t3", "s1r2"])
+def test_mixed_against_fp64(steps, oracle, mode, N):
+    """Mixed precision against FP64 on every row (the pair-sum bar, p99 1e-5),
+    close pairs and pairs across the box edge included; deterministic."""
+    print(f"case pair-symmetric mixed {mode} N={N}", flush=True)
+    x, M, h, L = particles(mode, N, N)
+    if mode != "r3":
+        x[300:330, 2] = 1e-9 * np.arange(30)              # either side of the wrap
+        x[330:360, 2] = L / 2 + 1e-8 * (np.arange(30) - 15)  # half a period away
+    (d, keep), _ = descriptor(steps, oracle, mode, L)
+    d.cosmology = 0
+    F = steps.force_eval(d, x, M, h)
+    d.precision = steps.PREC_MIXED
+    Fm = steps.force_eval(d, x, M, h)
+    e = rel_err(Fm, F)
+    report(f"pair-symmetric mixed {mode} N={N} vs fp64", e)
+    assert np.all(np.isfinite(Fm)) and np.median(e) <= 2e-6 and np.percentile(e, 99) <= 1e-5 and e.max() <= 1e-3
+    assert not np.array_equal(Fm, F) and np.array_equal(steps.force_eval(d, x, M, h), Fm)
+
+
 @pytest.mark.parametrize("N", [1024, 1087, 3000, 40001, 66000, 107001])
 def test_t3_ewald_against_oracle(steps, oracle, N):
     """Every rows-per-workgroup choice of the T3 Ewald kernel (64, 128, 256
