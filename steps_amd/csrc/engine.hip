@@ -286,7 +286,12 @@ int make_plan(const steps_force_desc &d, int64_t N, int64_t id_min, int64_t id_m
     const int64_t nib = std::max<int64_t>(1, (p.nrows + rows_per_block - 1) / rows_per_block);
     const int64_t target = (int64_t)cu_count(d.device) * 8;
     int64_t splits = (target + nib - 1) / nib;
-    splits = std::max<int64_t>(1, std::min<int64_t>(splits, std::max<int64_t>(1, N / 256)));
+    // at least kMinChunk sources a split: below N = 4096 one tile, above it
+    // two.  Chunks of 256 and more left the chip idle in small evaluations
+    // (N = 1500: 6 row blocks x 5 splits, the pair kernel 57 us, now ~15; one
+    // call 133 -> 109 us, N = 4500 170 -> 149, T3 nearest 12^3 132 -> 92).
+    const int64_t kMinChunk = N < 4096 ? kTile : 2 * kTile;
+    splits = std::max<int64_t>(1, std::min<int64_t>(splits, (N + kMinChunk - 1) / kMinChunk));
     // Source chunks of at most kL2Sources (2.6 MB of records + 0.5 MB of
     // softening lengths, under the 4 MB L2 of an XCD): workgroups resident at
     // the same time work on the same chunk (row blocks vary fastest in the

@@ -1344,8 +1344,8 @@ constexpr int kSymNI = 4;
 // tasks to fill the chip (N = 9000: 0.129 against 0.167 ms).
 constexpr int64_t kSymMinN = 8192;
 constexpr int64_t kSymMixedMinN = 12288;  // the same in mixed precision (sym_mixed_kernel)
-constexpr int64_t kSymS1MinN = 4096;  // S1R2 with a table
-constexpr int64_t kSymT3MinN = 1024;  // T3 Ewald (13^3: 0.57 against 2.8 ms)
+constexpr int64_t kSymS1MinN = 1024;      // S1R2 with a table (N = 1536, CIC: 0.110 against 0.131 ms)
+constexpr int64_t kSymT3MinN = 128;       // T3 Ewald (N = 216: 0.32 against 0.70 ms, 13^3: 0.57 against 2.8)
 // Scratch the slots may take; the offsets go in as many launches as that
 // needs (128 MiB: 4.5 against 4.3 ms at N = 100003, 33.2 against 31.0 ms for
 // the 64^3 nearest image).
