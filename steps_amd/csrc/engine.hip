@@ -548,8 +548,13 @@ struct OneShot {
     int device = -1;
     hipStream_t stream = nullptr;
     DevBuf x, M, soft, jrec, jsoft, part, F;
+    double *pin = nullptr;  // kPinBytes of pinned host memory (small evaluations)
     TableCopy t3, s1r2, radial, radial_bh;
 };
+// Evaluations whose inputs and forces fit this go through one pinned block
+// and two copies: three copies from and one to pageable memory cost ~40 us of
+// the ~110 us a call at N = 1500 takes.
+constexpr size_t kPinBytes = (size_t)1 << 20;
 OneShot g_oneshot;
 
 }  // namespace
@@ -601,7 +606,7 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
         o.device = d->device;
     }
     const size_t nb = (size_t)N * sizeof(double);
-    if ((rc = o.x.reserve(3 * nb, "alloc x")) || (rc = o.M.reserve(nb, "alloc M")) ||
+    if ((rc = o.x.reserve(5 * nb, "alloc x")) || (rc = o.M.reserve(nb, "alloc M")) ||
         (rc = o.soft.reserve(nb, "alloc soft")) || (rc = o.jrec.reserve((size_t)N * sizeof(double4), "alloc jrec")) ||
         (rc = o.jsoft.reserve(nb, "alloc jsoft")) || (rc = reserve_scratch(o.part, p)) ||
         (rc = o.F.reserve(3 * (size_t)p.nrows * sizeof(double), "alloc F")))
@@ -623,16 +628,30 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
     p.s1r2_odd = o.s1r2.odd;
     p.radial = o.radial.ptr();
     p.bh_radial = o.radial_bh.ptr();
-    STEPS_HIP(hipMemcpyAsync(o.x.ptr, x, 3 * nb, hipMemcpyHostToDevice, st), "copy x");
-    STEPS_HIP(hipMemcpyAsync(o.M.ptr, M, nb, hipMemcpyHostToDevice, st), "copy M");
-    STEPS_HIP(hipMemcpyAsync(o.soft.ptr, soft, nb, hipMemcpyHostToDevice, st), "copy soft");
+    const size_t fb = 3 * (size_t)p.nrows * sizeof(double);
+    const bool pinned = 5 * nb + fb <= kPinBytes;
+    if (pinned && !o.pin) STEPS_HIP(hipHostMalloc((void **)&o.pin, kPinBytes, hipHostMallocDefault), "pinned block");
+    const double *dx = o.x.as<double>(), *dM = o.M.as<double>(), *dsoft = o.soft.as<double>();
+    if (pinned) {
+        // x, M, soft in one block, one copy
+        std::memcpy(o.pin, x, 3 * nb);
+        std::memcpy(o.pin + 3 * N, M, nb);
+        std::memcpy(o.pin + 4 * N, soft, nb);
+        STEPS_HIP(hipMemcpyAsync(o.x.ptr, o.pin, 5 * nb, hipMemcpyHostToDevice, st), "copy particles");
+        dM = dx + 3 * N;
+        dsoft = dx + 4 * N;
+    } else {
+        STEPS_HIP(hipMemcpyAsync(o.x.ptr, x, 3 * nb, hipMemcpyHostToDevice, st), "copy x");
+        STEPS_HIP(hipMemcpyAsync(o.M.ptr, M, nb, hipMemcpyHostToDevice, st), "copy M");
+        STEPS_HIP(hipMemcpyAsync(o.soft.ptr, soft, nb, hipMemcpyHostToDevice, st), "copy soft");
+    }
     DeviceParticles dp{o.jrec.as<double4>(), o.jsoft.as<double>(), N};
-    STEPS_HIP(launch_pack(o.x.as<double>(), o.M.as<double>(), o.soft.as<double>(), N, dp, st), "pack");
+    STEPS_HIP(launch_pack(dx, dM, dsoft, N, dp, st), "pack");
     STEPS_HIP(launch_forces(p, dp, o.part.as<double>(), o.F.as<double>(), st, nullptr, nullptr, nullptr),
               "force kernels");
-    STEPS_HIP(hipMemcpyAsync(F, o.F.ptr, 3 * (size_t)p.nrows * sizeof(double), hipMemcpyDeviceToHost, st),
-              "copy F");
+    STEPS_HIP(hipMemcpyAsync(pinned ? o.pin + 5 * N : F, o.F.ptr, fb, hipMemcpyDeviceToHost, st), "copy F");
     STEPS_HIP(hipStreamSynchronize(st), "force evaluation");
+    if (pinned) std::memcpy(F, o.pin + 5 * N, fb);
     return STEPS_OK;
 }
 
