@@ -460,33 +460,34 @@ hipError_t sim_enqueue_forces(steps_sim *s, const EvalPlan &p, hipStream_t st, b
                          events ? s->ev1 : nullptr, events ? s->ev2 : nullptr);
 }
 
-hipError_t sim_enqueue_step_before(steps_sim *s, hipStream_t st) {
-    // step.cc:128-181: params in, kick + drift + periodic wrap
+hipError_t sim_enqueue_step_before(steps_sim *s, hipStream_t st, bool captured) {
+    // step.cc:128-181: kick + drift + periodic wrap; a captured step copies its
+    // parameters in, so that each replay takes the block's present values
     hipError_t e;
-    if ((e = hipMemcpyAsync(s->dparams.ptr, s->hparams, sizeof(KdkParams), hipMemcpyHostToDevice, st)) != hipSuccess)
+    if (captured && (e = hipMemcpyAsync(s->dparams.ptr, s->hparams, sizeof(KdkParams), hipMemcpyHostToDevice, st)) !=
+                        hipSuccess)
         return e;
-    return launch_kick_drift(s->dp, s->v.as<double>(), s->F.as<double>(), s->dparams.as<const KdkParams>(),
-                             s->desc.topology, s->desc.L, st);
+    return launch_kick_drift(s->dp, s->v.as<double>(), s->F.as<double>(),
+                             captured ? s->dparams.as<const KdkParams>() : nullptr, *s->hparams, s->desc.topology,
+                             s->desc.L, st);
 }
 
-hipError_t sim_enqueue_step_after(steps_sim *s, hipStream_t st) {
+hipError_t sim_enqueue_step_after(steps_sim *s, hipStream_t st, bool captured) {
     // step.cc:250-269: second kick + errmax, errmax out
     const int nb = kdk_reduce_blocks(s->N);
-    double *bm = s->blockmax.as<double>();
-    hipError_t e = launch_kick_errmax(s->dp, s->v.as<double>(), s->F.as<double>(), s->dparams.as<const KdkParams>(),
-                                      bm, nb, bm + nb, st, true);
-    if (e != hipSuccess) return e;
-    return hipMemcpyAsync(s->herrmax, bm + nb, sizeof(double), hipMemcpyDeviceToHost, st);
+    return launch_kick_errmax(s->dp, s->v.as<double>(), s->F.as<double>(),
+                              captured ? s->dparams.as<const KdkParams>() : nullptr, *s->hparams,
+                              s->blockmax.as<double>(), nb, s->herrmax, st, true);
 }
 
-hipError_t sim_enqueue_step(steps_sim *s, const EvalPlan &p, hipStream_t st) {
+hipError_t sim_enqueue_step(steps_sim *s, const EvalPlan &p, hipStream_t st, bool captured) {
     // step.cc:100-312
     hipError_t e;
-    if ((e = sim_enqueue_step_before(s, st)) != hipSuccess) return e;
+    if ((e = sim_enqueue_step_before(s, st, captured)) != hipSuccess) return e;
     if ((e = launch_forces(p, s->dp, s->part.as<double>(), s->F.as<double>(), st, nullptr, nullptr, nullptr)) !=
         hipSuccess)
         return e;
-    return sim_enqueue_step_after(s, st);
+    return sim_enqueue_step_after(s, st, captured);
 }
 
 int sim_fill_params(steps_sim *s, const steps_step_params &sp) {
@@ -767,7 +768,7 @@ int steps_sim_step(steps_sim *s, const steps_step_params *sp, double *errmax) {
         return fail(STEPS_ERR_STATE, "a KDK step needs the full-range forces of the current positions "
                                      "(call steps_sim_forces(s, 0, N-1) first)");
     s->evaluated = s->full = s->timed = false;
-    STEPS_HIP(sim_enqueue_step(s, p, s->stream), "KDK step");
+    STEPS_HIP(sim_enqueue_step(s, p, s->stream, false), "KDK step");
     STEPS_HIP(hipStreamSynchronize(s->stream), "KDK step");
     s->last_nrows = p.nrows;
     s->evaluated = s->full = true;  // the step's second force evaluation, all rows (no timing events)
@@ -783,14 +784,9 @@ int steps_sim_errmax(steps_sim *s, double a, double hubble, double G, double rho
     steps_step_params sp{0.0, a, hubble, a, hubble, G, rho_part};
     int rc = sim_fill_params(s, sp);
     if (rc) return rc;
-    const int nb = kdk_reduce_blocks(s->N);
-    double *bm = s->blockmax.as<double>();
-    STEPS_HIP(hipMemcpyAsync(s->dparams.ptr, s->hparams, sizeof(KdkParams), hipMemcpyHostToDevice, s->stream),
-              "params");
-    STEPS_HIP(launch_kick_errmax(s->dp, s->v.as<double>(), s->F.as<double>(), s->dparams.as<const KdkParams>(), bm,
-                                 nb, bm + nb, s->stream, false),
+    STEPS_HIP(launch_kick_errmax(s->dp, s->v.as<double>(), s->F.as<double>(), nullptr, *s->hparams,
+                                 s->blockmax.as<double>(), kdk_reduce_blocks(s->N), s->herrmax, s->stream, false),
               "errmax");
-    STEPS_HIP(hipMemcpyAsync(s->herrmax, bm + nb, sizeof(double), hipMemcpyDeviceToHost, s->stream), "errmax");
     STEPS_HIP(hipStreamSynchronize(s->stream), "errmax");
     if (errmax) *errmax = *s->herrmax;
     return STEPS_OK;

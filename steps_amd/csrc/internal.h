@@ -220,10 +220,12 @@ struct KdkParams {
     double const_beta;        // 3/(4 pi rho_part)
     double pad;
 };
-hipError_t launch_kick_drift(DeviceParticles &dp, double *v, const double *F, const KdkParams *prm,
-                             int topology, double L, hipStream_t stream);
-hipError_t launch_kick_errmax(const DeviceParticles &dp, double *v, const double *F, const KdkParams *prm,
-                              double *block_max, int nblocks_max, double *errmax_dev,
+// `dev` non-null: the parameters are read there, else `val` is used; errmax may
+// be pinned host memory.
+hipError_t launch_kick_drift(DeviceParticles &dp, double *v, const double *F, const KdkParams *dev,
+                             const KdkParams &val, int topology, double L, hipStream_t stream);
+hipError_t launch_kick_errmax(const DeviceParticles &dp, double *v, const double *F, const KdkParams *dev,
+                              const KdkParams &val, double *block_max, int nblocks_max, double *errmax,
                               hipStream_t stream, bool kick);
 int kdk_reduce_blocks(int64_t n);
 

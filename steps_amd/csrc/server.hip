@@ -362,7 +362,7 @@ struct steps_server {
             if (!g) {
                 hipGraph_t graph = nullptr;
                 STEPS_HIP(hipStreamBeginCapture(sl.stream, hipStreamCaptureModeRelaxed), "begin capture");
-                he = (r.kind == STEPS_REQ_STEP) ? sim_enqueue_step(s, p, sl.stream)
+                he = (r.kind == STEPS_REQ_STEP) ? sim_enqueue_step(s, p, sl.stream, true)
                                                 : sim_enqueue_forces(s, p, sl.stream, false);
                 hipError_t he2 = hipStreamEndCapture(sl.stream, &graph);
                 if (he != hipSuccess) return hip_fail(he, "capture");
@@ -377,7 +377,7 @@ struct steps_server {
             }
             STEPS_HIP(hipGraphLaunch(g, sl.stream), "graph launch");
         } else {
-            he = (r.kind == STEPS_REQ_STEP) ? sim_enqueue_step(s, p, sl.stream)
+            he = (r.kind == STEPS_REQ_STEP) ? sim_enqueue_step(s, p, sl.stream, false)
                                             : sim_enqueue_forces(s, p, sl.stream, false);
             if (he != hipSuccess) return hip_fail(he, "enqueue");
         }
@@ -403,7 +403,7 @@ struct steps_server {
         const hipStream_t qs = sl.stream;
         hipError_t he = hipSuccess;
         for (size_t i = 0; i < n && he == hipSuccess; ++i)
-            if (a.rs[i]->kind == STEPS_REQ_STEP) he = sim_enqueue_step_before(a.es[i]->res, qs);
+            if (a.rs[i]->kind == STEPS_REQ_STEP) he = sim_enqueue_step_before(a.es[i]->res, qs, false);
         for (size_t i = 0; i < n && he == hipSuccess; ++i) {
             steps_sim *s = a.es[i]->res;
             he = launch_forces_prepare(plans[i], s->dp, s->part.as<double>(), qs);
@@ -426,7 +426,7 @@ struct steps_server {
             he = launch_forces_finish(plans[i], s->dp, s->part.as<double>(), s->F.as<double>(), qs);
         }
         for (size_t i = 0; i < n && he == hipSuccess; ++i)
-            if (a.rs[i]->kind == STEPS_REQ_STEP) he = sim_enqueue_step_after(a.es[i]->res, qs);
+            if (a.rs[i]->kind == STEPS_REQ_STEP) he = sim_enqueue_step_after(a.es[i]->res, qs, false);
         if (he == hipSuccess) he = hipEventRecord(sl.done, qs);
         if (he != hipSuccess) {
             // work already queued on this stream must drain before the

@@ -68,8 +68,8 @@ struct steps_sim {
     steps::DeviceParticles dp;
     steps::DevBuf jrec, jsoft, v, F, part, stage, blockmax, dparams;
     steps::TableCopy t3, s1r2, radial, radial_bh;
-    steps::KdkParams *hparams = nullptr;   // pinned: copied to dparams by the step sequence
-    double *herrmax = nullptr;             // pinned: errmax copied back by the step sequence
+    steps::KdkParams *hparams = nullptr;   // pinned: the step's scalars (a captured step copies them to dparams)
+    double *herrmax = nullptr;             // pinned: errmax, written by the step sequence
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;
     hipGraphExec_t graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // [kind][precision]
@@ -91,11 +91,13 @@ int sim_plan(steps_sim *s, int64_t id_min, int64_t id_max, int precision, EvalPl
 // Enqueue (no synchronisation): forces of all rows, or a whole KDK step whose
 // scalars the caller has written to s->hparams.  Both are graph-capturable.
 hipError_t sim_enqueue_forces(steps_sim *s, const EvalPlan &p, hipStream_t st, bool events);
-hipError_t sim_enqueue_step(steps_sim *s, const EvalPlan &p, hipStream_t st);
-// The step around its force evaluation: parameters in, first kick and drift
-// (before); second kick, errmax and its copy to the pinned host block (after).
-hipError_t sim_enqueue_step_before(steps_sim *s, hipStream_t st);
-hipError_t sim_enqueue_step_after(steps_sim *s, hipStream_t st);
+hipError_t sim_enqueue_step(steps_sim *s, const EvalPlan &p, hipStream_t st, bool captured);
+// The step around its force evaluation: first kick and drift (before); second
+// kick and errmax into the pinned host block (after).  captured: the sequence
+// is being captured, so it copies the pinned parameters in at each replay; else
+// their present values go by value.
+hipError_t sim_enqueue_step_before(steps_sim *s, hipStream_t st, bool captured);
+hipError_t sim_enqueue_step_after(steps_sim *s, hipStream_t st, bool captured);
 // Fill the pinned parameter block from the public step parameters.
 int sim_fill_params(steps_sim *s, const steps_step_params &sp);
 // Host <-> device state (synchronous on the sim's stream).
