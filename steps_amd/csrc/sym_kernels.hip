@@ -1364,10 +1364,11 @@ bool sym_variant(const EvalPlan &p) {
 // Measured (ms, 256 / 128 / 64 rows): 56^3 (c = 44) 443 / 471 / -, 48^3 (28)
 // 216 / 207 / 239, 44^3 (21) 251 / 131 / 150, 40^3 (16) 172 / 86 / 90, 36^3
 // (12) 95 / 92 / 52; 512 rows: 618 against 621 at 60^3, 538 against 443 at 56^3.
+// Mixed, 256 / 128: 44^3 65.4 / 71.2, 42^3 51.4 / 55.3, 40^3 41.8 / 42.6.
 int sym_t3_rows(const EvalPlan &p) {
     const double c = (double)p.N / ((double)p.t3_ng * p.t3_ng);
     const bool mx = p.precision == STEPS_PREC_MIXED;
-    return 320 <= (mx ? 14 : 12) * c ? 256 : (192 <= (mx ? 18 : 12) * c ? 128 : 64);
+    return 320 <= (mx ? 20 : 12) * c ? 256 : (192 <= (mx ? 18 : 12) * c ? 128 : 64);
 }
 
 int64_t sym_min_n(const EvalPlan &p) {
