@@ -780,6 +780,8 @@ __device__ __forceinline__ double bh_radial_bh(double r, double R, const double 
 // it, since it took an ancestor).  So each lane sees exactly the items of its
 // own traversal, in the same order: the interactions and their summation
 // order are those of a lane walking alone.
+typedef double v8d __attribute__((ext_vector_type(8)));
+
 template <int MODE, int ORD>
 __device__ __forceinline__ void bh_walk(const BhNode *__restrict__ nodes, int total, bool mine, int i, double xi,
                                         double yi, double zi, double hi, double theta, double L, double cut,
@@ -787,34 +789,40 @@ __device__ __forceinline__ void bh_walk(const BhNode *__restrict__ nodes, int to
     int wait = mine ? 0 : INT32_MAX;  // the next item this lane takes part in
     int it = 0;
     if constexpr (MODE == BH_R3) {
-        // The R3 walk with selects in place of branches: the item's test and
-        // interaction are formed for every lane and kept where the lane takes
-        // part (the scalar unit, not the vector unit, bounds this walk, and
-        // each branch costs it exec-mask work); only the softened branch stays.
+        // The R3 walk: the item's test for every lane, the wave's decisions as
+        // scalar masks, and the interaction only where a lane takes the item
+        // (where all of them open it, the branch skips it).  Vector issue and
+        // the scalar unit bound this walk about equally; the whole record comes
+        // in one scalar load.  N = 2^21, theta = 0.5: 7.6 ms, against 8.65 with
+        // the interaction formed at every item and selected.
         // side / r < theta as side^2 / theta^2 < r^2, r >= beta as r^2 >= beta^2
         // (the same decisions to rounding), and m r^-3 from the v_rsq_f64 seed y
         // with one correction, y^3 (1 + 1.5 e), e = 1 - r^2 y^2: within 2.1e-14
         // (one-sided).
         while (it < total) {
-            const BhNode q = nodes[it];
-            const bool active = wait <= it && q.pidx != i && q.pidx != kBhMassless;
+            v8d rec = *(const v8d *)(nodes + (uint32_t)it);
+            asm volatile("" : "+s"(rec));  // one 64-byte scalar load, not its parts at their uses
+            const BhNode q = __builtin_bit_cast(BhNode, rec);
             const double dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
             const double r2 = dx * dx + dy * dy + dz * dz;
-            const bool take = q.pidx >= 0 || q.open2 < r2;
-            const double beta = q.msoft + hi;
-            const double y0 = __builtin_amdgcn_rsq(r2);
-            const double t = y0 * y0;
-            const double e = fma(-r2, t, 1.0);
-            double wm = (t * (y0 * q.m)) * fma(e, 1.5, 1.0);
-            const bool soft = active && take && !(r2 >= beta * beta);
-            if (soft) wm = q.m * bh_soft(sqrt(r2), beta);
-            wm = (active && take) ? wm : 0.0;
-            f[0] = fma(wm, dx, f[0]);
-            f[1] = fma(wm, dy, f[1]);
-            f[2] = fma(wm, dz, f[2]);
-            const bool open = active && !take;
-            if (wait <= it && !open) wait = q.next;  // took or skipped it: wait for its skip link
-            it = __ballot(open) ? it + 1 : q.next;
+            const uint64_t active = q.pidx == kBhMassless ? 0ull
+                                                          : __builtin_amdgcn_ballot_w64(wait <= it) &
+                                                                __builtin_amdgcn_ballot_w64(q.pidx != i);
+            const uint64_t far = __builtin_amdgcn_ballot_w64(q.open2 < r2) | (q.pidx >= 0 ? ~0ull : 0ull);
+            const uint64_t use = active & far;
+            if (__builtin_amdgcn_inverse_ballot_w64(use)) {
+                const double beta = q.msoft + hi;
+                const double y0 = __builtin_amdgcn_rsq(r2);
+                const double t = y0 * y0;
+                const double e = fma(-r2, t, 1.0);
+                double wm = (t * (y0 * q.m)) * fma(e, 1.5, 1.0);
+                if (!(r2 >= beta * beta)) wm = q.m * bh_soft(sqrt(r2), beta);
+                f[0] = fma(wm, dx, f[0]);
+                f[1] = fma(wm, dy, f[1]);
+                f[2] = fma(wm, dz, f[2]);
+                wait = q.next;  // took it: wait for its skip link
+            }
+            it = (active & ~far) ? it + 1 : q.next;
         }
         return;
     }
