@@ -161,6 +161,17 @@ int make_plan(const steps_force_desc &d, int64_t N, int64_t id_min, int64_t id_m
     if (N < 0) return fail(STEPS_ERR_ARG, "N < 0");
     if (N > (int64_t)INT32_MAX * 4) return fail(STEPS_ERR_ARG, "N too large");
     if (id_max < id_min - 1) return fail(STEPS_ERR_RANGE, "id_max < id_min - 1");
+namespace {
+
+// At most `splits` source chunks of whole tiles.
+void set_splits(EvalPlan &p, int64_t splits) {
+    const int64_t chunk = std::max<int64_t>(1, (p.N + splits - 1) / splits);
+    p.jchunk = ((chunk + kTile - 1) / kTile) * kTile;  // splits start on tile boundaries
+    p.splits = (int)std::max<int64_t>(1, (p.N + p.jchunk - 1) / p.jchunk);
+}
+
+}  // namespace
+
     if (id_max >= id_min && (id_min < 0 || id_max >= N))
         return fail(STEPS_ERR_RANGE, "row range outside [0, N)");
     if (d.precision != STEPS_PREC_FP64 && d.precision != STEPS_PREC_MIXED)
@@ -302,11 +313,7 @@ int make_plan(const steps_force_desc &d, int64_t N, int64_t id_min, int64_t id_m
     constexpr int64_t kMaxPartialBytes = (int64_t)2 << 30;
     splits = std::max<int64_t>(splits, (N + kL2Sources - 1) / kL2Sources);
     splits = std::min<int64_t>(splits, std::max<int64_t>(1, kMaxPartialBytes / (24 * std::max<int64_t>(p.nrows, 1))));
-    int64_t jchunk = std::max<int64_t>(1, (N + splits - 1) / splits);
-    jchunk = ((jchunk + kTile - 1) / kTile) * kTile;  // splits start on tile boundaries
-    splits = std::max<int64_t>(1, (N + jchunk - 1) / jchunk);
-    p.splits = (int)splits;
-    p.jchunk = jchunk;
+    set_splits(p, splits);
     if (t3_slab_plan(p)) {
         // one split per XCD; the packed (server) launches, which keep the
         // generic kernel, split the sources into eight equal chunks instead
@@ -375,7 +382,7 @@ int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool 
     if ((rc = s->jrec.reserve((size_t)N * sizeof(double4), "alloc jrec")) ||
         (rc = s->jsoft.reserve(nb, "alloc soft")) || (rc = s->v.reserve(3 * nb, "alloc v")) ||
         (rc = s->F.reserve(3 * nb, "alloc F")) ||
-        (rc = s->part.reserve(lean ? least : scratch, "alloc partials") && (rc = s->part.reserve(least, "alloc partials"))) ||
+        ((lean || s->part.reserve(scratch, "alloc partials")) && (rc = s->part.reserve(least, "alloc partials"))) ||
         (rc = s->stage.reserve(std::max(3 * nb, (size_t)1024), "alloc stage")) ||
         (rc = s->blockmax.reserve((size_t)(kdk_reduce_blocks(N) + 1) * sizeof(double), "alloc blockmax")) ||
         (rc = s->dparams.reserve(sizeof(KdkParams), "alloc step params")))
@@ -450,6 +457,12 @@ int sim_plan(steps_sim *s, int64_t id_min, int64_t id_max, int precision, EvalPl
     p.t3_odd = s->t3.odd;
     p.s1r2 = s->s1r2.ptr();
     p.s1r2_odd = s->s1r2.odd;
+    // a part of the rows may be split finer than the whole (more workgroups
+    // for the chip): no finer than the scratch holds
+    const bool sym = p.sym;
+    p.sym = false;
+    while (!p.bh && p.splits > 1 && scratch_bytes(p) > s->part.cap) set_splits(p, p.splits - 1);
+    p.sym = sym;
     p.radial = s->radial.ptr();
     p.bh_radial = s->radial_bh.ptr();
     return STEPS_OK;
