@@ -388,13 +388,14 @@ int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool 
         (rc = s->dparams.reserve(sizeof(KdkParams), "alloc step params")))
         return cleanup(rc);
     hipError_t e;
-    if ((e = hipHostMalloc((void **)&s->hparams, sizeof(KdkParams) + sizeof(double), hipHostMallocDefault)) !=
+    if ((e = hipHostMalloc((void **)&s->hparams, sizeof(KdkParams) + 2 * sizeof(double), hipHostMallocDefault)) !=
         hipSuccess) {
         s->hparams = nullptr;
         return cleanup(hip_fail(e, "pinned step block"));
     }
     s->herrmax = (double *)(s->hparams + 1);
-    std::memset(s->hparams, 0, sizeof(KdkParams) + sizeof(double));
+    s->hflag = (int *)(s->herrmax + 1);
+    std::memset(s->hparams, 0, sizeof(KdkParams) + 2 * sizeof(double));
     if ((e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking)) != hipSuccess ||
         (e = hipEventCreate(&s->ev0)) != hipSuccess || (e = hipEventCreate(&s->ev1)) != hipSuccess ||
         (e = hipEventCreate(&s->ev2)) != hipSuccess)
@@ -709,10 +710,18 @@ int steps_sim_set_state(steps_sim *s, const double *x, const double *v, const do
 
 int steps_sim_set_positions(steps_sim *s, const double *x) {
     if (!s || !x) return fail(STEPS_ERR_ARG, "null argument");
-    int rc = check_finite(x, 3 * s->N);
-    if (rc) return rc;
+    const bool on_device = s->N >= kDeviceCheckN;
+    int rc;
+    if (!on_device && (rc = check_finite(x, 3 * s->N))) return rc;
     STEPS_HIP(hipSetDevice(s->device), "hipSetDevice");
     const size_t nb = (size_t)s->N * sizeof(double);
+namespace {
+// New positions are checked on the device from here on: at N = 2^21 the host's
+// loop took 1.5 of a call's 3.4 ms, which is ~47 us at this size, against the
+// ~20 us of a kernel and a wait.
+constexpr int64_t kDeviceCheckN = 65536;
+}  // namespace
+
     STEPS_HIP(hipMemcpyAsync(s->stage.ptr, x, 3 * nb, hipMemcpyHostToDevice, s->stream), "copy x");
     STEPS_HIP(launch_pack_positions(s->stage.as<double>(), s->N, s->dp, s->stream), "pack positions");
     STEPS_HIP(hipStreamSynchronize(s->stream), "set positions");
@@ -720,6 +729,13 @@ int steps_sim_set_positions(steps_sim *s, const double *x) {
     return STEPS_OK;
 }
 
+    if (on_device) {
+        // before the particles change
+        *s->hflag = 0;
+        STEPS_HIP(launch_check_finite(s->stage.as<double>(), 3 * s->N, s->hflag, s->stream), "check x");
+        STEPS_HIP(hipStreamSynchronize(s->stream), "check x");
+        if (*s->hflag) return fail(STEPS_ERR_NONFINITE, "non-finite input value");
+    }
 int steps_sim_get_state(steps_sim *s, double *x, double *v) {
     if (!s) return fail(STEPS_ERR_ARG, "null sim");
     return sim_download(s, x, v, nullptr);

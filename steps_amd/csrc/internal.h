@@ -209,6 +209,8 @@ hipError_t launch_pack_positions(const double *x, int64_t n, DeviceParticles &dp
                                  hipStream_t stream);
 // DeviceParticles positions -> AoS x [3n] (device).
 hipError_t launch_unpack_positions(const DeviceParticles &dp, double *x, hipStream_t stream);
+// Writes 1 to *flag (pinned host memory) when one of x[0..count) is not finite.
+hipError_t launch_check_finite(const double *x, int64_t count, int *flag, hipStream_t stream);
 
 // KDK pieces (kdk_kernels.hip).  Per-step scalars live in device memory
 // (written by the host before the launch) so that captured graphs replay.

@@ -1134,6 +1134,14 @@ __global__ void pack_positions_kernel(const double *__restrict__ x, double4 *__r
     jrec[i] = make_double4(x[3 * i], x[3 * i + 1], x[3 * i + 2], m);
 }
 
+__global__ __launch_bounds__(256) void check_finite_kernel(const double *__restrict__ x, int64_t count,
+                                                           int *__restrict__ flag) {
+    bool bad = false;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
+        bad = bad || !isfinite(x[i]);
+    if (bad) *flag = 1;
+}
+
 __global__ void unpack_positions_kernel(const double4 *__restrict__ jrec, double *__restrict__ x,
                                         int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1643,6 +1651,13 @@ hipError_t launch_pack(const double *x, const double *M, const double *soft, int
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(pack_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, M,
                        soft, dp.jrec, dp.soft, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_check_finite(const double *x, int64_t count, int *flag, hipStream_t st) {
+    if (count <= 0) return hipSuccess;
+    const unsigned nb = (unsigned)std::min<int64_t>(4096, (count + 255) / 256);
+    hipLaunchKernelGGL(check_finite_kernel, dim3(nb), dim3(256), 0, st, x, count, flag);
     return hipGetLastError();
 }
 
