@@ -780,14 +780,53 @@ __device__ __forceinline__ double bh_radial_bh(double r, double R, const double 
 // it, since it took an ancestor).  So each lane sees exactly the items of its
 // own traversal, in the same order: the interactions and their summation
 // order are those of a lane walking alone.
+//
+// A walk over the items [first, total) alone starts with bh_enter: what the
+// lanes decided at the cubes that hold item `first`, without their
+// interactions (those belong to the walk that has the cube).  So the walks of
+// consecutive ranges have the interactions of one walk, each once.
 typedef double v8d __attribute__((ext_vector_type(8)));
 
+// The walk up to item `first`: returns the item to go on from.
+template <int MODE>
+__device__ __forceinline__ int bh_enter(const BhNode *__restrict__ nodes, int first, double xi, double yi, double zi,
+                                        double theta, double L, int &wait) {
+    int it = 0;
+    while (it < first) {
+        const BhNode q = nodes[it];
+        if (q.next <= first || q.pidx == kBhMassless) {  // does not hold it, or is skipped whole
+            it = q.next;
+            continue;
+        }
+        double dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
+        if (MODE == BH_T3_NEAR || MODE == BH_T3_EWALD) {
+            if (fabs(dx) > 0.5 * L) dx -= copysign(L, dx);
+            if (fabs(dy) > 0.5 * L) dy -= copysign(L, dy);
+        }
+        if (MODE >= BH_T3_NEAR && MODE <= BH_S1R2_TABLE)
+            if (fabs(dz) > 0.5 * L) dz -= copysign(L, dz);
+        const double r2 = dx * dx + dy * dy + dz * dz;  // the walks' displacement and tests
+        bool take;
+        if (MODE == BH_R3) {
+            take = q.open2 < r2;
+        } else {
+            double y, dist;
+            bh_rsq(r2, y, dist);
+            take = q.side * y < theta;
+        }
+        const bool active = wait <= it;
+        if (active && take) wait = q.next;
+        it = __builtin_amdgcn_ballot_w64(active && !take) ? it + 1 : q.next;
+    }
+    return __builtin_amdgcn_readfirstlane(it);
+}
+
 template <int MODE, int ORD>
-__device__ __forceinline__ void bh_walk(const BhNode *__restrict__ nodes, int total, bool mine, int i, double xi,
-                                        double yi, double zi, double hi, double theta, double L, double cut,
+__device__ __forceinline__ void bh_walk(const BhNode *__restrict__ nodes, int first, int total, bool mine, int i,
+                                        double xi, double yi, double zi, double hi, double theta, double L, double cut,
                                         const BhTables &tb, double *f) {
     int wait = mine ? 0 : INT32_MAX;  // the next item this lane takes part in
-    int it = 0;
+    int it = first > 0 ? bh_enter<MODE>(nodes, first, xi, yi, zi, theta, L, wait) : 0;
     if constexpr (MODE == BH_R3) {
         // The R3 walk: the item's test for every lane, the wave's decisions as
         // scalar masks, and the interaction only where a lane takes the item
@@ -915,36 +954,8 @@ __device__ __forceinline__ void bh_walk(const BhNode *__restrict__ nodes, int to
 // image sum walks the tree once per z image m = -(P+1) .. P+1 with the row
 // moved by m L and no wrap, and adds the walks in that order (forces.cc:
 // 1108-1118).
-template <int MODE, int ORD>
-__global__ __launch_bounds__(256) void bh_force_kernel(const double4 *__restrict__ srec,
-                                                       const double *__restrict__ ssoft,
-                                                       const uint32_t *__restrict__ sidx, int64_t n,
-                                                       const int *__restrict__ info,
-                                                       const BhNode *__restrict__ nodes, double theta, double L,
-                                                       int images, BhTables tb, BhFrame fr, int ext_mode,
-                                                       double ext_coeff, int64_t id_min, int64_t id_max,
-                                                       double *__restrict__ F) {
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t sc = min(s, n - 1);
-    const int i = (int)sidx[sc];
-    const bool mine = s < n && i >= id_min && i <= id_max;
-    const double4 me = srec[sc];
-    const double hi = ssoft[sc];
-    double f[3] = {0.0, 0.0, 0.0};
-    const int total = info[0];
-    if (MODE == BH_S1R2_IMAGES) {
-        const double cut = ((double)images - 0.4) * L;  // main.cc:1270-1271, forces.cc:1100
-        for (int m = -images; m < images + 1; ++m) {
-            double g[3] = {0.0, 0.0, 0.0};
-            bh_walk<MODE, ORD>(nodes, total, mine, i, me.x, me.y, me.z + (double)m * L, hi, theta, L, cut, tb, g);
-            f[0] += g[0];
-            f[1] += g[1];
-            f[2] += g[2];
-        }
-    } else {
-        bh_walk<MODE, ORD>(nodes, total, mine, i, me.x, me.y, me.z, hi, theta, L, 0.0, tb, f);
-    }
-    if (!mine) return;
+__device__ __forceinline__ void bh_finish_row(double *f, const double4 &me, const BhTables &tb, const BhFrame &fr,
+                                              int ext_mode, double ext_coeff, double *__restrict__ o) {
     if (ext_mode == 1) {
         f[0] += ext_coeff * me.x;
         f[1] += ext_coeff * me.y;
@@ -972,10 +983,73 @@ __global__ __launch_bounds__(256) void bh_force_kernel(const double4 *__restrict
     }
     if (fr.kind == 1) bh_rodrigues(f[0], f[1], f[2], fr.ax, fr.ay, fr.az, fr.cb, fr.sb);
     else if (fr.kind == 3) bh_rotate_xy(f[0], f[1], fr.cb, fr.sb);
-    double *o = F + 3 * (i - id_min);
     o[0] = f[0];
     o[1] = f[1];
     o[2] = f[2];
+}
+
+// RANGES: workgroup row y walks the y-th of gridDim.y equal ranges of the
+// items and stores its sums to part [range][3][n] (bh_split has the rule).
+template <int MODE, int ORD, bool RANGES>
+__global__ __launch_bounds__(256) void bh_force_kernel(const double4 *__restrict__ srec,
+                                                       const double *__restrict__ ssoft,
+                                                       const uint32_t *__restrict__ sidx, int64_t n,
+                                                       const int *__restrict__ info,
+                                                       const BhNode *__restrict__ nodes, double theta, double L,
+                                                       int images, BhTables tb, BhFrame fr, int ext_mode,
+                                                       double ext_coeff, int64_t id_min, int64_t id_max,
+                                                       double *__restrict__ part, double *__restrict__ F) {
+    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t sc = min(s, n - 1);
+    const int i = (int)sidx[sc];
+    const bool mine = s < n && i >= id_min && i <= id_max;
+    const double4 me = srec[sc];
+    const double hi = ssoft[sc];
+    double f[3] = {0.0, 0.0, 0.0};
+    int first = 0, total = info[0];
+    if (RANGES) {
+        first = (int)((int64_t)info[0] * blockIdx.y / gridDim.y);
+        total = (int)((int64_t)info[0] * (blockIdx.y + 1) / gridDim.y);
+    }
+    if (MODE == BH_S1R2_IMAGES) {
+        const double cut = ((double)images - 0.4) * L;  // main.cc:1270-1271, forces.cc:1100
+        for (int m = -images; m < images + 1; ++m) {
+            double g[3] = {0.0, 0.0, 0.0};
+            bh_walk<MODE, ORD>(nodes, first, total, mine, i, me.x, me.y, me.z + (double)m * L, hi, theta, L, cut, tb,
+                               g);
+            f[0] += g[0];
+            f[1] += g[1];
+            f[2] += g[2];
+        }
+    } else {
+        bh_walk<MODE, ORD>(nodes, first, total, mine, i, me.x, me.y, me.z, hi, theta, L, 0.0, tb, f);
+    }
+    if (!mine) return;
+    if (RANGES) {
+        double *o = part + (size_t)blockIdx.y * 3u * (size_t)n + s;
+        o[0] = f[0];
+        o[n] = f[1];
+        o[2 * n] = f[2];
+        return;
+    }
+    bh_finish_row(f, me, tb, fr, ext_mode, ext_coeff, F + 3 * (i - id_min));
+}
+
+// The ranges' sums of a row in their order, then its external terms.
+__global__ __launch_bounds__(256) void bh_finish_kernel(const double4 *__restrict__ srec,
+                                                        const uint32_t *__restrict__ sidx, int64_t n, int ranges,
+                                                        const double *__restrict__ part, BhTables tb, BhFrame fr,
+                                                        int ext_mode, double ext_coeff, int64_t id_min, int64_t id_max,
+                                                        double *__restrict__ F) {
+    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= n) return;
+    const int i = (int)sidx[s];
+    if (i < id_min || i > id_max) return;
+    double f[3] = {0.0, 0.0, 0.0};
+#pragma unroll 8
+    for (int r = 0; r < ranges; ++r)
+        for (int c = 0; c < 3; ++c) f[c] += part[((size_t)r * 3u + c) * (size_t)n + s];
+    bh_finish_row(f, srec[s], tb, fr, ext_mode, ext_coeff, F + 3 * (i - id_min));
 }
 
 struct BhView {
@@ -1103,6 +1177,24 @@ size_t bh_scratch_bytes(int64_t n) {
     return b + 256;
 }
 
+// Ranges of the item list, each walked by workgroups of its own.  A walk is a
+// serial chain of ~3400 items (theta 0.5) whatever N: at N = 20000 its 313
+// waves leave two of three SIMDs empty and take as long as 32768 waves take
+// for a quarter of theirs.  With R ranges there are R times the waves, each
+// with ~1/R of the chain and the cubes around its first item to decide again
+// (bh_enter).  One evaluation (ms, 1 / 8 / 64 ranges): N = 20000 1.41 / 0.92 /
+// 0.76, 65536 1.77 / 1.38 / 1.21, 300000 3.13 / 2.93 / 3.11, 800000 6.13 (2:
+// 5.92), 2^21 16.5 (2: 16.6).  S1R2 walks whole: its rows' z forces nearly
+// cancel, and the one walk adds them in the reference's order.
+int bh_split(int topology, int64_t n) {
+    if (topology == STEPS_TOPO_S1R2 || n <= 0) return 1;
+    return (int)std::min<int64_t>(64, std::max<int64_t>(1, ((int64_t)1 << 21) / n));
+}
+
+size_t bh_part_bytes(int64_t n, int ranges) {
+    return ranges > 1 ? 256 + (size_t)ranges * 3u * (size_t)std::max<int64_t>(n, 1) * sizeof(double) : 0;
+}
+
 hipError_t launch_bh_forces(const EvalPlan &p, const DeviceParticles &dp, void *scratch, double *F,
                             hipStream_t st, hipEvent_t ev_tree_end) {
     const int64_t n = p.N;
@@ -1147,18 +1239,27 @@ hipError_t launch_bh_forces(const EvalPlan &p, const DeviceParticles &dp, void *
     BhTables tb{p.t3, p.t3_ng, p.t3_lo, p.s1r2, p.s1r2_nrho, p.s1r2_nz, kRadialExtent * p.Rsim, p.radial,
                 p.radial_size, p.Rsim, p.bh_radial_size > 0 ? p.bh_radial : nullptr, p.bh_radial_size};
     const int64_t id_max = p.id_min + p.nrows - 1;
-#define STEPS_BH_LAUNCH(MODE, ORD)                                                                                  \
-    hipLaunchKernelGGL((bh_force_kernel<MODE, ORD>), dim3(ng), dim3(256), 0, st, v.srec, v.ssoft, v.sidx, n, v.info, \
-                       v.nodes, p.bh_theta, p.L, p.images, tb, fr, p.ext_mode, p.ext_coeff, p.id_min, id_max, F)
+    const int ranges = p.bh_ranges;
+    double *const part = ranges > 1 ? (double *)((char *)scratch + a256(bh_scratch_bytes(n))) : nullptr;
+#define STEPS_BH_KERNEL(MODE, ORD, RANGES)                                                                          \
+    hipLaunchKernelGGL((bh_force_kernel<MODE, ORD, RANGES>), dim3(ng, (unsigned)ranges), dim3(256), 0, st, v.srec,  \
+                       v.ssoft, v.sidx, n, v.info, v.nodes, p.bh_theta, p.L, p.images, tb, fr, p.ext_mode,          \
+                       p.ext_coeff, p.id_min, id_max, part, F)
+#define STEPS_BH_LAUNCH(MODE, ORD) STEPS_BH_KERNEL(MODE, ORD, false)
+#define STEPS_BH_RANGES(MODE, ORD)                     \
+    do {                                               \
+        if (part) STEPS_BH_KERNEL(MODE, ORD, true);    \
+        else STEPS_BH_KERNEL(MODE, ORD, false);        \
+    } while (0)
     switch (p.variant) {
-    case PV_R3: STEPS_BH_LAUNCH(BH_R3, 0); break;
-    case PV_T3_NEAREST: STEPS_BH_LAUNCH(BH_T3_NEAR, 0); break;
+    case PV_R3: STEPS_BH_RANGES(BH_R3, 0); break;
+    case PV_T3_NEAREST: STEPS_BH_RANGES(BH_T3_NEAR, 0); break;
     case PV_T3_EWALD:
         switch (p.bh_order) {
-        case 4: STEPS_BH_LAUNCH(BH_T3_EWALD, 4); break;
-        case 6: STEPS_BH_LAUNCH(BH_T3_EWALD, 6); break;
-        case 8: STEPS_BH_LAUNCH(BH_T3_EWALD, 8); break;
-        default: STEPS_BH_LAUNCH(BH_T3_EWALD, 2); break;
+        case 4: STEPS_BH_RANGES(BH_T3_EWALD, 4); break;
+        case 6: STEPS_BH_RANGES(BH_T3_EWALD, 6); break;
+        case 8: STEPS_BH_RANGES(BH_T3_EWALD, 8); break;
+        default: STEPS_BH_RANGES(BH_T3_EWALD, 2); break;
         }
         break;
     case PV_S1R2_NEAREST: STEPS_BH_LAUNCH(BH_S1R2_NEAR, 0); break;
@@ -1168,7 +1269,12 @@ hipError_t launch_bh_forces(const EvalPlan &p, const DeviceParticles &dp, void *
     case PV_S1R2_IMAGES: STEPS_BH_LAUNCH(BH_S1R2_IMAGES, 0); break;
     default: return hipErrorInvalidValue;
     }
+#undef STEPS_BH_RANGES
 #undef STEPS_BH_LAUNCH
+#undef STEPS_BH_KERNEL
+    if (part)
+        hipLaunchKernelGGL(bh_finish_kernel, dim3(ng), dim3(256), 0, st, v.srec, v.sidx, n, ranges, part, tb, fr,
+                           p.ext_mode, p.ext_coeff, p.id_min, id_max, F);
     return hipGetLastError();
 }
 

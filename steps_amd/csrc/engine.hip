@@ -42,10 +42,14 @@ int cu_count(int device) {
     return n;
 }
 
+void least_scratch(EvalPlan &p) {
+    p.sym_launch_cells = std::min(p.sym_launch_cells, 1);
+    p.bh_ranges = 1;
+}
+
 int reserve_scratch(DevBuf &b, EvalPlan &p) {
     if (b.reserve(scratch_bytes(p), "alloc partials") == STEPS_OK) return STEPS_OK;
-    // the slots of fewer cells at a time take less (and give the same sums)
-    if (p.sym) p.sym_launch_cells = 1;
+    least_scratch(p);
     return b.reserve(scratch_bytes(p), "alloc partials");
 }
 
@@ -157,10 +161,6 @@ int TableCopy::sync_s1r2(const double *h, int nrho, int nz, double L_, double Rs
     return STEPS_OK;
 }
 
-int make_plan(const steps_force_desc &d, int64_t N, int64_t id_min, int64_t id_max, EvalPlan &p) {
-    if (N < 0) return fail(STEPS_ERR_ARG, "N < 0");
-    if (N > (int64_t)INT32_MAX * 4) return fail(STEPS_ERR_ARG, "N too large");
-    if (id_max < id_min - 1) return fail(STEPS_ERR_RANGE, "id_max < id_min - 1");
 namespace {
 
 // At most `splits` source chunks of whole tiles.
@@ -172,6 +172,10 @@ void set_splits(EvalPlan &p, int64_t splits) {
 
 }  // namespace
 
+int make_plan(const steps_force_desc &d, int64_t N, int64_t id_min, int64_t id_max, EvalPlan &p) {
+    if (N < 0) return fail(STEPS_ERR_ARG, "N < 0");
+    if (N > (int64_t)INT32_MAX * 4) return fail(STEPS_ERR_ARG, "N too large");
+    if (id_max < id_min - 1) return fail(STEPS_ERR_RANGE, "id_max < id_min - 1");
     if (id_max >= id_min && (id_min < 0 || id_max >= N))
         return fail(STEPS_ERR_RANGE, "row range outside [0, N)");
     if (d.precision != STEPS_PREC_FP64 && d.precision != STEPS_PREC_MIXED)
@@ -263,6 +267,7 @@ void set_splits(EvalPlan &p, int64_t splits) {
         p.bh_particle_radius = d.bh_particle_radius;
         // the CPU build's T3 table interpolation (ewald_space.cc:452-466): even
         // orders up to 8, anything else falls back to 2
+        p.bh_ranges = bh_split(d.topology, N);
         p.bh_order = d.interp_order;
         if (p.bh_order < 2 || p.bh_order % 2 != 0) p.bh_order = 2;
         if (p.bh_order > 8) p.bh_order = 8;
@@ -325,7 +330,7 @@ void set_splits(EvalPlan &p, int64_t splits) {
 }
 
 size_t scratch_bytes(const EvalPlan &p) {
-    if (p.bh) return bh_scratch_bytes(p.N);
+    if (p.bh) return bh_scratch_bytes(p.N) + bh_part_bytes(p.N, p.bh_ranges);
     return ((partial_bytes(p) + 255) & ~(size_t)255) + tile_extra_bytes(p);
 }
 
@@ -355,7 +360,7 @@ int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool 
     int rc = make_plan(d, N, 0, N - 1, p);
     if (rc) return rc;
     size_t scratch = scratch_bytes(p);
-    p.sym_launch_cells = std::min(p.sym_launch_cells, 1);
+    least_scratch(p);
     size_t least = scratch_bytes(p);
     if (both_precisions && desc_mixed_capable(d)) {
         // the scratch serves either precision (neither plan's need bounds the other's)
@@ -364,7 +369,7 @@ int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool 
         EvalPlan q;
         if ((rc = make_plan(dd, N, 0, N - 1, q))) return rc;
         scratch = std::max(scratch, scratch_bytes(q));
-        q.sym_launch_cells = std::min(q.sym_launch_cells, 1);
+        least_scratch(q);
         least = std::max(least, scratch_bytes(q));
     }
     if ((rc = set_device(d.device))) return rc;
@@ -452,18 +457,19 @@ int sim_plan(steps_sim *s, int64_t id_min, int64_t id_max, int precision, EvalPl
     d.precision = precision;
     int rc = make_plan(d, s->N, id_min, id_max, p);
     if (rc) return rc;
-    if (!sym_fit(p, s->part.cap) || scratch_bytes(p) > s->part.cap) return fail(STEPS_ERR_STATE, "scratch too small for this precision");
-    p.t3 = s->t3.ptr();
-    p.t3_lo = s->t3.lo;
-    p.t3_odd = s->t3.odd;
-    p.s1r2 = s->s1r2.ptr();
-    p.s1r2_odd = s->s1r2.odd;
     // a part of the rows may be split finer than the whole (more workgroups
     // for the chip): no finer than the scratch holds
     const bool sym = p.sym;
     p.sym = false;
     while (!p.bh && p.splits > 1 && scratch_bytes(p) > s->part.cap) set_splits(p, p.splits - 1);
     p.sym = sym;
+    if (p.bh && scratch_bytes(p) > s->part.cap) least_scratch(p);
+    if (!sym_fit(p, s->part.cap) || scratch_bytes(p) > s->part.cap) return fail(STEPS_ERR_STATE, "scratch too small for this precision");
+    p.t3 = s->t3.ptr();
+    p.t3_lo = s->t3.lo;
+    p.t3_odd = s->t3.odd;
+    p.s1r2 = s->s1r2.ptr();
+    p.s1r2_odd = s->s1r2.odd;
     p.radial = s->radial.ptr();
     p.bh_radial = s->radial_bh.ptr();
     return STEPS_OK;
@@ -708,13 +714,6 @@ int steps_sim_set_state(steps_sim *s, const double *x, const double *v, const do
     return sim_upload(s, x, v, M, soft, nullptr);
 }
 
-int steps_sim_set_positions(steps_sim *s, const double *x) {
-    if (!s || !x) return fail(STEPS_ERR_ARG, "null argument");
-    const bool on_device = s->N >= kDeviceCheckN;
-    int rc;
-    if (!on_device && (rc = check_finite(x, 3 * s->N))) return rc;
-    STEPS_HIP(hipSetDevice(s->device), "hipSetDevice");
-    const size_t nb = (size_t)s->N * sizeof(double);
 namespace {
 // New positions are checked on the device from here on: at N = 2^21 the host's
 // loop took 1.5 of a call's 3.4 ms, which is ~47 us at this size, against the
@@ -722,13 +721,14 @@ namespace {
 constexpr int64_t kDeviceCheckN = 65536;
 }  // namespace
 
+int steps_sim_set_positions(steps_sim *s, const double *x) {
+    if (!s || !x) return fail(STEPS_ERR_ARG, "null argument");
+    const bool on_device = s->N >= kDeviceCheckN;
+    int rc;
+    if (!on_device && (rc = check_finite(x, 3 * s->N))) return rc;
+    STEPS_HIP(hipSetDevice(s->device), "hipSetDevice");
+    const size_t nb = (size_t)s->N * sizeof(double);
     STEPS_HIP(hipMemcpyAsync(s->stage.ptr, x, 3 * nb, hipMemcpyHostToDevice, s->stream), "copy x");
-    STEPS_HIP(launch_pack_positions(s->stage.as<double>(), s->N, s->dp, s->stream), "pack positions");
-    STEPS_HIP(hipStreamSynchronize(s->stream), "set positions");
-    s->evaluated = s->full = s->timed = false;
-    return STEPS_OK;
-}
-
     if (on_device) {
         // before the particles change
         *s->hflag = 0;
@@ -736,6 +736,12 @@ constexpr int64_t kDeviceCheckN = 65536;
         STEPS_HIP(hipStreamSynchronize(s->stream), "check x");
         if (*s->hflag) return fail(STEPS_ERR_NONFINITE, "non-finite input value");
     }
+    STEPS_HIP(launch_pack_positions(s->stage.as<double>(), s->N, s->dp, s->stream), "pack positions");
+    STEPS_HIP(hipStreamSynchronize(s->stream), "set positions");
+    s->evaluated = s->full = s->timed = false;
+    return STEPS_OK;
+}
+
 int steps_sim_get_state(steps_sim *s, double *x, double *v) {
     if (!s) return fail(STEPS_ERR_ARG, "null sim");
     return sim_download(s, x, v, nullptr);

@@ -88,6 +88,7 @@ struct EvalPlan {
     bool bh = false;
     double bh_theta = 0, bh_particle_radius = 0;  // opening angle, ParticleRadi
     int bh_order = 2;
+    int bh_ranges = 1;     // ranges of the item list walked by workgroups of their own (bh_split)
     // the randomised octree (RANDOMIZE_BH) and its draws u0..u5
     bool bh_randomize = false;
     double bh_u[6] = {0, 0, 0, 0, 0, 0};
@@ -198,6 +199,9 @@ hipError_t launch_sort_words(const uint32_t *const *words, int nwords, int64_t n
 // recorded between the tree build and the traversal.
 int64_t bh_item_capacity(int64_t n);
 size_t bh_scratch_bytes(int64_t n);
+int bh_split(int topology, int64_t n);
+void least_scratch(EvalPlan &p);  // the choices that take the least scratch
+size_t bh_part_bytes(int64_t n, int ranges);  // the ranges' sums, after it; 0 for one range
 hipError_t launch_bh_forces(const EvalPlan &p, const DeviceParticles &dp, void *scratch, double *F,
                             hipStream_t stream, hipEvent_t ev_tree_end);
 
@@ -205,12 +209,12 @@ hipError_t launch_bh_forces(const EvalPlan &p, const DeviceParticles &dp, void *
 hipError_t launch_pack(const double *x, const double *M, const double *soft, int64_t n,
                        DeviceParticles &dp, hipStream_t stream);
 // Replace positions only (AoS x [3n], device) keeping masses.
+// Writes 1 to *flag (pinned host memory) when one of x[0..count) is not finite.
+hipError_t launch_check_finite(const double *x, int64_t count, int *flag, hipStream_t stream);
 hipError_t launch_pack_positions(const double *x, int64_t n, DeviceParticles &dp,
                                  hipStream_t stream);
 // DeviceParticles positions -> AoS x [3n] (device).
 hipError_t launch_unpack_positions(const DeviceParticles &dp, double *x, hipStream_t stream);
-// Writes 1 to *flag (pinned host memory) when one of x[0..count) is not finite.
-hipError_t launch_check_finite(const double *x, int64_t count, int *flag, hipStream_t stream);
 
 // KDK pieces (kdk_kernels.hip).  Per-step scalars live in device memory
 // (written by the host before the launch) so that captured graphs replay.

@@ -128,6 +128,11 @@ extern "C" int steps_force_eval_noalloc(const steps_force_desc *d, int64_t N, co
         return n;
     };
     size_t need = total();
+    if (need > kNoAllocScratchBytes && p.bh) {
+        least_scratch(p);
+        pieces[6] = scratch_bytes(p);
+        need = total();
+    }
     if (need > kNoAllocScratchBytes && p.sym) {
         // fewer cells of a pair-symmetric evaluation at a time: the same sums
         const size_t rest = need - ((pieces[6] + 255) & ~(size_t)255);

@@ -95,7 +95,7 @@ size_t footprint(const steps_force_desc &d, int64_t N, bool lean) {
         if (prec == STEPS_PREC_MIXED && !desc_mixed_capable(d)) continue;
         dd.precision = prec;
         if (make_plan(dd, N, 0, N - 1, p) != STEPS_OK) continue;
-        if (lean) p.sym_launch_cells = std::min(p.sym_launch_cells, 1);
+        if (lean) least_scratch(p);
         scratch = std::max(scratch, scratch_bytes(p));
     }
     b += scratch;
