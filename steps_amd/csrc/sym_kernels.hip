@@ -636,9 +636,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // 192 table values per pair, and those reads are what the pair costs; here
 // they serve both sides.  Records are in z pencils.  Before each source tile
 // the workgroup copies the table window that its rows' and the tile's cell
-// columns can reach into LDS, unfolded, so that a stencil is 16 rows at fixed
-// strides from one address: no mirror or wrap per row (638 -> 468 VALU per
-// pair against the folded window of body_t3_win).  A window that does not fit
+// columns can reach into LDS, unfolded in x and y, so that a stencil is 16
+// rows at fixed strides from one address: no mirror or wrap per row (638 ->
+// 468 VALU per pair against the folded window of body_t3_win).  ZF: a table
+// mirrored in z as well is looked up at |dz| and its z component takes the sign
+// of dz, so a window row holds the nodes of z >= 0 only and the window 1.65
+// times the rows (FP64 24^3 9.7 -> 7.0 ms, 32^3 34 -> 22.7, 40^3 80 -> 68, 56^3
+// 443 -> 411; mixed 24^3 5.0 -> 3.6, 40^3 42 -> 36.8).  A window that does not fit
 // is taken in up to three bands of y rows, each its own pass over the steps in
 // which the lanes whose stencils lie in the band take part (32^3 46 -> 34 ms;
 // more bands gain nothing); a wider one leaves the tile on the global table,
@@ -655,28 +659,35 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // words) and rows 4, planes 8 words apart mod 16.  Measured at 60^3: folded
 // body_t3_win rows 737 ms, this layout 615; planes at 4 or 2 mod 16 695 / 652,
 // rows of 104 or 108 words 630 / 633, z components as single 8-byte reads 710.
-// Measured against the one-sided kernels (ms): 24^3 22.8 -> 9.7, 32^3 91 -> 34,
-// 40^3 310 -> 80, 48^3 739 -> 194, 56^3 1440 -> 443, 64^3 2000 -> 850.
+// Measured against the one-sided kernels (ms): 24^3 22.7 -> 7.0, 32^3 91 -> 22.7,
+// 40^3 310 -> 68, 48^3 739 -> 178, 56^3 1440 -> 411.
 //
 // MX, mixed precision: the displacement is formed and wrapped in FP64 and
 // rounded once, the rest of a pair is FP32, with 16-byte nodes (64 reads a
 // pair); FP32 sums run over one wave's steps of a tile and are added in FP64,
 // pairs within the softening bound are done again in FP64 (body_t3_mixed's
 // scheme).  VALU (420 per pair) and LDS (490 cycles) are about even there:
-// 24^3 14.6 -> 5.0 ms, 40^3 190 -> 42, 48^3 490 -> 103, 56^3 1092 -> 235.
+// 24^3 14.6 -> 3.6 ms, 40^3 190 -> 36.8, 48^3 490 -> 97, 56^3 1092 -> 230.
 // ---------------------------------------------------------------------------
 constexpr int kSymT3Win = 9800;   // 16-byte words: 153 KB, one workgroup per CU
 constexpr int kT3Waves = 8;
 constexpr int kT3Bands = 3;       // most bands of a window (see sym_t3_kernel)
 constexpr int kT3MaxWinNg = 63;   // the window row is laid out for tables up to this grid
-constexpr int kT3Row = 100;       // words a window row: 66 (x, y) nodes and 34 z pairs
-constexpr int kT3Row32 = 68;      // ... of FP32 nodes, one word each
-constexpr int kT3RunOff[4] = {0, 17, 34, 50};  // (x, y) nodes by z mod 4: start of each run
-constexpr int kT3ZPairs = 66;     // start of the z components, two nodes a word
 
-__device__ __forceinline__ unsigned t3_run_start(unsigned r) {
-    return r == 0u ? kT3RunOff[0] : (r == 1u ? kT3RunOff[1] : (r == 2u ? kT3RunOff[2] : kT3RunOff[3]));
-}
+// A window row, in words: the (x, y) nodes in four runs by z mod 4, then the z
+// components, two nodes a word; FP32 nodes take one word each and have no z
+// part.  All z nodes (66), or those of z >= 0 (35).
+template <bool ZF> struct T3Row;
+template <> struct T3Row<false> {
+    static constexpr int words = 100, words32 = 68, zpairs = 66;
+    static __device__ __forceinline__ constexpr unsigned run(unsigned r) {
+        return r == 0u ? 0u : (r == 1u ? 17u : (r == 2u ? 34u : 50u));
+    }
+};
+template <> struct T3Row<true> {
+    static constexpr int words = 60, words32 = 36, zpairs = 36;
+    static __device__ __forceinline__ constexpr unsigned run(unsigned r) { return 9u * r; }
+};
 
 // Words from one x plane of window rows to the next: 8 (mod 16), which with
 // rows 4 (mod 16) apart spreads the 2 x 2 neighbouring rows that the lanes
@@ -725,11 +736,28 @@ __device__ __forceinline__ int t3_weights(float d, const KScalars &k, float w[4]
     return (int)uf;
 }
 
-template <int G, bool MX>
+// The z axis of a window that holds z >= 0: d >= 0, indices from node `first`
+// (the one at or below z = 0, which rounding must not pass).
+template <class T> __device__ __forceinline__ int t3_weights_from(T d, const KScalars &k, int first, T w[4]) {
+    T u;
+    if constexpr (sizeof(T) == 8) u = (d + k.L * 0.5) * k.inv_gs - 0.5;
+    else u = (d + k.halfLf) * k.inv_gsf - 0.5f;
+    u -= (T)first;
+    const T uf = fmax(floor(u), (T)0);
+    const T t = u - uf;
+    const T t2 = t * t, t3 = t * t2;
+    w[0] = (T)-0.5 * t3 + t2 - (T)0.5 * t;
+    w[1] = (T)1.5 * t3 - (T)2.5 * t2 + (T)1.0;
+    w[2] = (T)-1.5 * t3 + (T)2.0 * t2 + (T)0.5 * t;
+    w[3] = (T)0.5 * t3 - (T)0.5 * t2;
+    return (int)uf;
+}
+
+template <int G, bool MX, bool ZF>
 __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) {
     constexpr int W = kT3Waves, RW = W / G;  // waves; waves of different rows
     constexpr int kSteps = kTile / G;
-    constexpr int kRow = MX ? kT3Row32 : kT3Row;
+    constexpr int kRow = MX ? T3Row<ZF>::words32 : T3Row<ZF>::words, kZPairs = T3Row<ZF>::zpairs;
     using real = std::conditional_t<MX, float, double>;
     __shared__ __align__(16) double win[2 * kSymT3Win];
     __shared__ __align__(16) double2 jbuf[2][kTile];
@@ -754,6 +782,9 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
     double fx = 0.0, fy = 0.0, fz = 0.0;
     const int Ng = k.ng, lo = k.t3_lo;
     const unsigned NY = (unsigned)(Ng - lo), NZ = (unsigned)(Ng + 3), NZ3 = 3u * NZ;
+    // the window's z nodes: entries zf .. of a table row (ZF: from one below z = 0)
+    const int zf = ZF ? (Ng - 1) / 2 : 0;
+    const unsigned wz = NZ - (unsigned)zf, wz3 = 3u * wz;
 
     int bxmin = 0, bxmax = 0, bymin = 0, bymax = 0;  // the rows' cell columns
     {
@@ -831,26 +862,26 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                     const unsigned mx = (unsigned)(fx_ ? Ng - 1 - lo - jx : jx - lo);
                     const unsigned my = (unsigned)(fy_ ? Ng - 1 - lo - jy : jy - lo);
                     if constexpr (MX) {
-                        const float4 *src = a.tab32 + (mx * NY + my) * NZ;
+                        const float4 *src = a.tab32 + (mx * NY + my) * NZ + zf;
                         float4 *dst = (float4 *)win + ax * plane + ay * kRow;
-                        for (unsigned z = lane; z < NZ; z += 64) {
+                        for (unsigned z = lane; z < wz; z += 64) {
                             float4 v = src[z];
                             if (fx_) v.x = -v.x;
                             if (fy_) v.y = -v.y;
-                            dst[t3_run_start(z & 3u) + (z >> 2)] = v;
+                            dst[T3Row<ZF>::run(z & 3u) + (z >> 2)] = v;
                         }
                     } else {
-                        const double *src = a.table + (mx * NY + my) * NZ3;
+                        const double *src = a.table + (mx * NY + my) * NZ3 + 3 * zf;
                         double *dst = win + 2 * (ax * plane + ay * kRow);
-                        for (unsigned o = lane; o < NZ3; o += 64) {
+                        for (unsigned o = lane; o < wz3; o += 64) {
                             const unsigned z = o / 3u, c = o - 3u * z;
                             double v = src[o];
                             if (c == 0u && fx_) v = -v;
                             if (c == 1u && fy_) v = -v;
-                            dst[c < 2u ? 2u * (t3_run_start(z & 3u) + (z >> 2)) + c : 2u * kT3ZPairs + z] = v;
+                            dst[c < 2u ? 2u * (T3Row<ZF>::run(z & 3u) + (z >> 2)) + c : 2u * kZPairs + z] = v;
                         }
                         // z values past the run meet zero weights
-                        const unsigned pad = 2u * kT3ZPairs + NZ + lane;
+                        const unsigned pad = 2u * kZPairs + wz + lane;
                         if (pad < 2u * kRow) dst[pad] = 0.0;
                     }
                 }
@@ -871,10 +902,18 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                 unsigned rx = 0, ry = 0, iz = 0;
                 bool in = false, out = band == 0;
                 if (bands > 0) {
-                    const int ix = t3_weights(dx, k, wxs), iy = t3_weights(dy, k, wys), izi = t3_weights(dz, k, wzs);
-                    iz = min((unsigned)izi, (unsigned)(izi + Ng));  // layout z index of the stencil's first node
+                    const int ix = t3_weights(dx, k, wxs), iy = t3_weights(dy, k, wys);
+                    unsigned nz = (unsigned)Ng;
+                    if constexpr (ZF) {
+                        // |dz|: the z component changes sign with dz, the others are even in it
+                        iz = (unsigned)t3_weights_from(dz < 0 ? -dz : dz, k, zf, wzs);
+                        nz -= (unsigned)zf;
+                    } else {
+                        const int izi = t3_weights(dz, k, wzs);
+                        iz = min((unsigned)izi, (unsigned)(izi + Ng));  // layout z index of the stencil's first node
+                    }
                     const bool inx = t3_win_rel(ix, wx0, nx, Ng, rx), iny = t3_win_rel(iy, wy0, ny, Ng, ry);
-                    const bool held = inx && iny && iz < (unsigned)Ng;
+                    const bool held = inx && iny && iz < nz;
                     ry -= (unsigned)y0;
                     in = held && ry < (unsigned)bys;
                     out = band == 0 && !held;
@@ -907,7 +946,7 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                     const unsigned base = rx * (unsigned)plane + ry * (unsigned)kRow;
                     unsigned at[4];
 #pragma unroll
-                    for (unsigned q = 0; q < 4; ++q) at[q] = base + kT3RunOff[q] + blk + (q < r ? 1u : 0u);
+                    for (unsigned q = 0; q < 4; ++q) at[q] = base + T3Row<ZF>::run(q) + blk + (q < r ? 1u : 0u);
                     real s0 = 0, s1 = 0, s2 = 0;
                     if constexpr (MX) {
 #pragma unroll
@@ -939,7 +978,7 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                         const double wz5[5] = {r1 ? 0.0 : wzs[0], r1 ? wzs[0] : wzs[1], r1 ? wzs[1] : wzs[2],
                                                r1 ? wzs[2] : wzs[3], r1 ? wzs[3] : 0.0};
                         const double2 *w2 = (const double2 *)win;
-                        const unsigned zat = base + kT3ZPairs + (iz >> 1);
+                        const unsigned zat = base + kZPairs + (iz >> 1);
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             const double2 *pk[4], *pz = w2 + zat + i * plane;
@@ -966,7 +1005,7 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                     }
                     Dx = s0;
                     Dy = s1;
-                    Dz = s2;
+                    Dz = ZF && dz < 0 ? -s2 : s2;
                 } else if (out) {
                     if constexpr (MX) {
                         T3Stencil32 st;
@@ -1359,16 +1398,16 @@ bool sym_variant(const EvalPlan &p) {
 
 // Rows of a T3 Ewald workgroup: with c particles per cell column, R rows and
 // a tile span about (R + 64) / c columns in y, and a window of 5 planes holds
-// 98 / 5 = 19 rows of it, 5 + 2 of them the stencil's and the partial columns
-// (FP32 nodes: 28).
-// Measured (ms, 256 / 128 / 64 rows): 56^3 (c = 44) 443 / 471 / -, 48^3 (28)
-// 216 / 207 / 239, 44^3 (21) 251 / 131 / 150, 40^3 (16) 172 / 86 / 90, 36^3
-// (12) 95 / 92 / 52; 512 rows: 618 against 621 at 60^3, 538 against 443 at 56^3.
-// Mixed, 256 / 128: 44^3 65.4 / 71.2, 42^3 51.4 / 55.3, 40^3 41.8 / 42.6.
+// 163 / 5 = 32 rows of it (FP32 nodes: 54), 5 + 2 of them the stencil's and
+// the partial columns.  More rows share a window until it needs bands.
+// Measured (ms, 64 / 128 / 256 rows): 24^3 (c = 3.5) 7.0 / 7.1 / 9.5, 28^3
+// (5.5) 12.7 / 14.3 / 15.1, 32^3 (8.3) 23.7 / 22.7 / 27.2, 36^3 (11.8) 44.7 /
+// 40.0 / 45.5, 40^3 (16.1) 79 / 71 / 68, 48^3 (28) 212 / 188 / 178.  Mixed: 24^3
+// 3.6 / 4.0 / 4.0, 28^3 7.6 / 6.6 / 8.4, 32^3 14.1 / 12.4 / 12.0, 40^3 48 / 40 / 37.
 int sym_t3_rows(const EvalPlan &p) {
     const double c = (double)p.N / ((double)p.t3_ng * p.t3_ng);
     const bool mx = p.precision == STEPS_PREC_MIXED;
-    return 320 <= (mx ? 20 : 12) * c ? 256 : (192 <= (mx ? 18 : 12) * c ? 128 : 64);
+    return c >= (mx ? 8.0 : 14.0) ? 256 : (c >= (mx ? 4.5 : 7.0) ? 128 : 64);
 }
 
 int64_t sym_min_n(const EvalPlan &p) {
@@ -1405,17 +1444,19 @@ void launch_sym_kernel(const EvalPlan &p, const SymArgs &a, int cells, hipStream
     if (p.variant == PV_T3_EWALD) {
         const dim3 block(64 * kT3Waves);
         const bool mx = p.precision == STEPS_PREC_MIXED;
-        const int rows = p.sym_block_rows;
-        if (rows == 256) {
-            if (mx) hipLaunchKernelGGL((sym_t3_kernel<2, true>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((sym_t3_kernel<2, false>), grid, block, 0, st, a);
-        } else if (rows == 128) {
-            if (mx) hipLaunchKernelGGL((sym_t3_kernel<4, true>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((sym_t3_kernel<4, false>), grid, block, 0, st, a);
-        } else {
-            if (mx) hipLaunchKernelGGL((sym_t3_kernel<8, true>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((sym_t3_kernel<8, false>), grid, block, 0, st, a);
-        }
+        auto go = [&](auto g) {
+            constexpr int G = decltype(g)::value;
+            if (p.t3_lo > 0) {  // even and odd through z = 0 too (odd, and mirrored in x and y)
+                if (mx) hipLaunchKernelGGL((sym_t3_kernel<G, true, true>), grid, block, 0, st, a);
+                else hipLaunchKernelGGL((sym_t3_kernel<G, false, true>), grid, block, 0, st, a);
+            } else {
+                if (mx) hipLaunchKernelGGL((sym_t3_kernel<G, true, false>), grid, block, 0, st, a);
+                else hipLaunchKernelGGL((sym_t3_kernel<G, false, false>), grid, block, 0, st, a);
+            }
+        };
+        if (p.sym_block_rows == 256) go(IntC<2>{});
+        else if (p.sym_block_rows == 128) go(IntC<4>{});
+        else go(IntC<8>{});
         return;
     }
     if (is_s1r2_lookup(p.variant)) {

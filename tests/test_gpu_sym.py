@@ -163,3 +163,30 @@ def test_scratch_does_not_change_the_sums(steps, N):
     rc = lib.steps_force_eval_noalloc(C.byref(d), N, _abi._ptr(x), _abi._ptr(M), _abi._ptr(h), _abi._ptr(G), 0, N - 1)
     assert rc == 0, lib.steps_last_error()
     assert np.array_equal(G.reshape(-1, 3), F)
+
+
+@pytest.mark.parametrize("ng", [3, 4, 8, 31, 62, 63])
+@pytest.mark.parametrize("N", [700, 30011])
+def test_t3_ewald_grids_against_oracle(steps, oracle, ng, N):
+    """Tables of even and odd grids that are mirrored in x, y and z, which the
+    window holds for z >= 0 only; pairs at dz = 0, at half a period and around."""
+    print(f"case pair-symmetric t3 ewald ng={ng} N={N}", flush=True)
+    x, M, h, L = particles("t3", N, N)
+    x[400:460, 2] = 10.0 + 1e-13 * (np.arange(60) % 5)
+    x[460:520, 2] = 10.0 + L / 2 + 1e-9 * (np.arange(60) - 30)
+    x %= L
+    g = (np.arange(ng) - (ng - 1) / 2) * (L / ng)
+    X, Y, Z = np.meshgrid(g, g, g, indexing="ij")
+    f = 1e-6 * np.exp(-(X * X + Y * Y + Z * Z) / (0.1 * L * L))
+    T = np.ascontiguousarray(np.stack([X * f, Y * f, Z * f], axis=-1).reshape(-1))
+    d, keep = steps.make_desc(steps.TOPO_T3, is_periodic=2, L=L, t3_table=T)
+    p = oracle.params(1, is_periodic=2, L=L, t3_table=T, interp_order=4)
+    rows = np.unique(np.concatenate([np.arange(395, 525, 3), np.linspace(0, N - 1, 24).astype(int)])).astype(np.int32)
+    F = steps.force_eval(d, x, M, h)
+    e = rel_err(F[rows], oracle.forces_rows(p, x, M, h, rows))
+    report(f"pair-symmetric t3 ewald ng={ng} N={N}", e)
+    assert np.all(np.isfinite(F)) and np.median(e) <= 1e-12 and e.max() <= 1e-9
+    dm, keepm = steps.make_desc(steps.TOPO_T3, is_periodic=2, L=L, t3_table=T, precision=steps.PREC_MIXED)
+    em = rel_err(steps.force_eval(dm, x, M, h), F)
+    report(f"pair-symmetric t3 ewald ng={ng} N={N} mixed vs fp64", em)
+    assert np.median(em) <= 2e-6 and np.percentile(em, 99) <= 1e-5
