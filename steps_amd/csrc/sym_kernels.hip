@@ -39,6 +39,7 @@
 #include "pair_device.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace steps {
@@ -640,9 +641,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // rows at fixed strides from one address: no mirror or wrap per row (638 ->
 // 468 VALU per pair against the folded window of body_t3_win).  ZF: a table
 // mirrored in z as well is looked up at |dz| and its z component takes the sign
-// of dz, so a window row holds the nodes of z >= 0 only and the window 1.65
-// times the rows (FP64 24^3 9.7 -> 7.0 ms, 32^3 34 -> 22.7, 40^3 80 -> 68, 56^3
-// 443 -> 411; mixed 24^3 5.0 -> 3.6, 40^3 42 -> 36.8).  A window that does not fit
+// of dz, so a window row holds the nodes of z >= 0 only and the window 1.3
+// times the rows, 1.9 in FP32 (FP64 24^3 9.7 -> 7.0 ms, 32^3 34 -> 21.4, 40^3 80
+// -> 61, 56^3 443 -> 349; mixed 24^3 5.0 -> 3.6, 40^3 42 -> 35.5).  A window that does not fit
 // is taken in up to three bands of y rows, each its own pass over the steps in
 // which the lanes whose stencils lie in the band take part (32^3 46 -> 34 ms;
 // more bands gain nothing); a wider one leaves the tile on the global table,
@@ -651,23 +652,24 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // sparse boxes (few particles per column) take G = 4 or 8.  After the tile
 // the window's memory takes the waves' source sums.
 //
-// Bound by LDS: ~107 reads of 16 bytes per pair, 4.3 cycles each, and as much
-// again in bank conflicts (876 LDS cycles of 978 per wave step at 60^3).  In
+// Bound by LDS: 96 reads of 16 bytes per pair (ZF; 112 else), 4.3 cycles each,
+// and as much again in bank conflicts (876 LDS cycles of 978 per wave step at
+// 60^3 with 112).  In
 // the lanes of one read the source and row indices both advance, so their
 // stencils sit a few z nodes apart on 2 x 2 neighbouring rows; the (x, y)
 // nodes are therefore stored by z mod 4 (lanes a few nodes apart then share
-// words) and rows 4, planes 8 words apart mod 16.  Measured at 60^3: folded
+// words) and rows 4 (ZF: 12), planes 8 words apart mod 16.  Measured at 60^3: folded
 // body_t3_win rows 737 ms, this layout 615; planes at 4 or 2 mod 16 695 / 652,
 // rows of 104 or 108 words 630 / 633, z components as single 8-byte reads 710.
-// Measured against the one-sided kernels (ms): 24^3 22.7 -> 7.0, 32^3 91 -> 22.7,
-// 40^3 310 -> 68, 48^3 739 -> 178, 56^3 1440 -> 411.
+// Measured against the one-sided kernels (ms): 16^3 3.0 -> 1.3, 24^3 22.7 -> 7.0,
+// 32^3 91 -> 21.4, 40^3 310 -> 61, 48^3 739 -> 155, 56^3 1440 -> 349.
 //
 // MX, mixed precision: the displacement is formed and wrapped in FP64 and
 // rounded once, the rest of a pair is FP32, with 16-byte nodes (64 reads a
 // pair); FP32 sums run over one wave's steps of a tile and are added in FP64,
 // pairs within the softening bound are done again in FP64 (body_t3_mixed's
 // scheme).  VALU (420 per pair) and LDS (490 cycles) are about even there:
-// 24^3 14.6 -> 3.6 ms, 40^3 190 -> 36.8, 48^3 490 -> 97, 56^3 1092 -> 230.
+// 24^3 14.6 -> 3.6 ms, 40^3 190 -> 35.5, 48^3 490 -> 93, 56^3 1092 -> 221.
 // ---------------------------------------------------------------------------
 constexpr int kSymT3Win = 9800;   // 16-byte words: 153 KB, one workgroup per CU
 constexpr int kT3Waves = 8;
@@ -676,16 +678,19 @@ constexpr int kT3MaxWinNg = 63;   // the window row is laid out for tables up to
 
 // A window row, in words: the (x, y) nodes in four runs by z mod 4, then the z
 // components, two nodes a word; FP32 nodes take one word each and have no z
-// part.  All z nodes (66), or those of z >= 0 (35).
+// part.  All z nodes (66), or those of z >= 0 (35), whose z components then
+// stand twice, in pairs from even and (zodd) from odd nodes: a stencil's four
+// are two words at either start, where one run takes three (FP64 36^3 40 ->
+// 35 ms, 56^3 405 -> 349).
 template <bool ZF> struct T3Row;
 template <> struct T3Row<false> {
-    static constexpr int words = 100, words32 = 68, zpairs = 66;
+    static constexpr int words = 100, words32 = 68, zpairs = 66, zodd = 0;
     static __device__ __forceinline__ constexpr unsigned run(unsigned r) {
         return r == 0u ? 0u : (r == 1u ? 17u : (r == 2u ? 34u : 50u));
     }
 };
 template <> struct T3Row<true> {
-    static constexpr int words = 60, words32 = 36, zpairs = 36;
+    static constexpr int words = 76, words32 = 36, zpairs = 36, zodd = 54;
     static __device__ __forceinline__ constexpr unsigned run(unsigned r) { return 9u * r; }
 };
 
@@ -757,7 +762,8 @@ template <int G, bool MX, bool ZF>
 __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) {
     constexpr int W = kT3Waves, RW = W / G;  // waves; waves of different rows
     constexpr int kSteps = kTile / G;
-    constexpr int kRow = MX ? T3Row<ZF>::words32 : T3Row<ZF>::words, kZPairs = T3Row<ZF>::zpairs;
+    constexpr int kRow = MX ? T3Row<ZF>::words32 : T3Row<ZF>::words, kZPairs = T3Row<ZF>::zpairs,
+                  kZOdd = T3Row<ZF>::zodd;
     using real = std::conditional_t<MX, float, double>;
     __shared__ __align__(16) double win[2 * kSymT3Win];
     __shared__ __align__(16) double2 jbuf[2][kTile];
@@ -879,10 +885,13 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                             if (c == 0u && fx_) v = -v;
                             if (c == 1u && fy_) v = -v;
                             dst[c < 2u ? 2u * (T3Row<ZF>::run(z & 3u) + (z >> 2)) + c : 2u * kZPairs + z] = v;
+                            if (ZF && c == 2u && z > 0u) dst[2u * kZOdd + z - 1u] = v;
                         }
-                        // z values past the run meet zero weights
-                        const unsigned pad = 2u * kZPairs + wz + lane;
-                        if (pad < 2u * kRow) dst[pad] = 0.0;
+                        if constexpr (!ZF) {
+                            // z values past the run meet zero weights
+                            const unsigned pad = 2u * kZPairs + wz + lane;
+                            if (pad < 2u * kRow) dst[pad] = 0.0;
+                        }
                     }
                 }
             }
@@ -978,7 +987,7 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                         const double wz5[5] = {r1 ? 0.0 : wzs[0], r1 ? wzs[0] : wzs[1], r1 ? wzs[1] : wzs[2],
                                                r1 ? wzs[2] : wzs[3], r1 ? wzs[3] : 0.0};
                         const double2 *w2 = (const double2 *)win;
-                        const unsigned zat = base + kZPairs + (iz >> 1);
+                        const unsigned zat = base + (unsigned)(ZF && r1 ? kZOdd : kZPairs) + (iz >> 1);
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             const double2 *pk[4], *pz = w2 + zat + i * plane;
@@ -989,11 +998,15 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                             for (int jj = 0; jj < 4; ++jj) {
                                 const double2 a0 = pk[0][jj * kRow], a1 = pk[1][jj * kRow], a2 = pk[2][jj * kRow],
                                               a3 = pk[3][jj * kRow];
-                                const double2 z0 = pz[jj * kRow], z1 = pz[jj * kRow + 1], z2 = pz[jj * kRow + 2];
+                                const double2 z0 = pz[jj * kRow], z1 = pz[jj * kRow + 1];
                                 const double t0 = fma(wk[3], a3.x, fma(wk[2], a2.x, fma(wk[1], a1.x, wk[0] * a0.x)));
                                 const double t1 = fma(wk[3], a3.y, fma(wk[2], a2.y, fma(wk[1], a1.y, wk[0] * a0.y)));
-                                const double t2 = fma(wz5[4], z2.x,
-                                                      fma(wz5[3], z1.y, fma(wz5[2], z1.x, fma(wz5[1], z0.y, wz5[0] * z0.x))));
+                                double t2;
+                                if constexpr (ZF)
+                                    t2 = fma(wzs[3], z1.y, fma(wzs[2], z1.x, fma(wzs[1], z0.y, wzs[0] * z0.x)));
+                                else
+                                    t2 = fma(wz5[4], pz[jj * kRow + 2].x,
+                                             fma(wz5[3], z1.y, fma(wz5[2], z1.x, fma(wz5[1], z0.y, wz5[0] * z0.x))));
                                 u0 = fma(wys[jj], t0, u0);
                                 u1 = fma(wys[jj], t1, u1);
                                 u2 = fma(wys[jj], t2, u2);
@@ -1396,18 +1409,30 @@ bool sym_variant(const EvalPlan &p) {
     return p.variant == PV_R3 || p.variant == PV_T3_NEAREST || p.variant == PV_S1R2_NEAREST;
 }
 
-// Rows of a T3 Ewald workgroup: with c particles per cell column, R rows and
-// a tile span about (R + 64) / c columns in y, and a window of 5 planes holds
-// 163 / 5 = 32 rows of it (FP32 nodes: 54), 5 + 2 of them the stencil's and
-// the partial columns.  More rows share a window until it needs bands.
-// Measured (ms, 64 / 128 / 256 rows): 24^3 (c = 3.5) 7.0 / 7.1 / 9.5, 28^3
-// (5.5) 12.7 / 14.3 / 15.1, 32^3 (8.3) 23.7 / 22.7 / 27.2, 36^3 (11.8) 44.7 /
-// 40.0 / 45.5, 40^3 (16.1) 79 / 71 / 68, 48^3 (28) 212 / 188 / 178.  Mixed: 24^3
-// 3.6 / 4.0 / 4.0, 28^3 7.6 / 6.6 / 8.4, 32^3 14.1 / 12.4 / 12.0, 40^3 48 / 40 / 37.
+// Rows of a T3 Ewald workgroup: with c particles per cell column, R rows and a
+// tile span about (R + 64) / c columns in y, and their stencils start on 4
+// rows more (a partial column at either end).  A window of 5 planes holds
+// 25 y rows (FP32 nodes: 54), 3 of them for the last stencils.  The most rows
+// that share a window need the fewest copies; the fewest bands go first.
+// Measured (ms, 64 / 128 / 256 / 512 rows): 24^3 (c = 3.5) 7.0 / 8.0 / 9.8 /
+// 9.9, 28^3 (5.5) 14.2 / 13.2 / 18.1 / 24.6, 32^3 (8.3) 21.5 / 25.9 / 27.1 / 53,
+// 40^3 (16) 71 / 62 / 68 / 75, 48^3 (28) 192 / 165 / 155 / 190, 56^3 (44) 448 /
+// 383 / 361 / 349.  Mixed: 24^3 3.6 / 4.0 / 4.0, 28^3 7.6 / 6.6 / 8.4, 32^3 14.2 /
+// 12.4 / 12.0 / 17.7, 40^3 48 / 40 / 37 / 36, 56^3 306 / 253 / 231 / 221.
 int sym_t3_rows(const EvalPlan &p) {
     const double c = (double)p.N / ((double)p.t3_ng * p.t3_ng);
-    const bool mx = p.precision == STEPS_PREC_MIXED;
-    return c >= (mx ? 8.0 : 14.0) ? 256 : (c >= (mx ? 4.5 : 7.0) ? 128 : 64);
+    const int row = p.precision == STEPS_PREC_MIXED ? T3Row<true>::words32 : T3Row<true>::words;
+    const int starts = (kSymT3Win / 5 - 12) / row - 3;
+    int best = 64;
+    double fewest = INFINITY;
+    for (int rows = 64; rows <= 64 * kT3Waves; rows *= 2) {
+        const double bands = std::ceil(((rows + 64) / c + 4.0) / starts);
+        if (bands <= kT3Bands && bands <= fewest) {
+            best = rows;
+            fewest = bands;
+        }
+    }
+    return best;
 }
 
 int64_t sym_min_n(const EvalPlan &p) {
@@ -1454,7 +1479,8 @@ void launch_sym_kernel(const EvalPlan &p, const SymArgs &a, int cells, hipStream
                 else hipLaunchKernelGGL((sym_t3_kernel<G, false, false>), grid, block, 0, st, a);
             }
         };
-        if (p.sym_block_rows == 256) go(IntC<2>{});
+        if (p.sym_block_rows == 512) go(IntC<1>{});
+        else if (p.sym_block_rows == 256) go(IntC<2>{});
         else if (p.sym_block_rows == 128) go(IntC<4>{});
         else go(IntC<8>{});
         return;
