@@ -386,7 +386,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // ---------------------------------------------------------------------------
 template <int V, int NI>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_mixed_kernel(const SymArgs a) {
-    constexpr int kFlush = 64 / NI;
+    constexpr int kFlush = V == PV_R3 ? 64 / NI : 32 / NI;
     __shared__ __align__(1024) float4 jbuf[2][kTile];
     __shared__ double gsum[2][kSymWaves][3][kTile];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -486,6 +486,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             bnd = bnd || fabsf(h) < k.wrap_epsf;
             return h > 0.0f ? d - copysignf(k.Lf, d) : d;
         };
+        auto end_rows = [&] {
+#pragma unroll
+            for (int q = 0; q < NI; ++q) {
+                fx[q] += (double)ax[q];
+                fy[q] += (double)ay[q];
+                fz[q] += (double)az[q];
+                ax[q] = ay[q] = az[q] = 0.0f;
+            }
+        };
         auto steps = [&](auto near, auto wm) {
             constexpr int NEAR = decltype(near)::value;
             constexpr int WM = decltype(wm)::value;
@@ -536,6 +545,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                     __builtin_amdgcn_wave_barrier();
                 }
                 gx = gy = gz = 0.0f;
+                if (V != PV_R3) end_rows();
             }
         };
         auto variants = [&](auto near) {
@@ -551,12 +561,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         };
         if (far) variants(IntC<0>{});
         else variants(IntC<1>{});
-#pragma unroll
-        for (int q = 0; q < NI; ++q) {
-            fx[q] += (double)ax[q];
-            fy[q] += (double)ay[q];
-            fz[q] += (double)az[q];
-        }
+        if (V == PV_R3) end_rows();
         if (__any(close)) {
             // rare: those pairs in FP64 from the FP64 records
             double cx = 0.0, cy = 0.0, cz = 0.0;
@@ -666,13 +671,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 //
 // MX, mixed precision: the displacement is formed and wrapped in FP64 and
 // rounded once, the rest of a pair is FP32, with 16-byte nodes (64 reads a
-// pair); FP32 sums run over one wave's steps of a tile and are added in FP64,
+// pair); FP32 sums run over eight steps and are added in FP64,
 // pairs within the softening bound are done again in FP64 (body_t3_mixed's
 // scheme).  VALU (420 per pair) and LDS (490 cycles) are about even there:
 // 24^3 14.6 -> 3.6 ms, 40^3 190 -> 35.5, 48^3 490 -> 93, 56^3 1092 -> 221.
 // ---------------------------------------------------------------------------
 constexpr int kSymT3Win = 9800;   // 16-byte words: 153 KB, one workgroup per CU
 constexpr int kT3Waves = 8;
+constexpr int kMxRun = 8;         // mixed: steps of an FP32 sum
 constexpr int kT3Bands = 3;       // most bands of a window (see sym_t3_kernel)
 constexpr int kT3MaxWinNg = 63;   // the window row is laid out for tables up to this grid
 
@@ -730,7 +736,9 @@ __device__ __forceinline__ int t3_weights(double d, const KScalars &k, double w[
     return (int)uf;
 }
 __device__ __forceinline__ int t3_weights(float d, const KScalars &k, float w[4]) {
-    const float u = (d + k.halfLf) * k.inv_gsf - 0.5f;
+    // from the centre node, not the edge: u is at most half as large, and small
+    // where d is, so t keeps more of its bits
+    const float u = fmaf(d, k.inv_gsf, (k.ng & 1) ? 0.0f : 0.5f);
     const float uf = floorf(u);
     const float t = u - uf;
     const float t2 = t * t, t3 = t * t2;
@@ -738,16 +746,15 @@ __device__ __forceinline__ int t3_weights(float d, const KScalars &k, float w[4]
     w[1] = 1.5f * t3 - 2.5f * t2 + 1.0f;
     w[2] = -1.5f * t3 + 2.0f * t2 + 0.5f * t;
     w[3] = 0.5f * t3 - 0.5f * t2;
-    return (int)uf;
+    return (int)uf + (k.ng - 1) / 2;
 }
 
 // The z axis of a window that holds z >= 0: d >= 0, indices from node `first`
 // (the one at or below z = 0, which rounding must not pass).
 template <class T> __device__ __forceinline__ int t3_weights_from(T d, const KScalars &k, int first, T w[4]) {
     T u;
-    if constexpr (sizeof(T) == 8) u = (d + k.L * 0.5) * k.inv_gs - 0.5;
-    else u = (d + k.halfLf) * k.inv_gsf - 0.5f;
-    u -= (T)first;
+    if constexpr (sizeof(T) == 8) u = (d + k.L * 0.5) * k.inv_gs - 0.5 - (double)first;
+    else u = fmaf(d, k.inv_gsf, (k.ng & 1) ? 0.0f : 0.5f);
     const T uf = fmax(floor(u), (T)0);
     const T t = u - uf;
     const T t2 = t * t, t3 = t * t2;
@@ -897,8 +904,23 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
             }
             __syncthreads();  // the window is complete
             real gx = 0, gy = 0, gz = 0, ax = 0, ay = 0, az = 0;
+            // mixed: the FP32 sums of a run of steps onto FP64 ones; a run moves
+            // the sources kMxRun lanes down, and their sums with them
+            constexpr bool kRuns = MX && kSteps > kMxRun;
+            double bx = 0.0, by = 0.0, bz = 0.0;
+            auto end_run = [&] {
+                fx += (double)ax;
+                fy += (double)ay;
+                fz += (double)az;
+                const int from = (lane + kMxRun) & 63;
+                bx = __shfl(bx, from, 64) + (double)gx;
+                by = __shfl(by, from, 64) + (double)gy;
+                bz = __shfl(bz, from, 64) + (double)gz;
+                ax = ay = az = gx = gy = gz = 0;
+            };
 #pragma unroll 1
             for (int s = 0; s < kSteps; ++s) {
+                if (kRuns && s > 0 && s % kMxRun == 0) end_run();
                 const int id = (lane + s0 + s) & 63;
                 const double2 pa = jbuf[0][id], pb = jbuf[1][id];
                 // the displacement is formed and wrapped in FP64 (mixed: then rounded once)
@@ -1047,13 +1069,13 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
                 gy = from_next_lane(mad(mr, py, gy));
                 gz = from_next_lane(mad(mr, pz, gz));
             }
-            // the tile's sums (mixed: FP32 over at most 64 pairs) onto the FP64 ones
+            if (kRuns) end_run();
             fx += (double)ax;
             fy += (double)ay;
             fz += (double)az;
-            hx += (double)gx;
-            hy += (double)gy;
-            hz += (double)gz;
+            hx += kRuns ? bx : (double)gx;
+            hy += kRuns ? by : (double)gy;
+            hz += kRuns ? bz : (double)gz;
         }
         if (MX && __any(near)) {
             // rare: the pairs within the bound, in FP64 with the FP64 table
