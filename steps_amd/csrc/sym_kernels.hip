@@ -1161,8 +1161,8 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
 // displacement is formed and wrapped in FP64 and rounded once -- the lanes of
 // a step hold different sources, so there is no common centre to take FP32
 // offsets from, and no image can be chosen differently than in FP64 -- the
-// rest of a pair is FP32 (FP32 copy of the table), FP32 sums run over the 64
-// pairs of a tile and are added in FP64, and pairs within the softening bound
+// rest of a pair is FP32 (FP32 copy of the table), FP32 sums run over eight
+// steps and are added in FP64 (over a tile's 64, three times the error of a row), and pairs within the softening bound
 // are done again in FP64.  Measured against the one-sided kernels (resident
 // calls on the cylinder, ms): N = 262144 FP64 CIC 182 -> 92, TSC 296 -> 146,
 // mixed CIC 111 -> 66, TSC 183 -> 94; N = 32799 FP64 CIC 6.6 -> 2.1, TSC 10.3
@@ -1250,9 +1250,22 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         const double B = bb * bb;
         const float Bf = (float)(bb * (1.0 + 1e-5)) * (float)(bb * (1.0 + 1e-5));  // mixed: widened
         real gx = 0, gy = 0, gz = 0, ax = 0, ay = 0, az = 0;
+        double hx = 0.0, hy = 0.0, hz = 0.0;
+        // a run's sums onto the FP64 ones (sym_t3_kernel's end_run)
+        auto end_run = [&] {
+            fx += (double)ax;
+            fy += (double)ay;
+            fz += (double)az;
+            const int from = (lane + kMxRun) & 63;
+            hx = __shfl(hx, from, 64) + (double)gx;
+            hy = __shfl(hy, from, 64) + (double)gy;
+            hz = __shfl(hz, from, 64) + (double)gz;
+            ax = ay = az = gx = gy = gz = 0;
+        };
         bool near = false;
 #pragma unroll 1
         for (int s = 0; s < kTile; ++s) {
+            if (MX && s > 0 && s % kMxRun == 0) end_run();
             const int id = (lane + s) & 63;
             const double2 pa = jbuf[0][id], pb = jbuf[1][id];
             const real dx = (real)(pa.x - xi), dy = (real)(pa.y - yi), dz = (real)wrap_half(pb.x - zi, k);
@@ -1287,10 +1300,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             gy = from_next_lane(mad(si, dy, gy));
             gz = from_next_lane(mad(mr, pz, gz));
         }
-        fx += (double)ax;
-        fy += (double)ay;
-        fz += (double)az;
-        double hx = (double)gx, hy = (double)gy, hz = (double)gz;
+        if (MX) {
+            end_run();
+        } else {
+            fx += ax;
+            fy += ay;
+            fz += az;
+            hx = gx;
+            hy = gy;
+            hz = gz;
+        }
         if (MX && __any(near)) {
             // rare: the pairs within the bound, in FP64 with the FP64 table
             double cx = 0.0, cy = 0.0, cz = 0.0;
