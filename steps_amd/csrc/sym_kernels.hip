@@ -1601,11 +1601,14 @@ void sym_plan(EvalPlan &p) {
     p.sym_blocks = (int)((p.N + p.sym_block_rows - 1) / p.sym_block_rows);
     const int tb = p.sym_block_rows / kTile, offsets = p.sym_blocks / 2 + 1;
     // Tasks of several offsets where there are plenty (fewer row-sum slots),
-    // of parts of an offset where there are few (workgroups to fill the chip).
+    // of parts of an offset where there are few: at 4 workgroups a CU the chip
+    // holds 1024, and twice that leaves a short last wave (at least 1100 / 2200
+    // tasks, ms: R3 N = 16384 0.239 / 0.226, 30000 0.554 / 0.522, mixed 30000
+    // 0.411 / 0.390, T3 nearest 32^3 0.750 / 0.727; 4400 gains nothing).
     int tiles = tb;
     if ((int64_t)p.sym_blocks * offsets >= 16384) tiles = 2 * tb;
     if ((int64_t)p.sym_blocks * offsets >= 4 * 16384) tiles = 4 * tb;
-    while (tiles > 1 && tiles <= tb && (int64_t)p.sym_blocks * offsets * (tb / tiles) < 1100) tiles /= 2;
+    while (tiles > 1 && tiles <= tb && (int64_t)p.sym_blocks * offsets * (tb / tiles) < 2200) tiles /= 2;
     p.sym_task_tiles = tiles;
     const SymShape s = sym_shape(p);
     p.sym_cells = s.cells;
