@@ -1162,13 +1162,86 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
 // a step hold different sources, so there is no common centre to take FP32
 // offsets from, and no image can be chosen differently than in FP64 -- the
 // rest of a pair is FP32 (FP32 copy of the table), FP32 sums run over eight
-// steps and are added in FP64 (over a tile's 64, three times the error of a row), and pairs within the softening bound
-// are done again in FP64.  Measured against the one-sided kernels (resident
-// calls on the cylinder, ms): N = 262144 FP64 CIC 182 -> 92, TSC 296 -> 146,
-// mixed CIC 111 -> 66, TSC 183 -> 94; N = 32799 FP64 CIC 6.6 -> 2.1, TSC 10.3
-// -> 4.3, mixed TSC 7.0 -> 2.6.  Bound by VALU issue.
+// steps and are added in FP64 (over a tile's 64, three times the error of a
+// row), and pairs within the softening bound are done again in FP64.  A tile
+// whose window holds every row and whose |dz| all end within half a period
+// takes the short lookup s1r2_window (CIC 93.5 -> 86 ms at N = 262144, mixed
+// CIC 11.6 -> 10.9 and TSC 17.7 -> 16.6 at N = 102400).  Against the one-sided
+// kernels (resident calls on the cylinder, ms): N = 262144 FP64 CIC 182 -> 86;
+// N = 38220 mixed TSC 8.1 -> 2.9.  Bound by VALU issue and LDS reads together.
 // ---------------------------------------------------------------------------
 constexpr int kSymS1Win = 2368;  // 16-byte words (37 KB: four workgroups per CU), two FP32 nodes a word
+
+__device__ __forceinline__ double fract_of(double v) { return __builtin_amdgcn_fract(v); }
+__device__ __forceinline__ float fract_of(float v) { return __builtin_amdgcn_fractf(v); }
+
+// s1r2_interp_win for a pair whose rho rows lie in the window (rows w0 .. w0 +
+// nw - 1, which the caller's bounds on rho ensure; the clamp only keeps a read
+// inside it) and whose |dz| is at most half a period: no test of the row or of
+// the z wrap, one address for the whole stencil, cells and offsets from one
+// coordinate each.  rxy2 = dx^2 + dy^2.
+template <int ORD, class real, class node>
+__device__ __forceinline__ void s1r2_window(const node *win, int w0, int nw, unsigned nz3, const KScalars &k,
+                                            const real rxy2, const real dz, real &q, real &Dz) {
+    constexpr bool F64 = sizeof(real) == 8;
+    constexpr int kRows = ORD == 2 ? 2 : 3;  // the stencil's rho rows, the first one at or below rho (CIC), below it (TSC)
+    real inv_rho, rho, fz, ur;
+    int iz;
+    if constexpr (F64) {
+        const double r = fmax(rxy2, 1e-300);  // on the axis: q finite, times dx = dy = 0
+        inv_rho = rsqrt_f64(r);
+        rho = r * inv_rho;
+        ur = fmin(rho * k.inv_drho, k.last_r);
+        const double half = 0.5 * (double)k.nz;
+        const double uz = ORD == 2 ? fma(dz, k.inv_dzg, half + 0.5) : fmax(fma(dz, k.inv_dzg, half), 0.0);
+        iz = (int)uz;
+        fz = fract_of(uz);
+    } else {
+        inv_rho = rxy2 > 0.0f ? __builtin_amdgcn_rsqf(rxy2) : 0.0f;
+        rho = rxy2 * inv_rho;
+        ur = fminf(rho * k.inv_drhof, k.last_rf);
+        // from the centre of the z axis: cell coordinates keep more bits there
+        const bool shift = (ORD == 2) != ((k.nz & 1) != 0);
+        const int base = ORD == 2 ? (k.nz + 1) / 2 : k.nz / 2;
+        float uz = fmaf(dz, k.inv_dzgf, shift ? 0.5f : 0.0f);
+        if (ORD != 2) uz = fmaxf(uz, -(float)base);
+        iz = (int)floorf(uz) + base;
+        fz = fract_of(uz);
+    }
+    const real um = ORD == 2 ? ur : ur + (real)0.5;
+    const int ir = (int)um - (ORD == 2 ? 0 : 1);
+    const real fr = fract_of(um);
+    const int rel = min(max(ir - w0, 0), nw - kRows);
+    const node *p = win + (__umul24((unsigned)rel, nz3) + (unsigned)iz);
+    auto mad = [](real a, real b, real c) {
+        if constexpr (F64) return fma(a, b, c);
+        else return fmaf(a, b, c);
+    };
+    real Dr;
+    if constexpr (ORD == 2) {
+        const node t00 = p[0], t01 = p[1], t10 = p[nz3], t11 = p[nz3 + 1];
+        const real a0 = mad(fr, t10.x - t00.x, t00.x), b0 = mad(fr, t11.x - t01.x, t01.x);
+        const real a1 = mad(fr, t10.y - t00.y, t00.y), b1 = mad(fr, t11.y - t01.y, t01.y);
+        Dr = mad(fz, b0 - a0, a0);
+        Dz = mad(fz, b1 - a1, a1);
+    } else {
+        const real sr = fr - (real)0.5, sz = fz - (real)0.5;
+        const real wr[3] = {(real)0.5 * ((real)0.5 - sr) * ((real)0.5 - sr), (real)0.75 - sr * sr,
+                            (real)0.5 * ((real)0.5 + sr) * ((real)0.5 + sr)};
+        const real wz[3] = {(real)0.5 * ((real)0.5 - sz) * ((real)0.5 - sz), (real)0.75 - sz * sz,
+                            (real)0.5 * ((real)0.5 + sz) * ((real)0.5 + sz)};
+        Dr = 0;
+        Dz = 0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const node *r = p + c * nz3;
+            const node a = r[0], b = r[1], d = r[2];
+            Dr = mad(wr[c], mad(wz[2], d.x, mad(wz[1], b.x, wz[0] * a.x)), Dr);
+            Dz = mad(wr[c], mad(wz[2], d.y, mad(wz[1], b.y, wz[0] * a.y)), Dz);
+        }
+    }
+    q = Dr * inv_rho;
+}
 
 template <int V, bool MX>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_s1r2_kernel(const SymArgs a) {
@@ -1263,43 +1336,55 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             ax = ay = az = gx = gy = gz = 0;
         };
         bool near = false;
+        auto steps = [&](auto fast) {
+            unsigned o = (unsigned)lane * 16u;
 #pragma unroll 1
-        for (int s = 0; s < kTile; ++s) {
-            if (MX && s > 0 && s % kMxRun == 0) end_run();
-            const int id = (lane + s) & 63;
-            const double2 pa = jbuf[0][id], pb = jbuf[1][id];
-            const real dx = (real)(pa.x - xi), dy = (real)(pa.y - yi), dz = (real)wrap_half(pb.x - zi, k);
-            real wp, mj, mr, qd, Dz;
-            if constexpr (MX) {
-                const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                const bool nr = r2 < Bf;  // left to the FP64 redo (r2 may be 0 here)
-                near = near || nr;
-                const float y = __builtin_amdgcn_rsqf(r2);
-                wp = nr ? 0.0f : (y * y) * y;
-                mj = nr ? 0.0f : (float)pb.y;
-                mr = nr ? 0.0f : (float)mi;
-                s1r2_interp_f32<ORD, true>(a.tab32s, k, dx, dy, dz, qd, Dz,
-                                           S1R2Win32{(const float2 *)win, w0, nw, wok});
-            } else {
-                const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-                wp = pair_w_tile(r2, B, hi, a.soft, min((int64_t)tile * kTile + id, N - 1), k);
-                mj = pb.y;
-                mr = mi;
-                s1r2_interp_win<ORD>(a.table, k, dx, dy, dz, qd, Dz, S1R2Win{win, w0, nw, wok});
+            for (int s = 0; s < kTile; ++s, o = (o + 16u) & (16u * kTile - 1u)) {
+                if (MX && s > 0 && s % kMxRun == 0) end_run();
+                const char *at = (const char *)&jbuf[0][0] + o;
+                const double2 pa = *(const double2 *)at, pb = *(const double2 *)(at + sizeof(jbuf[0]));
+                const real dx = (real)(pa.x - xi), dy = (real)(pa.y - yi), dz = (real)wrap_half(pb.x - zi, k);
+                real wp, mj, mr, qd, Dz, rxy2;
+                if constexpr (MX) {
+                    rxy2 = fmaf(dx, dx, dy * dy);
+                    const float r2 = fmaf(dz, dz, rxy2);
+                    const bool nr = r2 < Bf;  // left to the FP64 redo (r2 may be 0 here)
+                    near = near || nr;
+                    const float y = __builtin_amdgcn_rsqf(r2);
+                    wp = nr ? 0.0f : (y * y) * y;
+                    mj = nr ? 0.0f : (float)pb.y;
+                    mr = nr ? 0.0f : (float)mi;
+                } else {
+                    rxy2 = fma(dx, dx, dy * dy);
+                    const double r2 = fma(dz, dz, rxy2);
+                    wp = pair_w_tile(r2, B, hi, a.soft, min((int64_t)tile * kTile + (o >> 4), N - 1), k);
+                    mj = pb.y;
+                    mr = mi;
+                }
+                if constexpr (decltype(fast)::value)
+                    s1r2_window<ORD, real, node>((const node *)win, w0, nw, nz3, k, rxy2, dz, qd, Dz);
+                else if constexpr (MX)
+                    s1r2_interp_f32<ORD, true>(a.tab32s, k, dx, dy, dz, qd, Dz,
+                                               S1R2Win32{(const float2 *)win, w0, nw, wok});
+                else
+                    s1r2_interp_win<ORD>(a.table, k, dx, dy, dz, qd, Dz, S1R2Win{win, w0, nw, wok});
+                // m (w d - D) with D_x = q dx, D_y = q dy: x and y share m (w - q)
+                auto mad = [](real m, real v, real acc) {
+                    if constexpr (MX) return fmaf(m, v, acc);
+                    else return fma(m, v, acc);
+                };
+                const real sxy = wp - qd, pz = mad(wp, dz, -Dz), sj = mj * sxy, si = mr * sxy;
+                ax = mad(sj, dx, ax);
+                ay = mad(sj, dy, ay);
+                az = mad(mj, pz, az);
+                gx = from_next_lane(mad(si, dx, gx));
+                gy = from_next_lane(mad(si, dy, gy));
+                gz = from_next_lane(mad(mr, pz, gz));
             }
-            // m (w d - D) with D_x = q dx, D_y = q dy: x and y share m (w - q)
-            auto mad = [](real m, real v, real acc) {
-                if constexpr (MX) return fmaf(m, v, acc);
-                else return fma(m, v, acc);
-            };
-            const real sxy = wp - qd, pz = mad(wp, dz, -Dz), sj = mj * sxy, si = mr * sxy;
-            ax = mad(sj, dx, ax);
-            ay = mad(sj, dy, ay);
-            az = mad(mj, pz, az);
-            gx = from_next_lane(mad(si, dx, gx));
-            gy = from_next_lane(mad(si, dy, gy));
-            gz = from_next_lane(mad(mr, pz, gz));
-        }
+        };
+        // every |dz| within half a period after one wrap (else the general path)
+        if (wok && __all(fabs(zi - tc.z) + te.z <= k.L * (1.5 - 1e-9))) steps(std::true_type{});
+        else steps(std::false_type{});
         if (MX) {
             end_run();
         } else {

@@ -190,3 +190,35 @@ def test_t3_ewald_grids_against_oracle(steps, oracle, ng, N):
     em = rel_err(steps.force_eval(dm, x, M, h), F)
     report(f"pair-symmetric t3 ewald ng={ng} N={N} mixed vs fp64", em)
     assert np.median(em) <= 2e-6 and np.percentile(em, 99) <= 1e-5
+
+
+@pytest.mark.parametrize("order", [2, 4])
+@pytest.mark.parametrize("shape", [(40, 33), (64, 8)])
+def test_s1r2_lookup_edges(steps, oracle, order, shape):
+    """Odd and even z grids, pairs on the axis, half a period apart, beyond the
+    last rho node, and particles outside the box, which take the general lookup."""
+    N, L, Rsim = 3001, 100.0, 20.0
+    print(f"case pair-symmetric s1r2 edges order={order} shape={shape}", flush=True)
+    x, M, h, _ = particles("s1r2", N, 9)
+    x[:, :2] *= 0.3
+    x = x[np.argsort(np.hypot(x[:, 0], x[:, 1]), kind="stable")]
+    x[100:160, :2] = x[100, :2]
+    x[130:160, 2] = (x[100:130, 2] + L / 2 + 1e-9 * (np.arange(30) - 15)) % L
+    nrho, nz = shape
+    rho = np.arange(nrho)[:, None] * (2.25 * Rsim / (nrho - 1))
+    z = (np.arange(nz)[None, :] + 0.5) * (L / nz) - 0.5 * L
+    T = np.stack([1e-6 * rho * np.exp(-(z / L) ** 2), 1e-6 * z * np.exp(-rho / L)], axis=-1)
+    T = np.ascontiguousarray(T.reshape(-1))
+    kw = dict(is_periodic=2, L=L, Rsim=Rsim, s1r2_lookup=1, interp_order=order, s1r2_table=T, s1r2_shape=shape)
+    for label, y in (("in the box", x), ("outside", x + np.where(np.arange(N)[:, None] % 7 == 0, [0.0, 0.0, 1.75 * L], 0.0))):
+        d, keep = steps.make_desc(steps.TOPO_S1R2, **kw)
+        F = steps.force_eval(d, y, M, h)
+        rows = np.unique(np.concatenate([np.arange(95, 165), np.linspace(0, N - 1, 60).astype(int)])).astype(np.int32)
+        e = rel_err(F[rows], oracle.forces_rows(oracle.params(2, **kw), y, M, h, rows))
+        report(f"pair-symmetric s1r2 edges order={order} {shape} {label}", e)
+        # pairs exactly half a period apart may take either image: the median only
+        assert np.all(np.isfinite(F)) and np.median(e) <= 1e-12 and np.percentile(e, 80) <= 1e-9
+        dm, keepm = steps.make_desc(steps.TOPO_S1R2, precision=steps.PREC_MIXED, **kw)
+        em = rel_err(steps.force_eval(dm, y, M, h), F)
+        report(f"pair-symmetric s1r2 edges order={order} {shape} {label} mixed vs fp64", em)
+        assert np.median(em) <= 2e-6 and np.percentile(em, 99) <= 1e-5
