@@ -468,6 +468,7 @@ int sim_plan(steps_sim *s, int64_t id_min, int64_t id_max, int precision, EvalPl
     p.t3 = s->t3.ptr();
     p.t3_lo = s->t3.lo;
     p.t3_odd = s->t3.odd;
+    p.equal_mass = s->equal_mass;
     p.s1r2 = s->s1r2.ptr();
     p.s1r2_odd = s->s1r2.odd;
     p.radial = s->radial.ptr();
@@ -529,6 +530,7 @@ int sim_upload(steps_sim *s, const double *x, const double *v, const double *M, 
     STEPS_HIP(hipSetDevice(s->device), "hipSetDevice");
     const size_t nb = (size_t)s->N * sizeof(double);
     double *xs = s->stage.as<double>();
+    s->equal_mass = masses_equal(M, s->N);
     // M and soft are staged in the v buffer (v is written right after)
     double *ms = s->v.as<double>();
     double *hs = ms + s->N;
@@ -645,6 +647,7 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
     p.t3 = o.t3.ptr();
     p.t3_lo = o.t3.lo;
     p.t3_odd = o.t3.odd;
+    p.equal_mass = p.sym && masses_equal(M, N);
     p.s1r2 = o.s1r2.ptr();
     p.s1r2_odd = o.s1r2.odd;
     p.radial = o.radial.ptr();

@@ -101,6 +101,7 @@ struct EvalPlan {
     bool sym = false;
     int sym_blocks = 0, sym_block_rows = 0, sym_task_tiles = 0;
     int sym_cells = 0, sym_launch_cells = 0;
+    bool equal_mass = false;  // every particle has the same mass (sym_kernel)
 };
 
 // The T3 Ewald evaluation deals its sources out to the eight XCDs by table
@@ -127,6 +128,7 @@ void sym_plan(EvalPlan &p);
 bool sym_fit(EvalPlan &p, size_t bytes);
 size_t sym_bytes(const EvalPlan &p);  // of the partial sums; 0 without sym
 bool sym_selected(const EvalPlan &p);
+bool masses_equal(const double *M, int64_t n);
 hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t stream);
 hipError_t launch_sym_finish(const EvalPlan &p, const SymBuffers &b, double *F, hipStream_t stream);
 

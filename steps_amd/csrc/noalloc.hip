@@ -153,6 +153,7 @@ extern "C" int steps_force_eval_noalloc(const steps_force_desc *d, int64_t N, co
     double *radd = cv.take<double>(rad);
     double *rbhd = cv.take<double>(rbh);
 
+    p.equal_mass = p.sym && masses_equal(M, N);
     const hipStream_t st = nullptr;  // the null stream: no stream is created
     if (t3) {
         STEPS_HIP(hipMemcpyAsync(t3r, d->t3_table, t3_raw, hipMemcpyHostToDevice, st), "copy T3 table");

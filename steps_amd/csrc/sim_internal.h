@@ -70,6 +70,7 @@ struct steps_sim {
     steps::TableCopy t3, s1r2, radial, radial_bh;
     steps::KdkParams *hparams = nullptr;   // pinned: the step's scalars (a captured step copies them to dparams)
     double *herrmax = nullptr;             // pinned: errmax, written by the step sequence
+    bool equal_mass = false;               // masses_equal of the state in use
     int *hflag = nullptr;                  // pinned: a non-finite position was found
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;

@@ -222,3 +222,25 @@ def test_s1r2_lookup_edges(steps, oracle, order, shape):
         em = rel_err(steps.force_eval(dm, y, M, h), F)
         report(f"pair-symmetric s1r2 edges order={order} {shape} {label} mixed vs fp64", em)
         assert np.median(em) <= 2e-6 and np.percentile(em, 99) <= 1e-5
+
+
+@pytest.mark.parametrize("N", [MIN_N, MIN_N + 63, 10 * 1024 - 1, 33000])
+@pytest.mark.parametrize("mode", ["r3", "t3", "s1r2"])
+def test_equal_masses_against_oracle(steps, oracle, mode, N):
+    """Particles of one mass, whose products leave the pairs: whole and ragged
+    last blocks and tiles, close and coincident pairs; resident and one-shot
+    calls, and the masses changed in between."""
+    print(f"case pair-symmetric equal masses {mode} N={N}", flush=True)
+    x, M, h, L = particles(mode, N, N)
+    (d, keep), p = descriptor(steps, oracle, mode, L)
+    rows = np.unique(np.concatenate([np.arange(0, 40), np.arange(N - 70, N),
+                                     np.linspace(0, N - 1, 40).astype(int)])).astype(np.int32)
+    sim = steps.Sim(d, N)
+    for label, m in (("equal", np.full(N, 0.37)), ("mixed", M), ("equal again", np.full(N, 1.6))):
+        F = steps.force_eval(d, x, m, h)
+        e = rel_err(F[rows], oracle.forces_rows(p, x, m, h, rows))
+        report(f"pair-symmetric equal masses {mode} N={N} {label}", e)
+        assert np.all(np.isfinite(F)) and np.median(e) <= 1e-12 and e.max() <= 1e-10
+        sim.set_state(x, m, h)
+        sim.forces()
+        assert np.array_equal(sim.get_forces(), F)
