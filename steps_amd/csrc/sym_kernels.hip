@@ -395,7 +395,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // them are FMAs on three VGPR operands, where the one-sided kernel has three
 // and takes its sources from SGPRs, so the gain stays below FP64's.
 // ---------------------------------------------------------------------------
-template <int V, int NI>
+// EQ: sym_kernel's, the masses 1 or 0 and one product at the end.
+template <int V, int NI, bool EQ>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_mixed_kernel(const SymArgs a) {
     constexpr int kFlush = V == PV_R3 ? 64 / NI : 32 / NI;
     __shared__ __align__(1024) float4 jbuf[2][kTile];
@@ -417,15 +418,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 #pragma unroll
     for (int q = 0; q < NI; ++q) {
         const int64_t r = row0 + q * 64;
-        m[q] = r < N ? (float)a.rec[min(r, N - 1)].w : 0.0f;
+        m[q] = r < N ? (EQ ? 1.0f : (float)a.rec[min(r, N - 1)].w) : 0.0f;
         fx[q] = fy[q] = fz[q] = 0.0;
     }
     auto stage = [&](int buf, int tile) {  // wave 0: one source per lane
         const int64_t j = (int64_t)tile * kTile + lane;
         float4 p = a.jrel[min(j, N - 1)];
+        if (EQ) p.w = 1.0f;
         if (j >= N) p.w = 0.0f;
         jbuf[buf][lane] = p;
     };
+    const double mass = EQ ? a.rec[0].w : 1.0;
+    const bool whole = EQ && (int64_t)(b + 1) * (kSymWaves * 64 * NI) <= N;  // no row past the end
     bool have = w.settle(a, b, ntiles);
     if (have && wave == 0) stage(0, w.tile);
     __syncthreads();
@@ -506,9 +510,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                 ax[q] = ay[q] = az[q] = 0.0f;
             }
         };
-        auto steps = [&](auto near, auto wm) {
+        auto steps = [&](auto near, auto wm, auto unit) {
             constexpr int NEAR = decltype(near)::value;
             constexpr int WM = decltype(wm)::value;
+            constexpr bool UNIT = decltype(unit)::value;
             unsigned o = (unsigned)lane * 16u;
             const char *base = (const char *)&jbuf[buf][0];
             float4 nj = *(const float4 *)(base + o);
@@ -533,7 +538,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                             close = close || c;
                             y3 = c ? 0.0f : y3;
                         }
-                        const float sj = y3 * pj.w, si = y3 * m[q];
+                        const float sj = UNIT ? y3 : y3 * pj.w, si = UNIT ? y3 : y3 * m[q];
                         ax[q] = fmaf(sj, dx, ax[q]);
                         ay[q] = fmaf(sj, dy, ay[q]);
                         az[q] = fmaf(sj, dz, az[q]);
@@ -559,19 +564,21 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                 if (V != PV_R3) end_rows();
             }
         };
-        auto variants = [&](auto near) {
+        auto variants = [&](auto near, auto unit) {
             const int wm = (wx ? 1 : 0) | (wy ? 2 : 0) | (wz ? 4 : 0);
-            if (wm == 0) steps(near, IntC<0>{});
-            else if (V == PV_S1R2_NEAREST) steps(near, IntC<4>{});
+            if (wm == 0) steps(near, IntC<0>{}, unit);
+            else if (V == PV_S1R2_NEAREST) steps(near, IntC<4>{}, unit);
             else if (V == PV_T3_NEAREST) {
-                if (wm == 1) steps(near, IntC<1>{});
-                else if (wm == 2) steps(near, IntC<2>{});
-                else if (wm == 4) steps(near, IntC<4>{});
-                else steps(near, IntC<7>{});
+                if (wm == 1) steps(near, IntC<1>{}, unit);
+                else if (wm == 2) steps(near, IntC<2>{}, unit);
+                else if (wm == 4) steps(near, IntC<4>{}, unit);
+                else steps(near, IntC<7>{}, unit);
             }
         };
-        if (far) variants(IntC<0>{});
-        else variants(IntC<1>{});
+        if (far) {
+            if (whole && (int64_t)(tile + 1) * kTile <= N) variants(IntC<0>{}, std::bool_constant<EQ>{});
+            else variants(IntC<0>{}, std::false_type{});
+        } else variants(IntC<1>{}, std::false_type{});
         if (V == PV_R3) end_rows();
         if (__any(close)) {
             // rare: those pairs in FP64 from the FP64 records
@@ -602,7 +609,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                         const double beta = a.soft[i] + a.soft[j];
                         double u = inv_r3(r2, 1.5);
                         if (r2 < beta * beta) u = softening_exact(sqrt(r2), beta);
-                        const double sj = (pj.w == 0.0f ? 0.0 : pd.w) * u, si = (m[q] == 0.0f ? 0.0 : pi.w) * u;
+                        const double sj = (pj.w == 0.0f ? 0.0 : (EQ ? 1.0 : pd.w)) * u,
+                                     si = (m[q] == 0.0f ? 0.0 : (EQ ? 1.0 : pi.w)) * u;
                         fx[q] = fma(sj, ex, fx[q]);
                         fy[q] = fma(sj, ey, fy[q]);
                         fz[q] = fma(sj, ez, fz[q]);
@@ -630,7 +638,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             for (int v = 1; v < kSymWaves; ++v) g += gsum[buf][v][wave][lane];
             if (j < N)
                 a.part[sym_slot(N, cell_l, a.cell_tasks, a.cell_offs, a.cell_tasks + off - cell * a.cell_offs) +
-                       (size_t)wave * N + j] = g;
+                       (size_t)wave * N + j] = EQ ? g * mass : g;
         }
         w = nw;
         have = more;
@@ -641,9 +649,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     for (int q = 0; q < NI; ++q) {
         const int64_t r = row0 + q * 64;
         if (r < N) {
-            out[r] = fx[q];
-            out[N + r] = fy[q];
-            out[2 * N + r] = fz[q];
+            out[r] = EQ ? fx[q] * mass : fx[q];
+            out[N + r] = EQ ? fy[q] * mass : fy[q];
+            out[2 * N + r] = EQ ? fz[q] * mass : fz[q];
         }
     }
 }
@@ -1634,12 +1642,15 @@ void launch_sym_kernel(const EvalPlan &p, const SymArgs &a, int cells, hipStream
         return;
     }
     if (p.precision == STEPS_PREC_MIXED) {
+        auto go = [&](auto v) {
+            constexpr int V = decltype(v)::value;
+            if (p.equal_mass) hipLaunchKernelGGL((sym_mixed_kernel<V, kSymNI, true>), grid, dim3(kBlock), 0, st, a);
+            else hipLaunchKernelGGL((sym_mixed_kernel<V, kSymNI, false>), grid, dim3(kBlock), 0, st, a);
+        };
         switch (p.variant) {
-        case PV_R3: hipLaunchKernelGGL((sym_mixed_kernel<PV_R3, kSymNI>), grid, dim3(kBlock), 0, st, a); break;
-        case PV_T3_NEAREST:
-            hipLaunchKernelGGL((sym_mixed_kernel<PV_T3_NEAREST, kSymNI>), grid, dim3(kBlock), 0, st, a);
-            break;
-        default: hipLaunchKernelGGL((sym_mixed_kernel<PV_S1R2_NEAREST, kSymNI>), grid, dim3(kBlock), 0, st, a); break;
+        case PV_R3: go(IntC<PV_R3>{}); break;
+        case PV_T3_NEAREST: go(IntC<PV_T3_NEAREST>{}); break;
+        default: go(IntC<PV_S1R2_NEAREST>{}); break;
         }
         return;
     }

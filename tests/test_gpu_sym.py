@@ -224,7 +224,7 @@ def test_s1r2_lookup_edges(steps, oracle, order, shape):
         assert np.median(em) <= 2e-6 and np.percentile(em, 99) <= 1e-5
 
 
-@pytest.mark.parametrize("N", [MIN_N, MIN_N + 63, 10 * 1024 - 1, 33000])
+@pytest.mark.parametrize("N", [MIN_N, MIN_N + 63, 10 * 1024 - 1, 13 * 1024, 33000])
 @pytest.mark.parametrize("mode", ["r3", "t3", "s1r2"])
 def test_equal_masses_against_oracle(steps, oracle, mode, N):
     """Particles of one mass, whose products leave the pairs: whole and ragged
@@ -244,3 +244,8 @@ def test_equal_masses_against_oracle(steps, oracle, mode, N):
         sim.set_state(x, m, h)
         sim.forces()
         assert np.array_equal(sim.get_forces(), F)
+        (dm, keepm), _ = descriptor(steps, oracle, mode, L)
+        dm.precision = steps.PREC_MIXED
+        em = rel_err(steps.force_eval(dm, x, m, h), F)
+        report(f"pair-symmetric equal masses {mode} N={N} {label} mixed vs fp64", em)
+        assert np.median(em) <= 2e-6 and np.percentile(em, 99) <= 1e-5 and em.max() <= 1e-3
