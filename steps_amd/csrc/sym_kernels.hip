@@ -30,9 +30,9 @@
 // order do not depend on the grouping.
 //
 // Measured against the one-sided kernels (resident or one-shot calls, copies
-// included): R3 N = 16384 KDK runs 1.33 -> 1.04 ms, N = 100003 6.8 -> 4.5 ms,
-// N = 10^6 511 -> 387 ms (1.34 T pair evaluations/s, 2.67 T interactions/s;
-// the loop alone reaches 1.41); T3 nearest image at 64^3 50.0 -> 32.5 ms.
+// included): R3 N = 16384 KDK runs 1.32 -> 0.98 ms, N = 100003 6.7 -> 4.4 ms,
+// N = 10^6 487 -> 373 ms (1.34 T pair evaluations/s, 2.67 T interactions/s;
+// the loop alone reaches 1.41); T3 nearest image at 64^3 50.2 -> 29.1 ms.
 // Errors against 64-bit sums are smaller (shorter addition chains).  Bound by
 // FP64 VALU issue: ~100 of the ~107 cycles a pair evaluation takes per SIMD
 // are its 18 FP64 instructions and the quarter-rate v_rsq_f64.
@@ -380,15 +380,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // Mixed precision, R3 and nearest image: the scheme of sym_kernel with FP32
 // pairs.  A tile's sources are FP32 offsets from the tile's centre (jrel), a
 // row's offset is formed in FP64 (its image nearest the tile on periodic
-// axes) and rounded once per tile.  FP32 sums: a row's run over the 64 sources
-// of a tile, a source's over kFlush steps of NI rows (at most 64 pairs); both
-// are then added in FP64, the source's in LDS.  Pairs within the bound, or
+// axes) and rounded once per tile.  FP32 sums: a source's run over eight steps
+// of NI rows (32 pairs), a row's over 32 sources, or eight in the nearest-image
+// modes, whose forces are small residuals; both are then added in FP64, the
+// source's in LDS.  (Over 64 pairs each: 4% faster in R3, 3% in T3, but a
+// median row's error 4.8e-7 instead of 3.3e-7 at N = 100000, where the
+// one-sided kernel has 4.6e-7, and 4.7e-7 instead of 3.1e-7 on a lattice.)  Pairs within the bound, or
 // within 1e-6 L of half a period on an axis that is wrapped per pair (where
 // FP32 could take the other image), are done again in FP64.
 //
 // Measured against the one-sided kernels (ms): R3 N = 16384 0.235 -> 0.192,
-// 100003 4.0 -> 2.8, 1.5 10^6 575 -> 468; T3 nearest 24^3 0.471 -> 0.423,
-// 45^3 6.3 -> 3.8, 64^3 38.3 -> 27.5; below N = 12288 the one-sided kernel is
+// 100003 4.0 -> 2.8, 1.5 10^6 576 -> 488; T3 nearest, one mass, 40^3 2.40 ->
+// 2.17 and 64^3 28.4 -> 27.7 against this kernel with the products, 38.3
+// one-sided; below N = 12288 the one-sided kernel is
 // as fast (R3 N = 9000: 0.189 against 0.217).  Bound by VALU issue at ~65
 // cycles a pair evaluation and SIMD for 17.5 instructions: fewer or more waves
 // (2, 3, 5, 6 per SIMD) and 8 rows per lane all measured 0-15% slower.  Six of
@@ -398,7 +402,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // EQ: sym_kernel's, the masses 1 or 0 and one product at the end.
 template <int V, int NI, bool EQ>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_mixed_kernel(const SymArgs a) {
-    constexpr int kFlush = V == PV_R3 ? 64 / NI : 32 / NI;
+    constexpr int kFlush = 32 / NI, kRowFlush = V == PV_R3 ? 4 * kFlush : kFlush;  // steps of an FP32 sum
     __shared__ __align__(1024) float4 jbuf[2][kTile];
     __shared__ double gsum[2][kSymWaves][3][kTile];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -561,7 +565,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                     __builtin_amdgcn_wave_barrier();
                 }
                 gx = gy = gz = 0.0f;
-                if (V != PV_R3) end_rows();
+                if ((s0 + kFlush) % kRowFlush == 0) end_rows();
             }
         };
         auto variants = [&](auto near, auto unit) {
@@ -579,7 +583,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             if (whole && (int64_t)(tile + 1) * kTile <= N) variants(IntC<0>{}, std::bool_constant<EQ>{});
             else variants(IntC<0>{}, std::false_type{});
         } else variants(IntC<1>{}, std::false_type{});
-        if (V == PV_R3) end_rows();
         if (__any(close)) {
             // rare: those pairs in FP64 from the FP64 records
             double cx = 0.0, cy = 0.0, cz = 0.0;
