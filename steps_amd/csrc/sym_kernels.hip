@@ -377,7 +377,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 }
 
 // ---------------------------------------------------------------------------
-// Mixed precision, R3 and nearest image: the scheme of sym_kernel with FP32
+// Mixed precision, R3 and T3 nearest image: the scheme of sym_kernel with FP32
 // pairs.  A tile's sources are FP32 offsets from the tile's centre (jrel), a
 // row's offset is formed in FP64 (its image nearest the tile on periodic
 // axes) and rounded once per tile.  FP32 sums: a source's run over eight steps
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // Measured against the one-sided kernels (ms): R3 N = 16384 0.235 -> 0.192,
 // 100003 4.0 -> 2.8, 1.5 10^6 576 -> 488; T3 nearest, one mass, 40^3 2.40 ->
 // 2.17 and 64^3 28.4 -> 27.7 against this kernel with the products, 38.3
-// one-sided; below N = 12288 the one-sided kernel is
+// one-sided; below N = 14336 the one-sided kernel is
 // as fast (R3 N = 9000: 0.189 against 0.217).  Bound by VALU issue at ~65
 // cycles a pair evaluation and SIMD for 17.5 instructions: fewer or more waves
 // (2, 3, 5, 6 per SIMD) and 8 rows per lane all measured 0-15% slower.  Six of
@@ -571,7 +571,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         auto variants = [&](auto near, auto unit) {
             const int wm = (wx ? 1 : 0) | (wy ? 2 : 0) | (wz ? 4 : 0);
             if (wm == 0) steps(near, IntC<0>{}, unit);
-            else if (V == PV_S1R2_NEAREST) steps(near, IntC<4>{}, unit);
             else if (V == PV_T3_NEAREST) {
                 if (wm == 1) steps(near, IntC<1>{}, unit);
                 else if (wm == 2) steps(near, IntC<2>{}, unit);
@@ -1543,7 +1542,7 @@ constexpr int kSymNI = 4;
 // Below this many particles the triangle of block pairs leaves too few equal
 // tasks to fill the chip (N = 9000: 0.129 against 0.167 ms).
 constexpr int64_t kSymMinN = 8192;
-constexpr int64_t kSymMixedMinN = 12288;  // the same in mixed precision (sym_mixed_kernel)
+constexpr int64_t kSymMixedMinN = 14336;  // mixed (R3 N = 13000: 0.228 against 0.234 ms, 16384: 0.235 against 0.194)
 constexpr int64_t kSymS1MinN = 1024;      // S1R2 with a table (N = 1536, CIC: 0.110 against 0.131 ms)
 constexpr int64_t kSymT3MinN = 128;       // T3 Ewald (N = 216: 0.32 against 0.70 ms, 13^3: 0.57 against 2.8)
 // Scratch the slots may take; the offsets go in as many launches as that
@@ -1554,7 +1553,10 @@ constexpr size_t kSymBytes = (size_t)256 << 20;
 bool sym_variant(const EvalPlan &p) {
     if (p.variant == PV_T3_EWALD) return p.t3_ng <= kT3MaxWinNg;  // either precision
     if (p.variant == PV_S1R2_CIC || p.variant == PV_S1R2_TSC) return true;
-    return p.variant == PV_R3 || p.variant == PV_T3_NEAREST || p.variant == PV_S1R2_NEAREST;
+    if (p.variant == PV_R3 || p.variant == PV_T3_NEAREST) return true;
+    // mixed: the one-sided kernel wraps one axis only and is the faster and the
+    // more exact (N = 524288: 84 against 90 ms, median error 9.1e-8 against 1.2e-7)
+    return p.variant == PV_S1R2_NEAREST && p.precision == STEPS_PREC_FP64;
 }
 
 // Rows of a T3 Ewald workgroup: with c particles per cell column, R rows and a
@@ -1650,11 +1652,8 @@ void launch_sym_kernel(const EvalPlan &p, const SymArgs &a, int cells, hipStream
             if (p.equal_mass) hipLaunchKernelGGL((sym_mixed_kernel<V, kSymNI, true>), grid, dim3(kBlock), 0, st, a);
             else hipLaunchKernelGGL((sym_mixed_kernel<V, kSymNI, false>), grid, dim3(kBlock), 0, st, a);
         };
-        switch (p.variant) {
-        case PV_R3: go(IntC<PV_R3>{}); break;
-        case PV_T3_NEAREST: go(IntC<PV_T3_NEAREST>{}); break;
-        default: go(IntC<PV_S1R2_NEAREST>{}); break;
-        }
+        if (p.variant == PV_R3) go(IntC<PV_R3>{});
+        else go(IntC<PV_T3_NEAREST>{});
         return;
     }
     auto go = [&](auto v) {

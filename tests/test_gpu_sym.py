@@ -64,7 +64,7 @@ def test_against_oracle(steps, oracle, mode, N):
     assert np.median(rel_err(few, F[:N // 2 + 1])) <= 1e-12
 
 
-@pytest.mark.parametrize("N", [12288, 12289, 15 * 1024 - 63, 66001])
+@pytest.mark.parametrize("N", [12288, 12289, 14336, 15 * 1024 - 63, 66001])
 @pytest.mark.parametrize("mode", ["r3", "t3", "s1r2"])
 def test_mixed_against_fp64(steps, oracle, mode, N):
     """Mixed precision against FP64 on every row (the pair-sum bar, p99 1e-5),
@@ -224,7 +224,7 @@ def test_s1r2_lookup_edges(steps, oracle, order, shape):
         assert np.median(em) <= 2e-6 and np.percentile(em, 99) <= 1e-5
 
 
-@pytest.mark.parametrize("N", [MIN_N, MIN_N + 63, 10 * 1024 - 1, 13 * 1024, 33000])
+@pytest.mark.parametrize("N", [MIN_N, MIN_N + 63, 10 * 1024 - 1, 15 * 1024, 33000])
 @pytest.mark.parametrize("mode", ["r3", "t3", "s1r2"])
 def test_equal_masses_against_oracle(steps, oracle, mode, N):
     """Particles of one mass, whose products leave the pairs: whole and ragged
