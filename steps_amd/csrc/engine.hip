@@ -136,7 +136,7 @@ int TableCopy::sync_t3(const double *h, int ng, hipStream_t st) {
     n = count;
     fp = f;
     lo = l;
-    odd = t3_table_odd(h, ng);
+    sym = t3_symmetry(h, ng);
     return STEPS_OK;
 }
 
@@ -467,7 +467,7 @@ int sim_plan(steps_sim *s, int64_t id_min, int64_t id_max, int precision, EvalPl
     if (!sym_fit(p, s->part.cap) || scratch_bytes(p) > s->part.cap) return fail(STEPS_ERR_STATE, "scratch too small for this precision");
     p.t3 = s->t3.ptr();
     p.t3_lo = s->t3.lo;
-    p.t3_odd = s->t3.odd;
+    p.t3_sym = s->t3.sym;
     p.equal_mass = s->equal_mass;
     p.s1r2 = s->s1r2.ptr();
     p.s1r2_odd = s->s1r2.odd;
@@ -646,7 +646,7 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
         return rc;
     p.t3 = o.t3.ptr();
     p.t3_lo = o.t3.lo;
-    p.t3_odd = o.t3.odd;
+    p.t3_sym = o.t3.sym;
     p.equal_mass = p.sym && masses_equal(M, N);
     p.s1r2 = o.s1r2.ptr();
     p.s1r2_odd = o.s1r2.odd;

@@ -59,6 +59,15 @@ struct DeviceParticles {
     int64_t n = 0;
 };
 
+// Symmetries of a T3 table at every node (components below 2^-52 max|T| count
+// as zero).  odd: T(-d) = -T(d), so the correction of a pair serves both sides.
+// mirror_z: odd, and T(x, y, -z) = (Tx, Ty, -Tz), so |dz| alone is looked up;
+// the x / y fold and oddness do not imply it, since the fold leaves the planes
+// a mirror maps onto themselves (odd Ng) as they are.
+struct T3Symmetry {
+    bool odd = false, mirror_z = false;
+};
+
 // Everything one force evaluation needs on the device.
 struct EvalPlan {
     int variant = PV_R3;
@@ -76,7 +85,7 @@ struct EvalPlan {
     // tables (device)
     const double *t3 = nullptr; int t3_ng = 0;
     int t3_lo = 0;         // first x/y node of the T3 device layout (t3_device_layout)
-    bool t3_odd = false;   // the table in use is odd (t3_table_odd)
+    T3Symmetry t3_sym;     // of the table in use (t3_symmetry)
     const double *s1r2 = nullptr; int s1r2_nrho = 0, s1r2_nz = 0;
     bool s1r2_odd = false; // the table in use is odd in z (s1r2_table_odd)
     const double *radial = nullptr; int radial_size = 0;
@@ -247,9 +256,7 @@ int kdk_reduce_blocks(int64_t n);
 int t3_device_layout(const double *T, int ng, std::vector<double> &out);
 // The lo t3_device_layout picks for this table (Ng/2 when it folds, else 0).
 int t3_layout_lo(const double *T, int ng);
-// The table is odd through its centre, T(-d) = -T(d) (components below 2^-52
-// max|T| count as zero): the correction of a pair then serves both sides.
-bool t3_table_odd(const double *T, int ng);
+T3Symmetry t3_symmetry(const double *T, int ng);
 inline size_t t3_device_entries(int ng, int lo) {
     return (size_t)(ng - lo) * (size_t)(ng - lo) * (size_t)(ng + 3) * 3u;
 }

@@ -161,7 +161,7 @@ extern "C" int steps_force_eval_noalloc(const steps_force_desc *d, int64_t N, co
         STEPS_HIP(hipGetLastError(), "T3 table layout");
         p.t3 = t3d;
         p.t3_lo = lo;
-        p.t3_odd = t3_table_odd(d->t3_table, d->t3_ngrid);
+        p.t3_sym = t3_symmetry(d->t3_table, d->t3_ngrid);
     }
     if (s1r2) {
         STEPS_HIP(hipMemcpyAsync(s1r, d->s1r2_table, s1_raw, hipMemcpyHostToDevice, st), "copy S1R2 table");

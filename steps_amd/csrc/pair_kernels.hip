@@ -1444,18 +1444,31 @@ static bool t3_antisymmetric_xy(const double *T, int ng) {
     return true;
 }
 
-bool t3_table_odd(const double *T, int ng) {
-    const size_t n3 = (size_t)ng * ng * ng;
+T3Symmetry t3_symmetry(const double *T, int ng) {
+    T3Symmetry s;
+    const size_t n = (size_t)ng, n3 = n * n * n;
     double tmax = 0.0;
     for (size_t i = 0; i < n3 * 3u; ++i) tmax = std::max(tmax, std::fabs(T[i]));
-    if (!(tmax < INFINITY)) return false;
+    if (!(tmax < INFINITY)) return s;
     const double eps0 = std::ldexp(tmax, -52);
-    for (size_t i = 0; i < n3; ++i) {  // node n3 - 1 - i is node i seen through the centre
-        const double *a = T + 3u * i, *b = T + 3u * (n3 - 1 - i);
-        for (int c = 0; c < 3; ++c)
-            if (!(b[c] == -a[c] || (std::fabs(a[c]) <= eps0 && std::fabs(b[c]) <= eps0))) return false;
+    auto same = [eps0](double b, double a) {
+        return b == a || (std::fabs(a) <= eps0 && std::fabs(b) <= eps0);
+    };
+    s.odd = s.mirror_z = true;
+    for (size_t i = 0; i < n3 && s.odd; ++i) {
+        const double *a = T + 3u * i;
+        if (2 * i < n3) {  // node n3 - 1 - i is node i seen through the centre
+            const double *b = T + 3u * (n3 - 1 - i);
+            s.odd = same(b[0], -a[0]) && same(b[1], -a[1]) && same(b[2], -a[2]);
+        }
+        const size_t iz = i % n;
+        if (2 * iz < n) {
+            const double *b = a + 3u * (n - 1 - 2 * iz);
+            s.mirror_z = s.mirror_z && same(b[0], a[0]) && same(b[1], a[1]) && same(b[2], -a[2]);
+        }
     }
-    return true;
+    s.mirror_z = s.mirror_z && s.odd;
+    return s;
 }
 
 int t3_layout_lo(const double *T, int ng) { return t3_antisymmetric_xy(T, ng) ? ng / 2 : 0; }

@@ -36,7 +36,8 @@ struct TableCopy {
     double L = 0, Rsim = 0;  // S1R2 tables: the box the oddness was checked for
     DevBuf dev;
     int lo = 0;        // T3 tables: first x/y node of the device layout
-    bool odd = false;  // T3 / S1R2 tables: t3_table_odd, s1r2_table_odd
+    T3Symmetry sym;    // T3 tables
+    bool odd = false;  // S1R2 tables: s1r2_table_odd
     int sync(const double *h, size_t count, hipStream_t st, const char *what);
     // T3 / S1R2: upload the table in the pair kernels' layout
     // (t3_device_layout, s1r2_device_layout)

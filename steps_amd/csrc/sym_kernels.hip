@@ -1621,7 +1621,7 @@ void launch_sym_kernel(const EvalPlan &p, const SymArgs &a, int cells, hipStream
         const bool mx = p.precision == STEPS_PREC_MIXED;
         auto go = [&](auto g) {
             constexpr int G = decltype(g)::value;
-            if (p.t3_lo > 0) {  // even and odd through z = 0 too (odd, and mirrored in x and y)
+            if (p.t3_lo > 0 && p.t3_sym.mirror_z) {
                 if (mx) hipLaunchKernelGGL((sym_t3_kernel<G, true, true>), grid, block, 0, st, a);
                 else hipLaunchKernelGGL((sym_t3_kernel<G, false, true>), grid, block, 0, st, a);
             } else {
@@ -1749,7 +1749,7 @@ bool masses_equal(const double *M, int64_t n) {
 }
 
 bool sym_selected(const EvalPlan &p) {
-    return p.sym && (p.variant != PV_T3_EWALD || p.t3_odd) && (!is_s1r2_lookup(p.variant) || p.s1r2_odd);
+    return p.sym && (p.variant != PV_T3_EWALD || p.t3_sym.odd) && (!is_s1r2_lookup(p.variant) || p.s1r2_odd);
 }
 
 hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t st) {
