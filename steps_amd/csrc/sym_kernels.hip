@@ -390,7 +390,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // FP32 could take the other image), are done again in FP64.
 //
 // Measured against the one-sided kernels (ms): R3 N = 16384 0.235 -> 0.192,
-// 100003 4.0 -> 2.8, 1.5 10^6 576 -> 488; T3 nearest, one mass, 40^3 2.40 ->
+// 100003 4.0 -> 2.8, 1.5 10^6 576 -> 499 (492 with r^-3 formed before the masses); T3 nearest, one mass, 40^3 2.40 ->
 // 2.17 and 64^3 28.4 -> 27.7 against this kernel with the products, 38.3
 // one-sided; below N = 14336 the one-sided kernel is
 // as fast (R3 N = 9000: 0.189 against 0.217).  Bound by VALU issue at ~65
@@ -399,7 +399,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // them are FMAs on three VGPR operands, where the one-sided kernel has three
 // and takes its sources from SGPRs, so the gain stays below FP64's.
 // ---------------------------------------------------------------------------
-// EQ: sym_kernel's, the masses 1 or 0 and one product at the end.
+// The power of two at or below |m|, in the FP32 range (1 for no mass).
+__device__ __forceinline__ double unit_mass(double m) {
+    return m == 0.0 ? 1.0 : ldexp(1.0, max(-126, min(127, ilogb(m))));
+}
+
+// EQ: sym_kernel's, the masses one value (R3: unit_mass) or 0 and one product
+// at the end.
 template <int V, int NI, bool EQ>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_mixed_kernel(const SymArgs a) {
     constexpr int kFlush = 32 / NI, kRowFlush = V == PV_R3 ? 4 * kFlush : kFlush;  // steps of an FP32 sum
@@ -417,22 +423,23 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 
     KScalars k = a.k;
     const int64_t row0 = ((int64_t)b * kSymWaves + wave) * (64 * NI) + lane;
+    const double um = EQ && V == PV_R3 ? unit_mass(a.rec[0].w) : 1.0;  // what a particle of EQ has in the pairs
     double fx[NI], fy[NI], fz[NI];
     float m[NI];
 #pragma unroll
     for (int q = 0; q < NI; ++q) {
         const int64_t r = row0 + q * 64;
-        m[q] = r < N ? (EQ ? 1.0f : (float)a.rec[min(r, N - 1)].w) : 0.0f;
+        m[q] = r < N ? (EQ ? (float)um : (float)a.rec[min(r, N - 1)].w) : 0.0f;
         fx[q] = fy[q] = fz[q] = 0.0;
     }
     auto stage = [&](int buf, int tile) {  // wave 0: one source per lane
         const int64_t j = (int64_t)tile * kTile + lane;
         float4 p = a.jrel[min(j, N - 1)];
-        if (EQ) p.w = 1.0f;
+        if (EQ) p.w = (float)um;
         if (j >= N) p.w = 0.0f;
         jbuf[buf][lane] = p;
     };
-    const double mass = EQ ? a.rec[0].w : 1.0;
+    const double mass = EQ ? a.rec[0].w / um : 1.0;
     const bool whole = EQ && (int64_t)(b + 1) * (kSymWaves * 64 * NI) <= N;  // no row past the end
     bool have = w.settle(a, b, ntiles);
     if (have && wave == 0) stage(0, w.tile);
@@ -535,14 +542,23 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                         if (WM & 2) dy = wrap(dy, c);
                         if (WM & 4) dz = wrap(dz, c);
                         const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                        const float yr = __builtin_amdgcn_rsqf(r2);
-                        float y3 = (yr * yr) * yr;
+                        float yr = __builtin_amdgcn_rsqf(r2);
                         if (NEAR || WM) {
                             if (NEAR) c = c || r2 < B;
                             close = close || c;
-                            y3 = c ? 0.0f : y3;
+                            yr = c ? 0.0f : yr;
                         }
-                        const float sj = UNIT ? y3 : y3 * pj.w, si = UNIT ? y3 : y3 * m[q];
+                        const float t = yr * yr;
+                        float sj, si;
+                        if constexpr (V == PV_R3) {
+                            // the mass before r^-3, which alone leaves the FP32 range at 4e12 length units
+                            sj = t * (yr * (UNIT ? (float)um : pj.w));
+                            si = UNIT ? sj : t * (yr * m[q]);
+                        } else {
+                            const float y3 = t * yr;
+                            sj = UNIT ? y3 : y3 * pj.w;
+                            si = UNIT ? y3 : y3 * m[q];
+                        }
                         ax[q] = fmaf(sj, dx, ax[q]);
                         ay[q] = fmaf(sj, dy, ay[q]);
                         az[q] = fmaf(sj, dz, az[q]);
@@ -611,8 +627,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                         const double beta = a.soft[i] + a.soft[j];
                         double u = inv_r3(r2, 1.5);
                         if (r2 < beta * beta) u = softening_exact(sqrt(r2), beta);
-                        const double sj = (pj.w == 0.0f ? 0.0 : (EQ ? 1.0 : pd.w)) * u,
-                                     si = (m[q] == 0.0f ? 0.0 : (EQ ? 1.0 : pi.w)) * u;
+                        const double sj = (pj.w == 0.0f ? 0.0 : (EQ ? um : pd.w)) * u,
+                                     si = (m[q] == 0.0f ? 0.0 : (EQ ? um : pi.w)) * u;
                         fx[q] = fma(sj, ex, fx[q]);
                         fy[q] = fma(sj, ey, fy[q]);
                         fz[q] = fma(sj, ez, fz[q]);
