@@ -31,6 +31,9 @@ int fail(int code, const std::string &msg) {
 int hip_fail(hipError_t e, const char *what) {
     std::string m = std::string(what) + ": " + hipGetErrorString(e);
     set_error(m);
+    // the thread's last error stays until it is read, past later successes: the
+    // next launch's check would report this one again
+    (void)hipGetLastError();
     return (e == hipErrorOutOfMemory || e == hipErrorMemoryAllocation) ? STEPS_ERR_NOMEM
                                                                         : STEPS_ERR_DEVICE;
 }
@@ -387,7 +390,6 @@ int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool 
     if ((rc = s->jrec.reserve((size_t)N * sizeof(double4), "alloc jrec")) ||
         (rc = s->jsoft.reserve(nb, "alloc soft")) || (rc = s->v.reserve(3 * nb, "alloc v")) ||
         (rc = s->F.reserve(3 * nb, "alloc F")) ||
-        ((lean || s->part.reserve(scratch, "alloc partials")) && (rc = s->part.reserve(least, "alloc partials"))) ||
         (rc = s->stage.reserve(std::max(3 * nb, (size_t)1024), "alloc stage")) ||
         (rc = s->blockmax.reserve((size_t)(kdk_reduce_blocks(N) + 1) * sizeof(double), "alloc blockmax")) ||
         (rc = s->dparams.reserve(sizeof(KdkParams), "alloc step params")))
@@ -415,6 +417,9 @@ int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool 
         return cleanup(rc);
     if (p.bh_radial_size > 0 &&
         (rc = s->radial_bh.sync(d.radial_bh_table, (size_t)d.radial_bh_table_size, s->stream, "radial octree table")))
+        return cleanup(rc);
+    // last: what does not fit beside the rest is done with the least
+    if ((lean || s->part.reserve(scratch, "alloc partials")) && (rc = s->part.reserve(least, "alloc partials")))
         return cleanup(rc);
     // the sim owns device copies: host table pointers are not kept
     s->desc.t3_table = nullptr;
@@ -631,7 +636,7 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
     const size_t nb = (size_t)N * sizeof(double);
     if ((rc = o.x.reserve(5 * nb, "alloc x")) || (rc = o.M.reserve(nb, "alloc M")) ||
         (rc = o.soft.reserve(nb, "alloc soft")) || (rc = o.jrec.reserve((size_t)N * sizeof(double4), "alloc jrec")) ||
-        (rc = o.jsoft.reserve(nb, "alloc jsoft")) || (rc = reserve_scratch(o.part, p)) ||
+        (rc = o.jsoft.reserve(nb, "alloc jsoft")) ||
         (rc = o.F.reserve(3 * (size_t)p.nrows * sizeof(double), "alloc F")))
         return rc;
     hipStream_t st = o.stream;
@@ -644,6 +649,7 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
     if (p.bh_radial_size > 0 &&
         (rc = o.radial_bh.sync(d->radial_bh_table, (size_t)d->radial_bh_table_size, st, "radial octree table")))
         return rc;
+    if ((rc = reserve_scratch(o.part, p))) return rc;  // last, as in sim_create
     p.t3 = o.t3.ptr();
     p.t3_lo = o.t3.lo;
     p.t3_sym = o.t3.sym;
@@ -653,8 +659,12 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
     p.radial = o.radial.ptr();
     p.bh_radial = o.radial_bh.ptr();
     const size_t fb = 3 * (size_t)p.nrows * sizeof(double);
-    const bool pinned = 5 * nb + fb <= kPinBytes;
-    if (pinned && !o.pin) STEPS_HIP(hipHostMalloc((void **)&o.pin, kPinBytes, hipHostMallocDefault), "pinned block");
+    bool pinned = 5 * nb + fb <= kPinBytes;
+    if (pinned && !o.pin && hipHostMalloc((void **)&o.pin, kPinBytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        o.pin = nullptr;
+        pinned = false;
+    }
     const double *dx = o.x.as<double>(), *dM = o.M.as<double>(), *dsoft = o.soft.as<double>();
     if (pinned) {
         // x, M, soft in one block, one copy
