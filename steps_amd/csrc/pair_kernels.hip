@@ -1090,7 +1090,7 @@ __global__ void t3_f32_kernel(const double *__restrict__ T, float4 *__restrict__
 // ---------------------------------------------------------------------------
 // perm (or null): partial-sum row r belongs to input row perm[r] (rows taken
 // in spatial order; id_min is 0 then).
-__global__ __launch_bounds__(256) void reduce_kernel(const double *__restrict__ part,
+__global__ __launch_bounds__(64) void reduce_kernel(const double *__restrict__ part,
                                                      const double4 *__restrict__ jrec,
                                                      const uint32_t *__restrict__ perm,
                                                      const double *__restrict__ radial,
@@ -1102,11 +1102,23 @@ __global__ __launch_bounds__(256) void reduce_kernel(const double *__restrict__ 
     if (k >= nrows) return;
     const int64_t r = perm ? (int64_t)perm[k] : k;  // output row
     double f[3] = {0.0, 0.0, 0.0};
-    for (int s = 0; s < splits; ++s) {
-        const double *p = part + (size_t)s * 3u * (size_t)nrows;
-        f[0] += p[k];
-        f[1] += p[nrows + k];
-        f[2] += p[2 * nrows + k];
+    // Bound by the latency of its loads where there are few rows, so those of
+    // kAhead splits are on the way at once and a workgroup has 64 rows (47
+    // splits of N = 3000: 17 us one split after another, 8.0 ahead, 6.2 with 64
+    // rows instead of 256); the additions stay in split order
+    constexpr int kAhead = 8;
+    for (int s0 = 0; s0 < splits; s0 += kAhead) {
+        double v[kAhead][3];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const double *p = part + (size_t)min(s0 + u, splits - 1) * 3u * (size_t)nrows + k;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) v[u][c] = p[(size_t)c * (size_t)nrows];
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) f[c] = s0 + u < splits ? f[c] + v[u][c] : f[c];
     }
     add_external(f, jrec[id_min + r], radial, ext_mode, ext_coeff, Rsim, radial_size);
     F[3 * r + 0] = f[0];
@@ -1613,7 +1625,7 @@ hipError_t launch_forces_finish(const EvalPlan &p, const DeviceParticles &dp, do
     const int splits = (p.N > 0) ? p.splits : 0;
     const uint32_t *perm =
         (sorted_rows(p) && has_pairs(p)) ? spatial_order_perm(scratch_view(p, partials).order, p.N) : nullptr;
-    hipLaunchKernelGGL(reduce_kernel, dim3((unsigned)((p.nrows + 255) / 256)), dim3(256), 0, st, partials,
+    hipLaunchKernelGGL(reduce_kernel, dim3((unsigned)((p.nrows + 63) / 64)), dim3(64), 0, st, partials,
                        dp.jrec, perm, p.radial, F, p.nrows, p.id_min, splits, p.ext_mode, p.ext_coeff, p.Rsim,
                        p.radial_size);
     return hipGetLastError();
