@@ -229,7 +229,8 @@ int steps_radial_bh_table_finish(int32_t size, double *sum, const int32_t *count
  * submission order per simulation), each simulation's force/step sequence is
  * replayed from a captured hipGraph, and the pair kernels of ready requests
  * of small simulations (N <= pack_max_n, same variant and precision) are
- * packed into one launch.  Results do not depend on the mix. */
+ * packed into one launch of each kernel that several of them take.  Results do
+ * not depend on the mix. */
 typedef struct steps_server steps_server;
 
 typedef struct steps_server_config {

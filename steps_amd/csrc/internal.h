@@ -140,6 +140,11 @@ bool sym_selected(const EvalPlan &p);
 bool masses_equal(const double *M, int64_t n);
 hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t stream);
 hipError_t launch_sym_finish(const EvalPlan &p, const SymBuffers &b, double *F, hipStream_t stream);
+// Packed launches of pair-symmetric evaluations (pack_kind and its fellows below).
+const void *sym_pack_kind(const EvalPlan &p);
+size_t sym_desc_bytes();
+int64_t sym_describe(const EvalPlan &p, const SymBuffers &b, void *host_descs, int idx, int64_t blk_begin);
+hipError_t launch_sym_packed(const EvalPlan &p, const void *dev_descs, int nseg, int64_t blocks, hipStream_t stream);
 
 // Scratch of one evaluation: partial sums [splits][3][nrows] (FP64), followed
 // (256-byte aligned) by the source-tile table and, for STEPS_PREC_MIXED, the
@@ -167,16 +172,20 @@ hipError_t launch_forces_finish(const EvalPlan &p, const DeviceParticles &dp, do
                                 hipStream_t stream);
 
 // Packed launches: the pair kernels of up to kMaxPack evaluations of one
-// (variant, precision) in one grid.  pack_describe writes the descriptor of
-// evaluation idx (host memory, pack_desc_bytes() each) whose workgroups start
-// at blk_begin and returns its workgroup count; launch_pair_packed runs the
-// descriptors after they have been copied to device memory.  Each evaluation
-// runs exactly the kernel body, plan and reduction order it runs alone.
+// (variant, precision) and one pack_kind in one grid.  pack_kind is null for an
+// evaluation that has to go alone (a pair-symmetric one of several launches).
+// pack_describe writes the descriptor of the group's evaluation idx (host
+// memory, pack_desc_bytes() each at most) whose workgroups start at blk_begin
+// and returns its workgroup count; launch_pair_packed runs the group's
+// descriptors after they have been copied to device memory, p being any plan of
+// the group.  Each evaluation runs exactly the kernel body, plan and reduction
+// order it runs alone.
 constexpr int kMaxPack = 16;
 size_t pack_desc_bytes();
+const void *pack_kind(const EvalPlan &p);
 int64_t pack_describe(const EvalPlan &p, const DeviceParticles &dp, double *partials, void *host_descs, int idx,
                       int64_t blk_begin);
-hipError_t launch_pair_packed(int variant, int precision, const void *dev_descs, int nseg, int64_t total_blocks,
+hipError_t launch_pair_packed(const EvalPlan &p, const void *dev_descs, int nseg, int64_t total_blocks,
                               hipStream_t stream);
 
 // Spatial ordering of n particles into sorted copies jrec_s / soft_s: Morton

@@ -1650,24 +1650,31 @@ hipError_t launch_forces(const EvalPlan &p, const DeviceParticles &dp, double *p
     return hipSuccess;
 }
 
-size_t pack_desc_bytes() { return sizeof(PackSeg); }
+size_t pack_desc_bytes() { return (std::max(sizeof(PackSeg), sym_desc_bytes()) + 15) & ~(size_t)15; }
+
+const void *pack_kind(const EvalPlan &p) {
+    static const char one_sided = 0;  // the group's variant and precision say which kernel
+    if (!has_pairs(p)) return nullptr;
+    return sym_selected(p) ? sym_pack_kind(p) : &one_sided;
+}
 
 int64_t pack_describe(const EvalPlan &p, const DeviceParticles &dp, double *partials, void *host_descs, int idx,
                       int64_t blk_begin) {
+    if (sym_selected(p)) return sym_describe(p, sym_buffers(p, dp, partials), host_descs, idx, blk_begin);
     PackSeg g;
     g.a = make_args(p, dp, scratch_view(p, partials));
     g.nbx = std::max(1u, row_blocks(p));
     g.blk_begin = (int)blk_begin;
     ((PackSeg *)host_descs)[idx] = g;
-    // a pair-symmetric evaluation is launched by itself (its segment owns no workgroup)
-    return (has_pairs(p) && !sym_selected(p)) ? (int64_t)g.nbx * p.splits : 0;
+    return (int64_t)g.nbx * p.splits;
 }
 
-hipError_t launch_pair_packed(int variant, int precision, const void *dev_descs, int nseg, int64_t total_blocks,
+hipError_t launch_pair_packed(const EvalPlan &p, const void *dev_descs, int nseg, int64_t total_blocks,
                               hipStream_t st) {
     if (nseg <= 0 || total_blocks <= 0) return hipSuccess;
     if (nseg > kMaxPack || total_blocks > INT32_MAX) return hipErrorInvalidValue;
-    return launch_pair(variant, precision, nullptr, (const PackSeg *)dev_descs, nseg, (unsigned)total_blocks, 1,
+    if (sym_selected(p)) return launch_sym_packed(p, dev_descs, nseg, total_blocks, st);
+    return launch_pair(p.variant, p.precision, nullptr, (const PackSeg *)dev_descs, nseg, (unsigned)total_blocks, 1,
                        st);
 }
 

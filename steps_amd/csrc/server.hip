@@ -16,9 +16,9 @@
 //     precision in a hipGraph and replayed (one launch per request); the
 //     per-step scalars travel through a pinned block the graph copies in;
 //   * ready requests of small simulations (N <= pack_max_n) with the same
-//     pair variant and precision are packed: their pair kernels run as one
-//     launch (a flat grid over all their row blocks and splits), the cheap
-//     per-simulation kernels around it are launched directly.
+//     pair variant and precision are packed: those that take the same pair
+//     kernel run it as one launch (a flat grid over the workgroups of all), the
+//     cheap per-simulation kernels around it are launched directly.
 // The scheduler takes its decisions under the server mutex and does the
 // device work they imply (allocation, state copies, graph capture, launches)
 // after releasing it, so submit, wait, get_stats and get_state never wait for
@@ -218,6 +218,7 @@ struct steps_server {
         bool admit = false;           // es[0] has to become resident first
         steps_sim *admitted = nullptr;
         int rc = STEPS_OK;            // admission or launch status
+        int packed_launches = 0, packed_requests = 0;  // launches that several members shared, and those members
     };
 
     // Room for e (not resident) within the budget: least-recently-used idle
@@ -385,11 +386,11 @@ struct steps_server {
         return STEPS_OK;
     }
 
-    // One packed launch for the head requests of the group: per simulation
-    // the step's first half and the source preparation, one pair kernel over
-    // all, per simulation the reduction and the step's second half.  No graphs
-    // (the composition changes from launch to launch).
-    int issue_batch(const Action &a) {
+    // The head requests of a group together: per simulation the step's first
+    // half and the source preparation, one pair kernel over all that take the
+    // same one (pack_kind), per simulation the reduction and the step's second
+    // half.  No graphs (the composition changes from launch to launch).
+    int issue_batch(Action &a) {
         const size_t n = a.es.size();
         std::vector<EvalPlan> plans(n);
         for (size_t i = 0; i < n; ++i) {
@@ -408,19 +409,52 @@ struct steps_server {
             steps_sim *s = a.es[i]->res;
             he = launch_forces_prepare(plans[i], s->dp, s->part.as<double>(), qs);
         }
-        int64_t blocks = 0;
-        for (size_t i = 0; i < n && he == hipSuccess; ++i) {
-            steps_sim *s = a.es[i]->res;
-            blocks += pack_describe(plans[i], s->dp, s->part.as<double>(), sl.hseg, (int)i, blocks);
-        }
-        if (he == hipSuccess)
-            he = hipMemcpyAsync(sl.dseg.ptr, sl.hseg, n * pack_desc_bytes(), hipMemcpyHostToDevice, qs);
-        if (he == hipSuccess) he = launch_pair_packed(plans[0].variant, plans[0].precision, sl.dseg.ptr, (int)n, blocks, qs);
-        for (size_t i = 0; i < n && he == hipSuccess; ++i)
-            if (sym_selected(plans[i])) {  // owns no workgroup of the packed launch
-                steps_sim *s = a.es[i]->res;
-                he = launch_forces_pairs(plans[i], s->dp, s->part.as<double>(), qs);
+        // the members of each kernel, in their order; a kernel of one member and
+        // members that go alone are launched directly
+        struct Pack {
+            const void *kind;
+            std::vector<size_t> of;
+        };
+        std::vector<Pack> packs;
+        for (size_t i = 0; i < n; ++i) {
+            const void *kind = pack_kind(plans[i]);
+            Pack *to = nullptr;
+            for (Pack &k : packs)
+                if (kind && k.kind == kind) to = &k;
+            if (!to) {
+                packs.push_back(Pack{kind, {}});
+                to = &packs.back();
             }
+            to->of.push_back(i);
+        }
+        std::vector<int64_t> blocks(packs.size(), 0);
+        size_t used_descs = 0;
+        for (size_t k = 0; k < packs.size(); ++k) {
+            if (packs[k].of.size() < 2) continue;
+            char *descs = (char *)sl.hseg + used_descs * pack_desc_bytes();
+            int idx = 0;
+            for (size_t i : packs[k].of) {
+                steps_sim *s = a.es[i]->res;
+                blocks[k] += pack_describe(plans[i], s->dp, s->part.as<double>(), descs, idx++, blocks[k]);
+            }
+            used_descs += packs[k].of.size();
+        }
+        if (he == hipSuccess && used_descs > 0)
+            he = hipMemcpyAsync(sl.dseg.ptr, sl.hseg, used_descs * pack_desc_bytes(), hipMemcpyHostToDevice, qs);
+        used_descs = 0;
+        for (size_t k = 0; k < packs.size() && he == hipSuccess; ++k) {
+            const std::vector<size_t> &of = packs[k].of;
+            if (of.size() < 2) {
+                steps_sim *s = a.es[of[0]]->res;
+                he = launch_forces_pairs(plans[of[0]], s->dp, s->part.as<double>(), qs);
+                continue;
+            }
+            const char *descs = (const char *)sl.dseg.ptr + used_descs * pack_desc_bytes();
+            he = launch_pair_packed(plans[of[0]], descs, (int)of.size(), blocks[k], qs);
+            used_descs += of.size();
+            a.packed_launches++;
+            a.packed_requests += (int)of.size();
+        }
         for (size_t i = 0; i < n && he == hipSuccess; ++i) {
             steps_sim *s = a.es[i]->res;
             he = launch_forces_finish(plans[i], s->dp, s->part.as<double>(), s->F.as<double>(), qs);
@@ -487,10 +521,8 @@ struct steps_server {
                 }
             }
             if (a.rc == STEPS_OK) {
-                if (a.es.size() >= 2) {
-                    st.packed_launches++;
-                    st.packed_requests += (int64_t)a.es.size();
-                }
+                st.packed_launches += a.packed_launches;
+                st.packed_requests += a.packed_requests;
                 a.slot->batch.clear();
                 for (Request *r : a.rs) a.slot->batch.push_back(r->ticket);
                 a.slot->ticket = a.rs[0]->ticket;

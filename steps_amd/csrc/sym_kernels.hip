@@ -168,14 +168,13 @@ template <int K> struct IntC { static constexpr int value = K; };
 // between masses are 1, or 0 for rows and sources past the end, whose tiles
 // keep the products.
 template <int V, int NI, bool EQ>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_kernel(const SymArgs a) {
+__device__ __forceinline__ void sym_body(const SymArgs &a, const int b, const int by) {
     __shared__ __align__(2048) double2 jbuf[2][2][kTile];  // (x, y) and (z, -1.5 m) of the tile's sources
     __shared__ double gsum[2][kSymWaves][3][kTile];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t N = a.k.N;
     const int ntiles = (int)((N + kTile - 1) / kTile);
-    const int b = blockIdx.x;
-    const int cell_l = blockIdx.y / a.cell_tasks, task = blockIdx.y % a.cell_tasks;
+    const int cell_l = by / a.cell_tasks, task = by % a.cell_tasks;
     const int cell = a.cell0 + cell_l;
     SymWalk w;
     w.r = cell * a.cell_offs * a.tb + task * a.tpt;
@@ -407,15 +406,14 @@ __device__ __forceinline__ double unit_mass(double m) {
 // EQ: sym_kernel's, the masses one value (R3: unit_mass) or 0 and one product
 // at the end.
 template <int V, int NI, bool EQ>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_mixed_kernel(const SymArgs a) {
+__device__ __forceinline__ void sym_mixed_body(const SymArgs &a, const int b, const int by) {
     constexpr int kFlush = 32 / NI, kRowFlush = V == PV_R3 ? 4 * kFlush : kFlush;  // steps of an FP32 sum
     __shared__ __align__(1024) float4 jbuf[2][kTile];
     __shared__ double gsum[2][kSymWaves][3][kTile];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t N = a.k.N;
     const int ntiles = (int)((N + kTile - 1) / kTile);
-    const int b = blockIdx.x;
-    const int cell_l = blockIdx.y / a.cell_tasks, task = blockIdx.y % a.cell_tasks;
+    const int cell_l = by / a.cell_tasks, task = by % a.cell_tasks;
     const int cell = a.cell0 + cell_l;
     SymWalk w;
     w.r = cell * a.cell_offs * a.tb + task * a.tpt;
@@ -803,7 +801,7 @@ template <class T> __device__ __forceinline__ int t3_weights_from(T d, const KSc
 }
 
 template <int G, bool MX, bool ZF>
-__global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) {
+__device__ __forceinline__ void sym_t3_body(const SymArgs &a, const int b, const int by) {
     constexpr int W = kT3Waves, RW = W / G;  // waves; waves of different rows
     constexpr int kSteps = kTile / G;
     constexpr int kRow = MX ? T3Row<ZF>::words32 : T3Row<ZF>::words, kZPairs = T3Row<ZF>::zpairs,
@@ -815,8 +813,7 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t N = a.k.N;
     const int ntiles = (int)((N + kTile - 1) / kTile);
-    const int b = blockIdx.x;
-    const int cell_l = blockIdx.y / a.cell_tasks, task = blockIdx.y % a.cell_tasks;
+    const int cell_l = by / a.cell_tasks, task = by % a.cell_tasks;
     const int cell = a.cell0 + cell_l;
     SymWalk w;
     w.r = cell * a.cell_offs * a.tb + task * a.tpt;
@@ -1281,7 +1278,7 @@ __device__ __forceinline__ void s1r2_window(const node *win, int w0, int nw, uns
 }
 
 template <int V, bool MX>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_s1r2_kernel(const SymArgs a) {
+__device__ __forceinline__ void sym_s1r2_body(const SymArgs &a, const int b, const int by) {
     constexpr int W = kSymWaves;
     constexpr int ORD = V == PV_S1R2_CIC ? 2 : 4;
     constexpr int kNodes = MX ? 2 * kSymS1Win : kSymS1Win;
@@ -1293,8 +1290,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t N = a.k.N;
     const int ntiles = (int)((N + kTile - 1) / kTile);
-    const int b = blockIdx.x;
-    const int cell_l = blockIdx.y / a.cell_tasks, task = blockIdx.y % a.cell_tasks;
+    const int cell_l = by / a.cell_tasks, task = by % a.cell_tasks;
     const int cell = a.cell0 + cell_l;
     SymWalk w;
     w.r = cell * a.cell_offs * a.tb + task * a.tpt;
@@ -1493,6 +1489,69 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     }
 }
 
+// ---------------------------------------------------------------------------
+// kernels: one evaluation per launch (blocks x tasks of the launch's cells), or
+// several evaluations of one kernel packed into one launch (flat grid, each
+// workgroup finds its evaluation among at most kMaxPack).  Packed, small
+// evaluations share the chip: a server wave of 16 T3 nearest 21^3 1.40 ms (2.36 one
+// after another), of 16 S1R2 CIC N = 1536 0.52 (0.85), of 16 T3 Ewald N = 216 1.30
+// (3.5).
+// ---------------------------------------------------------------------------
+struct SymSeg {
+    SymArgs a;
+    int blk_begin;
+};
+
+__device__ __forceinline__ SymArgs sym_segment(const SymSeg *__restrict__ segs, int nseg, int &local) {
+    const int b = blockIdx.x;
+    int s = 0;
+    for (int q = 1; q < nseg; ++q)
+        if (segs[q].blk_begin <= b) s = q;
+    local = b - segs[s].blk_begin;
+    return segs[s].a;
+}
+
+template <int V, int NI, bool EQ>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_kernel(const SymArgs a) {
+    sym_body<V, NI, EQ>(a, blockIdx.x, blockIdx.y);
+}
+template <int V, int NI, bool EQ>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_kernel_packed(const SymSeg *__restrict__ segs, int nseg) {
+    int local;
+    const SymArgs a = sym_segment(segs, nseg, local);
+    sym_body<V, NI, EQ>(a, local % a.blocks, local / a.blocks);
+}
+template <int V, int NI, bool EQ>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_mixed_kernel(const SymArgs a) {
+    sym_mixed_body<V, NI, EQ>(a, blockIdx.x, blockIdx.y);
+}
+template <int V, int NI, bool EQ>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_mixed_kernel_packed(const SymSeg *__restrict__ segs, int nseg) {
+    int local;
+    const SymArgs a = sym_segment(segs, nseg, local);
+    sym_mixed_body<V, NI, EQ>(a, local % a.blocks, local / a.blocks);
+}
+template <int G, bool MX, bool ZF>
+__global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) {
+    sym_t3_body<G, MX, ZF>(a, blockIdx.x, blockIdx.y);
+}
+template <int G, bool MX, bool ZF>
+__global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel_packed(const SymSeg *__restrict__ segs, int nseg) {
+    int local;
+    const SymArgs a = sym_segment(segs, nseg, local);
+    sym_t3_body<G, MX, ZF>(a, local % a.blocks, local / a.blocks);
+}
+template <int V, bool MX>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_s1r2_kernel(const SymArgs a) {
+    sym_s1r2_body<V, MX>(a, blockIdx.x, blockIdx.y);
+}
+template <int V, bool MX>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_s1r2_kernel_packed(const SymSeg *__restrict__ segs, int nseg) {
+    int local;
+    const SymArgs a = sym_segment(segs, nseg, local);
+    sym_s1r2_body<V, MX>(a, local % a.blocks, local / a.blocks);
+}
+
 // The slots of one launch onto the running sums: cell by cell, the row sums
 // of its tasks, then its source sums (with the sign of the other side).  The
 // last launch's reduction adds the external term (reduce_kernel's) and writes
@@ -1630,58 +1689,82 @@ size_t sym_acc_bytes(const EvalPlan &p) {
     return p.sym_launch_cells < p.sym_cells ? 3u * (size_t)p.N * sizeof(double) : 0;
 }
 
-void launch_sym_kernel(const EvalPlan &p, const SymArgs &a, int cells, hipStream_t st) {
-    const dim3 grid((unsigned)a.blocks, (unsigned)(cells * a.cell_tasks));
+struct SymKernel {
+    void (*one)(const SymArgs);
+    void (*packed)(const SymSeg *, int);
+    unsigned threads;
+};
+
+// The kernel of an evaluation.
+SymKernel sym_kernel_of(const EvalPlan &p) {
+    const bool mx = p.precision == STEPS_PREC_MIXED;
     if (p.variant == PV_T3_EWALD) {
-        const dim3 block(64 * kT3Waves);
-        const bool mx = p.precision == STEPS_PREC_MIXED;
-        auto go = [&](auto g) {
+        const bool zf = p.t3_lo > 0 && p.t3_sym.mirror_z;
+        auto of = [&](auto g) {
             constexpr int G = decltype(g)::value;
-            if (p.t3_lo > 0 && p.t3_sym.mirror_z) {
-                if (mx) hipLaunchKernelGGL((sym_t3_kernel<G, true, true>), grid, block, 0, st, a);
-                else hipLaunchKernelGGL((sym_t3_kernel<G, false, true>), grid, block, 0, st, a);
-            } else {
-                if (mx) hipLaunchKernelGGL((sym_t3_kernel<G, true, false>), grid, block, 0, st, a);
-                else hipLaunchKernelGGL((sym_t3_kernel<G, false, false>), grid, block, 0, st, a);
-            }
+            constexpr unsigned T = 64 * kT3Waves;
+            if (mx) return zf ? SymKernel{sym_t3_kernel<G, true, true>, sym_t3_kernel_packed<G, true, true>, T}
+                              : SymKernel{sym_t3_kernel<G, true, false>, sym_t3_kernel_packed<G, true, false>, T};
+            return zf ? SymKernel{sym_t3_kernel<G, false, true>, sym_t3_kernel_packed<G, false, true>, T}
+                      : SymKernel{sym_t3_kernel<G, false, false>, sym_t3_kernel_packed<G, false, false>, T};
         };
-        if (p.sym_block_rows == 512) go(IntC<1>{});
-        else if (p.sym_block_rows == 256) go(IntC<2>{});
-        else if (p.sym_block_rows == 128) go(IntC<4>{});
-        else go(IntC<8>{});
-        return;
+        switch (p.sym_block_rows) {
+        case 512: return of(IntC<1>{});
+        case 256: return of(IntC<2>{});
+        case 128: return of(IntC<4>{});
+        default: return of(IntC<8>{});
+        }
     }
     if (is_s1r2_lookup(p.variant)) {
-        const bool mx = p.precision == STEPS_PREC_MIXED;
-        if (p.variant == PV_S1R2_CIC) {
-            if (mx) hipLaunchKernelGGL((sym_s1r2_kernel<PV_S1R2_CIC, true>), grid, dim3(kBlock), 0, st, a);
-            else hipLaunchKernelGGL((sym_s1r2_kernel<PV_S1R2_CIC, false>), grid, dim3(kBlock), 0, st, a);
-        } else {
-            if (mx) hipLaunchKernelGGL((sym_s1r2_kernel<PV_S1R2_TSC, true>), grid, dim3(kBlock), 0, st, a);
-            else hipLaunchKernelGGL((sym_s1r2_kernel<PV_S1R2_TSC, false>), grid, dim3(kBlock), 0, st, a);
-        }
-        return;
-    }
-    if (p.precision == STEPS_PREC_MIXED) {
-        auto go = [&](auto v) {
+        auto of = [&](auto v) {
             constexpr int V = decltype(v)::value;
-            if (p.equal_mass) hipLaunchKernelGGL((sym_mixed_kernel<V, kSymNI, true>), grid, dim3(kBlock), 0, st, a);
-            else hipLaunchKernelGGL((sym_mixed_kernel<V, kSymNI, false>), grid, dim3(kBlock), 0, st, a);
+            return mx ? SymKernel{sym_s1r2_kernel<V, true>, sym_s1r2_kernel_packed<V, true>, kBlock}
+                      : SymKernel{sym_s1r2_kernel<V, false>, sym_s1r2_kernel_packed<V, false>, kBlock};
         };
-        if (p.variant == PV_R3) go(IntC<PV_R3>{});
-        else go(IntC<PV_T3_NEAREST>{});
-        return;
+        return p.variant == PV_S1R2_CIC ? of(IntC<PV_S1R2_CIC>{}) : of(IntC<PV_S1R2_TSC>{});
     }
-    auto go = [&](auto v) {
+    if (mx) {
+        auto of = [&](auto v) {
+            constexpr int V = decltype(v)::value;
+            return p.equal_mass
+                       ? SymKernel{sym_mixed_kernel<V, kSymNI, true>, sym_mixed_kernel_packed<V, kSymNI, true>, kBlock}
+                       : SymKernel{sym_mixed_kernel<V, kSymNI, false>, sym_mixed_kernel_packed<V, kSymNI, false>, kBlock};
+        };
+        return p.variant == PV_R3 ? of(IntC<PV_R3>{}) : of(IntC<PV_T3_NEAREST>{});
+    }
+    auto of = [&](auto v) {
         constexpr int V = decltype(v)::value;
-        if (p.equal_mass) hipLaunchKernelGGL((sym_kernel<V, kSymNI, true>), grid, dim3(kBlock), 0, st, a);
-        else hipLaunchKernelGGL((sym_kernel<V, kSymNI, false>), grid, dim3(kBlock), 0, st, a);
+        return p.equal_mass ? SymKernel{sym_kernel<V, kSymNI, true>, sym_kernel_packed<V, kSymNI, true>, kBlock}
+                            : SymKernel{sym_kernel<V, kSymNI, false>, sym_kernel_packed<V, kSymNI, false>, kBlock};
     };
     switch (p.variant) {
-    case PV_R3: go(IntC<PV_R3>{}); break;
-    case PV_T3_NEAREST: go(IntC<PV_T3_NEAREST>{}); break;
-    default: go(IntC<PV_S1R2_NEAREST>{}); break;
+    case PV_R3: return of(IntC<PV_R3>{});
+    case PV_T3_NEAREST: return of(IntC<PV_T3_NEAREST>{});
+    default: return of(IntC<PV_S1R2_NEAREST>{});
     }
+}
+
+SymArgs sym_args(const EvalPlan &p, const SymBuffers &b) {
+    const SymShape s = sym_shape(p);
+    SymArgs a{};
+    a.rec = b.rec;
+    a.soft = b.soft;
+    a.tiles = b.tiles;
+    a.ext = b.ext;
+    a.table = b.table;
+    a.keys = b.keys;
+    a.tab32 = b.tab32;
+    a.jrel = b.jrel;
+    a.tab32s = (const float2 *)b.tab32;
+    a.part = b.part;
+    a.k = make_scalars(p);
+    a.blocks = p.sym_blocks;
+    a.half = s.half;
+    a.tb = s.tb;
+    a.tpt = p.sym_task_tiles;
+    a.cell_tasks = s.cell_tasks;
+    a.cell_offs = s.cell_offs;
+    return a;
 }
 
 hipError_t launch_sym_reduce(const EvalPlan &p, const SymBuffers &b, int cell0, int cells, double *F, hipStream_t st) {
@@ -1769,34 +1852,37 @@ bool sym_selected(const EvalPlan &p) {
 }
 
 hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t st) {
-    const SymShape s = sym_shape(p);
-    SymArgs a{};
-    a.rec = b.rec;
-    a.soft = b.soft;
-    a.tiles = b.tiles;
-    a.ext = b.ext;
-    a.table = b.table;
-    a.keys = b.keys;
-    a.tab32 = b.tab32;
-    a.jrel = b.jrel;
-    a.tab32s = (const float2 *)b.tab32;
-    a.part = b.part;
-    a.k = make_scalars(p);
-    a.blocks = p.sym_blocks;
-    a.half = s.half;
-    a.tb = s.tb;
-    a.tpt = p.sym_task_tiles;
-    a.cell_tasks = s.cell_tasks;
-    a.cell_offs = s.cell_offs;
+    const SymKernel k = sym_kernel_of(p);
+    SymArgs a = sym_args(p, b);
     for (int c0 = 0; c0 < p.sym_cells; c0 += p.sym_launch_cells) {
         const int cells = std::min(p.sym_launch_cells, p.sym_cells - c0);
         a.cell0 = c0;
-        launch_sym_kernel(p, a, cells, st);
+        hipLaunchKernelGGL(k.one, dim3((unsigned)a.blocks, (unsigned)(cells * a.cell_tasks)), dim3(k.threads), 0, st, a);
         hipError_t e = hipGetLastError();
         if (e == hipSuccess && c0 + cells < p.sym_cells) e = launch_sym_reduce(p, b, c0, cells, nullptr, st);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+const void *sym_pack_kind(const EvalPlan &p) {
+    return p.sym_launch_cells >= p.sym_cells ? (const void *)sym_kernel_of(p).packed : nullptr;
+}
+
+size_t sym_desc_bytes() { return sizeof(SymSeg); }
+
+int64_t sym_describe(const EvalPlan &p, const SymBuffers &b, void *host_descs, int idx, int64_t blk_begin) {
+    SymSeg g;
+    g.a = sym_args(p, b);
+    g.blk_begin = (int)blk_begin;
+    ((SymSeg *)host_descs)[idx] = g;
+    return (int64_t)p.sym_blocks * p.sym_cells * g.a.cell_tasks;
+}
+
+hipError_t launch_sym_packed(const EvalPlan &p, const void *dev_descs, int nseg, int64_t blocks, hipStream_t st) {
+    const SymKernel k = sym_kernel_of(p);
+    hipLaunchKernelGGL(k.packed, dim3((unsigned)blocks), dim3(k.threads), 0, st, (const SymSeg *)dev_descs, nseg);
+    return hipGetLastError();
 }
 
 hipError_t launch_sym_finish(const EvalPlan &p, const SymBuffers &b, double *F, hipStream_t st) {

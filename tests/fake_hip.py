@@ -15,7 +15,9 @@ fake.fake_set_limit.argtypes = fake.fake_set_capacity.argtypes = [ctypes.c_size_
 sys.path.insert(0, sys.argv[2])
 import numpy as np
 import steps_amd as steps
-MB = 1 << 20
+fake.fake_launches.restype = ctypes.c_long
+def launches(part, blocks=0):
+    return fake.fake_launches(part.encode(), blocks)
 NO_LIMIT = (1 << 64) - 1
 def cloud(N, L=None):
     rng = np.random.default_rng(N)

@@ -1,6 +1,7 @@
 /* A HIP runtime of host memory for tests of the engine's error paths: loaded
  * with RTLD_GLOBAL before libsteps_amd.so, its functions take the place of
- * libamdhip64's.  Kernels do not run.  hipMalloc fails above a limit for
+ * libamdhip64's.  Kernels do not run, but their launches are counted by name.
+ * While `busy` is set no event has happened yet.  hipMalloc fails above a limit for
  * one allocation or a capacity for all, and an
  * error stays the thread's last error until hipGetLastError reads it, past
  * later calls that succeed, as the HIP 7 documentation states. */
@@ -13,10 +14,12 @@ typedef struct { unsigned x, y, z; } dim3_t;
 static _Thread_local int last_error;
 static size_t limit = (size_t)-1, capacity = (size_t)-1, largest, live;
 static int pinned_fails;
+static volatile int busy;
 
 void fake_set_limit(size_t bytes) { limit = bytes; }
 void fake_set_capacity(size_t bytes) { capacity = bytes; }
 void fake_set_pinned_fails(int on) { pinned_fails = on; }
+void fake_set_busy(int on) { busy = on; }
 size_t fake_largest(void) { size_t v = largest; largest = 0; return v; }  /* since the last call */
 size_t fake_live(void) { return live; }
 
@@ -67,17 +70,59 @@ int hipEventCreate(void **e) { *e = (void *)1; return 0; }
 int hipEventCreateWithFlags(void **e, unsigned f) { (void)f; *e = (void *)1; return 0; }
 int hipEventDestroy(void *e) { (void)e; return 0; }
 int hipEventRecord(void *e, void *s) { (void)e; (void)s; return 0; }
-int hipEventQuery(void *e) { (void)e; return 0; }
+int hipEventQuery(void *e) { (void)e; return busy ? 600 : 0; } /* hipErrorNotReady */
 int hipEventSynchronize(void *e) { (void)e; return 0; }
 int hipEventElapsedTime(float *ms, void *a, void *b) { (void)a; (void)b; *ms = 0; return 0; }
-int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t sh, void *st) { (void)g; (void)b; (void)sh; (void)st; return 0; }
+
+/* launches by kernel name */
+#define MAX_KERNELS 4096
+static struct { const void *f; const char *name; long launches, blocks; } kernels[MAX_KERNELS];
+static int nkernels;
+static _Thread_local struct { dim3_t g, b; size_t sh; void *st; } config;
+
+void **__hipRegisterFatBinary(const void *data) { (void)data; return (void **)&nkernels; }
+void __hipUnregisterFatBinary(void **m) { (void)m; }
+void __hipRegisterFunction(void **m, const void *f, char *device_fun, const char *name, unsigned limit_, void *tid,
+                           void *bid, dim3_t *bd, dim3_t *gd, int *ws) {
+    (void)m; (void)device_fun; (void)limit_; (void)tid; (void)bid; (void)bd; (void)gd; (void)ws;
+    if (nkernels == MAX_KERNELS) abort();
+    kernels[nkernels].f = f;
+    kernels[nkernels++].name = name;
+}
+void __hipRegisterVar(void **m, void *var, char *host, char *device, int ext, size_t size, int constant, int global) {
+    (void)m; (void)var; (void)host; (void)device; (void)ext; (void)size; (void)constant; (void)global;
+}
+/* launches (or, blocks != 0, workgroups) of the kernels whose names hold `part`, since the last reset */
+long fake_launches(const char *part, int blocks) {
+    long n = 0;
+    for (int i = 0; i < nkernels; ++i)
+        if (strstr(kernels[i].name, part)) n += blocks ? kernels[i].blocks : kernels[i].launches;
+    return n;
+}
+void fake_reset_launches(void) {
+    for (int i = 0; i < nkernels; ++i) kernels[i].launches = kernels[i].blocks = 0;
+}
+int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t sh, void *st) {
+    config.g = g;
+    config.b = b;
+    config.sh = sh;
+    config.st = st;
+    return 0;
+}
 int __hipPopCallConfiguration(dim3_t *g, dim3_t *b, size_t *sh, void **st) {
-    g->x = g->y = g->z = b->x = b->y = b->z = 1;
-    *sh = 0;
-    *st = NULL;
+    *g = config.g;
+    *b = config.b;
+    *sh = config.sh;
+    *st = config.st;
     return 0;
 }
 int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t sh, void *st) {
-    (void)f; (void)g; (void)b; (void)args; (void)sh; (void)st;
-    return 0;
+    (void)b; (void)args; (void)sh; (void)st;
+    for (int i = 0; i < nkernels; ++i)
+        if (kernels[i].f == f) {
+            kernels[i].launches++;
+            kernels[i].blocks += (long)g.x * g.y * g.z;
+            return 0;
+        }
+    return last_error = 98; /* hipErrorInvalidDeviceFunction */
 }
