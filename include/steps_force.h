@@ -277,7 +277,8 @@ int steps_server_destroy(steps_server *s);
 int steps_server_add_sim(steps_server *s, const steps_force_desc *d, int64_t N, const double *x,
                          const double *v, const double *M, const double *soft, int64_t *sim_id);
 int steps_server_remove_sim(steps_server *s, int64_t sim_id);
-/* Device bytes the simulation takes while resident (state + scratch + tables). */
+/* Device bytes the simulation needs to be resident (state + tables + scratch;
+ * more scratch is used where the whole ensemble fits the budget with it). */
 int64_t steps_server_sim_bytes(steps_server *s, int64_t sim_id);
 /* kind: STEPS_REQ_FORCE (all rows) or STEPS_REQ_STEP (p required); precision
  * per request (enum steps_precision).  A step kicks with the forces of the

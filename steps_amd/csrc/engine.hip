@@ -45,14 +45,15 @@ int cu_count(int device) {
     return n;
 }
 
-void least_scratch(EvalPlan &p) {
-    p.sym_launch_cells = std::min(p.sym_launch_cells, 1);
-    p.bh_ranges = 1;
+void limit_scratch(EvalPlan &p, Scratch s) {
+    if (s == Scratch::FULL) return;
+    if (p.sym) p.sym_launch_cells = std::min(p.sym_launch_cells, s == Scratch::LEAN ? sym_lean_cells(p) : 1);
+    if (s == Scratch::LEAST) p.bh_ranges = 1;
 }
 
 int reserve_scratch(DevBuf &b, EvalPlan &p) {
     if (b.reserve(scratch_bytes(p), "alloc partials") == STEPS_OK) return STEPS_OK;
-    least_scratch(p);
+    limit_scratch(p, Scratch::LEAST);
     return b.reserve(scratch_bytes(p), "alloc partials");
 }
 
@@ -356,14 +357,15 @@ int check_finite(const double *x, int64_t n) {
 // resident simulation
 // ---------------------------------------------------------------------------
 
-int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool lean, steps_sim **out) {
+int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, Scratch want, steps_sim **out) {
     *out = nullptr;
     if (N <= 0) return fail(STEPS_ERR_ARG, "N must be positive");
     EvalPlan p;
     int rc = make_plan(d, N, 0, N - 1, p);
     if (rc) return rc;
+    limit_scratch(p, want);
     size_t scratch = scratch_bytes(p);
-    least_scratch(p);
+    limit_scratch(p, Scratch::LEAST);
     size_t least = scratch_bytes(p);
     if (both_precisions && desc_mixed_capable(d)) {
         // the scratch serves either precision (neither plan's need bounds the other's)
@@ -371,8 +373,9 @@ int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool 
         dd.precision = (d.precision == STEPS_PREC_MIXED) ? STEPS_PREC_FP64 : STEPS_PREC_MIXED;
         EvalPlan q;
         if ((rc = make_plan(dd, N, 0, N - 1, q))) return rc;
+        limit_scratch(q, want);
         scratch = std::max(scratch, scratch_bytes(q));
-        least_scratch(q);
+        limit_scratch(q, Scratch::LEAST);
         least = std::max(least, scratch_bytes(q));
     }
     if ((rc = set_device(d.device))) return rc;
@@ -419,7 +422,7 @@ int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool 
         (rc = s->radial_bh.sync(d.radial_bh_table, (size_t)d.radial_bh_table_size, s->stream, "radial octree table")))
         return cleanup(rc);
     // last: what does not fit beside the rest is done with the least
-    if ((lean || s->part.reserve(scratch, "alloc partials")) && (rc = s->part.reserve(least, "alloc partials")))
+    if (s->part.reserve(scratch, "alloc partials") && (rc = s->part.reserve(least, "alloc partials")))
         return cleanup(rc);
     // the sim owns device copies: host table pointers are not kept
     s->desc.t3_table = nullptr;
@@ -468,7 +471,7 @@ int sim_plan(steps_sim *s, int64_t id_min, int64_t id_max, int precision, EvalPl
     p.sym = false;
     while (!p.bh && p.splits > 1 && scratch_bytes(p) > s->part.cap) set_splits(p, p.splits - 1);
     p.sym = sym;
-    if (p.bh && scratch_bytes(p) > s->part.cap) least_scratch(p);
+    if (p.bh && scratch_bytes(p) > s->part.cap) limit_scratch(p, Scratch::LEAST);
     if (!sym_fit(p, s->part.cap) || scratch_bytes(p) > s->part.cap) return fail(STEPS_ERR_STATE, "scratch too small for this precision");
     p.t3 = s->t3.ptr();
     p.t3_lo = s->t3.lo;
@@ -693,7 +696,7 @@ int steps_force_eval(const steps_force_desc *d, int64_t N, const double *x, cons
 
 int steps_sim_create(const steps_force_desc *d, int64_t N, steps_sim **out) {
     if (!d || !out) return fail(STEPS_ERR_ARG, "null argument");
-    return sim_create(*d, N, true, false, out);
+    return sim_create(*d, N, true, Scratch::FULL, out);
 }
 
 int steps_sim_destroy(steps_sim *s) {

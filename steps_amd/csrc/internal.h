@@ -137,6 +137,7 @@ void sym_plan(EvalPlan &p);
 bool sym_fit(EvalPlan &p, size_t bytes);
 size_t sym_bytes(const EvalPlan &p);  // of the partial sums; 0 without sym
 bool sym_selected(const EvalPlan &p);
+int sym_lean_cells(const EvalPlan &p);
 bool masses_equal(const double *M, int64_t n);
 hipError_t launch_sym_pairs(const EvalPlan &p, const SymBuffers &b, hipStream_t stream);
 hipError_t launch_sym_finish(const EvalPlan &p, const SymBuffers &b, double *F, hipStream_t stream);
@@ -220,7 +221,11 @@ hipError_t launch_sort_words(const uint32_t *const *words, int nwords, int64_t n
 int64_t bh_item_capacity(int64_t n);
 size_t bh_scratch_bytes(int64_t n);
 int bh_split(int topology, int64_t n);
-void least_scratch(EvalPlan &p);  // the choices that take the least scratch
+// How much scratch a resident simulation holds (scratch_bytes of its plan after
+// limit_scratch): all it can use; what keeps the launches of a pair-symmetric
+// evaluation filling the chip; or the least it can do with.
+enum class Scratch { FULL, LEAN, LEAST };
+void limit_scratch(EvalPlan &p, Scratch s);
 size_t bh_part_bytes(int64_t n, int ranges);  // the ranges' sums, after it; 0 for one range
 hipError_t launch_bh_forces(const EvalPlan &p, const DeviceParticles &dp, void *scratch, double *F,
                             hipStream_t stream, hipEvent_t ev_tree_end);

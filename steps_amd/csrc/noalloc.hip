@@ -129,7 +129,7 @@ extern "C" int steps_force_eval_noalloc(const steps_force_desc *d, int64_t N, co
     };
     size_t need = total();
     if (need > kNoAllocScratchBytes && p.bh) {
-        least_scratch(p);
+        limit_scratch(p, Scratch::LEAST);
         pieces[6] = scratch_bytes(p);
         need = total();
     }

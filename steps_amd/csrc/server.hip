@@ -7,7 +7,9 @@
 //   * admission: a simulation becomes resident (state + scratch in HBM) when
 //     it has work and fits the memory budget; idle resident simulations are
 //     evicted least-recently-used to host memory to make room, and re-admitted
-//     with their state (x, v, F) when they get work again;
+//     with their state (x, v, F) when they get work again.  A simulation holds
+//     all the scratch it can use where the rest of the ensemble still fits
+//     beside it, else what keeps its launches filling the chip;
 //   * up to `streams` requests are on the device at once, each on its own
 //     stream, at most one per simulation (a simulation's requests run in
 //     submission order); requests that arrive while others run are issued as
@@ -59,8 +61,10 @@ struct SimEntry {
     std::vector<double> x, v, M, soft, F;   // host copy, authoritative while not resident
     std::vector<double> t3, s1r2, radial;   // host tables, needed to (re)admit
     steps_sim *res = nullptr;
-    size_t bytes = 0;
-    bool lean = false;            // resident with the least scratch (it would not fit the budget otherwise)
+    size_t bytes[3] = {0, 0, 0};  // device bytes while resident, by the scratch it holds
+    Scratch least = Scratch::LEAN;    // the least it is resident with (LEAST only where LEAN exceeds the budget)
+    Scratch scratch = Scratch::FULL;  // of this residence, and its bytes (0: not resident)
+    size_t held = 0;
     // busy: its device state is in use (a request in flight, an admission
     // or eviction in progress, a get_state copy); has_F: the host F copy is
     // the forces of the host positions; lost: an eviction failed to copy the
@@ -80,7 +84,7 @@ struct Slot {
 };
 
 // Device bytes a resident simulation takes (what sim_create allocates).
-size_t footprint(const steps_force_desc &d, int64_t N, bool lean) {
+size_t footprint(const steps_force_desc &d, int64_t N, Scratch want) {
     EvalPlan p;
     steps_force_desc dd = d;
     // tables only have to look present for the size computation
@@ -95,7 +99,7 @@ size_t footprint(const steps_force_desc &d, int64_t N, bool lean) {
         if (prec == STEPS_PREC_MIXED && !desc_mixed_capable(d)) continue;
         dd.precision = prec;
         if (make_plan(dd, N, 0, N - 1, p) != STEPS_OK) continue;
-        if (lean) least_scratch(p);
+        limit_scratch(p, want);
         scratch = std::max(scratch, scratch_bytes(p));
     }
     b += scratch;
@@ -221,13 +225,25 @@ struct steps_server {
         int packed_launches = 0, packed_requests = 0;  // launches that several members shared, and those members
     };
 
+    // The scratch a simulation is admitted with: the most that leaves room for
+    // every other one with its least, so that an ensemble that fits the budget
+    // stays resident.
+    Scratch choose_scratch(const SimEntry &e) const {
+        int64_t others = (int64_t)used;
+        for (const SimEntry &o : sims)
+            if (&o != &e && !o.removed && o.held == 0) others += (int64_t)o.bytes[(int)o.least];
+        return others + (int64_t)e.bytes[(int)Scratch::FULL] <= cfg.hbm_budget_bytes ? Scratch::FULL : e.least;
+    }
+
     // Room for e (not resident) within the budget: least-recently-used idle
     // residents are detached as victims (their device state is downloaded and
     // freed with the action).  0: reserved; 1: no room now (victims already
     // detached still go); <0: it can never fit.
     int plan_admission(SimEntry &e, std::vector<Evict> &victims) {
-        if ((int64_t)e.bytes > cfg.hbm_budget_bytes) return fail(STEPS_ERR_ADMISSION, "simulation larger than the budget");
-        while ((int64_t)(used + e.bytes) > cfg.hbm_budget_bytes) {
+        e.scratch = choose_scratch(e);
+        const size_t bytes = e.bytes[(int)e.scratch];
+        if ((int64_t)bytes > cfg.hbm_budget_bytes) return fail(STEPS_ERR_ADMISSION, "simulation larger than the budget");
+        while ((int64_t)(used + bytes) > cfg.hbm_budget_bytes) {
             SimEntry *lru = nullptr;
             for (SimEntry &o : sims) {
                 if (&o == &e || !o.res || o.busy) continue;
@@ -237,9 +253,11 @@ struct steps_server {
             victims.push_back(Evict{lru, lru->res});
             lru->res = nullptr;
             lru->busy = true;
-            used -= lru->bytes;
+            used -= lru->held;
+            lru->held = 0;
         }
-        used += e.bytes;
+        e.held = bytes;
+        used += bytes;
         return 0;
     }
 
@@ -286,7 +304,8 @@ struct steps_server {
             if (e.removed && !e.busy && e.res) {
                 reap.push_back(e.res);
                 e.res = nullptr;
-                used -= e.bytes;
+                used -= e.held;
+                e.held = 0;
                 progressed = true;
             }
         }
@@ -488,7 +507,7 @@ struct steps_server {
             d.s1r2_table = e.s1r2.empty() ? nullptr : e.s1r2.data();
             d.radial_table = e.radial.empty() ? nullptr : e.radial.data();
             steps_sim *s = nullptr;
-            a.rc = sim_create(d, e.N, true, e.lean, &s);
+            a.rc = sim_create(d, e.N, true, e.scratch, &s);
             if (!a.rc) {
                 a.rc = sim_upload(s, e.x.data(), e.v.data(), e.M.data(), e.soft.data(), e.has_F ? e.F.data() : nullptr);
                 if (a.rc) sim_destroy(s);
@@ -517,7 +536,8 @@ struct steps_server {
                     e.res = a.admitted;
                     st.admissions++;
                 } else {
-                    used -= e.bytes;
+                    used -= e.held;
+                    e.held = 0;
                 }
             }
             if (a.rc == STEPS_OK) {
@@ -701,10 +721,9 @@ int steps_server_add_sim(steps_server *S, const steps_force_desc *d, int64_t N, 
     if (p.ext_mode == 3) e.radial.assign(d->radial_table, d->radial_table + d->radial_table_size);
     e.desc.t3_table = e.desc.s1r2_table = e.desc.radial_table = nullptr;
     e.variant = p.variant;
-    e.bytes = footprint(*d, N, false);
-    e.lean = (int64_t)e.bytes > S->cfg.hbm_budget_bytes;
-    if (e.lean) e.bytes = footprint(*d, N, true);
-    if ((int64_t)e.bytes > S->cfg.hbm_budget_bytes)
+    for (Scratch s : {Scratch::FULL, Scratch::LEAN, Scratch::LEAST}) e.bytes[(int)s] = footprint(*d, N, s);
+    if ((int64_t)e.bytes[(int)Scratch::LEAN] > S->cfg.hbm_budget_bytes) e.least = Scratch::LEAST;
+    if ((int64_t)e.bytes[(int)e.least] > S->cfg.hbm_budget_bytes)
         return fail(STEPS_ERR_ADMISSION, "simulation larger than the whole memory budget");
     std::lock_guard<std::mutex> lk(S->mu);
     *sim_id = (int64_t)S->sims.size();
@@ -727,7 +746,8 @@ int64_t steps_server_sim_bytes(steps_server *S, int64_t sim) {
     if (!S) return fail(STEPS_ERR_ARG, "null server");
     std::lock_guard<std::mutex> lk(S->mu);
     if (sim < 0 || sim >= (int64_t)S->sims.size()) return fail(STEPS_ERR_ARG, "unknown simulation");
-    return (int64_t)S->sims[(size_t)sim].bytes;
+    const SimEntry &e = S->sims[(size_t)sim];
+    return (int64_t)e.bytes[(int)e.least];
 }
 
 int steps_server_submit(steps_server *S, int64_t sim, int32_t kind, int32_t precision, const steps_step_params *sp,

@@ -85,9 +85,9 @@ struct steps_sim {
 namespace steps {
 
 // Create/destroy without touching the global error state of other sims.
-// lean: the least scratch its evaluations can do with (one cell of a
-// pair-symmetric evaluation at a time; the same results).
-int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, bool lean, steps_sim **out);
+// want: the scratch to hold (the results are the same with any; the least
+// where it does not fit the device).
+int sim_create(const steps_force_desc &d, int64_t N, bool both_precisions, Scratch want, steps_sim **out);
 void sim_destroy(steps_sim *s);
 // Plan of one evaluation of this sim at the given precision.
 int sim_plan(steps_sim *s, int64_t id_min, int64_t id_max, int precision, EvalPlan &p);

@@ -1833,6 +1833,18 @@ size_t sym_bytes(const EvalPlan &p) {
     return p.sym ? sym_cell_bytes(p) * (size_t)p.sym_launch_cells + sym_acc_bytes(p) : 0;
 }
 
+// Cells a launch with which its workgroups fill the chip once (one a CU for T3
+// Ewald, whose window takes a CU's LDS, else four).  Evaluations (ms) with as
+// many cells as 256 MiB hold / these / one at a time / the one-sided kernel:
+// R3 N = 30000 0.43 / 0.51 / 0.70 / 0.63, 100003 3.9 / 4.5 / 6.1 / 6.2, 300000
+// 32.8 / 35.4 / 57 / 46 (mixed 21.2 / 24.1 / 44 / 28.8); T3 Ewald 32^3 21.3 / 22.9
+// / 22.9 / 91; S1R2 CIC N = 102400 15.6 / 20.9 / 31.9 / 44.9; T3 nearest 64^3 29.2 /
+// 32.0 / 43.7 / 48.3 (mixed 30.2 / 40.5 / 99.6 / 37.2).
+int sym_lean_cells(const EvalPlan &p) {
+    const int fill = p.variant == PV_T3_EWALD ? 256 : 1024, each = p.sym_blocks * sym_shape(p).cell_tasks;
+    return std::max(1, (fill + each - 1) / each);
+}
+
 bool sym_fit(EvalPlan &p, size_t bytes) {
     while (p.sym && scratch_bytes(p) > bytes) {
         if (p.sym_launch_cells == 1) return false;
