@@ -783,9 +783,40 @@ __device__ __forceinline__ double bh_radial_bh(double r, double R, const double 
 //
 // A walk over the items [first, total) alone starts with bh_enter: what the
 // lanes decided at the cubes that hold item `first`, without their
-// interactions (those belong to the walk that has the cube).  So the walks of
-// consecutive ranges have the interactions of one walk, each once.
+// interactions (those belong to the walk that has the cube), by the same
+// displacement, r^2 and test to the bit.  So the walks of consecutive ranges
+// have the interactions of one walk, each once.
 typedef double v8d __attribute__((ext_vector_type(8)));
+
+// Displacement from the row to an item: nearest image on the periodic axes
+// (forces.cc:594-601, 941-942; the image sum moves the row instead).
+template <int MODE>
+__device__ __forceinline__ void bh_displacement(double qx, double qy, double qz, double xi, double yi, double zi,
+                                                double L, double &dx, double &dy, double &dz) {
+    dx = qx - xi;
+    dy = qy - yi;
+    dz = qz - zi;
+    if (MODE == BH_T3_NEAR || MODE == BH_T3_EWALD) {
+        if (fabs(dx) > 0.5 * L) dx -= copysign(L, dx);
+        if (fabs(dy) > 0.5 * L) dy -= copysign(L, dy);
+    }
+    if (MODE >= BH_T3_NEAR && MODE <= BH_S1R2_TABLE)
+        if (fabs(dz) > 0.5 * L) dz -= copysign(L, dz);
+}
+
+// r^2 with its roundings fixed: left to the compiler's contraction, the walk
+// and bh_enter rounded it differently, and a row within an ulp of a cube's
+// limit lost or doubled that cube's force.
+__device__ __forceinline__ double bh_r2(double dx, double dy, double dz) {
+#pragma clang fp contract(off)
+    return fma(dz, dz, fma(dx, dx, dy * dy));
+}
+
+// A cube is taken whole (y = 1 / r, which R3 does without).
+template <int MODE>
+__device__ __forceinline__ bool bh_far(double open2, double side, double r2, double y, double theta) {
+    return MODE == BH_R3 ? open2 < r2 : side * y < theta;
+}
 
 // The walk up to item `first`: returns the item to go on from.
 template <int MODE>
@@ -798,22 +829,11 @@ __device__ __forceinline__ int bh_enter(const BhNode *__restrict__ nodes, int fi
             it = q.next;
             continue;
         }
-        double dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
-        if (MODE == BH_T3_NEAR || MODE == BH_T3_EWALD) {
-            if (fabs(dx) > 0.5 * L) dx -= copysign(L, dx);
-            if (fabs(dy) > 0.5 * L) dy -= copysign(L, dy);
-        }
-        if (MODE >= BH_T3_NEAR && MODE <= BH_S1R2_TABLE)
-            if (fabs(dz) > 0.5 * L) dz -= copysign(L, dz);
-        const double r2 = dx * dx + dy * dy + dz * dz;  // the walks' displacement and tests
-        bool take;
-        if (MODE == BH_R3) {
-            take = q.open2 < r2;
-        } else {
-            double y, dist;
-            bh_rsq(r2, y, dist);
-            take = q.side * y < theta;
-        }
+        double dx, dy, dz, y = 0.0, dist;
+        bh_displacement<MODE>(q.x, q.y, q.z, xi, yi, zi, L, dx, dy, dz);
+        const double r2 = bh_r2(dx, dy, dz);
+        if (MODE != BH_R3) bh_rsq(r2, y, dist);
+        const bool take = bh_far<MODE>(q.open2, q.side, r2, y, theta);
         const bool active = wait <= it;
         if (active && take) wait = q.next;
         it = __builtin_amdgcn_ballot_w64(active && !take) ? it + 1 : q.next;
@@ -842,12 +862,13 @@ __device__ __forceinline__ void bh_walk(const BhNode *__restrict__ nodes, int fi
             v8d rec = *(const v8d *)(nodes + (uint32_t)it);
             asm volatile("" : "+s"(rec));  // one 64-byte scalar load, not its parts at their uses
             const BhNode q = __builtin_bit_cast(BhNode, rec);
-            const double dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
-            const double r2 = dx * dx + dy * dy + dz * dz;
+            double dx, dy, dz;
+            bh_displacement<MODE>(q.x, q.y, q.z, xi, yi, zi, L, dx, dy, dz);
+            const double r2 = bh_r2(dx, dy, dz);
             const uint64_t active = q.pidx == kBhMassless ? 0ull
                                                           : __builtin_amdgcn_ballot_w64(wait <= it) &
                                                                 __builtin_amdgcn_ballot_w64(q.pidx != i);
-            const uint64_t far = __builtin_amdgcn_ballot_w64(q.open2 < r2) | (q.pidx >= 0 ? ~0ull : 0ull);
+            const uint64_t far = __builtin_amdgcn_ballot_w64(bh_far<MODE>(q.open2, q.side, r2, 0.0, theta)) | (q.pidx >= 0 ? ~0ull : 0ull);
             const uint64_t use = active & far;
             if (__builtin_amdgcn_inverse_ballot_w64(use)) {
                 const double beta = q.msoft + hi;
@@ -873,16 +894,11 @@ __device__ __forceinline__ void bh_walk(const BhNode *__restrict__ nodes, int fi
         while (it < total) {
             const BhNode q = nodes[it];
             const bool active = wait <= it && q.pidx != i && q.pidx != kBhMassless;
-            double dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
-            if (MODE == BH_T3_NEAR) {  // forces.cc:594-599
-                if (fabs(dx) > 0.5 * L) dx -= copysign(L, dx);
-                if (fabs(dy) > 0.5 * L) dy -= copysign(L, dy);
-            }
-            if (fabs(dz) > 0.5 * L) dz -= copysign(L, dz);  // forces.cc:600-601, 941-942
-            const double r2 = dx * dx + dy * dy + dz * dz;
-            double y, dist;
+            double dx, dy, dz, y, dist;
+            bh_displacement<MODE>(q.x, q.y, q.z, xi, yi, zi, L, dx, dy, dz);
+            const double r2 = bh_r2(dx, dy, dz);
             bh_rsq(r2, y, dist);
-            const bool take = q.pidx >= 0 || q.side * y < theta;
+            const bool take = q.pidx >= 0 || bh_far<MODE>(q.open2, q.side, r2, y, theta);
             const bool use = active && take;
             const double beta = q.msoft + hi;
             double w = (y * y) * y;
@@ -904,17 +920,11 @@ __device__ __forceinline__ void bh_walk(const BhNode *__restrict__ nodes, int fi
             if (q.pidx == i || q.pidx == kBhMassless) {  // the row's own leaf; a massless item
                 wait = q.next;
             } else {
-                double dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
-                if (MODE == BH_T3_NEAR || MODE == BH_T3_EWALD) {  // forces.cc:594-599
-                    if (fabs(dx) > 0.5 * L) dx -= copysign(L, dx);
-                    if (fabs(dy) > 0.5 * L) dy -= copysign(L, dy);
-                }
-                if (MODE >= BH_T3_NEAR && MODE <= BH_S1R2_TABLE)  // forces.cc:600-601, 941-942
-                    if (fabs(dz) > 0.5 * L) dz -= copysign(L, dz);
-                const double r2 = dx * dx + dy * dy + dz * dz;
-                double y, dist;
+                double dx, dy, dz, y, dist;
+                bh_displacement<MODE>(q.x, q.y, q.z, xi, yi, zi, L, dx, dy, dz);
+                const double r2 = bh_r2(dx, dy, dz);
                 bh_rsq(r2, y, dist);
-                if (q.pidx >= 0 || q.side * y < theta) {
+                if (q.pidx >= 0 || bh_far<MODE>(q.open2, q.side, r2, y, theta)) {
                     wait = q.next;
                     if (MODE != BH_S1R2_IMAGES || fabs(dz) <= cut) {  // forces.cc:915
                         const double beta = q.msoft + hi;
