@@ -1206,6 +1206,13 @@ __device__ __forceinline__ void sym_t3_body(const SymArgs &a, const int b, const
 // ---------------------------------------------------------------------------
 constexpr int kSymS1Win = 2368;  // 16-byte words (37 KB: four workgroups per CU), two FP32 nodes a word
 
+// r^2 of a mixed S1R2 pair, by which the main loop leaves a pair to the FP64
+// redo and the redo takes it: one order of roundings for both.
+__device__ __forceinline__ float s1r2_r2(float dx, float dy, float dz, float &rxy2) {
+    rxy2 = fmaf(dx, dx, dy * dy);
+    return fmaf(dz, dz, rxy2);
+}
+
 __device__ __forceinline__ double fract_of(double v) { return __builtin_amdgcn_fract(v); }
 __device__ __forceinline__ float fract_of(float v) { return __builtin_amdgcn_fractf(v); }
 
@@ -1379,8 +1386,7 @@ __device__ __forceinline__ void sym_s1r2_body(const SymArgs &a, const int b, con
                 const real dx = (real)(pa.x - xi), dy = (real)(pa.y - yi), dz = (real)wrap_half(pb.x - zi, k);
                 real wp, mj, mr, qd, Dz, rxy2;
                 if constexpr (MX) {
-                    rxy2 = fmaf(dx, dx, dy * dy);
-                    const float r2 = fmaf(dz, dz, rxy2);
+                    const float r2 = s1r2_r2(dx, dy, dz, rxy2);
                     const bool nr = r2 < Bf;  // left to the FP64 redo (r2 may be 0 here)
                     near = near || nr;
                     const float y = __builtin_amdgcn_rsqf(r2);
@@ -1437,7 +1443,8 @@ __device__ __forceinline__ void sym_s1r2_body(const SymArgs &a, const int b, con
                 const double2 pa = jbuf[0][id], pb = jbuf[1][id];
                 const double ex = pa.x - xi, ey = pa.y - yi, ez = wrap_half(pb.x - zi, k);
                 const float dx = (float)ex, dy = (float)ey, dz = (float)ez;
-                if (fmaf(dx, dx, fmaf(dy, dy, dz * dz)) < Bf) {
+                float rxy2;
+                if (s1r2_r2(dx, dy, dz, rxy2) < Bf) {
                     const double r2 = fma(ex, ex, fma(ey, ey, ez * ez));
                     const double wp = pair_w_tile(r2, B, hi, a.soft, min((int64_t)tile * kTile + id, N - 1), k);
                     double qd, Dz;
