@@ -176,6 +176,10 @@ void set_splits(EvalPlan &p, int64_t splits) {
 
 }  // namespace
 
+void coarse_splits(EvalPlan &p) {
+    if (!t3_slab_plan(p)) set_splits(p, std::min<int64_t>(p.splits, std::max<int64_t>(1, p.N / 256)));
+}
+
 int make_plan(const steps_force_desc &d, int64_t N, int64_t id_min, int64_t id_max, EvalPlan &p) {
     if (N < 0) return fail(STEPS_ERR_ARG, "N < 0");
     if (N > (int64_t)INT32_MAX * 4) return fail(STEPS_ERR_ARG, "N too large");

@@ -226,6 +226,9 @@ int bh_split(int topology, int64_t n);
 // evaluation filling the chip; or the least it can do with.
 enum class Scratch { FULL, LEAN, LEAST };
 void limit_scratch(EvalPlan &p, Scratch s);
+// Source splits of at least 256 sources: fewer partial sums of a small
+// evaluation (they add in another order then).
+void coarse_splits(EvalPlan &p);
 size_t bh_part_bytes(int64_t n, int ranges);  // the ranges' sums, after it; 0 for one range
 hipError_t launch_bh_forces(const EvalPlan &p, const DeviceParticles &dp, void *scratch, double *F,
                             hipStream_t stream, hipEvent_t ev_tree_end);

@@ -128,18 +128,20 @@ extern "C" int steps_force_eval_noalloc(const steps_force_desc *d, int64_t N, co
         return n;
     };
     size_t need = total();
-    if (need > kNoAllocScratchBytes && p.bh) {
-        limit_scratch(p, Scratch::LEAST);
+    auto over = [&] {
         pieces[6] = scratch_bytes(p);
         need = total();
-    }
-    if (need > kNoAllocScratchBytes && p.sym) {
-        // fewer cells of a pair-symmetric evaluation at a time: the same sums
+        return need > kNoAllocScratchBytes;
+    };
+    if (over() && p.bh) limit_scratch(p, Scratch::LEAST);
+    if (!p.bh && over()) coarse_splits(p);
+    if (over() && p.sym) {
+        // fewer cells of a pair-symmetric evaluation at a time (the same sums),
+        // or the one-sided kernel where not even one fits
         const size_t rest = need - ((pieces[6] + 255) & ~(size_t)255);
-        if (rest < kNoAllocScratchBytes) (void)sym_fit(p, (kNoAllocScratchBytes - rest) & ~(size_t)255);
-        pieces[6] = scratch_bytes(p);
-        need = total();
+        if (rest < kNoAllocScratchBytes && !sym_fit(p, (kNoAllocScratchBytes - rest) & ~(size_t)255)) p.sym = false;
     }
+    (void)over();
     if (need > kNoAllocScratchBytes)
         return fail(STEPS_ERR_ARG, "evaluation needs " + std::to_string(need) + " bytes of device scratch; " +
                                        "steps_force_eval_noalloc has " + std::to_string(kNoAllocScratchBytes));

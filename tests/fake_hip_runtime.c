@@ -74,6 +74,16 @@ int hipEventQuery(void *e) { (void)e; return busy ? 600 : 0; } /* hipErrorNotRea
 int hipEventSynchronize(void *e) { (void)e; return 0; }
 int hipEventElapsedTime(float *ms, void *a, void *b) { (void)a; (void)b; *ms = 0; return 0; }
 
+/* device variables (the engine has one, its static scratch) */
+static size_t var_size;
+static void *var;
+int hipGetSymbolAddress(void **p, const void *symbol) {
+    (void)symbol;
+    if (!var && !(var = malloc(var_size))) return last_error = 2;
+    *p = var;
+    return 0;
+}
+
 /* launches by kernel name */
 #define MAX_KERNELS 4096
 static struct { const void *f; const char *name; long launches, blocks; } kernels[MAX_KERNELS];
@@ -89,8 +99,9 @@ void __hipRegisterFunction(void **m, const void *f, char *device_fun, const char
     kernels[nkernels].f = f;
     kernels[nkernels++].name = name;
 }
-void __hipRegisterVar(void **m, void *var, char *host, char *device, int ext, size_t size, int constant, int global) {
-    (void)m; (void)var; (void)host; (void)device; (void)ext; (void)size; (void)constant; (void)global;
+void __hipRegisterVar(void **m, void *v, char *host, char *device, int ext, size_t size, int constant, int global) {
+    (void)m; (void)v; (void)host; (void)device; (void)ext; (void)constant; (void)global;
+    var_size = size;
 }
 /* launches (or, blocks != 0, workgroups) of the kernels whose names hold `part`, since the last reset */
 long fake_launches(const char *part, int blocks) {
