@@ -48,7 +48,10 @@ int cu_count(int device) {
 void limit_scratch(EvalPlan &p, Scratch s) {
     if (s == Scratch::FULL) return;
     if (p.sym) p.sym_launch_cells = std::min(p.sym_launch_cells, s == Scratch::LEAN ? sym_lean_cells(p) : 1);
-    if (s == Scratch::LEAST) p.bh_ranges = 1;
+    if (s == Scratch::LEAST) {
+        p.bh_ranges = 1;
+        if (!p.bh) coarse_splits(p);
+    }
 }
 
 int reserve_scratch(DevBuf &b, EvalPlan &p) {

@@ -71,3 +71,14 @@ print(code(lambda: serve(1, least // 3)), *serve(1, least - 1), least)
 """)
     rc, resident, evictions, most, admissions, least = [int(v) for v in out[0].split()]
     assert rc != 0 and resident == 1 and most < least
+
+
+def test_small_simulation_in_a_small_budget(tmp_path):
+    """N = 3000 takes 47 source splits where there is room; it needs the 11 of
+    256 sources: 1.25 MB."""
+    out = fake_hip.run(tmp_path, RUN + """
+N = 3000
+print(*serve(1, 1250000), code(lambda: serve(1, 1000000)))
+""")
+    resident, evictions, most, admissions, rc = [int(v) for v in out[0].split()]
+    assert resident == 1 and most <= 1250000 and rc != 0
