@@ -72,6 +72,37 @@ __host__ __device__ inline size_t sym_slot(int64_t n, int cell, int cell_tasks, 
     return ((size_t)cell * (size_t)(cell_tasks + cell_offs) + (size_t)slot) * 3u * (size_t)n;
 }
 
+// A kernel runs one evaluation per launch (blocks x tasks of the launch's
+// cells), or several evaluations packed into one launch (flat grid, each
+// workgroup finds its evaluation among at most kMaxPack).  Packed, small
+// evaluations share the chip: a server wave of 16 T3 nearest 21^3 1.40 ms (2.36 one
+// after another), of 16 S1R2 CIC N = 1536 0.52 (0.85), of 16 T3 Ewald N = 216 1.30
+// (3.5).
+struct SymSeg {
+    SymArgs a;
+    int blk_begin;
+};
+struct SymPack {
+    const SymSeg *segs;
+    int nseg;
+};
+
+__device__ __forceinline__ const SymArgs &sym_this(const SymArgs &in, int &b, unsigned &by) {
+    b = blockIdx.x;
+    by = blockIdx.y;
+    return in;
+}
+__device__ __forceinline__ SymArgs sym_this(const SymPack &in, int &b, unsigned &by) {
+    int s = 0;
+    for (int q = 1; q < in.nseg; ++q)
+        if (in.segs[q].blk_begin <= (int)blockIdx.x) s = q;
+    const SymArgs a = in.segs[s].a;
+    const unsigned local = blockIdx.x - (unsigned)in.segs[s].blk_begin;
+    b = (int)(local % (unsigned)a.blocks);
+    by = local / (unsigned)a.blocks;
+    return a;
+}
+
 __device__ __forceinline__ double from_next_lane(double v) {
     // lane l receives lane (l + 1) mod 64's value
     union { double d; int i[2]; } u;
@@ -167,8 +198,11 @@ template <int K> struct IntC { static constexpr int value = K; };
 // instead of each pair (16 FP64 VALU for 18; T3 nearest 64^3 31.1 -> 29.1 ms); in
 // between masses are 1, or 0 for rows and sources past the end, whose tiles
 // keep the products.
-template <int V, int NI, bool EQ>
-__device__ __forceinline__ void sym_body(const SymArgs &a, const int b, const int by) {
+template <int V, int NI, bool EQ, class In>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_kernel(const In in) {
+    int b;
+    unsigned by;
+    const SymArgs &a = sym_this(in, b, by);
     __shared__ __align__(2048) double2 jbuf[2][2][kTile];  // (x, y) and (z, -1.5 m) of the tile's sources
     __shared__ double gsum[2][kSymWaves][3][kTile];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -405,8 +439,11 @@ __device__ __forceinline__ double unit_mass(double m) {
 
 // EQ: sym_kernel's, the masses one value (R3: unit_mass) or 0 and one product
 // at the end.
-template <int V, int NI, bool EQ>
-__device__ __forceinline__ void sym_mixed_body(const SymArgs &a, const int b, const int by) {
+template <int V, int NI, bool EQ, class In>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_mixed_kernel(const In in) {
+    int b;
+    unsigned by;
+    const SymArgs &a = sym_this(in, b, by);
     constexpr int kFlush = 32 / NI, kRowFlush = V == PV_R3 ? 4 * kFlush : kFlush;  // steps of an FP32 sum
     __shared__ __align__(1024) float4 jbuf[2][kTile];
     __shared__ double gsum[2][kSymWaves][3][kTile];
@@ -800,8 +837,11 @@ template <class T> __device__ __forceinline__ int t3_weights_from(T d, const KSc
     return (int)uf;
 }
 
-template <int G, bool MX, bool ZF>
-__device__ __forceinline__ void sym_t3_body(const SymArgs &a, const int b, const int by) {
+template <int G, bool MX, bool ZF, class In>
+__global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const In in) {
+    int b;
+    unsigned by;
+    const SymArgs &a = sym_this(in, b, by);
     constexpr int W = kT3Waves, RW = W / G;  // waves; waves of different rows
     constexpr int kSteps = kTile / G;
     constexpr int kRow = MX ? T3Row<ZF>::words32 : T3Row<ZF>::words, kZPairs = T3Row<ZF>::zpairs,
@@ -1284,8 +1324,11 @@ __device__ __forceinline__ void s1r2_window(const node *win, int w0, int nw, uns
     q = Dr * inv_rho;
 }
 
-template <int V, bool MX>
-__device__ __forceinline__ void sym_s1r2_body(const SymArgs &a, const int b, const int by) {
+template <int V, bool MX, class In>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_s1r2_kernel(const In in) {
+    int b;
+    unsigned by;
+    const SymArgs &a = sym_this(in, b, by);
     constexpr int W = kSymWaves;
     constexpr int ORD = V == PV_S1R2_CIC ? 2 : 4;
     constexpr int kNodes = MX ? 2 * kSymS1Win : kSymS1Win;
@@ -1496,69 +1539,6 @@ __device__ __forceinline__ void sym_s1r2_body(const SymArgs &a, const int b, con
     }
 }
 
-// ---------------------------------------------------------------------------
-// kernels: one evaluation per launch (blocks x tasks of the launch's cells), or
-// several evaluations of one kernel packed into one launch (flat grid, each
-// workgroup finds its evaluation among at most kMaxPack).  Packed, small
-// evaluations share the chip: a server wave of 16 T3 nearest 21^3 1.40 ms (2.36 one
-// after another), of 16 S1R2 CIC N = 1536 0.52 (0.85), of 16 T3 Ewald N = 216 1.30
-// (3.5).
-// ---------------------------------------------------------------------------
-struct SymSeg {
-    SymArgs a;
-    int blk_begin;
-};
-
-__device__ __forceinline__ SymArgs sym_segment(const SymSeg *__restrict__ segs, int nseg, int &local) {
-    const int b = blockIdx.x;
-    int s = 0;
-    for (int q = 1; q < nseg; ++q)
-        if (segs[q].blk_begin <= b) s = q;
-    local = b - segs[s].blk_begin;
-    return segs[s].a;
-}
-
-template <int V, int NI, bool EQ>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_kernel(const SymArgs a) {
-    sym_body<V, NI, EQ>(a, blockIdx.x, blockIdx.y);
-}
-template <int V, int NI, bool EQ>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_kernel_packed(const SymSeg *__restrict__ segs, int nseg) {
-    int local;
-    const SymArgs a = sym_segment(segs, nseg, local);
-    sym_body<V, NI, EQ>(a, local % a.blocks, local / a.blocks);
-}
-template <int V, int NI, bool EQ>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_mixed_kernel(const SymArgs a) {
-    sym_mixed_body<V, NI, EQ>(a, blockIdx.x, blockIdx.y);
-}
-template <int V, int NI, bool EQ>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_mixed_kernel_packed(const SymSeg *__restrict__ segs, int nseg) {
-    int local;
-    const SymArgs a = sym_segment(segs, nseg, local);
-    sym_mixed_body<V, NI, EQ>(a, local % a.blocks, local / a.blocks);
-}
-template <int G, bool MX, bool ZF>
-__global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const SymArgs a) {
-    sym_t3_body<G, MX, ZF>(a, blockIdx.x, blockIdx.y);
-}
-template <int G, bool MX, bool ZF>
-__global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel_packed(const SymSeg *__restrict__ segs, int nseg) {
-    int local;
-    const SymArgs a = sym_segment(segs, nseg, local);
-    sym_t3_body<G, MX, ZF>(a, local % a.blocks, local / a.blocks);
-}
-template <int V, bool MX>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_s1r2_kernel(const SymArgs a) {
-    sym_s1r2_body<V, MX>(a, blockIdx.x, blockIdx.y);
-}
-template <int V, bool MX>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sym_s1r2_kernel_packed(const SymSeg *__restrict__ segs, int nseg) {
-    int local;
-    const SymArgs a = sym_segment(segs, nseg, local);
-    sym_s1r2_body<V, MX>(a, local % a.blocks, local / a.blocks);
-}
-
 // The slots of one launch onto the running sums: cell by cell, the row sums
 // of its tasks, then its source sums (with the sign of the other side).  The
 // last launch's reduction adds the external term (reduce_kernel's) and writes
@@ -1698,7 +1678,7 @@ size_t sym_acc_bytes(const EvalPlan &p) {
 
 struct SymKernel {
     void (*one)(const SymArgs);
-    void (*packed)(const SymSeg *, int);
+    void (*packed)(const SymPack);
     unsigned threads;
 };
 
@@ -1710,10 +1690,10 @@ SymKernel sym_kernel_of(const EvalPlan &p) {
         auto of = [&](auto g) {
             constexpr int G = decltype(g)::value;
             constexpr unsigned T = 64 * kT3Waves;
-            if (mx) return zf ? SymKernel{sym_t3_kernel<G, true, true>, sym_t3_kernel_packed<G, true, true>, T}
-                              : SymKernel{sym_t3_kernel<G, true, false>, sym_t3_kernel_packed<G, true, false>, T};
-            return zf ? SymKernel{sym_t3_kernel<G, false, true>, sym_t3_kernel_packed<G, false, true>, T}
-                      : SymKernel{sym_t3_kernel<G, false, false>, sym_t3_kernel_packed<G, false, false>, T};
+            if (mx) return zf ? SymKernel{sym_t3_kernel<G, true, true, SymArgs>, sym_t3_kernel<G, true, true, SymPack>, T}
+                              : SymKernel{sym_t3_kernel<G, true, false, SymArgs>, sym_t3_kernel<G, true, false, SymPack>, T};
+            return zf ? SymKernel{sym_t3_kernel<G, false, true, SymArgs>, sym_t3_kernel<G, false, true, SymPack>, T}
+                      : SymKernel{sym_t3_kernel<G, false, false, SymArgs>, sym_t3_kernel<G, false, false, SymPack>, T};
         };
         switch (p.sym_block_rows) {
         case 512: return of(IntC<1>{});
@@ -1725,8 +1705,8 @@ SymKernel sym_kernel_of(const EvalPlan &p) {
     if (is_s1r2_lookup(p.variant)) {
         auto of = [&](auto v) {
             constexpr int V = decltype(v)::value;
-            return mx ? SymKernel{sym_s1r2_kernel<V, true>, sym_s1r2_kernel_packed<V, true>, kBlock}
-                      : SymKernel{sym_s1r2_kernel<V, false>, sym_s1r2_kernel_packed<V, false>, kBlock};
+            return mx ? SymKernel{sym_s1r2_kernel<V, true, SymArgs>, sym_s1r2_kernel<V, true, SymPack>, kBlock}
+                      : SymKernel{sym_s1r2_kernel<V, false, SymArgs>, sym_s1r2_kernel<V, false, SymPack>, kBlock};
         };
         return p.variant == PV_S1R2_CIC ? of(IntC<PV_S1R2_CIC>{}) : of(IntC<PV_S1R2_TSC>{});
     }
@@ -1734,15 +1714,15 @@ SymKernel sym_kernel_of(const EvalPlan &p) {
         auto of = [&](auto v) {
             constexpr int V = decltype(v)::value;
             return p.equal_mass
-                       ? SymKernel{sym_mixed_kernel<V, kSymNI, true>, sym_mixed_kernel_packed<V, kSymNI, true>, kBlock}
-                       : SymKernel{sym_mixed_kernel<V, kSymNI, false>, sym_mixed_kernel_packed<V, kSymNI, false>, kBlock};
+                       ? SymKernel{sym_mixed_kernel<V, kSymNI, true, SymArgs>, sym_mixed_kernel<V, kSymNI, true, SymPack>, kBlock}
+                       : SymKernel{sym_mixed_kernel<V, kSymNI, false, SymArgs>, sym_mixed_kernel<V, kSymNI, false, SymPack>, kBlock};
         };
         return p.variant == PV_R3 ? of(IntC<PV_R3>{}) : of(IntC<PV_T3_NEAREST>{});
     }
     auto of = [&](auto v) {
         constexpr int V = decltype(v)::value;
-        return p.equal_mass ? SymKernel{sym_kernel<V, kSymNI, true>, sym_kernel_packed<V, kSymNI, true>, kBlock}
-                            : SymKernel{sym_kernel<V, kSymNI, false>, sym_kernel_packed<V, kSymNI, false>, kBlock};
+        return p.equal_mass ? SymKernel{sym_kernel<V, kSymNI, true, SymArgs>, sym_kernel<V, kSymNI, true, SymPack>, kBlock}
+                            : SymKernel{sym_kernel<V, kSymNI, false, SymArgs>, sym_kernel<V, kSymNI, false, SymPack>, kBlock};
     };
     switch (p.variant) {
     case PV_R3: return of(IntC<PV_R3>{});
@@ -1900,7 +1880,7 @@ int64_t sym_describe(const EvalPlan &p, const SymBuffers &b, void *host_descs, i
 
 hipError_t launch_sym_packed(const EvalPlan &p, const void *dev_descs, int nseg, int64_t blocks, hipStream_t st) {
     const SymKernel k = sym_kernel_of(p);
-    hipLaunchKernelGGL(k.packed, dim3((unsigned)blocks), dim3(k.threads), 0, st, (const SymSeg *)dev_descs, nseg);
+    hipLaunchKernelGGL(k.packed, dim3((unsigned)blocks), dim3(k.threads), 0, st, SymPack{(const SymSeg *)dev_descs, nseg});
     return hipGetLastError();
 }
 
