@@ -353,13 +353,23 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         else variants(IntC<1>{}, std::false_type{});
         if (__any(close)) {
             // rare: the pairs within the bound, with the exact softening
-            // (every lane goes round, so that the source sums do)
+            // (every lane goes round, so that the source sums do).  Not those
+            // of rows and sources past the end, copies of the last particle
+            // that would all take it (T3 nearest N = 8500: one workgroup held
+            // the kernel for twice its time, 0.18 ms a call, now 0.12); a
+            // periodic row is formed again for the next tile
+            if (V != PV_R3 && (int64_t)(b + 1) * (kSymWaves * 64 * NI) > N) {
+#pragma unroll
+                for (int q = 0; q < NI; ++q)
+                    if (row0 + q * 64 >= N) x[q] = NAN;
+            }
 #pragma unroll 1
             for (int s = 0; s < kTile; ++s) {
                 const int id = (lane + s) & 63;
                 double2 pa, pb;
                 source(buf, (unsigned)id * 16u, pa, pb);
-                const int64_t j = min((int64_t)tile * kTile + id, N - 1);
+                const int64_t jt = (int64_t)tile * kTile + id, j = min(jt, N - 1);
+                const double Bj = jt < N ? B : 0.0;
 #pragma unroll
                 for (int q = 0; q < NI; ++q) {
                     double dx = pa.x - x[q], dy = pa.y - y[q], dz = pb.x - z[q];
@@ -367,7 +377,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                     if (V == PV_T3_NEAREST && wy) dy = wrap_half(dy, a.k);
                     if (V != PV_R3 && wz) dz = wrap_half(dz, a.k);
                     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-                    if (r2 < B) sym_close_pair(r2, dx, dy, dz, m[q], pb.y, a.soft, min(row0 + q * 64, N - 1), j, cm53,
+                    if (r2 < Bj) sym_close_pair(r2, dx, dy, dz, m[q], pb.y, a.soft, min(row0 + q * 64, N - 1), j, cm53,
                                                fx[q], fy[q], fz[q], gx, gy, gz);
                 }
                 gx = from_next_lane(gx);
