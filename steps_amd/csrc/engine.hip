@@ -317,8 +317,14 @@ int make_plan(const steps_force_desc &d, int64_t N, int64_t id_min, int64_t id_m
     // two.  Chunks of 256 and more left the chip idle in small evaluations
     // (N = 1500: 6 row blocks x 5 splits, the pair kernel 57 us, now ~15; one
     // call 133 -> 109 us, N = 4500 170 -> 149, T3 nearest 12^3 132 -> 92).
+    // T3 Ewald past there to N = 4608: N / 256 splits, about one workgroup a CU,
+    // where finer ones start a second, partly empty wave (a table that is
+    // not odd, N = 4200: 3.30 against 3.64 ms, 4500 3.53 / 3.74, but 5000 5.66 /
+    // 4.83 and 8000 10.9 / 9.4).
     const int64_t kMinChunk = N < 4096 ? kTile : 2 * kTile;
-    splits = std::max<int64_t>(1, std::min<int64_t>(splits, (N + kMinChunk - 1) / kMinChunk));
+    int64_t most = (N + kMinChunk - 1) / kMinChunk;
+    if (p.variant == PV_T3_EWALD && N > 4096 && N < 4608) most = N / 256;
+    splits = std::max<int64_t>(1, std::min(splits, most));
     // Source chunks of at most kL2Sources (2.6 MB of records + 0.5 MB of
     // softening lengths, under the 4 MB L2 of an XCD): workgroups resident at
     // the same time work on the same chunk (row blocks vary fastest in the
