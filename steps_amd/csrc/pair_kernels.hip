@@ -1459,27 +1459,31 @@ static bool t3_antisymmetric_xy(const double *T, int ng) {
 T3Symmetry t3_symmetry(const double *T, int ng) {
     T3Symmetry s;
     const size_t n = (size_t)ng, n3 = n * n * n;
-    double tmax = 0.0;
-    for (size_t i = 0; i < n3 * 3u; ++i) tmax = std::max(tmax, std::fabs(T[i]));
+    // eight running maxima: a one-shot call with a new table waits for this
+    double top[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    size_t k = 0;
+    for (; k + 8 <= n3 * 3u; k += 8)
+        for (int l = 0; l < 8; ++l) top[l] = std::max(top[l], std::fabs(T[k + l]));
+    for (; k < n3 * 3u; ++k) top[0] = std::max(top[0], std::fabs(T[k]));
+    const double tmax = *std::max_element(top, top + 8);
     if (!(tmax < INFINITY)) return s;
     const double eps0 = std::ldexp(tmax, -52);
-    auto same = [eps0](double b, double a) {
-        return b == a || (std::fabs(a) <= eps0 && std::fabs(b) <= eps0);
+    auto differ = [eps0](double b, double a) {
+        return !(b == a) & !((std::fabs(a) <= eps0) & (std::fabs(b) <= eps0));
     };
-    s.odd = s.mirror_z = true;
-    for (size_t i = 0; i < n3 && s.odd; ++i) {
-        const double *a = T + 3u * i;
-        if (2 * i < n3) {  // node n3 - 1 - i is node i seen through the centre
-            const double *b = T + 3u * (n3 - 1 - i);
-            s.odd = same(b[0], -a[0]) && same(b[1], -a[1]) && same(b[2], -a[2]);
-        }
-        const size_t iz = i % n;
-        if (2 * iz < n) {
-            const double *b = a + 3u * (n - 1 - 2 * iz);
-            s.mirror_z = s.mirror_z && same(b[0], a[0]) && same(b[1], a[1]) && same(b[2], -a[2]);
-        }
+    bool bad = false;
+    for (size_t i = 0; 2 * i < n3; ++i) {  // node n3 - 1 - i is node i seen through the centre
+        const double *a = T + 3u * i, *b = T + 3u * (n3 - 1 - i);
+        bad |= differ(b[0], -a[0]) | differ(b[1], -a[1]) | differ(b[2], -a[2]);
     }
-    s.mirror_z = s.mirror_z && s.odd;
+    if (bad) return s;
+    s.odd = true;
+    for (const double *row = T; row < T + 3u * n3; row += 3u * n)
+        for (size_t z = 0; 2 * z < n; ++z) {
+            const double *a = row + 3u * z, *b = row + 3u * (n - 1 - z);
+            bad |= differ(b[0], a[0]) | differ(b[1], a[1]) | differ(b[2], -a[2]);
+        }
+    s.mirror_z = !bad;
     return s;
 }
 
