@@ -789,7 +789,9 @@ __device__ __forceinline__ int t3_plane(int ny, int row) { return ny * row + ((8
 
 // Unfolded nodes one axis of the window holds: n0 .. n0 + n - 1 (mod Ng), n0
 // in [0, Ng), for sources in cell columns [smin, smax] and rows in [bmin,
-// bmax] (see t3_win_axis).  n <= Ng + 3 keeps every node at most twice.
+// bmax] (see t3_win_axis).  n = 5 or 6 more than the columns the two span, up
+// to 2 Ng + 4 where each spans the box; nodes then repeat, which the copy and
+// t3_win_rel allow for (a window that wide fits on small grids only).
 __device__ __forceinline__ void t3_win_nodes(int smin, int smax, int bmin, int bmax, int Ng, int &n0, int &n) {
     const int nlo = (smin - bmax) + (Ng - 1) / 2 - 2, nhi = (smax - bmin) + Ng / 2 + 2;
     n = nhi - nlo + 1;
@@ -1242,9 +1244,9 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const In in) {
 // lane, records in input order, and the rho rows of each source tile staged in
 // LDS as in body_f64 (all waves on the same tile).  D_rho is even and D_z odd
 // in dz (s1r2_table_odd), so one interpolation serves both sides.  MX: the
-// displacement is formed and wrapped in FP64 and rounded once -- the lanes of
-// a step hold different sources, so there is no common centre to take FP32
-// offsets from, and no image can be chosen differently than in FP64 -- the
+// displacement is formed and wrapped in FP64 and rounded once (FP32 offsets
+// from the tile's centre, as in sym_mixed_kernel, would carry its extent into
+// the error and could take another image at half a period) -- the
 // rest of a pair is FP32 (FP32 copy of the table), FP32 sums run over eight
 // steps and are added in FP64 (over a tile's 64, three times the error of a
 // row), and pairs within the softening bound are done again in FP64.  A tile
@@ -1252,7 +1254,10 @@ __global__ __launch_bounds__(64 * kT3Waves) void sym_t3_kernel(const In in) {
 // takes the short lookup s1r2_window (CIC 93.5 -> 86 ms at N = 262144, mixed
 // CIC 11.6 -> 10.9 and TSC 17.7 -> 16.6 at N = 102400).  Against the one-sided
 // kernels (resident calls on the cylinder, ms): N = 262144 FP64 CIC 182 -> 86;
-// N = 38220 mixed TSC 8.1 -> 2.9.  Bound by VALU issue and LDS reads together.
+// N = 38220 mixed TSC 8.1 -> 2.9.  Particles in another order than by radius
+// have wide tiles, whose stencils come from the global table: N = 102400
+// shuffled, CIC 118.8 -> 61.4 (mixed 73.8 -> 39.0), TSC 172 -> 88 (213 -> 64).
+// Bound by VALU issue and LDS reads together.
 // ---------------------------------------------------------------------------
 constexpr int kSymS1Win = 2368;  // 16-byte words (37 KB: four workgroups per CU), two FP32 nodes a word
 
