@@ -151,7 +151,7 @@ int TableCopy::sync_s1r2(const double *h, int nrho, int nz, double L_, double Rs
     const size_t count = (size_t)nrho * nz * 2;
     if (!h || nrho < 1 || nz < 1) return STEPS_OK;
     const uint64_t f = fingerprint(h, count);
-    if (h == host && count == n && f == fp && dev.ptr && L_ == L && Rsim_ == Rsim) return STEPS_OK;
+    if (h == host && count == n && nrho == rho_nodes && f == fp && dev.ptr && L_ == L && Rsim_ == Rsim) return STEPS_OK;
     std::vector<double> layout;
     s1r2_device_layout(h, nrho, nz, layout);
     int rc = dev.reserve(layout.size() * sizeof(double), "S1R2 table");
@@ -162,6 +162,7 @@ int TableCopy::sync_s1r2(const double *h, int nrho, int nz, double L_, double Rs
     host = h;
     n = count;
     fp = f;
+    rho_nodes = nrho;
     L = L_;
     Rsim = Rsim_;
     odd = s1r2_table_odd(h, nrho, nz, L_, Rsim_);

@@ -33,7 +33,8 @@ struct TableCopy {
     const double *host = nullptr;
     size_t n = 0;
     uint64_t fp = 0;
-    double L = 0, Rsim = 0;  // S1R2 tables: the box the oddness was checked for
+    int rho_nodes = 0;       // S1R2 tables: the shape they were laid out for (with n),
+    double L = 0, Rsim = 0;  // and the box the oddness was checked for
     DevBuf dev;
     int lo = 0;        // T3 tables: first x/y node of the device layout
     T3Symmetry sym;    // T3 tables
