@@ -433,7 +433,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // FP32 could take the other image), are done again in FP64.
 //
 // Measured against the one-sided kernels (ms): R3 N = 16384 0.235 -> 0.192,
-// 100003 4.0 -> 2.8, 1.5 10^6 576 -> 499 (492 with r^-3 formed before the masses); T3 nearest, one mass, 40^3 2.40 ->
+// 100003 4.0 -> 2.8, 1.5 10^6 580 -> 492; T3 nearest, one mass, 40^3 2.40 ->
 // 2.17 and 64^3 28.4 -> 27.7 against this kernel with the products, 38.3
 // one-sided; below N = 14336 the one-sided kernel is
 // as fast (R3 N = 9000: 0.189 against 0.217).  Bound by VALU issue at ~65
@@ -500,6 +500,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 
         const double4 tc = a.tiles[tile], te = a.ext[tile];
         bool far = true, wx = false, wy = false, wz = false;  // as in sym_kernel
+        // R3: r^-3 of every pair is well inside the FP32 range (r from 1e-12, or
+        // the bound, to 3.5e12), so the masses may come after it
+        bool mid = true;
+        const float reach = 2e12f - (float)fmax(fmax(te.x, te.y), te.z);
         float B = 0.0f;
         if (V != PV_R3) {
 #pragma unroll
@@ -544,9 +548,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             const double gx = wx ? 0.0 : fmax(fabs(p.x - tc.x) - te.x, 0.0);
             const double gy = wy ? 0.0 : fmax(fabs(p.y - tc.y) - te.y, 0.0);
             const double gz = wz ? 0.0 : fmax(fabs(p.z - tc.z) - te.z, 0.0);
-            far = far && fma(gx, gx, fma(gy, gy, gz * gz)) > (double)(bq * bq) * (1.0 + 1e-3);
+            const double d2 = fma(gx, gx, fma(gy, gy, gz * gz));
+            far = far && d2 > (double)(bq * bq) * (1.0 + 1e-3);
+            if (V == PV_R3) mid = mid && fmax(d2, (double)(bq * bq)) > 1e-24 && fmaxf(fmaxf(fabsf(x[q]), fabsf(y[q])), fabsf(z[q])) < reach;
         }
         far = __all(far);
+        if (V == PV_R3) mid = __all(mid);
         if (off > 0) gsum[buf][wave][0][lane] = gsum[buf][wave][1][lane] = gsum[buf][wave][2][lane] = 0.0;
 
         bool close = false;
@@ -557,19 +564,21 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             bnd = bnd || fabsf(h) < k.wrap_epsf;
             return h > 0.0f ? d - copysignf(k.Lf, d) : d;
         };
-        auto end_rows = [&] {
+        auto end_rows = [&](const double scale) {
 #pragma unroll
             for (int q = 0; q < NI; ++q) {
-                fx[q] += (double)ax[q];
-                fy[q] += (double)ay[q];
-                fz[q] += (double)az[q];
+                fx[q] = fma((double)ax[q], scale, fx[q]);
+                fy[q] = fma((double)ay[q], scale, fy[q]);
+                fz[q] = fma((double)az[q], scale, fz[q]);
                 ax[q] = ay[q] = az[q] = 0.0f;
             }
         };
-        auto steps = [&](auto near, auto wm, auto unit) {
+        auto steps = [&](auto near, auto wm, auto unit, auto plain) {
             constexpr int NEAR = decltype(near)::value;
             constexpr int WM = decltype(wm)::value;
             constexpr bool UNIT = decltype(unit)::value;
+            constexpr bool PLAIN = decltype(plain)::value;  // r^-3 by itself, then the masses
+            const double scale = UNIT && PLAIN ? um : 1.0;
             unsigned o = (unsigned)lane * 16u;
             const char *base = (const char *)&jbuf[buf][0];
             float4 nj = *(const float4 *)(base + o);
@@ -595,8 +604,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                         }
                         const float t = yr * yr;
                         float sj, si;
-                        if constexpr (V == PV_R3) {
-                            // the mass before r^-3, which alone leaves the FP32 range at 4e12 length units
+                        if constexpr (!PLAIN) {
+                            // the mass before r^-3, which alone leaves the FP32 range at 4e12 length
+                            // units (one product more a pair: 3.5% at N = 10^6, so only where it has to be)
                             sj = t * (yr * (UNIT ? (float)um : pj.w));
                             si = UNIT ? sj : t * (yr * m[q]);
                         } else {
@@ -620,24 +630,25 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                     // wave's LDS operations are in order
                     const int id = (lane + s0 + kFlush) & 63;
                     __builtin_amdgcn_wave_barrier();
-                    gsum[buf][wave][0][id] += (double)gx;
-                    gsum[buf][wave][1][id] += (double)gy;
-                    gsum[buf][wave][2][id] += (double)gz;
+                    gsum[buf][wave][0][id] = fma((double)gx, scale, gsum[buf][wave][0][id]);
+                    gsum[buf][wave][1][id] = fma((double)gy, scale, gsum[buf][wave][1][id]);
+                    gsum[buf][wave][2][id] = fma((double)gz, scale, gsum[buf][wave][2][id]);
                     __builtin_amdgcn_wave_barrier();
                 }
                 gx = gy = gz = 0.0f;
-                if ((s0 + kFlush) % kRowFlush == 0) end_rows();
+                if ((s0 + kFlush) % kRowFlush == 0) end_rows(scale);
             }
         };
         auto variants = [&](auto near, auto unit) {
             const int wm = (wx ? 1 : 0) | (wy ? 2 : 0) | (wz ? 4 : 0);
-            if (wm == 0) steps(near, IntC<0>{}, unit);
-            else if (V == PV_T3_NEAREST) {
-                if (wm == 1) steps(near, IntC<1>{}, unit);
-                else if (wm == 2) steps(near, IntC<2>{}, unit);
-                else if (wm == 4) steps(near, IntC<4>{}, unit);
-                else steps(near, IntC<7>{}, unit);
-            }
+            if (V == PV_R3) {
+                if (mid) steps(near, IntC<0>{}, unit, std::true_type{});
+                else steps(near, IntC<0>{}, unit, std::false_type{});
+            } else if (wm == 0) steps(near, IntC<0>{}, unit, std::true_type{});
+            else if (wm == 1) steps(near, IntC<1>{}, unit, std::true_type{});
+            else if (wm == 2) steps(near, IntC<2>{}, unit, std::true_type{});
+            else if (wm == 4) steps(near, IntC<4>{}, unit, std::true_type{});
+            else steps(near, IntC<7>{}, unit, std::true_type{});
         };
         if (far) {
             if (whole && (int64_t)(tile + 1) * kTile <= N) variants(IntC<0>{}, std::bool_constant<EQ>{});
